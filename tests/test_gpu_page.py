@@ -177,6 +177,47 @@ def test_store_prefill_drops_tokens_beyond_the_listed_pages():
     assert np.array_equal(to_host_bits(dev.pool), want)
 
 
+@pytest.mark.parametrize("Hq,Hkv,D,dtype,kv_dtype,num_tokens", [
+    (0, 8, 128, BZ_BF16, BZ_BF16, None), (0, 5, 64, BZ_F16, BZ_F16, None), (4, 1, 128, BZ_F16, BZ_F16, None),
+    (0, 40, 128, BZ_F16, BZ_F16, None), (3, 2, 128, BZ_BF16, BZ_E4M3, None), (0, 2, 128, BZ_F16, BZ_F16, 1 << 20),
+    (0, 3, 64, BZ_BF16, BZ_BF16, 0xFFFFFFFF)])
+def test_store_prefill_several_tokens_per_workgroup(Hq, Hkv, D, dtype, kv_dtype, num_tokens):
+    """Calls long enough for a workgroup to take several tokens: requests that begin inside a workgroup's tokens, empty
+    ones, more than 64 of them, a last workgroup with few tokens, a count that is only an upper bound."""
+    rng = np.random.default_rng(70)
+    lens = [0, 1, 2, 0, 0, 7] + list(rng.integers(0, 90, size=150)) + [1, 0]
+    P, theta = 16, 1e4
+    p, fill = _setup(71, lens, max(Hq, Hkv), Hkv, D, P, dtype, BZ_LAYOUT_HND, kv_dtype=kv_dtype)
+    ri = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    n = int(ri[-1])
+    assert n > 4 * 1024
+    k, v = wl.randn_bits(rng, (n, Hkv, D), dtype), wl.randn_bits(rng, (n, Hkv, D), dtype)
+    q = wl.randn_bits(rng, (n, Hq, D), dtype) if Hq else None
+    want_raw, want = p.pool.copy(), p.pool.copy()
+    oracle.store_prefill_kv(p.oracle_kv(want_raw), k, v, dtype, ri, k_scale=p.k_scale, v_scale=p.v_scale)
+    oracle.store_prefill_kv(p.oracle_kv(want), k, v, dtype, ri, rope=True, rope_theta=theta, k_scale=p.k_scale, v_scale=p.v_scale)
+    rid = to_dev(ri.view(np.float32), 3).view(torch.int32)
+    dev = DeviceDecode(p)
+    kd, vd = to_dev(k, dtype), to_dev(v, dtype)
+    K.store_prefill_kv_cache(dev.pt, kd, vd, rid, num_tokens=num_tokens, k_scale=dev.k_scale, v_scale=dev.v_scale)
+    torch.cuda.synchronize()
+    assert np.array_equal(to_host_bits(dev.pool), want_raw) and np.array_equal(to_host_bits(kd), k)
+    qd = to_dev(q, dtype) if Hq else None
+    K.store_prefill_kv_cache(dev.pt, kd, vd, rid, num_tokens=num_tokens, q=qd, num_qo_heads=Hq, rope=True if Hq else 2,
+                             rope_theta=theta, k_scale=dev.k_scale, v_scale=dev.v_scale)
+    torch.cuda.synchronize()
+    checks = [(to_host_bits(dev.pool), want, kv_dtype), (to_host_bits(kd), oracle.rope_ragged(k, dtype, ri, Hkv, D, theta), dtype)]
+    if Hq:
+        checks.append((to_host_bits(qd), oracle.rope_ragged(q, dtype, ri, Hq, D, theta), dtype))
+    for got, ref, dt in checks:
+        g, w = wl.to_f32(got, dt), wl.to_f32(ref, dt)
+        # one step of the storage type on rare elements (the device's sincosf against the host's)
+        step = np.maximum(np.abs(w), 2.0 ** -6) * 2.0 ** {BZ_F16: -9, BZ_BF16: -6, BZ_E4M3: -2}[dt]
+        assert (np.abs(g - w) <= step).all()
+        assert (got != ref).mean() < 2e-3
+    assert np.array_equal(to_host_bits(vd), v)
+
+
 @pytest.mark.parametrize("with_q", [False, True])
 def test_store_prefill_rotates_in_place_also_what_it_cannot_cache(with_q):
     """Tokens beyond the listed pages are not cached, but a store that rotates in place (rope = 2, or the fused
