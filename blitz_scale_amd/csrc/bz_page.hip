@@ -39,8 +39,8 @@ struct PageWriteArgs {
 // asked for first and the chain runs while they travel; the request is found with one load per 64 requests (a lane
 // compares one entry, the wave counts) instead of a binary search; and several tokens share one such chain.  One token
 // per workgroup, a binary search and then the rows: 47.5 us for 12 700 tokens of 8 heads (2.7 TB/s); like this 27.1 us
-// (4.8 TB/s).  With 40 heads (28 231 tokens, 1.45 GB), where the rows of one token fill a workgroup anyway, 254.7 against
-// 249.6 us on one machine (5.8 TB/s).
+// (4.8 TB/s).  With 40 heads (28 231 tokens, 1.45 GB), where the rows of one token fill a workgroup anyway, 267 against
+// 262 us on one machine (5.5 TB/s).
 // Rows held: 5 need 117 registers and leave half the waves (29.6 us with 8 heads), 2 leave too little in flight (298
 // against 265 us with 40).
 constexpr int kPwRows = 3;      // rows a lane holds at a time
@@ -446,16 +446,17 @@ extern "C" int bz_store_prefill_kv(const bz_paged_kv_t* kv, void* k, const void*
     if (kv->batch_size == 0) return 0;
     if (kv->head_dim != 128 && kv->head_dim != 64) return BZ_ERR_UNSUPPORTED;
     if (num_tokens == 0 || kv->num_kv_heads == 0) return 0;
-    // Tokens per workgroup: the number whose rows fill the lanes best over up to five passes of kPwRows rows a lane
-    // (28 231 tokens of 40 heads: 284 us with 80 rows on room for 128, 264 us with 80 on 96, 1.5 % less when the passes
-    // come out full), but no more than leaves four workgroups per compute unit: with fewer the chip idles, and a short call is over after one chain anyway.
+    // Tokens per workgroup: the number whose rows fill the lanes best over up to two passes of kPwRows rows a lane (28 231
+    // tokens of 40 heads, 96 rows a pass: 264 us with one token, 262 with two, 265 with three, 271 with six), but no more
+    // than leaves four workgroups per compute unit: with fewer the chip idles, and a short call is over after one chain
+    // anyway.
     const uint32_t rows = (a.rope && q_inout ? num_qo_heads : 0) + 2 * kv->num_kv_heads; // of one token
     const uint32_t held = kPwRows * (256 / (kv->head_dim / 16));
     const bool counted = num_tokens != BZ_NUM_TOKENS_FROM_INDPTR;
     const uint32_t most = counted ? std::max(1u, std::min<uint32_t>(kPwTokens, num_tokens / 1024)) : kPwTokens;
     uint32_t T = 1;
     float best = 0.f;
-    for (uint32_t t = 1; t <= most && (t == 1 || t * rows <= 5 * held); ++t) {
+    for (uint32_t t = 1; t <= most && (t == 1 || t * rows <= 2 * held); ++t) {
         const float filled = (float)(t * rows) / (float)((t * rows + held - 1) / held * held);
         if (filled > best + 0.01f) { best = filled; T = t; }
     }
