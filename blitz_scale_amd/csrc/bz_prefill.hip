@@ -3,8 +3,8 @@
 // worker.  head_dim 128, f16 or bf16, any number of q heads per kv head; self-attention over each request, or
 // q rows for the last tokens of a request only over K/V rows for all of them (distinct ragged indices).
 //
-// One workgroup of 4 waves takes 128 consecutive q rows of one (request, q head); wave w owns rows
-// 32w..32w+31.  K/V tiles of 32 tokens travel global -> LDS four tiles deep and are shared by the four
+// One workgroup of 4 waves takes 128 consecutive q rows of one (request, q head), wave w rows 32w..32w+31 -- or, with
+// grouped heads, 64 rows of two heads or 32 of four.  K/V tiles of 32 tokens travel global -> LDS four tiles deep and are shared by the four
 // waves.  Both contractions are issued "transposed" on v_mfma_f32_32x32x16:
 //     S^T[kv][q] = K[kv][:] . Q[q][:]      (A = K tile from LDS,      B = Q rows from registers)
 //     O^T[d][q]  = V^T[d][kv] . P^T[kv][q] (A = V tile, transposed LDS read, B = P from registers)
@@ -77,6 +77,13 @@ struct PrefillArgs {
     const float4* rope_table; // ROPE_Q: [32 couples of pairs][rope_pitch positions] x (cos i, sin i, cos i+1, sin i+1), i even
     uint32_t rope_pitch;
     uint32_t num_qo_heads, num_kv_heads;
+    // Grouped-query attention: log2 of the heads whose tiles are worked on in slices of rows (0, 1 or 2: sets of 1, 2 or
+    // 4 q heads of one kv head).  A workgroup that takes 32 rows of four heads instead of 128 rows of one reads the same
+    // K/V tiles for as many rows, but its waves end on the same diagonal tile -- with 128 consecutive rows three of the
+    // four waves wait out the last tiles, 1.5 tiles of a job on average -- and a request that does not fill its last 128
+    // rows leaves at most 31 of each head empty.  61 prompts of 16 .. 400 tokens, 32/8 heads, bf16: 113.7 -> 102.7 us; three
+    // chunks of a few hundred rows on prefixes of 4 000 to 15 000: 384 -> 357 us.  Without groups nothing changes.
+    int head_shift;
     int causal;
     float sm_scale_log2;
 };
@@ -293,19 +300,23 @@ __global__ __launch_bounds__(256, 2) void prefill_kernel(PrefillArgs a, const ch
 #endif
 
     const PrefillItem it = a.items[blockIdx.x];
-    if (it.len <= 0) return;
+    // This workgroup's rows (see PrefillArgs::head_shift): of the 2^head_shift jobs that the list has for one tile of a set
+    // of heads, the s-th takes the s-th last slice of the tile's rows for all heads of the set, a wave per head.
+    const int set_mask = (1 << a.head_shift) - 1, sub = it.head & set_mask, slice = kBM >> a.head_shift;
+    const int q0 = it.q0 + slice * (set_mask - sub);
+    if (q0 >= it.len) return; // (padding entries have no rows at all)
     const int tid = threadIdx.x, lane = tid & 63;
     const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int head = it.head;
+    const int head = it.head - sub + (wv & set_mask);
     const int Hq = (int)a.num_qo_heads, Hkv = (int)a.num_kv_heads;
     const int kvh = head / (Hq / Hkv);
     const int qn = lane & 31, h = lane >> 5;
     // Lq q rows attend to L K/V rows (L >= Lq); q row i of the request sits at position off + i: it sees, when
     // causal, the tokens up to that position, and is rotated by that position.
     const int L = it.kv_len, Lq = it.len, off = L - Lq;
-    const int wave_q_lo = it.q0 + 32 * wv;
+    const int wave_q_lo = q0 + 32 * (wv >> a.head_shift);
     const int q_pos = wave_q_lo + qn;
-    const int kv_limit = a.causal ? min(L, off + it.q0 + kBM) : L; // tokens any row of this workgroup can see
+    const int kv_limit = a.causal ? min(L, off + q0 + slice) : L; // tokens any row of this workgroup can see
     const int n = (kv_limit + kSN - 1) / kSN;                      // tiles of the job
     // tiles this wave computes (causal: up to the diagonal tile of its last row; none for rows past the end of the
     // request); t_diag: the first tile in which one of its rows may have to be masked
@@ -385,8 +396,7 @@ __global__ __launch_bounds__(256, 2) void prefill_kernel(PrefillArgs a, const ch
         }
     }
     int copies = 0; // tile copies issued so far
-    if (L >= kSNK * kSN) {
-        // the common case: the first tiles all exist and are whole (kv_limit >= 128 as well, so n >= 4)
+    if (L >= kSNK * kSN && n >= kSNK) { // the common case: the first tiles all exist and are whole
 #pragma unroll
         for (int i = -kSNK; i < 0; ++i) {
             issue_k_fast(i + kSNK, i + kSNK);
@@ -1075,6 +1085,8 @@ extern "C" int bz_batch_prefill_ragged(bz_prefill_plan_t* plan_, void* q, const 
     a.rope_table = (const float4*)p->rope_table;
     a.rope_pitch = p->max_len;
     a.num_qo_heads = num_qo_heads; a.num_kv_heads = num_kv_heads;
+    const uint32_t group = num_qo_heads / num_kv_heads;
+    a.head_shift = group % 4 == 0 ? 2 : (group % 2 == 0 ? 1 : 0);
     a.causal = causal ? 1 : 0;
     if (!(sm_scale > 0.f)) sm_scale = 1.0f / sqrtf((float)head_dim);
     a.sm_scale_log2 = sm_scale * 1.4426950408889634f;

@@ -221,7 +221,9 @@ int bz_prefill_plan(bz_prefill_plan_t* plan, void* float_buffer, size_t float_bu
  * table of the in-register q rotation (512 per position of the longest request; optional, see
  * bz_batch_prefill_ragged), and the host copy of the list, one record of 8 ints per workgroup in launch order
  * {first q row of the request, q rows of the request (0 = padding entry), first q row of the tile inside the
- * request, q head, first K/V row of the request, K/V rows of the request, 0, 0}.  No GPU call. */
+ * request, q head, first K/V row of the request, K/V rows of the request, 0, 0}.  (With 2 or 4 | q heads per kv head
+ * the workgroups of 2 or 4 neighbouring heads' jobs for a tile divide its rows among them, each taking its slice of
+ * the tile for all of these heads.)  No GPU call. */
 int bz_prefill_plan_workspace(bz_prefill_plan_t* plan, const int32_t* qo_indptr_h, const int32_t* kv_indptr_h,
                               uint32_t batch_size, uint32_t num_qo_heads, uint32_t num_kv_heads, uint32_t head_dim,
                               size_t* float_buffer_bytes, size_t* int_buffer_bytes);

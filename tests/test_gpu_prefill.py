@@ -80,6 +80,21 @@ def test_small_ragged_full_check(kind, causal, Hq, Hkv):
         assert np.abs(got - ref).max() <= 2e-3
 
 
+@pytest.mark.parametrize("kind", [F16, BF16_WIDEN_V], ids=["f16", "bf16-widen-v"])
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("Hq,Hkv", [(4, 2), (6, 2), (12, 2), (8, 1)])
+def test_grouped_heads_share_a_workgroup(kind, causal, Hq, Hkv):
+    """Groups of 2, 3, 6 and 8 heads: a workgroup takes 64 rows of two heads, 128 rows of one, 64 of two, 32 of four;
+    prompts that end on either side of a slice's edge, the last slices of a tile empty."""
+    dtype = kind[0]
+    pf = Prefill(205 + Hq, [1, 31, 32, 33, 63, 64, 65, 95, 97, 127, 128, 129, 161, 190, 257], Hq, Hkv, 128, dtype, kind[1])
+    got = pf.run(causal=causal, rope_mode=BZ_ROPE_Q_ONLY)
+    ref = oracle.batch_prefill_ragged(pf.q_as_fed(1e4), pf.k, pf.v, dtype, pf.indptr, Hq, Hkv, 128, causal=causal, sm_scale=LN2,
+                                      parallel=True)
+    assert not np.isnan(got).any()
+    assert (np.abs(got - ref) <= kind_tol(ref, kind)).all(), np.abs(got - ref).max()
+
+
 @pytest.mark.parametrize("kind", KINDS, ids=KIND_IDS)
 @pytest.mark.parametrize("float_ws_bytes", [1 << 20, 1 << 10])
 def test_rope_inside_the_call(kind, float_ws_bytes):
