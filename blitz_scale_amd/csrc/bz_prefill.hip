@@ -55,6 +55,25 @@ struct PrefillItem { // one workgroup's job, in launch order
     int32_t pad[2];
 };
 
+// Few q rows over many K/V rows (a chunk of a long prompt, one prompt on a GPU by itself) make fewer workgroups than the
+// chip holds, and the longest of them sets the time.  The planner then cuts the K/V range of such jobs into parts that
+// different workgroups attend to, each leaving normalised fp32 rows and their base-2 log-sum-exps in the float
+// workspace, and prefill_combine_kernel joins them (split_prefill_items has the rule).  Three chunks of 269 .. 543 tokens
+// behind 4 700 .. 16 000, 32/8 heads, bf16: 357 -> 252 us and
+// 6.7 us for the joining (0.85 PFLOP/s, what a batch of long prompts reaches); one chunk of 512 behind 8 000: 160 -> 93 us.
+struct PrefillPart { // beside each entry of a cut job list
+    int32_t t_begin, t_end; // tiles of 32 K/V rows, counted from the request's first; t_end INT32_MAX: to the end of what the rows see
+    int32_t partial;        // where the rows go; -1: the job is whole, they go to the output
+    int32_t pad;
+};
+struct PrefillJoin { // one slice of rows whose parts are joined: rows and heads named as in PrefillItem
+    int32_t tok0, len, q0, head;
+    int32_t partial0, count; // its parts' rows: partial0 .. partial0 + count - 1
+    int32_t pad[2];
+};
+constexpr size_t kPartRows = (size_t)kBM * 128;               // floats of one part's rows
+constexpr size_t kPartBytes = (kPartRows + kBM) * sizeof(float); // ... with the log-sum-exps
+
 struct PrefillPlan {
     bool planned = false;
     bool bf16_head_tail = false; // bf16: probabilities as head + tail of bf16 instead of V widened to f16 (bz_prefill_plan_set_bf16_mode)
@@ -65,6 +84,15 @@ struct PrefillPlan {
     // every attention call that rotates q, on its own stream, in front of the attention kernel
     float* rope_table = nullptr; // [32 couples of pairs][max_len] x (cos, sin, cos, sin); nullptr: the float workspace has no room
     std::vector<PrefillItem> h_items; // host copy of the last job list (kept between calls)
+    // The cut list, when there is one.  Its scratch lies in the plan's workspace, so only calls on the stream that the
+    // plan was made on take it -- they run one after the other; a call on another stream takes the list of whole jobs,
+    // which shares nothing.
+    const PrefillItem* cut_items_d = nullptr;
+    const PrefillPart* cut_parts_d = nullptr;
+    const PrefillJoin* joins_d = nullptr;
+    uint32_t num_cut_items = 0, num_joins = 0;
+    float *part_o = nullptr, *part_lse = nullptr;
+    hipStream_t cut_stream = nullptr;
     void* staging = nullptr;
     size_t staging_bytes = 0;
     hipEvent_t upload_done = nullptr;
@@ -74,6 +102,9 @@ struct PrefillPlan {
 struct PrefillArgs {
     void* out;
     const PrefillItem* items;
+    const PrefillPart* parts; // nullptr: every job is whole
+    float* part_o;            // [parts][4 waves][16 groups of four floats][64 lanes]: registers as they are
+    float* part_lse;          // [parts][128 rows]
     const float4* rope_table; // ROPE_Q: [32 couples of pairs][rope_pitch positions] x (cos i, sin i, cos i+1, sin i+1), i even
     uint32_t rope_pitch;
     uint32_t num_qo_heads, num_kv_heads;
@@ -281,7 +312,9 @@ __device__ unsigned long long bz_pf_ph[kPftMaxWg * 2 * 8];
 // quarter of the tile), the probabilities are packed as f16 and the second contraction runs on the f16
 // instruction, one per step.  The widening is exact for |v| in f16's range (2^-24 .. 65504; smaller values round
 // to f16 subnormals or zero, larger ones become infinite), which is why SPLIT_P stays selectable.
-template <bool BF16, bool SPLIT_P, bool ROPE_Q>
+// PARTS: the list has cut jobs in it (PrefillPart).  An instantiation of its own: the range and the place of the parts
+// would cost the other one scalar registers, which it spills then (1 % of a long-prompt batch).
+template <bool BF16, bool SPLIT_P, bool ROPE_Q, bool PARTS>
 __global__ __launch_bounds__(256, 2) void prefill_kernel(PrefillArgs a, const char* __restrict__ q_ptr,
                                                             const char* __restrict__ k_ptr,
                                                             const char* __restrict__ v_ptr) {
@@ -300,6 +333,8 @@ __global__ __launch_bounds__(256, 2) void prefill_kernel(PrefillArgs a, const ch
 #endif
 
     const PrefillItem it = a.items[blockIdx.x];
+    PrefillPart part = {0, INT32_MAX, -1, 0};
+    if constexpr (PARTS) part = a.parts[blockIdx.x];
     // This workgroup's rows (see PrefillArgs::head_shift): of the 2^head_shift jobs that the list has for one tile of a set
     // of heads, the s-th takes the s-th last slice of the tile's rows for all heads of the set, a wave per head.
     const int set_mask = (1 << a.head_shift) - 1, sub = it.head & set_mask, slice = kBM >> a.head_shift;
@@ -313,11 +348,15 @@ __global__ __launch_bounds__(256, 2) void prefill_kernel(PrefillArgs a, const ch
     const int qn = lane & 31, h = lane >> 5;
     // Lq q rows attend to L K/V rows (L >= Lq); q row i of the request sits at position off + i: it sees, when
     // causal, the tokens up to that position, and is rotated by that position.
-    const int L = it.kv_len, Lq = it.len, off = L - Lq;
+    // A part's K/V rows are counted from its first one, which every row of the workgroup sees (the planner cuts nowhere
+    // else): `off` may then be negative, off + q0 is not.
+    const int skip = PARTS ? part.t_begin * kSN : 0;
+    const int L = it.kv_len - skip, Lq = it.len, off = L - Lq;
     const int wave_q_lo = q0 + 32 * (wv >> a.head_shift);
     const int q_pos = wave_q_lo + qn;
     const int kv_limit = a.causal ? min(L, off + q0 + slice) : L; // tokens any row of this workgroup can see
-    const int n = (kv_limit + kSN - 1) / kSN;                      // tiles of the job
+    const int n_all = (kv_limit + kSN - 1) / kSN;
+    const int n = PARTS ? min(n_all, part.t_end - part.t_begin) : n_all; // tiles of the job
     // tiles this wave computes (causal: up to the diagonal tile of its last row; none for rows past the end of the
     // request); t_diag: the first tile in which one of its rows may have to be masked
     const int n_w = wave_q_lo >= Lq ? 0 : (a.causal ? min(n, (off + wave_q_lo + 31) / kSN + 1) : n);
@@ -338,7 +377,7 @@ __global__ __launch_bounds__(256, 2) void prefill_kernel(PrefillArgs a, const ch
         kfast[i] = (uint32_t)(4 * i + r4) * row_stride + kcol[i] - (uint32_t)(i * 1024);
         vfast[i] = (uint32_t)(4 * i + r4) * row_stride + vcol - (uint32_t)(i * 1024);
     }
-    const size_t kv_row0 = ((size_t)it.kv0 * Hkv + kvh) * 256; // byte offset of the request's first K/V row
+    const size_t kv_row0 = ((size_t)(it.kv0 + skip) * Hkv + kvh) * 256; // byte offset of the first K/V row
     const char* const k_wave = k_ptr + kv_row0 + (size_t)(8 * wv) * row_stride;
     const char* const v_wave = v_ptr + kv_row0 + (size_t)(8 * wv) * row_stride;
     const uint32_t m0_wave = lds0 + (uint32_t)(8 * wv * 256);
@@ -390,7 +429,7 @@ __global__ __launch_bounds__(256, 2) void prefill_kernel(PrefillArgs a, const ch
             // d = 16 ks + 8 h + e (ks < 4) pairs with d + 64, which this lane holds at step ks + 4.  The table is
             // laid out couple of pairs by couple of pairs, so the 32 rows of a half-wave read 512 consecutive bytes
             // per load.
-            const float4* tab = a.rope_table + (off + min(q_pos, Lq - 1));
+            const float4* tab = a.rope_table + (skip + off + min(q_pos, Lq - 1));
 #pragma unroll
             for (int e = 0; e < 16; ++e) cs[e] = sp_load16(tab + (size_t)(8 * (e >> 2) + 4 * h + (e & 3)) * a.rope_pitch);
         }
@@ -708,6 +747,20 @@ __global__ __launch_bounds__(256, 2) void prefill_kernel(PrefillArgs a, const ch
     // row r at c ^ (r % 16)), store whole rows
     const float l_row = lane_sum_xor32(l_run);
     const float inv_l = l_row > 0.f ? 1.0f / l_row : 0.f;
+    if (PARTS && part.partial >= 0) { // one part of several: fp32 rows in register order, joined by prefill_combine_kernel
+        if (wave_q_lo < Lq) {
+            float4* po = reinterpret_cast<float4*>(a.part_o + (size_t)part.partial * kPartRows) + wv * (16 * 64) + lane;
+#pragma unroll
+            for (int db = 0; db < 4; ++db)
+#pragma unroll
+                for (int b = 0; b < 4; ++b)
+                    po[(4 * db + b) * 64] = make_float4(acc[db][4 * b] * inv_l, acc[db][4 * b + 1] * inv_l,
+                                                        acc[db][4 * b + 2] * inv_l, acc[db][4 * b + 3] * inv_l);
+            const float lse = l_row > 0.f ? (QSCALED ? m_run : m_run * a.sm_scale_log2) + log2f(l_row) : -INFINITY;
+            if (h == 0) a.part_lse[(size_t)part.partial * kBM + 32 * wv + qn] = lse;
+        }
+        return;
+    }
     unsigned char* o_lds = smem + wv * (32 * 256);
 #pragma unroll
     for (int db = 0; db < 4; ++db)
@@ -751,6 +804,58 @@ __global__ __launch_bounds__(256, 2) void prefill_kernel(PrefillArgs a, const ch
         bz_pf_wg[blockIdx.x * 8 + 7] = ((__builtin_amdgcn_s_memrealtime() - pft[7]) << 40) | (pft[7] & 0xffffffffffull);
     }
 #endif
+}
+
+// ---- joins the parts of cut jobs: o = sum_i o_i 2^(lse_i - M) / sum_i 2^(lse_i - M).  Grid (joined slices, 4 waves of the
+// attention kernel's workgroup); wave `db` of the block takes 32 of the 128 output columns of that wave's 32 rows, the
+// same lane for the same elements, so that every read is 1 KiB of consecutive addresses.  The parts have just been
+// written and mostly come out of the last-level cache; the launch itself is the larger half of its time.
+template <typename T> __device__ __forceinline__ uint32_t pack_pair(float lo, float hi) {
+    return PfMma<std::is_same<T, bf16_t>::value>::pack2(lo, hi);
+}
+template <typename T>
+__global__ __launch_bounds__(256) void prefill_combine_kernel(PrefillArgs a, const PrefillJoin* __restrict__ joins) {
+    const PrefillJoin jn = joins[blockIdx.x];
+    const int wv = blockIdx.y, db = threadIdx.x >> 6, lane = threadIdx.x & 63, qn = lane & 31, h = lane >> 5;
+    const int set_mask = (1 << a.head_shift) - 1, sub = jn.head & set_mask, slice = kBM >> a.head_shift;
+    const int pos = jn.q0 + slice * (set_mask - sub) + 32 * (wv >> a.head_shift) + qn;
+    const int head = jn.head - sub + (wv & set_mask);
+    if (pos - qn >= jn.len) return; // (nothing was left for these rows)
+    const float* lse = a.part_lse + (size_t)jn.partial0 * kBM + 32 * wv + qn;
+    float m = -INFINITY;
+    for (int i = 0; i < jn.count; ++i) m = fmaxf(m, lse[(size_t)i * kBM]);
+    m = fmaxf(m, -1e30f);
+    const float4* po = reinterpret_cast<const float4*>(a.part_o + (size_t)jn.partial0 * kPartRows) + (wv * 16 + 4 * db) * 64 + lane;
+    float o[16], total = 0.f;
+#pragma unroll
+    for (int e = 0; e < 16; ++e) o[e] = 0.f;
+#pragma unroll 2
+    for (int i = 0; i < jn.count; ++i) {
+        const float w = __builtin_amdgcn_exp2f(lse[(size_t)i * kBM] - m);
+        total += w;
+#pragma unroll
+        for (int b = 0; b < 4; ++b) {
+            const float4 x = po[(size_t)i * (kPartRows / 4) + b * 64];
+            o[4 * b] += w * x.x;
+            o[4 * b + 1] += w * x.y;
+            o[4 * b + 2] += w * x.z;
+            o[4 * b + 3] += w * x.w;
+        }
+    }
+    const float inv = total > 0.f ? 1.0f / total : 0.f;
+    // group b of this lane is d = 32 db + 8 b + 4 h .. +3: the half-waves exchange every second group, so that each lane
+    // holds eight elements of two groups and stores 16 bytes
+    uint2 w[4];
+#pragma unroll
+    for (int b = 0; b < 4; ++b) w[b] = make_uint2(pack_pair<T>(o[4 * b] * inv, o[4 * b + 1] * inv), pack_pair<T>(o[4 * b + 2] * inv, o[4 * b + 3] * inv));
+    char* row = (char*)a.out + (((size_t)jn.tok0 + pos) * a.num_qo_heads + head) * 256 + db * 64;
+#pragma unroll
+    for (int b = 0; b < 4; b += 2) {
+        const uint2 give = h ? w[b] : w[b + 1], keep = h ? w[b + 1] : w[b];
+        const uint2 got = make_uint2(__shfl_xor(give.x, 32, 64), __shfl_xor(give.y, 32, 64));
+        const uint4 v = h ? make_uint4(got.x, got.y, keep.x, keep.y) : make_uint4(keep.x, keep.y, got.x, got.y);
+        if (pos < jn.len) *reinterpret_cast<uint4*>(row + (b + h) * 16) = v;
+    }
 }
 
 // ---- in-place RoPE of ragged rows, one token per workgroup (used when the caller asks the attention call itself to
@@ -931,6 +1036,181 @@ static int build_prefill_items(PrefillPlan* p, const int32_t* qo_indptr_h, const
     return 0;
 }
 
+// ---- the cut list (PrefillPart): fewer, longer jobs than the chip has places are cut along their K/V range.
+static int prefill_places_per_xcd() { // two workgroups per compute unit
+    int dev = 0, cus = 256, v = 0;
+    if (hipGetDevice(&dev) == hipSuccess && hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && v > 0)
+        cus = v;
+    return std::max(2 * cus / 8, 1);
+}
+static int prefill_head_shift(uint32_t num_qo_heads, uint32_t num_kv_heads) {
+    const uint32_t group = num_qo_heads / num_kv_heads;
+    return group % 4 == 0 ? 2 : (group % 2 == 0 ? 1 : 0);
+}
+// Time of a list in tiles: a job takes its tiles and about ten more for its prologue and epilogue; jobs that all find a
+// place at once take as long as the longest, more of them as long as their sum over the places and, at the end, half of
+// a job that the others wait for.  (When there is a place free beside every job a tile takes 0.7 of the time.)
+struct PrefillLoad {
+    double jobs = 0, sum = 0, longest = 0;
+    void add(double tiles, double count) { jobs += count; sum += count * (tiles + 10); longest = std::max(longest, tiles + 10); }
+    double time(double places) const {
+        if (jobs <= places / 2) return 0.7 * longest;
+        if (jobs <= places) return std::max(longest, sum / places);
+        return std::max(longest, sum / places + 0.5 * longest);
+    }
+};
+struct PrefillCut {
+    std::vector<PrefillItem> items;
+    std::vector<PrefillPart> parts;
+    std::vector<PrefillJoin> joins;
+    uint32_t partials = 0;
+};
+// One slice of q rows (of all heads of a set) and the cuts of its K/V range.  Parts of one request start at the same
+// tiles for all its slices, so that workgroups of one part share its K/V through their XCD's L2.  Every row of a slice
+// has to see the first K/V row of each of its parts, also when causal (the call says only later whether it is): no part
+// starts behind the position of the slice's first row, and a remainder shorter than a third stays with the part before.
+struct PrefillSlices {
+    int32_t len, kv_len, slice, part_tiles; // part_tiles: tiles of a part
+    int32_t tiles(int32_t q0) const { return (std::min(kv_len, kv_len - len + q0 + slice) + kSN - 1) / kSN; }
+    int32_t count(int32_t q0) const {
+        const int32_t by_row = (kv_len - len + q0) / kSN / part_tiles, rest = tiles(q0) - part_tiles / 3;
+        return 1 + std::min(by_row, std::max(rest, 0) / part_tiles);
+    }
+    void cut_to(int32_t most_tiles) { // into equal parts of at most that many tiles
+        const int32_t all = (kv_len + kSN - 1) / kSN, n = (all + most_tiles - 1) / most_tiles;
+        part_tiles = (all + n - 1) / n;
+    }
+};
+// Returns false, and leaves `cut` alone, where whole jobs are as good or the scratch does not hold the parts.  The rule:
+// with at most four rounds of jobs, parts are tried that come to one, two, three and four rounds, and the cheapest by the
+// estimate above is taken if, with the joining kernel (its launch is worth a dozen tiles, a part's rows going out and
+// coming back a fiftieth of one), it saves a twelfth.
+// Against fixed part lengths on six such shapes (attention with the joining, us; tiles of a part): the three chunks 241 as
+// chosen, best 231 (103), 255 (52), 302 (24), whole 335; one chunk of 512 behind 8 000 with 32/8 heads 93, best 90, whole
+// 160; with 64/8 heads, which make twice the jobs, 158, 166 (73), whole 164.
+static bool split_prefill_items(PrefillCut& cut, const PrefillPlan* p, const int32_t* qo, const int32_t* kv, uint32_t batch_size,
+                                uint32_t num_qo_heads, uint32_t num_kv_heads, size_t scratch_bytes, int places_per_xcd) {
+    const int shift = prefill_head_shift(num_qo_heads, num_kv_heads), set_mask = (1 << shift) - 1;
+    const int32_t slice = kBM >> shift, sets = (int32_t)(num_qo_heads >> shift);
+    const double places = 8.0 * places_per_xcd;
+    std::vector<PrefillSlices> reqs(batch_size);
+    double jobs = 0;
+    int32_t longest = 0;
+    for (uint32_t b = 0; b < batch_size; ++b) {
+        const int32_t len = qo[b + 1] - qo[b], kv_len = kv[b + 1] - kv[b];
+        reqs[b] = {len, kv_len, slice, INT32_MAX / 2};
+        jobs += (double)((len + slice - 1) / slice) * sets;
+        if (len > 0) longest = std::max(longest, (kv_len + kSN - 1) / kSN);
+    }
+    constexpr int32_t kLeast = 12; // tiles of the shortest part worth its prologue
+    if (jobs == 0 || jobs > 4 * places || longest < 2 * kLeast) return false;
+    PrefillLoad whole[8]; // by XCD, as the list of whole jobs deals them
+    for (size_t i = 0; i < p->h_items.size(); ++i) {
+        const PrefillItem& it = p->h_items[i];
+        const int32_t q0 = it.q0 + slice * (set_mask - (it.head & set_mask));
+        if (q0 < it.len) whole[i % 8].add(PrefillSlices{it.len, it.kv_len, slice, 1}.tiles(q0), 1);
+    }
+    double whole_time = 0;
+    for (const PrefillLoad& l : whole) whole_time = std::max(whole_time, l.time(places_per_xcd));
+    auto load_of = [&](int32_t most_tiles, double& partials) {
+        PrefillLoad l;
+        partials = 0;
+        for (PrefillSlices r : reqs) {
+            if (r.len == 0) continue;
+            r.cut_to(most_tiles);
+            for (int32_t q0 = 0; q0 < r.len; q0 += slice) {
+                const int32_t n = r.count(q0);
+                if (n > 1) l.add(r.part_tiles, (double)(n - 1) * sets);
+                l.add(r.tiles(q0) - (n - 1) * r.part_tiles, sets);
+                if (n > 1) partials += (double)n * sets;
+            }
+        }
+        return l;
+    };
+    double best_time = whole_time * 11 / 12;
+    int32_t best = 0;
+    for (int rounds = 1; rounds <= 4; ++rounds) {
+        int32_t lo = kLeast, hi = longest; // the shortest parts that come to so many rounds
+        double partials;
+        while (lo < hi) {
+            const int32_t mid = (lo + hi) / 2;
+            if (load_of(mid, partials).jobs <= rounds * places) hi = mid; else lo = mid + 1;
+        }
+        const double time = load_of(lo, partials).time(places) + 12 + 0.02 * partials;
+        if (partials > 0 && partials * kPartBytes <= (double)scratch_bytes && time < best_time) {
+            best_time = time;
+            best = lo;
+        }
+    }
+    if (!best) return false;
+    // Jobs by (request, kv head, part): such a set shares K/V rows and goes to one XCD, the largest set first and each to
+    // the XCD with the least to do; on an XCD the jobs with most tiles come first.
+    struct Set { uint32_t req, kv_head; int32_t part; double load; };
+    std::vector<Set> order;
+    for (uint32_t b = 0; b < batch_size; ++b) {
+        if (reqs[b].len == 0) continue;
+        reqs[b].cut_to(best);
+        const PrefillSlices& r = reqs[b];
+        for (int32_t m = 0;; ++m) {
+            double load = 0;
+            for (int32_t q0 = 0; q0 < r.len; q0 += slice) {
+                const int32_t n = r.count(q0);
+                if (m < n) load += 10 + (m + 1 < n ? r.part_tiles : r.tiles(q0) - m * r.part_tiles);
+            }
+            if (load == 0) break;
+            for (uint32_t u = 0; u < num_kv_heads; ++u) order.push_back({b, u, m, load});
+        }
+    }
+    std::stable_sort(order.begin(), order.end(), [](const Set& x, const Set& y) { return x.load > y.load; });
+    struct Job { PrefillItem item; PrefillPart part; int32_t tiles; };
+    std::vector<Job> per_xcd[8];
+    double xcd_load[8] = {};
+    // where the parts of a slice leave their rows: the first place by (request, slice, set of heads)
+    std::vector<std::vector<int32_t>> first(batch_size);
+    for (uint32_t b = 0; b < batch_size; ++b) {
+        const PrefillSlices& r = reqs[b];
+        for (int32_t q0 = 0; q0 < r.len; q0 += slice) {
+            const int32_t n = r.count(q0);
+            for (int32_t set = 0; set < sets; ++set) {
+                first[b].push_back(n > 1 ? (int32_t)cut.partials : -1);
+                if (n == 1) continue;
+                cut.joins.push_back({qo[b], r.len, q0 / kBM * kBM, (set << shift) + set_mask - q0 % kBM / slice, (int32_t)cut.partials, n, {0, 0}});
+                cut.partials += (uint32_t)n;
+            }
+        }
+    }
+    const int32_t sets_per_kv = sets / (int32_t)num_kv_heads;
+    for (const Set& st : order) {
+        const int x = (int)(std::min_element(xcd_load, xcd_load + 8) - xcd_load);
+        xcd_load[x] += st.load * sets_per_kv;
+        const PrefillSlices& r = reqs[st.req];
+        for (int32_t q0 = (r.len - 1) / slice * slice; q0 >= 0; q0 -= slice) {
+            const int32_t n = r.count(q0);
+            if (st.part >= n) continue;
+            const bool last = st.part + 1 == n;
+            for (int32_t g = 0; g < sets_per_kv; ++g) {
+                const int32_t set = (int32_t)st.kv_head * sets_per_kv + g, at = first[st.req][(size_t)(q0 / slice) * sets + set];
+                per_xcd[x].push_back({{qo[st.req], r.len, q0 / kBM * kBM, (set << shift) + set_mask - q0 % kBM / slice, kv[st.req], r.kv_len, {0, 0}},
+                                      {st.part * r.part_tiles, last ? INT32_MAX : (st.part + 1) * r.part_tiles, at < 0 ? -1 : at + st.part, 0},
+                                      last ? r.tiles(q0) - st.part * r.part_tiles : r.part_tiles});
+            }
+        }
+    }
+    size_t rows = 0;
+    for (auto& v : per_xcd) {
+        std::stable_sort(v.begin(), v.end(), [](const Job& x, const Job& y) { return x.tiles > y.tiles; });
+        rows = std::max(rows, v.size());
+    }
+    cut.items.assign(rows * 8, PrefillItem{0, 0, 0, 0, 0, 0, {0, 0}});
+    cut.parts.assign(rows * 8, PrefillPart{0, INT32_MAX, -1, 0});
+    for (int x = 0; x < 8; ++x)
+        for (size_t k = 0; k < per_xcd[x].size(); ++k) {
+            cut.items[k * 8 + x] = per_xcd[x][k].item;
+            cut.parts[k * 8 + x] = per_xcd[x][k].part;
+        }
+    return true;
+}
+
 extern "C" int bz_prefill_plan_workspace(bz_prefill_plan_t* plan_, const int32_t* qo_indptr_h, const int32_t* kv_indptr_h,
                                          uint32_t batch_size, uint32_t num_qo_heads, uint32_t num_kv_heads,
                                          uint32_t head_dim, size_t* float_buffer_bytes, size_t* int_buffer_bytes) {
@@ -966,9 +1246,27 @@ extern "C" int bz_prefill_plan(bz_prefill_plan_t* plan_, void* float_buffer, siz
     const int rc0 = build_prefill_items(p, qo_indptr_h, kv_indptr_h, batch_size, num_qo_heads, num_kv_heads, head_dim);
     if (rc0) return rc0;
     const std::vector<PrefillItem>& items = p->h_items;
-    const size_t bytes = pf_align_up(items.size() * sizeof(PrefillItem), 256);
-    if (bytes > int_buffer_bytes) return BZ_ERR_WORKSPACE;
+    const size_t whole_bytes = pf_align_up(items.size() * sizeof(PrefillItem), 256);
+    if (whole_bytes > int_buffer_bytes) return BZ_ERR_WORKSPACE;
     hipStream_t s = (hipStream_t)stream;
+    uint32_t max_len = 0;
+    for (uint32_t b = 0; b < batch_size; ++b) max_len = std::max<uint32_t>(max_len, (uint32_t)(kv_indptr_h[b + 1] - kv_indptr_h[b]));
+    // the float workspace holds the angle table of the q rotation when it has room for it (512 bytes per position), and
+    // behind it the rows of cut jobs
+    const size_t table_bytes = (size_t)max_len * 512;
+    const bool table_fits = float_buffer && table_bytes <= float_buffer_bytes && (uintptr_t)float_buffer % 16 == 0;
+    PrefillCut cut;
+    bool use_cut = false;
+    try {
+        use_cut = table_fits && split_prefill_items(cut, p, qo_indptr_h, kv_indptr_h, batch_size, num_qo_heads, num_kv_heads,
+                                                    float_buffer_bytes - table_bytes, prefill_places_per_xcd());
+    } catch (const std::bad_alloc&) { // no memory on the host for the second list: the first does
+    }
+    const size_t parts_at = whole_bytes + pf_align_up(cut.items.size() * sizeof(PrefillItem), 256);
+    const size_t joins_at = parts_at + pf_align_up(cut.parts.size() * sizeof(PrefillPart), 256);
+    const size_t cut_bytes = joins_at + pf_align_up(cut.joins.size() * sizeof(PrefillJoin), 256);
+    if (cut_bytes > int_buffer_bytes) use_cut = false;
+    const size_t bytes = use_cut ? cut_bytes : whole_bytes;
     if (!p->upload_done) BZ_CHECK_HIP(hipEventCreateWithFlags(&p->upload_done, hipEventDisableTiming));
     else BZ_CHECK_HIP(hipEventSynchronize(p->upload_done));
     if (bytes > p->staging_bytes) {
@@ -982,6 +1280,12 @@ extern "C" int bz_prefill_plan(bz_prefill_plan_t* plan_, void* float_buffer, siz
     if (bytes) {
         memset(p->staging, 0, bytes);
         memcpy(p->staging, items.data(), items.size() * sizeof(PrefillItem));
+        if (use_cut) {
+            char* to = (char*)p->staging;
+            memcpy(to + whole_bytes, cut.items.data(), cut.items.size() * sizeof(PrefillItem));
+            memcpy(to + parts_at, cut.parts.data(), cut.parts.size() * sizeof(PrefillPart));
+            memcpy(to + joins_at, cut.joins.data(), cut.joins.size() * sizeof(PrefillJoin));
+        }
         BZ_CHECK_HIP(hipMemcpyAsync(int_buffer, p->staging, bytes, hipMemcpyHostToDevice, s));
     }
     BZ_CHECK_HIP(hipEventRecord(p->upload_done, s));
@@ -991,20 +1295,26 @@ extern "C" int bz_prefill_plan(bz_prefill_plan_t* plan_, void* float_buffer, siz
     p->head_dim = head_dim;
     p->total_tokens = (uint32_t)qo_indptr_h[batch_size];
     p->total_kv_tokens = (uint32_t)kv_indptr_h[batch_size];
-    p->max_len = 0;
-    for (uint32_t b = 0; b < batch_size; ++b)
-        p->max_len = std::max<uint32_t>(p->max_len, (uint32_t)(kv_indptr_h[b + 1] - kv_indptr_h[b]));
-    // the float workspace holds the angle table of the q rotation when it has room for it (512 bytes per position)
-    p->rope_table = (float_buffer && (size_t)p->max_len * 512 <= float_buffer_bytes && (uintptr_t)float_buffer % 16 == 0)
-                        ? (float*)float_buffer : nullptr;
+    p->max_len = max_len;
+    p->rope_table = table_fits ? (float*)float_buffer : nullptr;
+    p->num_cut_items = use_cut ? (uint32_t)cut.items.size() : 0;
+    p->num_joins = use_cut ? (uint32_t)cut.joins.size() : 0;
+    if (use_cut) {
+        p->cut_items_d = (const PrefillItem*)((char*)int_buffer + whole_bytes);
+        p->cut_parts_d = (const PrefillPart*)((char*)int_buffer + parts_at);
+        p->joins_d = (const PrefillJoin*)((char*)int_buffer + joins_at);
+        p->part_o = (float*)((char*)float_buffer + table_bytes);
+        p->part_lse = p->part_o + (size_t)cut.partials * kPartRows;
+        p->cut_stream = s;
+    }
     p->planned = true;
     return 0;
 }
 
-template <bool BF16, bool SPLIT_P, bool ROPE_Q>
-static int launch_prefill(const PrefillPlan* p, const PrefillArgs& a, const void* q, const void* k, const void* v,
+template <bool BF16, bool SPLIT_P, bool ROPE_Q, bool PARTS>
+static int launch_prefill_kernel(const PrefillPlan* p, const PrefillArgs& a, const void* q, const void* k, const void* v,
                              hipStream_t s) {
-    auto kern = prefill_kernel<BF16, SPLIT_P, ROPE_Q>;
+    auto kern = prefill_kernel<BF16, SPLIT_P, ROPE_Q, PARTS>;
     static std::atomic<uint64_t> attr_done{0};
     int dev = 0;
     BZ_CHECK_HIP(hipGetDevice(&dev));
@@ -1014,10 +1324,22 @@ static int launch_prefill(const PrefillPlan* p, const PrefillArgs& a, const void
         attr_done.fetch_or(bit, std::memory_order_relaxed);
     }
     if (p->time_start) BZ_CHECK_HIP(hipEventRecord(p->time_start, s));
-    hipLaunchKernelGGL(kern, dim3(p->num_items), dim3(256), kSLds, s, a, (const char*)q, (const char*)k, (const char*)v);
+    hipLaunchKernelGGL(kern, dim3(PARTS ? p->num_cut_items : p->num_items), dim3(256), kSLds, s, a, (const char*)q,
+                       (const char*)k, (const char*)v);
     BZ_LAUNCH_CHECK();
+    if (PARTS) {
+        if (BF16) hipLaunchKernelGGL(prefill_combine_kernel<bf16_t>, dim3(p->num_joins, 4), dim3(256), 0, s, a, p->joins_d);
+        else hipLaunchKernelGGL(prefill_combine_kernel<f16_t>, dim3(p->num_joins, 4), dim3(256), 0, s, a, p->joins_d);
+        BZ_LAUNCH_CHECK();
+    }
     if (p->time_stop) BZ_CHECK_HIP(hipEventRecord(p->time_stop, s));
     return 0;
+}
+
+template <bool BF16, bool SPLIT_P, bool ROPE_Q>
+static int launch_prefill(const PrefillPlan* p, const PrefillArgs& a, const void* q, const void* k, const void* v, hipStream_t s) {
+    return a.parts ? launch_prefill_kernel<BF16, SPLIT_P, ROPE_Q, true>(p, a, q, k, v, s)
+                   : launch_prefill_kernel<BF16, SPLIT_P, ROPE_Q, false>(p, a, q, k, v, s);
 }
 
 #ifdef BZ_PF_PHASES
@@ -1081,12 +1403,15 @@ extern "C" int bz_batch_prefill_ragged(bz_prefill_plan_t* plan_, void* q, const 
     if (p->num_items == 0) return 0; // no q rows in the batch (K, if the call was to rotate it, has been rotated)
     PrefillArgs a;
     a.out = out;
-    a.items = p->items_d;
+    const bool cut = p->num_cut_items > 0 && s == p->cut_stream;
+    a.items = cut ? p->cut_items_d : p->items_d;
+    a.parts = cut ? p->cut_parts_d : nullptr;
+    a.part_o = p->part_o;
+    a.part_lse = p->part_lse;
     a.rope_table = (const float4*)p->rope_table;
     a.rope_pitch = p->max_len;
     a.num_qo_heads = num_qo_heads; a.num_kv_heads = num_kv_heads;
-    const uint32_t group = num_qo_heads / num_kv_heads;
-    a.head_shift = group % 4 == 0 ? 2 : (group % 2 == 0 ? 1 : 0);
+    a.head_shift = prefill_head_shift(num_qo_heads, num_kv_heads);
     a.causal = causal ? 1 : 0;
     if (!(sm_scale > 0.f)) sm_scale = 1.0f / sqrtf((float)head_dim);
     a.sm_scale_log2 = sm_scale * 1.4426950408889634f;

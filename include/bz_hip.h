@@ -206,6 +206,10 @@ int bz_batch_decode_noalloc(bz_decode_plan_t* plan, const void* q, int q_dtype, 
 /* ---------------------------------------------------------------------------------------
  * Prefill plan: replaces BatchPrefillRaggedHandler::plan (flashinfer_types.h:12-41,
  * flashinfer_types.cu:24-49).  Builds the (request, q-tile) work list, longest first.
+ * Where few q rows attend to many K/V rows, workgroups also share a job along its K/V range if both buffers hold more
+ * than bz_prefill_plan_workspace reports: 66 048 bytes of float_buffer behind the angle table per part (1 000 to 2 000 parts
+ * at most) and a second list in int_buffer.  Calls on the plan's own stream do so; calls on other streams, and plans
+ * without the room, attend to whole jobs.  (Like the angle table, the parts lie in float_buffer only during a call.)
  * ------------------------------------------------------------------------------------- */
 typedef struct bz_prefill_plan bz_prefill_plan_t;
 

@@ -361,6 +361,61 @@ def test_q_rows_for_the_last_tokens_of_a_request_only(kind, causal, rope_mode, f
     assert (np.abs(got - ref) <= kind_tol(ref, kind)).all(), np.abs(got - ref).max()
 
 
+@pytest.mark.parametrize("kind", KINDS, ids=KIND_IDS)
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("Hq,Hkv,rope_mode", [(8, 2, BZ_ROPE_Q_ONLY), (4, 4, BZ_ROPE_Q_ONLY), (6, 3, BZ_ROPE_NONE), (3, 1, BZ_ROPE_Q_ONLY)])
+def test_few_q_rows_over_many_kv_rows_in_parts(kind, causal, Hq, Hkv, rope_mode):
+    """A list of few long jobs is cut along the K/V range when the float workspace has room for the parts' rows behind
+    the angle table: chunks of prompts and a prompt without a prefix (parts that begin below the diagonal only), slices of
+    32, 64 and 128 rows, part ends inside and at the end of a request.  Against the checker; and a call on another stream
+    than the plan's takes the whole jobs, to the bits of a plan without the room."""
+    dtype, theta, D = kind[0], 1e4, 128
+    kv_lens, q_lens = np.array([2500, 900, 40, 1300, 1024]), np.array([130, 900, 3, 5, 33])
+    kv_indptr = np.concatenate([[0], np.cumsum(kv_lens)]).astype(np.int32)
+    qo_indptr = np.concatenate([[0], np.cumsum(q_lens)]).astype(np.int32)
+    rng = np.random.default_rng(280 + Hq)
+    Nkv, B, longest = int(kv_indptr[-1]), len(kv_lens), int(kv_lens.max())
+    q_full, k, v = (wl.randn_bits(rng, (Nkv, H, D), dtype) for H in (Hq, Hkv, Hkv))
+    rows = np.concatenate([np.arange(kv_indptr[b + 1] - q_lens[b], kv_indptr[b + 1]) for b in range(B)]).astype(np.int32)
+    qd, kd, vd = to_dev(q_full[rows], dtype), to_dev(k, dtype), to_dev(v, dtype)
+    qo_d, kv_d = torch.from_numpy(qo_indptr).cuda(), torch.from_numpy(kv_indptr).cuda()
+    int_ws = torch.empty(1 << 20, dtype=torch.uint8, device="cuda")
+
+    def run(handler, stream=None):
+        out = torch.full_like(qd, float("nan"))
+        torch.cuda.synchronize()
+        K.batch_prefill_attention(handler, qd, qo_d, kd, vd, kv_d, out, B, Hq, Hkv, D, causal=causal, rope_mode=rope_mode,
+                                  rope_theta=theta, stream=stream)
+        torch.cuda.synchronize()
+        return wl.to_f32(to_host_bits(out), dtype)
+
+    def planned(float_ws_bytes):
+        handler = K.BatchPrefillRaggedHandler()
+        if kind[1] is not None:
+            handler.set_bf16_mode(kind[1])
+        float_ws = torch.zeros(float_ws_bytes, dtype=torch.uint8, device="cuda")
+        handler.plan(float_ws, float_ws.numel(), int_ws, int_ws.numel(), qo_indptr, kv_indptr, B, Hq, Hkv, D, 16)
+        return handler, float_ws
+
+    handler, float_ws = planned(longest * 512)
+    whole = run(handler)
+    handler, float_ws = planned(64 << 20)
+    got = run(handler)
+    assert float_ws[longest * 512:].any()  # parts were left there
+    if rope_mode == BZ_ROPE_NONE:
+        ref = oracle.batch_prefill_ragged(q_full, k, v, dtype, kv_indptr, Hq, Hkv, D, causal=causal, rows=rows, parallel=True)
+    else:
+        q_fed = prefill_q_as_fed(q_full, dtype, kv_indptr, Hq, D, theta, prefill_angle_table(float_ws, longest, D))
+        ref = oracle.batch_prefill_ragged(q_fed, k, v, dtype, kv_indptr, Hq, Hkv, D, causal=causal, sm_scale=LN2, rows=rows,
+                                          parallel=True)
+    for out in (whole, got):
+        assert not np.isnan(out).any()
+        assert (np.abs(out - ref) <= kind_tol(ref, kind)).all(), np.abs(out - ref).max()
+    side = torch.cuda.Stream()
+    float_ws[longest * 512:] = 0
+    assert np.array_equal(run(handler, side.cuda_stream), whole) and not float_ws[longest * 512:].any()
+
+
 def test_a_batch_without_q_rows_still_rotates_k():
     """BZ_ROPE_FULL promises rotated k rows in the caller's buffer (the page store that follows copies them), also
     when no request of the batch has a q row."""
