@@ -441,13 +441,13 @@ int decode_step_fast_path(const DecodePlan* p, const void* q, const void* k_new,
 // both pairs may point at the same memory.
 struct PartialBufs {
     float *part_o, *part_lse;           // general kernel: [partials][Hq][D], [partials][Hq]
-    float *mfma_part_o, *mfma_part_lse; // matrix-core kernel: [partials][16][128], [partials][16]
+    float *mfma_part_o, *mfma_part_lse; // matrix-core kernel: [partials][16][D], [partials][16]
 };
 
 static int batch_decode_impl(DecodePlan* p, const void* q, int q_dtype, const bz_paged_kv_t* kv, void* out,
                              int out_dtype, uint32_t num_qo_heads, int rope_mode, float rope_theta, float sm_scale,
                              const float* k_scale, const float* v_scale, float* lse, const PartialBufs* bufs_or_null,
-                             void* stream) {
+                             void* stream, bool general_only = false) {
     if (!p || !kv || !q || !out) return BZ_ERR_BAD_ARG;
     if (!p->planned) return BZ_ERR_NOT_PLANNED;
     // a table whose device pointers were cleared after the previous step (src/blitz/stub.h:1361-1363)
@@ -488,7 +488,7 @@ static int batch_decode_impl(DecodePlan* p, const void* q, int q_dtype, const bz
 
     if (p->num_segments > 0) {
         int rc = BZ_ERR_UNSUPPORTED;
-        if (!p->force_general)
+        if (!p->force_general && !general_only)
             rc = decode_fast_path(p, q, out, lse, q_dtype, out_dtype, rope_mode, a.sm_scale_log2, a.freqs, kv,
                                   num_qo_heads, k_scale, v_scale, bufs.mfma_part_o, bufs.mfma_part_lse, false, s);
         if (rc == 0) {
@@ -661,9 +661,13 @@ extern "C" int bz_batch_decode_noalloc(bz_decode_plan_t* plan_, const void* q, i
     // is pinned to the general kernel.
     const size_t gen_o = scratch_align((size_t)p->num_partials * p->num_qo_heads * p->head_dim * sizeof(float));
     const size_t gen_l = scratch_align((size_t)p->num_partials * p->num_qo_heads * sizeof(float));
-    const size_t mf_o = (p->mfma_ok && !p->force_general) ? scratch_align((size_t)p->mfma_partials * 16 * 128 * sizeof(float)) : 0;
-    const size_t mf_l = (p->mfma_ok && !p->force_general) ? scratch_align((size_t)p->mfma_partials * 16 * sizeof(float)) : 0;
-    if (gen_o + gen_l > (size_t)BZ_DECODE_NOALLOC_SCRATCH_BYTES || mf_o + mf_l > (size_t)BZ_DECODE_NOALLOC_SCRATCH_BYTES)
+    const bool mfma = p->mfma_ok && !p->force_general;
+    const size_t mf_o = mfma ? scratch_align((size_t)p->mfma_partials * 16 * p->head_dim * sizeof(float)) : 0;
+    const size_t mf_l = mfma ? scratch_align((size_t)p->mfma_partials * 16 * sizeof(float)) : 0;
+    // (heads of 64, whose partials the general kernel packs more tightly: it takes what fits only there)
+    const bool general_only = p->head_dim == 64 && mf_o + mf_l > (size_t)BZ_DECODE_NOALLOC_SCRATCH_BYTES;
+    if (gen_o + gen_l > (size_t)BZ_DECODE_NOALLOC_SCRATCH_BYTES ||
+        (!general_only && mf_o + mf_l > (size_t)BZ_DECODE_NOALLOC_SCRATCH_BYTES))
         return BZ_ERR_WORKSPACE;
     unsigned char* base = nullptr;
     const int rc = decode_scratch_for_current_device(&base);
@@ -673,5 +677,5 @@ extern "C" int bz_batch_decode_noalloc(bz_decode_plan_t* plan_, const void* q, i
     const PartialBufs bufs = {reinterpret_cast<float*>(base), reinterpret_cast<float*>(base + gen_o),
                               reinterpret_cast<float*>(base), reinterpret_cast<float*>(base + mf_o)};
     return batch_decode_impl(p, q, q_dtype, kv, out, out_dtype, num_qo_heads, rope_mode, rope_theta, sm_scale, k_scale,
-                             v_scale, lse, &bufs, stream);
+                             v_scale, lse, &bufs, stream, general_only);
 }

@@ -1,4 +1,4 @@
-// MFMA paged decode for gfx950 (head_dim 128, page_size a multiple of 16, f16/bf16/e4m3 KV, up to 16
+// MFMA paged decode for gfx950 (head_dim 128, or 64 with a 16-bit pool, page_size a multiple of 16, f16/bf16/e4m3 KV, up to 16
 // query heads per scheduled unit; the planner cuts a larger group into equal parts).  One wave64 per
 // workgroup walks a list of "pieces" (contiguous runs of 32-token tiles of one (sequence, kv head)) that
 // the host planner balanced over the wave slots of the chip, so every K and V byte is read once and
@@ -52,8 +52,8 @@ typedef __attribute__((ext_vector_type(4))) float f32x4_t;
 typedef __attribute__((ext_vector_type(4))) short s16x4_t;
 
 constexpr int kTileTok = 32;     // tokens per tile
-constexpr int kVRowBytes = 288;  // LDS row stride of the V tile: 256 B of data + 32 B so that
-                                 // consecutive rows start 8 banks apart (conflict-free transposed reads)
+constexpr int kVRowPad = 32;     // the LDS row stride of the V tile is a row of 16-bit values + 32 B: eight consecutive
+                                 // rows then start in eight different groups of 8 banks (conflict-free transposed reads)
 
 struct MfmaDecodeArgs {
     const void* q;
@@ -68,7 +68,7 @@ struct MfmaDecodeArgs {
     const MfmaPiece* pieces;
     const MfmaTile* tiles;
     const MfmaSlotHead* heads;
-    float* part_o;   // [num_partials][16][128]
+    float* part_o;   // [num_partials][16][D]
     float* part_lse; // [num_partials][16]
     uint64_t stride_page, stride_n, stride_h; // elements
     uint32_t page_size, num_qo_heads, group; // group: q heads per scheduled unit (<= 16)
@@ -175,7 +175,11 @@ constexpr int kInfoChunk = 16; // tile descriptions fetched per round trip (one 
 // the final normalisation.  A lane then fetches 16 bytes = 16 elements of a K row, so the contraction
 // index of MFMA step ks, lane group j, element i is d = 64*(ks/2) + 16*j + 8*(ks%2) + i (q follows).
 // NT: K/V loads carry the non-temporal hint (see kNtK16 above); chosen by the planner.
-template <bool BF16, typename OT, bool ROPE_Q, bool KV8, bool NT>
+// D: head size; 64 with 16-bit pools only (their rows have the bytes that a row of 128 has in a one-byte pool).
+// Heads of 64 run the loop of the one-byte pools, two 8 KiB tiles in flight, without the widening: 96 sequences of 17 to
+// 2048 tokens, 32/8 heads, f16: 77 us on the general kernel (bound by its vector instructions), 40.8 us here (5.0 TB/s; a
+// slot has 12 tiles, so its first round trips and its last tile weigh more than in the larger batches).
+template <bool BF16, typename OT, bool ROPE_Q, bool KV8, bool NT, int D>
 __global__ __launch_bounds__(64, 2) void decode_mfma_kernel(const MfmaSlotHead* __restrict__ heads, MfmaDecodeArgs a,
                                                             const char* __restrict__ q_ptr,
                                                             const char* __restrict__ k_data,
@@ -185,13 +189,17 @@ __global__ __launch_bounds__(64, 2) void decode_mfma_kernel(const MfmaSlotHead* 
                                                             const MfmaTile* __restrict__ tiles,
                                                             const float* __restrict__ k_scale,
                                                             const float* __restrict__ v_scale) {
+    static_assert(D == 128 || (D == 64 && !KV8), "head sizes");
     using M = Mma<BF16>;
+    constexpr bool TWO_SETS = KV8 || D == 64;   // a tile is 8 KiB: two of them in flight per wave
+    constexpr int KS = D / 32, DB = D / 16;     // matrix steps of the scores; 16-wide blocks of the output
+    constexpr int kVRowBytes = 2 * D + kVRowPad;
     __shared__ __attribute__((aligned(16))) unsigned char v_lds[kTileTok * kVRowBytes];
     __shared__ __attribute__((aligned(16))) int info_lds[2][kInfoChunk][kInfoInts];
     // Normalised rows of finished pieces, kept here until the slot's last tile is done (or the space runs out):
-    // 16 rows of 128 floats (+ 4 per row, so that the four lane groups fall on different banks), one log-sum-exp
+    // 16 rows of D floats (+ 4 per row, so that the four lane groups fall on different banks), one log-sum-exp
     // per row, and for each parked piece where its rows go.
-    constexpr int kStageRow = 132, kStageRows = 16, kStagePieces = 8;
+    constexpr int kStageRow = D + 4, kStageRows = 16, kStagePieces = 8;
     struct StagedPiece { char* dst; float* lse; int row0, rows, f32, pad; };
     __shared__ __attribute__((aligned(16))) float stage_lds[kStageRows * kStageRow + kStageRows];
     __shared__ StagedPiece stage_desc[kStagePieces];
@@ -226,7 +234,7 @@ __global__ __launch_bounds__(64, 2) void decode_mfma_kernel(const MfmaSlotHead* 
     // while it travels.
     float lane_freq = 0.f;
     if (ROPE_Q) {
-        lane_freq = a.freqs.f[lane];
+        lane_freq = a.freqs.f[lane & (D / 2 - 1)];
         asm("" : "+v"(lane_freq)); // (kept in its register: not fetched again at the point of use)
     }
     // Left to the compiler, the slot head is fetched in two steps (its tile range, then, behind the test for an empty
@@ -308,7 +316,7 @@ __global__ __launch_bounds__(64, 2) void decode_mfma_kernel(const MfmaSlotHead* 
         return u;
     };
 
-    uint4 kreg[2][4], vreg[8], qnext[4];
+    uint4 kreg[2][4], vreg[8], qnext[KS];
     // byte offsets of the two 16-token subtiles of a tile inside the pool
     struct TileBase { size_t b[2]; };
     auto tile_base = [&](const TileUni& u) -> TileBase {
@@ -321,12 +329,12 @@ __global__ __launch_bounds__(64, 2) void decode_mfma_kernel(const MfmaSlotHead* 
         }
         return r;
     };
-    // One-byte pools: a tile is 8 KiB and lands in half of the registers a 16-bit tile needs, so the two halves
+    // One-byte pools and heads of 64: a tile is 8 KiB and lands in half of the registers a 16 KiB tile needs, so the two halves
     // are two sets (SET 0 / 1: kreg[u][2 SET + p], vreg[4 SET + w]) and two tiles are in flight per wave.
     // `live` false: the set has no tile to fetch; the loads are issued all the same, every lane at the tile's first
     // bytes (one cache line), so that the number of loads behind a set's own does not depend on the path taken
     // and the waits the compiler derives for the sets stay apart.
-    auto issue_loads_kv8 = [&](const TileBase& tb, auto set_c, bool live) __attribute__((always_inline)) {
+    auto issue_loads_two = [&](const TileBase& tb, auto set_c, bool live) __attribute__((always_inline)) {
         constexpr int SET = decltype(set_c)::value;
         const size_t base[2] = {tb.b[0], tb.b[1]};
         const size_t koff = live ? (size_t)n * row_bytes + (size_t)(j * 16) : 0;
@@ -359,9 +367,9 @@ __global__ __launch_bounds__(64, 2) void decode_mfma_kernel(const MfmaSlotHead* 
     // (every lane loads: columns past the group fetch its last head again and are zeroed where the piece is opened --
     // loads under a lane mask would make the compiler wait for them on the spot)
     auto issue_q = [&](const TileUni& u) {
-        const char* qrow = q_ptr + ((size_t)u.seq * a.num_qo_heads + (size_t)u.kvh * G + min(n, G - 1)) * 256;
+        const char* qrow = q_ptr + ((size_t)u.seq * a.num_qo_heads + (size_t)u.kvh * G + min(n, G - 1)) * (2 * D);
 #pragma unroll
-        for (int ks = 0; ks < 4; ++ks) qnext[ks] = *reinterpret_cast<const uint4*>(qrow + d_of(ks) * 2);
+        for (int ks = 0; ks < KS; ++ks) qnext[ks] = *reinterpret_cast<const uint4*>(qrow + d_of(ks) * 2);
     };
 
     // The records of the first tiles are requested together with the two page ids of the first tile (whose
@@ -386,7 +394,7 @@ __global__ __launch_bounds__(64, 2) void decode_mfma_kernel(const MfmaSlotHead* 
     if (multi) raw0 = fetch_dep(rec0);
     __builtin_amdgcn_sched_barrier(0);
     issue_q(un);
-    if constexpr (KV8) issue_loads_kv8(tile_base(un), std::integral_constant<int, 0>{}, true);
+    if constexpr (TWO_SETS) issue_loads_two(tile_base(un), std::integral_constant<int, 0>{}, true);
     else issue_loads(tile_base(un));
     __builtin_amdgcn_sched_barrier(0);
     if (multi) {
@@ -396,9 +404,9 @@ __global__ __launch_bounds__(64, 2) void decode_mfma_kernel(const MfmaSlotHead* 
     int chunk_base = g_begin, buf = 0;
     Desc dnext;
 
-    uint4 qhi[4], qlo[4];
+    uint4 qhi[KS], qlo[KS];
     float m_run = -INFINITY, l_run = 0.f;
-    f32x4_t acc[8];
+    f32x4_t acc[DB];
 
     // descriptions of the next chunk of tiles: fetched a quarter into this chunk, parked in the other LDS
     // buffer at three quarters
@@ -413,7 +421,7 @@ __global__ __launch_bounds__(64, 2) void decode_mfma_kernel(const MfmaSlotHead* 
     // ================= first tile of a piece =================
     auto open_piece = [&](const TileUni& uc) __attribute__((always_inline)) {
 #pragma unroll
-        for (int ks = 0; ks < 4; ++ks) { qhi[ks] = n < G ? qnext[ks] : make_uint4(0, 0, 0, 0); qlo[ks] = make_uint4(0, 0, 0, 0); }
+        for (int ks = 0; ks < KS; ++ks) { qhi[ks] = n < G ? qnext[ks] : make_uint4(0, 0, 0, 0); qlo[ks] = make_uint4(0, 0, 0, 0); }
         if (ROPE_Q) {
             float sn1, cs1;
             sincosf((float)(uc.seq_len - 1 + a.step_mode) * lane_freq, &sn1, &cs1); // q sits at the last token
@@ -426,11 +434,11 @@ __global__ __launch_bounds__(64, 2) void decode_mfma_kernel(const MfmaSlotHead* 
             // the rotated q is split into a storage-precision head and tail (q = hi + lo) and both are
             // contracted, so rotating inside the kernel costs no precision
 #pragma unroll
-            for (int ks = 0; ks < 2; ++ks) { // dims d = 32ks+8j+e pair with d+64, held at ks+2
+            for (int ks = 0; ks < KS / 2; ++ks) { // dims d = d_of(ks)+e pair with d + D/2, held at ks + KS/2
 #pragma unroll
                 for (int w = 0; w < 4; ++w) {
                     float x[2] = {M::unpack_lo(u4(qhi[ks], w)), M::unpack_hi(u4(qhi[ks], w))};
-                    float y[2] = {M::unpack_lo(u4(qhi[ks + 2], w)), M::unpack_hi(u4(qhi[ks + 2], w))};
+                    float y[2] = {M::unpack_lo(u4(qhi[ks + KS / 2], w)), M::unpack_hi(u4(qhi[ks + KS / 2], w))};
                     float xr[2], yr[2];
 #pragma unroll
                     for (int e = 0; e < 2; ++e) {
@@ -439,27 +447,27 @@ __global__ __launch_bounds__(64, 2) void decode_mfma_kernel(const MfmaSlotHead* 
                     }
                     const uint32_t xh = M::pack2(xr[0], xr[1]), yh = M::pack2(yr[0], yr[1]);
                     u4(qhi[ks], w) = xh;
-                    u4(qhi[ks + 2], w) = yh;
+                    u4(qhi[ks + KS / 2], w) = yh;
                     u4(qlo[ks], w) = M::pack2(xr[0] - M::unpack_lo(xh), xr[1] - M::unpack_hi(xh));
-                    u4(qlo[ks + 2], w) = M::pack2(yr[0] - M::unpack_lo(yh), yr[1] - M::unpack_hi(yh));
+                    u4(qlo[ks + KS / 2], w) = M::pack2(yr[0] - M::unpack_lo(yh), yr[1] - M::unpack_hi(yh));
                 }
             }
         }
         m_run = -INFINITY;
         l_run = 0.f;
 #pragma unroll
-        for (int d = 0; d < 8; ++d) acc[d] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+        for (int d = 0; d < DB; ++d) acc[d] = f32x4_t{0.f, 0.f, 0.f, 0.f};
     };
     // ---- scores: S^T[token][head], lane (head n, group j) gets tokens 16u + 4j + r
-    auto scores = [&](const uint4 (&kop)[2][4], f32x4_t (&s)[2]) __attribute__((always_inline)) {
+    auto scores = [&](const uint4 (&kop)[2][KS], f32x4_t (&s)[2]) __attribute__((always_inline)) {
 #pragma unroll
         for (int u = 0; u < 2; ++u) {
             s[u] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-            for (int ks = 0; ks < 4; ++ks) s[u] = M::run(kop[u][ks], qhi[ks], s[u]);
+            for (int ks = 0; ks < KS; ++ks) s[u] = M::run(kop[u][ks], qhi[ks], s[u]);
             if (ROPE_Q) {
 #pragma unroll
-                for (int ks = 0; ks < 4; ++ks) s[u] = M::run(kop[u][ks], qlo[ks], s[u]);
+                for (int ks = 0; ks < KS; ++ks) s[u] = M::run(kop[u][ks], qlo[ks], s[u]);
             }
         }
     };
@@ -474,15 +482,15 @@ __global__ __launch_bounds__(64, 2) void decode_mfma_kernel(const MfmaSlotHead* 
         const float* src = stage_lds + row0 * kStageRow;
         if (f32) { // fp32 rows, four elements per lane; the rows lie side by side at the destination
             float* dst = reinterpret_cast<float*>(dst_c);
-            for (int c = lane; c < rows * 32; c += 64) {
-                const int row = c >> 5, w = c & 31;
+            for (int c = lane; c < rows * (D / 4); c += 64) {
+                const int row = c / (D / 4), w = c % (D / 4);
                 const float4 v = *reinterpret_cast<const float4*>(src + row * kStageRow + 4 * w);
-                store_global_16(dst + row * 128 + 4 * w, v.x, v.y, v.z, v.w);
+                store_global_16(dst + row * D + 4 * w, v.x, v.y, v.z, v.w);
             }
         } else if constexpr (!std::is_same<OT, float>::value) { // 16-bit rows, eight elements per lane
             OT* dst = reinterpret_cast<OT*>(dst_c);
-            for (int c = lane; c < rows * 16; c += 64) {
-                const int row = c >> 4, w = c & 15;
+            for (int c = lane; c < rows * (D / 8); c += 64) {
+                const int row = c / (D / 8), w = c % (D / 8);
                 const float4 x = *reinterpret_cast<const float4*>(src + row * kStageRow + 8 * w);
                 const float4 y = *reinterpret_cast<const float4*>(src + row * kStageRow + 8 * w + 4);
                 uint4 o;
@@ -490,7 +498,7 @@ __global__ __launch_bounds__(64, 2) void decode_mfma_kernel(const MfmaSlotHead* 
                 o.y = (uint32_t)StoreCvt<OT>::from(x.z).bits | ((uint32_t)StoreCvt<OT>::from(x.w).bits << 16);
                 o.z = (uint32_t)StoreCvt<OT>::from(y.x).bits | ((uint32_t)StoreCvt<OT>::from(y.y).bits << 16);
                 o.w = (uint32_t)StoreCvt<OT>::from(y.z).bits | ((uint32_t)StoreCvt<OT>::from(y.w).bits << 16);
-                store_global_16(dst + row * 128 + 8 * w, __uint_as_float(o.x), __uint_as_float(o.y), __uint_as_float(o.z),
+                store_global_16(dst + row * D + 8 * w, __uint_as_float(o.x), __uint_as_float(o.y), __uint_as_float(o.z),
                                 __uint_as_float(o.w));
             }
         }
@@ -558,13 +566,13 @@ __global__ __launch_bounds__(64, 2) void decode_mfma_kernel(const MfmaSlotHead* 
             for (int i = 0; i < 4; ++i) {
                 const float al = __shfl(alpha, 4 * j + i, 64);
 #pragma unroll
-                for (int d = 0; d < 8; ++d) acc[d][i] *= al;
+                for (int d = 0; d < DB; ++d) acc[d][i] *= al;
             }
         }
         wave_lds_sync(); // V tile written before the transposed reads
-        // ---- O[head][d] += P[head][tok] V[tok][d], eight 16-wide d blocks
+        // ---- O[head][d] += P[head][tok] V[tok][d], 16-wide d blocks
 #pragma unroll
-        for (int d = 0; d < 8; ++d) {
+        for (int d = 0; d < DB; ++d) {
             uint4 vb;
 #pragma unroll
             for (int u = 0; u < 2; ++u) {
@@ -592,7 +600,7 @@ __global__ __launch_bounds__(64, 2) void decode_mfma_kernel(const MfmaSlotHead* 
                 const float il = __shfl(inv_l, head, 64);
                 if (head < G) {
 #pragma unroll
-                    for (int d = 0; d < 8; ++d) rows[head * kStageRow + d * 16 + n] = acc[d][i] * il;
+                    for (int d = 0; d < DB; ++d) rows[head * kStageRow + d * 16 + n] = acc[d][i] * il;
                 }
             }
             if (j == 0 && n < G) stage_lds[kStageRows * kStageRow + pend_rows + n] = partial < 0 ? lse2 * 0.6931471805599453f : lse2;
@@ -600,10 +608,10 @@ __global__ __launch_bounds__(64, 2) void decode_mfma_kernel(const MfmaSlotHead* 
             char* dst_c;
             float* lse_p;
             if (partial >= 0) {
-                dst_c = reinterpret_cast<char*>(a.part_o + (size_t)partial * 16 * 128);
+                dst_c = reinterpret_cast<char*>(a.part_o + (size_t)partial * 16 * D);
                 lse_p = a.part_lse + (size_t)partial * 16;
             } else {
-                dst_c = reinterpret_cast<char*>(reinterpret_cast<OT*>(a.out) + ((size_t)b * a.num_qo_heads + kvh * G) * 128);
+                dst_c = reinterpret_cast<char*>(reinterpret_cast<OT*>(a.out) + ((size_t)b * a.num_qo_heads + kvh * G) * D);
                 lse_p = a.lse ? a.lse + (size_t)b * a.num_qo_heads + kvh * G : nullptr;
             }
             if (last_of_slot) { // nothing comes after these stores: out they go, behind whatever is still parked
@@ -625,14 +633,14 @@ __global__ __launch_bounds__(64, 2) void decode_mfma_kernel(const MfmaSlotHead* 
         }
     };
 
-    if constexpr (KV8) {
-        // ---- one-byte pools: two tiles in flight.  Tile g lives in set (g - g_begin) % 2; its set is refilled with
+    if constexpr (TWO_SETS) {
+        // ---- one-byte pools, heads of 64: two tiles in flight.  Tile g lives in set (g - g_begin) % 2; its set is refilled with
         // tile g + 2 as soon as its bytes have been widened into operand registers (K) and parked in LDS (V).
         TileUni dA = un, dB = un; // descriptions of the tiles in sets 0 and 1
         {
             const bool second = g_begin + 1 < g_end;
             if (second) dB = read_info(0, 1);
-            issue_loads_kv8(tile_base(dB), std::integral_constant<int, 1>{}, second);
+            issue_loads_two(tile_base(dB), std::integral_constant<int, 1>{}, second);
         }
         auto body = [&](int g, auto set_c, auto last_c) __attribute__((always_inline)) {
             constexpr int SET = decltype(set_c)::value;
@@ -652,41 +660,50 @@ __global__ __launch_bounds__(64, 2) void decode_mfma_kernel(const MfmaSlotHead* 
             const int tile_tok0 = uc.t * kTileTok;
             const bool ragged = tile_tok0 + kTileTok > uc.tok_end; // wave-uniform
             wave_lds_sync(); // transposed reads of the previous tile come before V is overwritten
+            auto park_v = [&](int w, const uint4& v) __attribute__((always_inline)) {
+                if constexpr (KV8) { // 16 e4m3 bytes -> 16 operand-type values -> 32 B of the LDS row
+                    unsigned char* dst = v_lds + (8 * w + (lane >> 3)) * kVRowBytes + (lane & 7) * 32;
+                    *reinterpret_cast<uint4*>(dst) = fp8x8_to_op<BF16>(v, 0);
+                    *reinterpret_cast<uint4*>(dst + 16) = fp8x8_to_op<BF16>(v, 1);
+                } else {
+                    *reinterpret_cast<uint4*>(v_lds + (8 * w + (lane >> 3)) * kVRowBytes + (lane & 7) * 16) = v;
+                }
+            };
             if (!ragged) {
 #pragma unroll
-                for (int w = 0; w < 4; ++w) { // 16 e4m3 bytes -> 16 operand-type values -> 32 B of the LDS row
-                    unsigned char* dst = v_lds + (8 * w + (lane >> 3)) * kVRowBytes + (lane & 7) * 32;
-                    *reinterpret_cast<uint4*>(dst) = fp8x8_to_op<BF16>(vreg[4 * SET + w], 0);
-                    *reinterpret_cast<uint4*>(dst + 16) = fp8x8_to_op<BF16>(vreg[4 * SET + w], 1);
-                }
+                for (int w = 0; w < 4; ++w) park_v(w, vreg[4 * SET + w]);
             } else {
 #pragma unroll
                 for (int w = 0; w < 4; ++w) {
                     uint4 v = vreg[4 * SET + w];
-                    const int row = 8 * w + (lane >> 3);
-                    if (tile_tok0 + row >= uc.tok_end) v = make_uint4(0, 0, 0, 0); // 0 * garbage must be 0
-                    unsigned char* dst = v_lds + row * kVRowBytes + (lane & 7) * 32;
-                    *reinterpret_cast<uint4*>(dst) = fp8x8_to_op<BF16>(v, 0);
-                    *reinterpret_cast<uint4*>(dst + 16) = fp8x8_to_op<BF16>(v, 1);
+                    if (tile_tok0 + 8 * w + (lane >> 3) >= uc.tok_end) v = make_uint4(0, 0, 0, 0); // 0 * garbage must be 0
+                    park_v(w, v);
                 }
             }
-            uint4 kcur[2][4];
+            uint4 kcur[2][KS];
+            f32x4_t s[2];
 #pragma unroll
             for (int u = 0; u < 2; ++u)
 #pragma unroll
-                for (int ks = 0; ks < 4; ++ks) kcur[u][ks] = fp8x8_to_op<BF16>(kreg[u][2 * SET + (ks >> 1)], ks & 1);
+                for (int ks = 0; ks < KS; ++ks) {
+                    if constexpr (KV8) kcur[u][ks] = fp8x8_to_op<BF16>(kreg[u][2 * SET + (ks >> 1)], ks & 1);
+                    else kcur[u][ks] = kreg[u][2 * SET + ks];
+                }
+            if constexpr (!KV8) { // the landing registers are the operands: contracted before they are refilled
+                scores(kcur, s);
+                __builtin_amdgcn_sched_barrier(0);
+            }
             // the set is free: q rows of the next tile's piece (one tile ahead), K/V of the tile after next
             if constexpr (!LAST) {
                 if (g + 1 < g_end) {
                     const TileUni& u1 = SET ? dA : dB;
                     if (u1.flags & 1) issue_q(u1);
                 }
-                issue_loads_kv8(nb, set_c, more);
+                issue_loads_two(nb, set_c, more);
                 if (SET) dB = u2; else dA = u2;
                 if (i + 1 == kInfoChunk) { chunk_base += kInfoChunk; buf ^= 1; }
             }
-            f32x4_t s[2];
-            scores(kcur, s);
+            if constexpr (KV8) scores(kcur, s);
             softmax_pv(uc, s, score_scale, g + 1 == g_end);
         };
         // (The loop has no exit between its halves, so that the only way into one set's half is through the
@@ -758,7 +775,7 @@ __global__ __launch_bounds__(64, 2) void decode_mfma_kernel(const MfmaSlotHead* 
 }
 
 // Combine the partials of one split (sequence, kv head): o = sum_i o_i 2^(lse_i - M) / sum_i 2^(lse_i - M).
-// One workgroup per (split, q head of the group): 128 lanes (one per output dimension) x S slices.  A
+// One workgroup per (split, q head of the group): D lanes (one per output dimension) x S slices.  A
 // slice fetches eight partials at a time with all loads issued before any is used and merges them with a
 // running maximum; slice s takes batches s, s+S, ...  With S = 1 (splits of up to 16 partials, what large
 // batches produce) that is two dependent memory round trips for up to eight partials.  A single long
@@ -766,8 +783,8 @@ __global__ __launch_bounds__(64, 2) void decode_mfma_kernel(const MfmaSlotHead* 
 // for one sequence on the whole chip): S = 4 or 8 slices then work side by side and are merged through
 // LDS, instead of 32 round trips one after the other.  (Batches of 32 per lane were measured as well:
 // slower on the large-batch workload, where most splits have two to four partials.)
-template <typename OT, int S>
-__global__ __launch_bounds__(128 * S) void decode_mfma_combine_kernel(const MfmaCombine* __restrict__ combos,
+template <typename OT, int S, int D>
+__global__ __launch_bounds__(D * S) void decode_mfma_combine_kernel(const MfmaCombine* __restrict__ combos,
                                                                       const float* __restrict__ part_o,
                                                                       const float* __restrict__ part_lse, void* out,
                                                                       float* lse, uint32_t num_qo_heads, uint32_t G) {
@@ -781,7 +798,7 @@ __global__ __launch_bounds__(128 * S) void decode_mfma_combine_kernel(const Mfma
             const bool live = i0 + k < c.count;
             const size_t slot = (size_t)(c.first + (live ? i0 + k : 0));
             li[k] = live ? part_lse[slot * 16 + g] : -INFINITY;
-            oi[k] = live ? part_o[(slot * 16 + g) * 128 + d] : 0.f;
+            oi[k] = live ? part_o[(slot * 16 + g) * D + d] : 0.f;
         }
         float m2 = M;
 #pragma unroll
@@ -799,7 +816,7 @@ __global__ __launch_bounds__(128 * S) void decode_mfma_combine_kernel(const Mfma
         M = m2;
     }
     if constexpr (S > 1) {
-        __shared__ float sm_m[S][128], sm_w[S][128], sm_o[S][128];
+        __shared__ float sm_m[S][D], sm_w[S][D], sm_o[S][D];
         sm_m[sl][d] = M;
         sm_w[sl][d] = wsum;
         sm_o[sl][d] = o;
@@ -822,7 +839,7 @@ __global__ __launch_bounds__(128 * S) void decode_mfma_combine_kernel(const Mfma
     }
     o = wsum > 0.f ? o / wsum : 0.f;
     const size_t hq = (size_t)c.seq * num_qo_heads + (size_t)c.kvh * G + g;
-    reinterpret_cast<OT*>(out)[hq * 128 + d] = StoreCvt<OT>::from(o);
+    reinterpret_cast<OT*>(out)[hq * D + d] = StoreCvt<OT>::from(o);
     if (lse && d == 0) lse[hq] = (M + log2f(wsum)) * 0.6931471805599453f;
 }
 
@@ -831,7 +848,7 @@ __global__ __launch_bounds__(128 * S) void decode_mfma_combine_kernel(const Mfma
 // result per piece.  This kernel takes the newest token from the caller's rows instead of from the pool: it
 // rotates the new K row (and q, in registers) at position seq_len-1, writes K and V into their page slot -- the
 // append -- and folds the token's own term exp(q.k) v into the merge of the partials.  One workgroup per
-// (sequence, scheduled unit, group of HB q heads): 32 lanes per head with four output dimensions each, x S slices
+// (sequence, scheduled unit, group of HB q heads): D/4 lanes per head with four output dimensions each, x S slices
 // over the partials (thread layout below).  The appended rows carry the same bits the append kernel writes.
 template <typename T> __device__ __forceinline__ float pool_to_f32(T v) { return to_f32(v); }
 template <> __device__ __forceinline__ float pool_to_f32<e4m3_t>(e4m3_t v) {
@@ -851,7 +868,7 @@ struct StepFinishArgs {
     const int32_t* last_page_len;
     const int32_t* steps_ahead;
     const MfmaUnit* units;
-    const float* part_o;   // [pieces][16][128]
+    const float* part_o;   // [pieces][16][D]
     const float* part_lse; // [pieces][16]
     void* out;
     float* lse;
@@ -864,7 +881,7 @@ struct StepFinishArgs {
     alignas(8) RopeFreqs freqs; // (read two at a time)
 };
 
-// Thread layout: 32 lanes per q head, four consecutive output dimensions per lane (16-byte loads of the partial
+// Thread layout: D/4 lanes per q head, four consecutive output dimensions per lane (16-byte loads of the partial
 // rows); HB heads of the unit share a workgroup (threadIdx.y) and with it the angles of the new token's
 // position; S slices (threadIdx.z) split a long list of partials.  The kernel is short enough that the number
 // of instructions its waves issue, not the bytes they move, sets its duration.
@@ -887,9 +904,10 @@ template <> __device__ __forceinline__ void store4<float>(float* p, const float*
     *reinterpret_cast<float4*>(p) = make_float4(v[0], v[1], v[2], v[3]);
 }
 
-template <typename QT, typename PT, typename OT, int S, int HB>
-__global__ __launch_bounds__(32 * HB * S) void decode_step_finish_kernel(const MfmaUnit* __restrict__ units_p,
+template <typename QT, typename PT, typename OT, int S, int HB, int D>
+__global__ __launch_bounds__(D / 4 * HB * S) void decode_step_finish_kernel(const MfmaUnit* __restrict__ units_p,
                                                                          const int32_t* __restrict__ ahead_p, StepFinishArgs a) {
+    constexpr int LPH = D / 4; // lanes of a head
     const uint32_t t = threadIdx.x, hl = threadIdx.y, sl = threadIdx.z;
     // The two pointers in front of the argument block arrive in registers with the wave (kernel-argument preload of
     // this target; the build asks for it), so the unit record and the step counter are asked for at once, while the
@@ -915,8 +933,8 @@ __global__ __launch_bounds__(32 * HB * S) void decode_step_finish_kernel(const M
     const int kvr = u.unit / (int)a.parts; // the kv head whose K/V the unit reads
     const uint32_t hq = (uint32_t)u.unit * a.group + g;
     const uint32_t d0 = 4 * t;             // this lane's four output dimensions
-    const bool upper = d0 >= 64;           // they are the second elements of their rotate-half pairs
-    const uint32_t i0 = d0 & 63, dp = upper ? d0 - 64 : d0 + 64;
+    const bool upper = d0 >= D / 2;           // they are the second elements of their rotate-half pairs
+    const uint32_t i0 = d0 & (D / 2 - 1), dp = upper ? d0 - D / 2 : d0 + D / 2;
     // Everything that depends on the unit record alone is requested at once: the caller's rows, the scales
     // and the first four partial results of this slice.  (The sequence's length and its place in the page
     // list come with the unit record, from the host table the plan was made from, like the lengths the
@@ -927,9 +945,9 @@ __global__ __launch_bounds__(32 * HB * S) void decode_step_finish_kernel(const M
     // and a load under a condition would be waited for on the spot)
     const bool appends = g_raw == 0 && sl == 0 && u.unit % (int)a.parts == 0; // one head's lanes per (sequence, kv head)
     const int64_t page = a.indices[u.ip0 + max(seq_len - 1, 0) / (int)a.page_size];
-    const QT* qrow = reinterpret_cast<const QT*>(a.q) + ((size_t)b * a.num_qo_heads + hq) * 128;
-    const QT* krow = reinterpret_cast<const QT*>(a.k_new) + ((size_t)b * a.num_kv_heads + kvr) * 128;
-    const QT* vrow = reinterpret_cast<const QT*>(a.v_new) + ((size_t)b * a.num_kv_heads + kvr) * 128;
+    const QT* qrow = reinterpret_cast<const QT*>(a.q) + ((size_t)b * a.num_qo_heads + hq) * D;
+    const QT* krow = reinterpret_cast<const QT*>(a.k_new) + ((size_t)b * a.num_kv_heads + kvr) * D;
+    const QT* vrow = reinterpret_cast<const QT*>(a.v_new) + ((size_t)b * a.num_kv_heads + kvr) * D;
     float q_own[4], q_par[4], k_own[4], k_par[4], v_in[4];
     load4_f32(qrow + d0, q_own);
     load4_f32(qrow + dp, q_par);
@@ -944,7 +962,7 @@ __global__ __launch_bounds__(32 * HB * S) void decode_step_finish_kernel(const M
             const bool live = j0 + k < u.count;
             const size_t slot = (size_t)(u.first_piece + (live ? j0 + k : 0));
             li[k] = live ? a.part_lse[slot * 16 + g] : -INFINITY;
-            oi[k] = *reinterpret_cast<const float4*>(a.part_o + (slot * 16 + g) * 128 + d0);
+            oi[k] = *reinterpret_cast<const float4*>(a.part_o + (slot * 16 + g) * D + d0);
         }
     };
     float li0[NB];
@@ -952,7 +970,7 @@ __global__ __launch_bounds__(32 * HB * S) void decode_step_finish_kernel(const M
     load_batch(NB * (int)sl, li0, oi0);
     asm("" : "+v"(freq2.x), "+v"(freq2.y)); // (asked for at the top, kept in their registers: not fetched again where used)
 
-    OT* orow = reinterpret_cast<OT*>(a.out) + ((size_t)b * a.num_qo_heads + hq) * 128;
+    OT* orow = reinterpret_cast<OT*>(a.out) + ((size_t)b * a.num_qo_heads + hq) * D;
     if (seq_len <= 0) { // no token at present: nothing to append, a zero row
         const OT z[4] = {StoreCvt<OT>::from(0.f), StoreCvt<OT>::from(0.f), StoreCvt<OT>::from(0.f), StoreCvt<OT>::from(0.f)};
         if (sl == 0 && head_live) store4(orow + d0, z);
@@ -974,7 +992,7 @@ __global__ __launch_bounds__(32 * HB * S) void decode_step_finish_kernel(const M
             const int src = (int)(i0 >> 1); // the lane of this head that holds pairs i0 and i0 + 1; the next one i0 + 2, i0 + 3
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
-                const float sn = __shfl(sn2[e & 1], src + (e >> 1), 32), cs = __shfl(cs2[e & 1], src + (e >> 1), 32);
+                const float sn = __shfl(sn2[e & 1], src + (e >> 1), LPH), cs = __shfl(cs2[e & 1], src + (e >> 1), LPH);
                 float xr, yr;
                 rope_pair(upper ? q_par[e] : q_own[e], upper ? q_own[e] : q_par[e], cs, sn, xr, yr);
                 qd[e] = upper ? yr : xr;
@@ -999,7 +1017,7 @@ __global__ __launch_bounds__(32 * HB * S) void decode_step_finish_kernel(const M
             store4(reinterpret_cast<PT*>(a.v_data) + off, v_st);
         }
 #pragma unroll
-        for (int o = 16; o > 0; o >>= 1) dot += __shfl_xor(dot, o, 64); // over the 32 lanes of the head
+        for (int o = LPH / 2; o > 0; o >>= 1) dot += __shfl_xor(dot, o, 64); // over the lanes of the head
         s_new = dot * a.sm_scale_log2 * ksc;
     }
 
@@ -1033,8 +1051,8 @@ __global__ __launch_bounds__(32 * HB * S) void decode_step_finish_kernel(const M
         merge_batch(li, oi);
     }
     if constexpr (S > 1) {
-        __shared__ float sm_m[S][HB][32], sm_w[S][HB][32];
-        __shared__ float4 sm_o[S][HB][32];
+        __shared__ float sm_m[S][HB][LPH], sm_w[S][HB][LPH];
+        __shared__ float4 sm_o[S][HB][LPH];
         sm_m[sl][hl][t] = M;
         sm_w[sl][hl][t] = wsum;
         sm_o[sl][hl][t] = make_float4(o[0], o[1], o[2], o[3]);
@@ -1073,45 +1091,45 @@ __global__ __launch_bounds__(32 * HB * S) void decode_step_finish_kernel(const M
 
 struct DecodeArgs; // general-kernel argument block (bz_decode.hip); only its scalar fields are forwarded here
 
-template <bool BF16, typename OT, bool ROPE_Q, bool KV8>
+template <bool BF16, typename OT, bool ROPE_Q, bool KV8, int D>
 static void launch_mfma_k(const DecodePlan* p, const MfmaDecodeArgs& a, hipStream_t s) {
     if (p->mfma_streaming)
-        hipLaunchKernelGGL((decode_mfma_kernel<BF16, OT, ROPE_Q, KV8, true>), dim3(p->mfma_slots), dim3(64), 0, s, a.heads, a,
+        hipLaunchKernelGGL((decode_mfma_kernel<BF16, OT, ROPE_Q, KV8, true, D>), dim3(p->mfma_slots), dim3(64), 0, s, a.heads, a,
                            (const char*)a.q, a.k_data, a.v_data, a.indices, a.pieces, a.tiles, a.k_scale,
                            a.v_scale);
     else
-        hipLaunchKernelGGL((decode_mfma_kernel<BF16, OT, ROPE_Q, KV8, false>), dim3(p->mfma_slots), dim3(64), 0, s, a.heads, a,
+        hipLaunchKernelGGL((decode_mfma_kernel<BF16, OT, ROPE_Q, KV8, false, D>), dim3(p->mfma_slots), dim3(64), 0, s, a.heads, a,
                            (const char*)a.q, a.k_data, a.v_data, a.indices, a.pieces, a.tiles, a.k_scale,
                            a.v_scale);
 }
 
-template <bool BF16, typename OT>
-static int launch_mfma(const DecodePlan* p, const MfmaDecodeArgs& a, bool kv8, hipStream_t s) {
+template <bool BF16, typename OT, bool KV8, int D>
+static int launch_mfma(const DecodePlan* p, const MfmaDecodeArgs& a, hipStream_t s) {
     if (p->time_start) BZ_CHECK_HIP(hipEventRecord(p->time_start, s));
-    if (kv8) {
-        if (a.rope_q) launch_mfma_k<BF16, OT, true, true>(p, a, s);
-        else launch_mfma_k<BF16, OT, false, true>(p, a, s);
-    } else {
-        if (a.rope_q) launch_mfma_k<BF16, OT, true, false>(p, a, s);
-        else launch_mfma_k<BF16, OT, false, false>(p, a, s);
-    }
+    if (a.rope_q) launch_mfma_k<BF16, OT, true, KV8, D>(p, a, s);
+    else launch_mfma_k<BF16, OT, false, KV8, D>(p, a, s);
     BZ_LAUNCH_CHECK();
     if (p->time_stop) BZ_CHECK_HIP(hipEventRecord(p->time_stop, s));
     if (a.step_mode) return 0; // the finishing kernel of the one-call step folds the partials
     if (p->mfma_combos > 0) {
         const dim3 cgrid(p->mfma_combos, a.group);
         if (p->mfma_max_count <= 16)
-            hipLaunchKernelGGL((decode_mfma_combine_kernel<OT, 1>), cgrid, dim3(128, 1), 0, s, p->mfma_combos_d,
+            hipLaunchKernelGGL((decode_mfma_combine_kernel<OT, 1, D>), cgrid, dim3(D, 1), 0, s, p->mfma_combos_d,
                                a.part_o, a.part_lse, a.out, a.lse, a.num_qo_heads, a.group);
         else if (p->mfma_max_count <= 64)
-            hipLaunchKernelGGL((decode_mfma_combine_kernel<OT, 4>), cgrid, dim3(128, 4), 0, s, p->mfma_combos_d,
+            hipLaunchKernelGGL((decode_mfma_combine_kernel<OT, 4, D>), cgrid, dim3(D, 4), 0, s, p->mfma_combos_d,
                                a.part_o, a.part_lse, a.out, a.lse, a.num_qo_heads, a.group);
         else
-            hipLaunchKernelGGL((decode_mfma_combine_kernel<OT, 8>), cgrid, dim3(128, 8), 0, s, p->mfma_combos_d,
+            hipLaunchKernelGGL((decode_mfma_combine_kernel<OT, 8, D>), cgrid, dim3(D, 8), 0, s, p->mfma_combos_d,
                                a.part_o, a.part_lse, a.out, a.lse, a.num_qo_heads, a.group);
         BZ_LAUNCH_CHECK();
     }
     return 0;
+}
+template <bool BF16, typename OT>
+static int launch_mfma_any(const DecodePlan* p, const MfmaDecodeArgs& a, bool kv8, hipStream_t s) {
+    if (p->head_dim == 64) return launch_mfma<BF16, OT, false, 64>(p, a, s);
+    return kv8 ? launch_mfma<BF16, OT, true, 128>(p, a, s) : launch_mfma<BF16, OT, false, 128>(p, a, s);
 }
 
 int decode_fast_path(const DecodePlan* p, const void* q, void* out, float* lse, int q_dtype, int out_dtype,
@@ -1122,6 +1140,7 @@ int decode_fast_path(const DecodePlan* p, const void* q, void* out, float* lse, 
     const bool kv8 = kv->kv_dtype == BZ_E4M3;
     if ((!kv8 && kv->kv_dtype != q_dtype) || rope_mode == BZ_ROPE_FULL) return BZ_ERR_UNSUPPORTED;
     if (!kv8 && (k_scale || v_scale)) return BZ_ERR_UNSUPPORTED;
+    if (kv8 && p->head_dim != 128) return BZ_ERR_UNSUPPORTED;
     const uint64_t es = kv8 ? 1 : 2;
     if ((kv->stride_n * es) % 16 || (kv->stride_h * es) % 16 || (kv->stride_page * es) % 16) return BZ_ERR_UNSUPPORTED;
     if (((uintptr_t)kv->k_data | (uintptr_t)kv->v_data | (uintptr_t)q | (uintptr_t)out) % 16) return BZ_ERR_UNSUPPORTED;
@@ -1141,30 +1160,30 @@ int decode_fast_path(const DecodePlan* p, const void* q, void* out, float* lse, 
     a.k_scale = k_scale; a.v_scale = v_scale;
     a.freqs = freqs;
     if (q_dtype == BZ_BF16)
-        return out_dtype == BZ_F32 ? launch_mfma<true, float>(p, a, kv8, s) : launch_mfma<true, bf16_t>(p, a, kv8, s);
-    return out_dtype == BZ_F32 ? launch_mfma<false, float>(p, a, kv8, s) : launch_mfma<false, f16_t>(p, a, kv8, s);
+        return out_dtype == BZ_F32 ? launch_mfma_any<true, float>(p, a, kv8, s) : launch_mfma_any<true, bf16_t>(p, a, kv8, s);
+    return out_dtype == BZ_F32 ? launch_mfma_any<false, float>(p, a, kv8, s) : launch_mfma_any<false, f16_t>(p, a, kv8, s);
 }
 
-template <typename QT, typename PT, typename OT>
+template <typename QT, typename PT, typename OT, int D>
 static int launch_step_finish(const DecodePlan* p, const StepFinishArgs& a, hipStream_t s) {
     // heads of a unit per workgroup: 4 where the group allows it (two waves), else 2 (one wave), 1 for single heads
     const uint32_t G = a.group;
     if (p->mfma_unit_max_count <= 16) { // what large batches produce
         if (G >= 4)
-            hipLaunchKernelGGL((decode_step_finish_kernel<QT, PT, OT, 1, 4>), dim3(p->mfma_units, (G + 3) / 4), dim3(32, 4, 1), 0, s, a.units, a.steps_ahead, a);
+            hipLaunchKernelGGL((decode_step_finish_kernel<QT, PT, OT, 1, 4, D>), dim3(p->mfma_units, (G + 3) / 4), dim3(D / 4, 4, 1), 0, s, a.units, a.steps_ahead, a);
         else if (G >= 2)
-            hipLaunchKernelGGL((decode_step_finish_kernel<QT, PT, OT, 1, 2>), dim3(p->mfma_units, (G + 1) / 2), dim3(32, 2, 1), 0, s, a.units, a.steps_ahead, a);
+            hipLaunchKernelGGL((decode_step_finish_kernel<QT, PT, OT, 1, 2, D>), dim3(p->mfma_units, (G + 1) / 2), dim3(D / 4, 2, 1), 0, s, a.units, a.steps_ahead, a);
         else
-            hipLaunchKernelGGL((decode_step_finish_kernel<QT, PT, OT, 1, 1>), dim3(p->mfma_units, G), dim3(32, 1, 1), 0, s, a.units, a.steps_ahead, a);
+            hipLaunchKernelGGL((decode_step_finish_kernel<QT, PT, OT, 1, 1, D>), dim3(p->mfma_units, G), dim3(D / 4, 1, 1), 0, s, a.units, a.steps_ahead, a);
     } else if (p->mfma_unit_max_count > 32 && p->mfma_unit_max_count <= 64) {
-        hipLaunchKernelGGL((decode_step_finish_kernel<QT, PT, OT, 4, 2>), dim3(p->mfma_units, (G + 1) / 2), dim3(32, 2, 4), 0, s, a.units, a.steps_ahead, a);
+        hipLaunchKernelGGL((decode_step_finish_kernel<QT, PT, OT, 4, 2, D>), dim3(p->mfma_units, (G + 1) / 2), dim3(D / 4, 2, 4), 0, s, a.units, a.steps_ahead, a);
     } else {
         // 17..32 partials (batches of eight sequences or so): eight slices, so one batch of four per slice and a single
         // round of loads, and one head per workgroup -- four waves.  Measured on 32 layers at batch 8: 497 us per step
         // against 505 with two heads per workgroup (eight waves), 527 with four (sixteen), 507 with four slices of two
         // heads.  More than 64 partials (a few very long sequences): the same shape (4 x 32 768 tokens: 90.8 against
         // 91.8 us with two heads).
-        hipLaunchKernelGGL((decode_step_finish_kernel<QT, PT, OT, 8, 1>), dim3(p->mfma_units, G), dim3(32, 1, 8), 0, s, a.units, a.steps_ahead, a);
+        hipLaunchKernelGGL((decode_step_finish_kernel<QT, PT, OT, 8, 1, D>), dim3(p->mfma_units, G), dim3(D / 4, 1, 8), 0, s, a.units, a.steps_ahead, a);
     }
     BZ_LAUNCH_CHECK();
     return 0;
@@ -1172,7 +1191,8 @@ static int launch_step_finish(const DecodePlan* p, const StepFinishArgs& a, hipS
 
 template <typename QT, typename OT>
 static int launch_step_finish_kv(const DecodePlan* p, const StepFinishArgs& a, bool kv8, hipStream_t s) {
-    return kv8 ? launch_step_finish<QT, e4m3_t, OT>(p, a, s) : launch_step_finish<QT, QT, OT>(p, a, s);
+    if (p->head_dim == 64) return launch_step_finish<QT, QT, OT, 64>(p, a, s);
+    return kv8 ? launch_step_finish<QT, e4m3_t, OT, 128>(p, a, s) : launch_step_finish<QT, QT, OT, 128>(p, a, s);
 }
 
 // The one-call decode step on the matrix-core kernel: BZ_ERR_UNSUPPORTED when the shape, the plan or the
@@ -1183,7 +1203,7 @@ int decode_step_fast_path(const DecodePlan* p, const void* q, const void* k_new,
                           const float* v_scale, hipStream_t s) {
     if (!p->mfma_ok || p->mfma_slots == 0 || !p->mfma_units_d || p->mfma_units == 0) return BZ_ERR_UNSUPPORTED;
     // one partial per piece, in the float workspace the plan was given
-    const size_t part_o_bytes = ((size_t)p->mfma_pieces * 16 * 128 * sizeof(float) + 255) / 256 * 256;
+    const size_t part_o_bytes = ((size_t)p->mfma_pieces * 16 * p->head_dim * sizeof(float) + 255) / 256 * 256;
     const size_t part_lse_bytes = ((size_t)p->mfma_pieces * 16 * sizeof(float) + 255) / 256 * 256;
     if (part_o_bytes + part_lse_bytes > p->float_buffer_bytes) return BZ_ERR_UNSUPPORTED;
     float* part_o = p->mfma_part_o;

@@ -57,10 +57,12 @@ struct ScheduleLayout {
     size_t unit_bytes, step_part_o_bytes, step_part_lse_bytes; // one-call decode step: unit list, one partial per piece
 };
 
-// Pure host work: fills the plan's host scratch (h_*) from the host copies of the page table.
+// Pure host work: fills the plan's host scratch (h_*) from the host copies of the page table.  small_heads: heads of 64 get
+// the matrix-core schedule as well -- a plan() for them takes it where the buffers have room for it, the sizes reported
+// beforehand are those of the general kernel's schedule, which is all that such a call needs.
 static int build_schedule(DecodePlan* p, const int32_t* indptr_h, const int32_t* last_page_len_h, uint32_t batch_size,
                           uint32_t num_qo_heads, uint32_t num_kv_heads, uint32_t head_dim, uint32_t page_size,
-                          uint32_t split_tokens, int cus, ScheduleCounts* counts) {
+                          uint32_t split_tokens, int cus, bool small_heads, ScheduleCounts* counts) {
     if (split_tokens == 0) split_tokens = 2048;
     // ---- choose the piece length (in pages) -------------------------------------------------
     // Pieces never exceed split_tokens (contexts longer than that are always split); they are
@@ -128,7 +130,7 @@ static int build_schedule(DecodePlan* p, const int32_t* indptr_h, const int32_t*
     const uint32_t group = num_qo_heads / num_kv_heads;
     uint32_t parts = (group + 15) / 16;
     while (parts < group && group % parts) ++parts;
-    const bool mfma_shape = head_dim == 128 && page_size % 16 == 0 && group / parts <= 16 && parts <= 8;
+    const bool mfma_shape = (head_dim == 128 || (head_dim == 64 && small_heads)) && page_size % 16 == 0 && group / parts <= 16 && parts <= 8;
     p->mfma_parts = mfma_shape ? parts : 1;
     const uint32_t num_units = num_kv_heads * (mfma_shape ? parts : 1); // kv heads as the matrix-core schedule sees them
     if (mfma_shape) {
@@ -258,10 +260,10 @@ static ScheduleLayout schedule_layout(const DecodePlan* p, const ScheduleCounts&
     L.mptr_bytes = align_up(L.nheads * sizeof(MfmaSlotHead), 256); // slot heads
     L.mc_bytes = align_up(p->h_mcombos.size() * sizeof(MfmaCombine), 256);
     L.cnt_bytes = align_up(p->h_tiles.size() * sizeof(MfmaTile), 256); // tile records
-    L.mpart_o_bytes = align_up((size_t)c.mfma_partials * 16 * 128 * sizeof(float), 256);
+    L.mpart_o_bytes = align_up((size_t)c.mfma_partials * 16 * head_dim * sizeof(float), 256);
     L.mpart_lse_bytes = align_up((size_t)c.mfma_partials * 16 * sizeof(float), 256);
     L.unit_bytes = align_up(p->h_units.size() * sizeof(MfmaUnit), 256);
-    L.step_part_o_bytes = align_up(p->h_pieces.size() * 16 * 128 * sizeof(float), 256);
+    L.step_part_o_bytes = align_up(p->h_pieces.size() * 16 * head_dim * sizeof(float), 256);
     L.step_part_lse_bytes = align_up(p->h_pieces.size() * 16 * sizeof(float), 256);
     return L;
 }
@@ -279,7 +281,7 @@ extern "C" int bz_decode_plan(bz_decode_plan_t* plan_, void* float_buffer, size_
     p->planned = false;
     ScheduleCounts counts;
     const int rc = build_schedule(p, indptr_h, last_page_len_h, batch_size, num_qo_heads, num_kv_heads, head_dim,
-                                  page_size, split_tokens, device_cu_count(), &counts);
+                                  page_size, split_tokens, device_cu_count(), true, &counts);
     if (rc) return rc;
     const std::vector<DecodeSegment>& segs = p->h_segs;
     const std::vector<DecodeCombine>& combos = p->h_combos;
@@ -402,7 +404,7 @@ extern "C" int bz_decode_plan(bz_decode_plan_t* plan_, void* float_buffer, size_
     // are whole (1024 sequences of 64 tokens: 63 us against 77 us).  The one call also needs room for one
     // partial per piece in the float workspace.
     {
-        const size_t part_o_bytes = ((size_t)p->mfma_pieces * 16 * 128 * sizeof(float) + 255) / 256 * 256;
+        const size_t part_o_bytes = ((size_t)p->mfma_pieces * 16 * head_dim * sizeof(float) + 255) / 256 * 256;
         const size_t part_lse_bytes = ((size_t)p->mfma_pieces * 16 * sizeof(float) + 255) / 256 * 256;
         const bool applies = p->mfma_ok && !p->force_general && p->mfma_slots > 0 && p->mfma_units_d &&
                              p->mfma_units > 0 && part_o_bytes + part_lse_bytes <= p->float_buffer_bytes;
@@ -427,7 +429,7 @@ extern "C" int bz_decode_plan_workspace(bz_decode_plan_t* plan_, const int32_t* 
     ScheduleCounts counts;
     const int cus = num_compute_units ? (int)num_compute_units : device_cu_count();
     const int rc = build_schedule(p, indptr_h, last_page_len_h, batch_size, num_qo_heads, num_kv_heads, head_dim,
-                                  page_size, split_tokens, cus, &counts);
+                                  page_size, split_tokens, cus, false, &counts);
     if (rc) return rc;
     const ScheduleLayout L = schedule_layout(p, counts, num_qo_heads, head_dim);
     const bool mfma = counts.mfma_shape && !p->h_pieces.empty();

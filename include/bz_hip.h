@@ -115,7 +115,9 @@ int bz_decode_plan(bz_decode_plan_t* plan, void* float_buffer, size_t float_buff
                    uint32_t page_size, uint32_t split_tokens, void* stream);
 /* Workspace sizing (no counterpart in the reference, which fixes 128 MiB + 8 MiB, src/model/llama.h:111-112):
  * runs the same host-side scheduling and reports how many bytes of the two workspaces bz_decode_plan would
- * use for this batch with the matrix-core kernel where the shape allows it.  Touches no GPU when
+ * use for this batch with the matrix-core kernel where the shape allows it (for heads of 64, what the general kernel
+ * would use: there the matrix-core kernel runs when both buffers have room left for its schedule and partials, as the
+ * reference's sizes do).  Touches no GPU when
  * num_compute_units is given (0 = ask the current device).  The handle must be planned again before the
  * next bz_batch_decode. */
 int bz_decode_plan_workspace(bz_decode_plan_t* plan, const int32_t* indptr_h, const int32_t* last_page_len_h,

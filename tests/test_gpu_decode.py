@@ -328,3 +328,35 @@ def test_rope_full_with_and_without_the_angle_table(Hq, Hkv, D):
     tight.plan(256)
     d = tight.decode(BZ_F32, BZ_ROPE_FULL, 5e5)
     assert np.abs(d - ref).max() <= 1e-4 and np.abs(d - a).max() <= 2e-6
+
+
+@pytest.mark.parametrize("dtype", [BZ_F16, BZ_BF16])
+@pytest.mark.parametrize("Hq,Hkv,P,layout", [(4, 4, 16, BZ_LAYOUT_HND), (8, 2, 64, BZ_LAYOUT_NHD), (12, 2, 48, BZ_LAYOUT_NHD),
+                                             (32, 1, 16, BZ_LAYOUT_HND)])
+def test_heads_of_64_on_the_matrix_core_kernel(dtype, Hq, Hkv, P, layout):
+    """16-bit pools with heads of 64: two tiles in flight, slots of one, two and an odd number of tiles, whole and split
+    sequences, ends inside and at a tile; against the checker at the fp32 bar and against the general kernel, as a call
+    and as the one-call step (groups of 1, 4, 6 and, in two parts, 32)."""
+    from test_gpu_decode_step import run_step
+    ctx = [1, 31, 32, 33, 64, 65, 1000, 0, 2049, 4096 + 17]
+    p = DecodeProblem(640 + Hq, ctx, Hq, Hkv, 64, P, dtype, layout=layout)
+    dev = DeviceDecode(p)
+    outs = {}
+    for path in ("", "general"):
+        if path:
+            os.environ["BZ_DECODE_PATH"] = path
+        try:
+            dev.plan(1024)
+        finally:
+            os.environ.pop("BZ_DECODE_PATH", None)
+        assert len(dev.handler.host_schedule(5)) > 0  # pieces: the schedule is there
+        outs[path] = [dev.decode(BZ_F32, mode, 1e4, want_lse=True) for mode in (BZ_ROPE_NONE, BZ_ROPE_Q_ONLY)]
+    live = p.ctx > 0
+    for i, mode in enumerate((oracle.ROPE_NONE, oracle.ROPE_Q_ONLY)):
+        ref, ref_lse = oracle.batch_decode(p.q, dtype, p.oracle_kv(), Hq, rope_mode=mode, rope_theta=1e4, want_lse=True)
+        for got, lse in (outs[""][i], outs["general"][i]):
+            assert np.abs(got - ref).max() <= 2e-5 and np.abs(lse[live] - ref_lse[live]).max() < 1e-3
+            assert not got[~live].any()
+    for split in (0, 1024):
+        dev2, _, _ = run_step(p, split_tokens=split, theta=1e4, expect_units=False)
+        assert dev2.form == "one_call"
