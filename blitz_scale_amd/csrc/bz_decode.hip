@@ -84,7 +84,12 @@ template <int N> __device__ __forceinline__ float row_sum(float v) {
 }
 
 // TABLE: BZ_ROPE_FULL with the angles of the cached K rows taken from a.rope_table (an instantiation of its own,
-// so that the registers the table rows travel through do not cost the other modes their occupancy).
+// so that the registers the table rows travel through do not cost the other modes their occupancy).  A lane then holds
+// four elements of the lower half of a K row and the four that they are rotated with (two loads of 8 bytes), so that the
+// rotation needs no exchange between lanes and 32 bytes of angles per lane and token, and the angles of the next set of
+// tokens are asked for behind that set's K and V and in front of the set after it: loads return in order, and angles asked
+// for behind the set after it wait for it to arrive.  48 sequences of 200 .. 2048 tokens, 32/8 heads, bf16, the whole call with
+// append and combine: 117.5 -> 71.1 us (64/8 heads, whose lanes had no registers for the wider rows of angles: 315 -> 97 us).
 template <typename QT, typename KVT, typename OT, int D, int G, bool TABLE = false>
 __global__ __launch_bounds__(256) void decode_general_kernel(DecodeArgs a) {
     using Geo = RowGeom<KVT, D>;
@@ -107,16 +112,53 @@ __global__ __launch_bounds__(256) void decode_general_kernel(DecodeArgs a) {
     const int tok_begin = seg.page_begin * (int)a.page_size;
     const int tok_end = min(seg.page_end * (int)a.page_size, seq_len);
 
+    // (a.rope_table: D/2 pairs of 8 bytes = D/4 float4 per position, two of them this lane's.  A sequence cannot be longer
+    // than its planned pages hold, which the table covers; the bound keeps the read inside the table whatever the
+    // device-side lengths say.)
+    auto table_row = [&](int pos, float4 (&cs)[2]) __attribute__((always_inline)) {
+        const float4* row = reinterpret_cast<const float4*>(a.rope_table) +
+                            (size_t)max(min(pos, a.rope_positions - 1), 0) * (D / 4) + lane_in_row * 2;
+        cs[0] = row[0];
+        cs[1] = row[1];
+    };
+    auto rotate = [&](float (&x)[8], const float4 (&cs)[2]) __attribute__((always_inline)) { // elements e and e + 4 are a pair
+        const float c[4] = {cs[0].x, cs[0].z, cs[1].x, cs[1].z}, sn[4] = {cs[0].y, cs[0].w, cs[1].y, cs[1].w};
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            float lo_r, hi_r;
+            rope_pair(x[e], x[e + 4], c[e], sn[e], lo_r, hi_r);
+            x[e] = lo_r;
+            x[e + 4] = hi_r;
+        }
+    };
+    // TABLE: four elements of each half of a row
+    auto load_halves = [&](auto& v, const auto* row, auto nt_c) __attribute__((always_inline)) {
+        typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
+        const u32x2 *lo = reinterpret_cast<const u32x2*>(row + lane_in_row * 4), *hi = reinterpret_cast<const u32x2*>(row + D / 2 + lane_in_row * 4);
+        if constexpr (decltype(nt_c)::value) {
+            const u32x2 l = __builtin_nontemporal_load(lo), h = __builtin_nontemporal_load(hi);
+            v.raw = make_uint4(l.x, l.y, h.x, h.y);
+        } else {
+            v.raw = make_uint4(lo->x, lo->y, hi->x, hi->y);
+        }
+    };
+
     // ---- q for the G heads of this kv head, as fp32, pre-rotated if asked ----
     float q[G][8];
 #pragma unroll
     for (int g = 0; g < G; ++g) {
-        const size_t qoff = ((size_t)b * a.num_qo_heads + (size_t)unit * G + g) * D + lane_in_row * 8;
+        const QT* row = reinterpret_cast<const QT*>(a.q) + ((size_t)b * a.num_qo_heads + (size_t)unit * G + g) * D;
         Vec8<QT> qv;
-        qv.load(reinterpret_cast<const QT*>(a.q) + qoff);
+        if constexpr (TABLE) load_halves(qv, row, std::false_type{});
+        else qv.load(row + lane_in_row * 8);
         qv.to_float(q[g]);
     }
-    if (a.rope_mode != BZ_ROPE_NONE) {
+    if constexpr (TABLE) {
+        float4 cs[2];
+        table_row(seq_len - 1, cs);
+#pragma unroll
+        for (int g = 0; g < G; ++g) rotate(q[g], cs);
+    } else if (a.rope_mode != BZ_ROPE_NONE) {
         // partner slice holds the other half of each rotate-half pair
         const bool upper = lane_in_row >= LANES / 2;
         const float pos = (float)(seq_len - 1);
@@ -146,16 +188,7 @@ __global__ __launch_bounds__(256) void decode_general_kernel(DecodeArgs a) {
     }
 
     const size_t esz = sizeof(KVT);
-    const size_t head_off = ((size_t)kvh * a.stride_h + (size_t)lane_in_row * 8) * esz;
-
-    // BZ_ROPE_FULL rotates every cached K row at its own position.  Evaluating sincosf per element makes the
-    // kernel compute-bound several times over, so the angles come from a table when the plan has room for one
-    // (64 bytes per lane and token, fetched TU tokens ahead; the groups of eight q heads have no registers left
-    // for that and keep the on-the-fly evaluation).
-    constexpr int TU = G <= 2 ? 4 : 2;
-    static_assert(!TABLE || G <= 4, "no registers for the table rows beside eight q heads");
-    constexpr bool table_rope = TABLE;
-    const float4* cs_lane = reinterpret_cast<const float4*>(a.rope_table) + (lane_in_row % (LANES / 2)) * 4;
+    const size_t head_off = (size_t)kvh * a.stride_h * esz, lane_off = (size_t)lane_in_row * 8 * esz;
 
     // Two register sets of UNROLL tokens per lane slot take turns: the loads of the next set go out before the
     // arithmetic of the present one.  They are issued whether or not the set has a live token (addresses are
@@ -167,64 +200,80 @@ __global__ __launch_bounds__(256) void decode_general_kernel(DecodeArgs a) {
         bool valid[UNROLL];
         int jj[UNROLL];
     };
-    auto issue = [&](int base, TokSet& S) __attribute__((always_inline)) {
+    // A wave's rows of one pass are kTokPerWave neighbouring tokens, and where pages hold a multiple of that they lie in
+    // one page (segments begin on pages): its id is a scalar load, fetched a set ahead.  As a vector load it would queue
+    // behind the K and V of the set in flight, and this set's loads would go out only when those have arrived (8-token pages
+    // without rotation, 48 such sequences: 86.5 -> 83.0 us; with it the larger part of the gain above).
+    constexpr int WTOK = Geo::kTokPerWave;
+    const int wave_slot = __builtin_amdgcn_readfirstlane(tid / 64) * WTOK;
+    int next_page[UNROLL], next_first[UNROLL]; // the next set's page ids, and the first tokens of the pages
+    auto fetch_pages = [&](int base, auto one_page) __attribute__((always_inline)) {
+        if constexpr (!decltype(one_page)::value) return;
 #pragma unroll
         for (int u = 0; u < UNROLL; ++u) {
-            const int j = base + u * TOK + slot;
-            S.jj[u] = j;
-            S.valid[u] = j < tok_end;
-            const int jc = S.valid[u] ? j : tok_begin; // any in-range token: keeps the load legal
-            const int64_t page = a.indices[ip0 + jc / (int)a.page_size];
-            const size_t off =
-                ((size_t)page * a.stride_page + (size_t)(jc % (int)a.page_size) * a.stride_n) * esz + head_off;
-            S.kv[u].load_nt(a.k_data + off); // read once per launch (+2 to 3 % over plain loads)
-            S.vv[u].load_nt(a.v_data + off);
+            const int j0 = base + u * TOK + wave_slot;
+            const int pg = (j0 < tok_end ? j0 : tok_begin) / (int)a.page_size;
+            next_first[u] = pg * (int)a.page_size;
+            next_page[u] = a.indices[ip0 + pg];
         }
     };
-    auto compute = [&](TokSet& S) __attribute__((always_inline)) {
+    auto issue = [&](int base, TokSet& S, auto one_page) __attribute__((always_inline)) {
+        constexpr bool ONE = decltype(one_page)::value;
+#pragma unroll
+        for (int u = 0; u < UNROLL; ++u) {
+            const int j = base + u * TOK + slot, j0 = base + u * TOK + wave_slot;
+            S.jj[u] = j;
+            S.valid[u] = j < tok_end;
+            // (any live token of the segment keeps the load legal and its values finite)
+            const int jc = S.valid[u] ? j : (ONE && j0 < tok_end ? j0 : tok_begin);
+            int64_t page;
+            int in_page;
+            if constexpr (ONE) {
+                page = next_page[u];
+                in_page = jc - next_first[u];
+            } else {
+                page = a.indices[ip0 + jc / (int)a.page_size];
+                in_page = jc % (int)a.page_size;
+            }
+            const size_t off = ((size_t)page * a.stride_page + (size_t)in_page * a.stride_n) * esz + head_off;
+            // (read once per launch: +2 to 3 % over plain loads)
+            if constexpr (TABLE) load_halves(S.kv[u], reinterpret_cast<const KVT*>(a.k_data + off), std::true_type{});
+            else S.kv[u].load_nt(a.k_data + off + lane_off);
+            S.vv[u].load_nt(a.v_data + off + lane_off);
+        }
+        fetch_pages(base + TOK * UNROLL, one_page);
+    };
+    float4 cs[TABLE ? UNROLL : 1][2]; // angles of this lane's four pairs at the positions of one set's tokens
+    auto fetch_cs = [&](TokSet& S) __attribute__((always_inline)) {
+        if constexpr (TABLE) {
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int u = 0; u < UNROLL; ++u) table_row(S.valid[u] ? S.jj[u] : tok_begin, cs[u]);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+    float sc_tok[UNROLL][G];
+    auto scores = [&](TokSet& S) __attribute__((always_inline)) {
         Vec8<KVT>(&kv)[UNROLL] = S.kv;
-        Vec8<KVT>(&vv)[UNROLL] = S.vv;
         bool(&valid)[UNROLL] = S.valid;
         int(&jj)[UNROLL] = S.jj;
-        float4 cs[TABLE ? TU : 1][4]; // (cos, sin) of this lane's eight pairs at the positions of TU tokens
-        auto fetch_cs = [&](int u) {
-            // (a sequence cannot be longer than its planned pages hold, which the table covers; the bound keeps the
-            // read inside the table whatever the device-side lengths say)
-            const int jc = min(valid[u] ? jj[u] : tok_begin, a.rope_positions - 1);
-            const float4* row = cs_lane + (size_t)jc * (D / 4); // D/2 pairs of 8 bytes = D/4 float4 per position
-#pragma unroll
-            for (int i = 0; i < 4; ++i) cs[u % TU][i] = row[i];
-        };
-        if constexpr (TABLE) {
-#pragma unroll
-            for (int u = 0; u < TU; ++u) fetch_cs(u);
-        }
         // Scores of the UNROLL tokens first (a token's row is spread over LANES lanes: products, then a sum across
         // the lanes of the row with DPP row rotations), then one softmax update per q head for all of them: one
         // maximum, one rescale of the accumulators per batch instead of per token, raw v_exp_f32.
-        float sc_tok[UNROLL][G];
 #pragma unroll
         for (int u = 0; u < UNROLL; ++u) {
             float kf[8];
             kv[u].to_float(kf);
-            if (a.rope_mode == BZ_ROPE_FULL) {
+            if constexpr (TABLE) {
+                rotate(kf, cs[u]);
+            } else if (a.rope_mode == BZ_ROPE_FULL) { // (no table: angles evaluated per element, several times the other work)
                 const bool upper = lane_in_row >= LANES / 2;
-                float cv[8], sv[8];
-                if constexpr (TABLE) {
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) {
-                        const float4 t = cs[u % TU][i];
-                        cv[2 * i] = t.x; sv[2 * i] = t.y; cv[2 * i + 1] = t.z; sv[2 * i + 1] = t.w;
-                    }
-                    if (u + TU < UNROLL) fetch_cs(u + TU);
-                }
 #pragma unroll
                 for (int e = 0; e < 8; ++e) {
                     const float other = __shfl_xor(kf[e], LANES / 2, 64);
                     const int fi = (lane_in_row % (LANES / 2)) * 8 + e;
                     float s, c;
-                    if constexpr (TABLE) { c = cv[e]; s = sv[e]; }
-                    else sincosf((float)jj[u] * a.freqs.f[fi], &s, &c);
+                    sincosf((float)jj[u] * a.freqs.f[fi], &s, &c);
                     float lo_r, hi_r;
                     rope_pair(upper ? other : kf[e], upper ? kf[e] : other, c, s, lo_r, hi_r);
                     kf[e] = upper ? hi_r : lo_r;
@@ -239,9 +288,11 @@ __global__ __launch_bounds__(256) void decode_general_kernel(DecodeArgs a) {
                 sc_tok[u][g] = valid[u] ? s * kscale : -INFINITY;
             }
         }
+    };
+    auto accumulate = [&](TokSet& S) __attribute__((always_inline)) {
         float vf[UNROLL][8];
 #pragma unroll
-        for (int u = 0; u < UNROLL; ++u) vv[u].to_float(vf[u]);
+        for (int u = 0; u < UNROLL; ++u) S.vv[u].to_float(vf[u]);
 #pragma unroll
         for (int g = 0; g < G; ++g) {
             float mx = m[g];
@@ -267,22 +318,38 @@ __global__ __launch_bounds__(256) void decode_general_kernel(DecodeArgs a) {
         }
     };
     constexpr int STEP = TOK * UNROLL;
-    if constexpr (G >= 2) {
-        TokSet A, B;
-        if (tok_begin < tok_end) issue(tok_begin, A);
-        for (int base = tok_begin; base < tok_end; base += 2 * STEP) {
-            issue(base + STEP, B);
-            compute(A);
-            issue(base + 2 * STEP, A);
-            if (base + STEP < tok_end) compute(B);
+    auto walk = [&](auto one_page) __attribute__((always_inline)) {
+        fetch_pages(tok_begin, one_page);
+        if constexpr (G >= 2) {
+            TokSet A, B;
+            if (tok_begin < tok_end) {
+                issue(tok_begin, A, one_page);
+                fetch_cs(A);
+            }
+            for (int base = tok_begin; base < tok_end; base += 2 * STEP) {
+                issue(base + STEP, B, one_page);
+                scores(A);
+                fetch_cs(B);
+                accumulate(A);
+                issue(base + 2 * STEP, A, one_page);
+                if (base + STEP < tok_end) {
+                    scores(B);
+                    fetch_cs(A);
+                    accumulate(B);
+                }
+            }
+        } else {
+            for (int base = tok_begin; base < tok_end; base += STEP) {
+                TokSet A;
+                issue(base, A, one_page);
+                fetch_cs(A);
+                scores(A);
+                accumulate(A);
+            }
         }
-    } else {
-        for (int base = tok_begin; base < tok_end; base += STEP) {
-            TokSet A;
-            issue(base, A);
-            compute(A);
-        }
-    }
+    };
+    if (a.page_size % WTOK == 0) walk(std::true_type{});
+    else walk(std::false_type{});
 
     // ---- merge the token slots: first inside the wave, then across the 4 waves through LDS ----
 #pragma unroll
@@ -379,11 +446,13 @@ __global__ void decode_zero_rows_kernel(const int32_t* empty_seqs, void* out, ui
 template <typename QT, typename KVT, typename OT, int D>
 static int launch_general_g(const DecodeArgs& a, int G, dim3 grid, hipStream_t s) {
     if constexpr (std::is_same<QT, KVT>::value) {
-        if (a.rope_mode == BZ_ROPE_FULL && a.rope_table && G <= 4) { // angles from the table
+        if (a.rope_mode == BZ_ROPE_FULL && a.rope_table) { // angles from the table
             switch (G) {
                 case 1: hipLaunchKernelGGL((decode_general_kernel<QT, KVT, OT, D, 1, true>), grid, dim3(256), 0, s, a); break;
                 case 2: hipLaunchKernelGGL((decode_general_kernel<QT, KVT, OT, D, 2, true>), grid, dim3(256), 0, s, a); break;
-                default: hipLaunchKernelGGL((decode_general_kernel<QT, KVT, OT, D, 4, true>), grid, dim3(256), 0, s, a); break;
+                case 4: hipLaunchKernelGGL((decode_general_kernel<QT, KVT, OT, D, 4, true>), grid, dim3(256), 0, s, a); break;
+                case 8: hipLaunchKernelGGL((decode_general_kernel<QT, KVT, OT, D, 8, true>), grid, dim3(256), 0, s, a); break;
+                default: return BZ_ERR_UNSUPPORTED;
             }
             BZ_LAUNCH_CHECK();
             return 0;

@@ -360,3 +360,13 @@ def test_heads_of_64_on_the_matrix_core_kernel(dtype, Hq, Hkv, P, layout):
     for split in (0, 1024):
         dev2, _, _ = run_step(p, split_tokens=split, theta=1e4, expect_units=False)
         assert dev2.form == "one_call"
+
+
+@pytest.mark.parametrize("D,P,Hq,Hkv", [(128, 16, 4, 4), (128, 2, 4, 2), (128, 4, 8, 2), (128, 3, 16, 2), (128, 64, 10, 2), (64, 8, 8, 1),
+                                        (64, 4, 4, 1), (64, 16, 3, 3)])
+@pytest.mark.parametrize("dtype", [BZ_F16, BZ_BF16])
+def test_raw_k_cache_with_angles_from_the_table(dtype, D, P, Hq, Hkv):
+    """BZ_ROPE_FULL in groups of 1, 2, 4, 5 and 8 heads over pages that a wave's rows of one pass share (and smaller ones,
+    that they do not), sequences that end inside a pass, split and whole, from one token on."""
+    p = DecodeProblem(660 + D + P, [1, 2, 3, 15, 16, 17, 63, 64, 65, 0, 500, 1031], Hq, Hkv, D, P, dtype)
+    check(p, split_tokens=256, rope_mode=BZ_ROPE_FULL)
