@@ -319,7 +319,7 @@ __global__ __launch_bounds__(256) void decode_general_kernel(DecodeArgs a) {
     };
     constexpr int STEP = TOK * UNROLL;
     auto walk = [&](auto one_page) __attribute__((always_inline)) {
-        fetch_pages(tok_begin, one_page);
+        if (tok_begin < tok_end) fetch_pages(tok_begin, one_page); // (no token on the device: no page entry is read)
         if constexpr (G >= 2) {
             TokSet A, B;
             if (tok_begin < tok_end) {
