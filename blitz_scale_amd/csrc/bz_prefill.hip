@@ -262,6 +262,12 @@ __device__ __forceinline__ void sp_wait_copies(int tiles) {
     }
     __builtin_amdgcn_sched_barrier(0);
 }
+// wait until at most BEHIND of this wave's LDS instructions are still in flight (they complete in order)
+template <int BEHIND> __device__ __forceinline__ void sp_wait_lds() {
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_waitcnt(0xC07F | (BEHIND << 8)); // lgkmcnt(BEHIND)
+    __builtin_amdgcn_sched_barrier(0);
+}
 // Copies are issued in pairs (K(i + kSNK), V(i + kSNV - 1)) at the top of iteration i, the first kSNK pairs
 // (i = -kSNK .. -1, tiles below 0 left out) in the prologue.  The tiles first read in iteration j are K(j+2) and
 // V(j); with V_NEXT also V(j+1), which is then converted in place during iteration j.  This counts the copies that
@@ -514,18 +520,32 @@ __global__ __launch_bounds__(256, 2) void prefill_kernel(PrefillArgs a, const ch
         const uint2 w0 = __builtin_bit_cast(uint2, t0), w1 = __builtin_bit_cast(uint2, t1);
         dst = make_uint4(w0.x, w0.y, w1.x, w1.y);
     };
-    // V_F16: this wave's quarter of the V tile in `slot` (the rows it copied), bf16 -> f16 in place
+    // V_F16: this wave's quarter of the V tile in `slot` (the rows it copied), bf16 -> f16 in place, as three steps that the
+    // halves of an iteration take between their matrix instructions: two 16-byte reads, eight words converted, two writes.
+    // The writer waits for its writes (sp_wait_lds) in front of the barrier behind which the tile is read.
+    // In one piece in front of the first half, the reads' latency and the conversions stood where the wave has no matrix
+    // instruction in flight: 780 of 2 520 cycles per tile where both workgroups of a compute unit keep step.  Whole calls, us,
+    // before and now: three chunks of 269 .. 543 tokens behind 4 700 .. 16 000, 32/8 heads, 246.7 -> 224.3 (f16: 209.7); 1 x
+    // 8 192, 32/8 heads, page store included, 590 -> 556; 8 x 1 000 123.9 -> 115.9; 16 prompts of 128 .. 4 096, 40 heads,
+    // 1 116 -> 1 078 (f16: 1 028).  What is left of the difference to f16 is the widening's 16 KiB of LDS traffic per tile.
+    typedef pf_u32x4 __attribute__((address_space(3)))* lds_u32x4_ptr;
+    auto widen_at = [&](int slot, int i) __attribute__((always_inline)) {
+        return (lds_u32x4_ptr)((unsigned char __attribute__((address_space(3)))*)(uintptr_t)(m0_wave + (uint32_t)((kSNK + slot) * kSTile)) +
+                               lane * 16 + i * 1024);
+    };
+    pf_u32x4 wide[2];
+    auto widen_words = [&](int i, int w0, int count) __attribute__((always_inline)) {
+#pragma unroll
+        for (int w = w0; w < w0 + count; ++w)
+            wide[i][w] = PfMma<false>::pack2(__uint_as_float(wide[i][w] << 16), __uint_as_float(wide[i][w] & 0xffff0000u));
+    };
     auto widen_v = [&](int slot) __attribute__((always_inline)) {
-        typedef pf_u32x4 __attribute__((address_space(3)))* lds_u32x4_ptr;
-        unsigned char __attribute__((address_space(3)))* base =
-            (unsigned char __attribute__((address_space(3)))*)(uintptr_t)(m0_wave + (uint32_t)((kSNK + slot) * kSTile)) + lane * 16;
+#pragma unroll
+        for (int i = 0; i < 2; ++i) wide[i] = *widen_at(slot, i);
 #pragma unroll
         for (int i = 0; i < 2; ++i) {
-            pf_u32x4 r = *(lds_u32x4_ptr)(base + i * 1024);
-#pragma unroll
-            for (int w = 0; w < 4; ++w)
-                r[w] = PfMma<false>::pack2(__uint_as_float(r[w] << 16), __uint_as_float(r[w] & 0xffff0000u));
-            *(lds_u32x4_ptr)(base + i * 1024) = r;
+            widen_words(i, 0, 4);
+            *widen_at(slot, i) = wide[i];
         }
     };
     auto k_at = [&](int slot) __attribute__((always_inline)) { return (uint32_t)(slot * kSTile); };
@@ -573,7 +593,8 @@ __global__ __launch_bounds__(256, 2) void prefill_kernel(PrefillArgs a, const ch
     // The first half of an iteration: scores of the next tile into s[PAR ^ 1] (QK) from K at k1 (steps 0..3 are in
     // the ring), probabilities of this tile from s[PAR] (EX), first V operands of this tile (at vj) into the ring.
     // The exponentials of step i are consumed in step i + 1 (their latency is longer than one instruction).
-    auto first_half = [&](auto par_c, auto qk_c, auto ex_c, uint32_t k1, uint32_t vj) __attribute__((always_inline)) {
+    // `wslot`: V_F16, the slot of the V tile whose widening starts here (negative: none).
+    auto first_half = [&](auto par_c, auto qk_c, auto ex_c, uint32_t k1, uint32_t vj, int wslot) __attribute__((always_inline)) {
         constexpr int PAR = decltype(par_c)::value;
         constexpr bool QK = decltype(qk_c)::value, EX = decltype(ex_c)::value;
         float e0 = 0.f, e1 = 0.f;
@@ -584,6 +605,7 @@ __global__ __launch_bounds__(256, 2) void prefill_kernel(PrefillArgs a, const ch
             if (QK) s[PAR ^ 1] = M::run(kring[i & 3], qreg[i], i == 0 ? cinit : s[PAR ^ 1]);
             if (i < 4) read_k(kring[i], k1, i + 4);
             else read_v(vring[i - 4], vj, i - 4);
+            if (V_F16 && (i == 4 || i == 5) && wslot >= 0) wide[i - 4] = *widen_at(wslot, i - 4);
             if (EX) {
                 const float n0 = exp_of(s[PAR][2 * i], 0.f), n1 = exp_of(s[PAR][2 * i + 1], 0.f);
                 if (i > 0) take_pair(e0, e1, i - 1);
@@ -596,8 +618,10 @@ __global__ __launch_bounds__(256, 2) void prefill_kernel(PrefillArgs a, const ch
         __builtin_amdgcn_sched_barrier(0);
     };
     // The second half: O += V^T P^T (PV), the rest of V (at vj) and the first K operands of the tile after the next
-    // (at k2) into the rings
-    auto second_half = [&](auto pv_c, uint32_t vj, uint32_t k2) __attribute__((always_inline)) {
+    // (at k2) into the rings.  V_F16: the widening ends here, in the shadow of the first six steps, whose matrix
+    // instructions have no vector work of their own beside them; behind its last write come kWidenBehind operand reads.
+    constexpr int kWidenBehind = 2;
+    auto second_half = [&](auto pv_c, uint32_t vj, uint32_t k2, int wslot) __attribute__((always_inline)) {
         constexpr bool PV = decltype(pv_c)::value;
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
@@ -608,6 +632,11 @@ __global__ __launch_bounds__(256, 2) void prefill_kernel(PrefillArgs a, const ch
             }
             if (i < 4) read_v(vring[i], vj, i + 4);
             else read_k(kring[i - 4], k2, i - 4);
+            if (V_F16 && i < 6 && wslot >= 0) {
+                if (i % 3 == 0) widen_words(i / 3, 0, 2);
+                else widen_words(i / 3, i % 3 + 1, 1);
+                if (i % 3 == 2) *widen_at(wslot, i / 3) = wide[i / 3];
+            }
             __builtin_amdgcn_sched_barrier(0);
         }
     };
@@ -664,7 +693,10 @@ __global__ __launch_bounds__(256, 2) void prefill_kernel(PrefillArgs a, const ch
         sp_barrier();
 #pragma unroll
         for (int i = 0; i < 4; ++i) read_k(kring[i], k_at(1 % kSNK), i);
-        if (V_F16) widen_v(0);
+        if (V_F16) {
+            widen_v(0);
+            sp_wait_lds<0>();
+        }
     }
     BZ_PF_WG(3);
 
@@ -677,6 +709,7 @@ __global__ __launch_bounds__(256, 2) void prefill_kernel(PrefillArgs a, const ch
         constexpr int PAR = decltype(par_c)::value, SL = decltype(sl_c)::value;
         BZ_PF_PH_START();
         sp_wait_copies(sp_copies_behind_steady(V_F16)); // K(j+2) and V(j) have landed (V_F16: V(j+1) too)
+        if (V_F16) sp_wait_lds<kWidenBehind>();         // V(j) is widened
         BZ_PF_PH(0);
         sp_barrier();
         BZ_PF_PH(1);
@@ -684,13 +717,13 @@ __global__ __launch_bounds__(256, 2) void prefill_kernel(PrefillArgs a, const ch
         lds_direct_load16x2(v_next, vfast[0], vfast[1], m0_wave + (uint32_t)((kSNK + (SL + kSNV - 1) % kSNV) * kSTile));
         k_next += tile_stride;
         v_next += tile_stride;
-        if (V_F16) widen_v((SL + 1) % kSNV); // V(j+1), first read after the next barrier
         BZ_PF_PH(2);
-        first_half(par_c, std::true_type{}, std::true_type{}, k_at((SL + 1) % kSNK), v_at(SL));
+        constexpr int WSLOT = V_F16 ? (SL + 1) % kSNV : -1; // V(j+1), first read after the next barrier
+        first_half(par_c, std::true_type{}, std::true_type{}, k_at((SL + 1) % kSNK), v_at(SL), WSLOT);
         BZ_PF_PH(3);
         if (__any(!(psum < 32768.0f))) move_maximum(s[PAR], s[PAR ^ 1]);
         l_run += psum;
-        second_half(std::true_type{}, v_at(SL), k_at((SL + 2) % kSNK));
+        second_half(std::true_type{}, v_at(SL), k_at((SL + 2) % kSNK), WSLOT);
         BZ_PF_PH(4);
     };
     // ---- the same with every condition checked (the slots are still compile-time constants: j % 4 == SL).  The operand
@@ -700,20 +733,22 @@ __global__ __launch_bounds__(256, 2) void prefill_kernel(PrefillArgs a, const ch
         constexpr int PAR = decltype(par_c)::value, SL = decltype(sl_c)::value;
         const bool has_cur = j < n_w, has_next = j + 1 < n_w;
         sp_wait_copies(sp_copies_behind(j, n, V_F16));
+        if (V_F16) sp_wait_lds<kWidenBehind>();
         sp_barrier();
         if (j + kSNK < n) issue_k(j + kSNK, SL);
         if (j + kSNV - 1 < n) issue_v(j + kSNV - 1, (SL + kSNV - 1) % kSNV);
-        if (V_F16 && j + 1 < n) widen_v((SL + 1) % kSNV);
+        // (V(j+1) is widened whether there is one or not: the slot is this wave's to write, what it holds then is read by nobody)
+        constexpr int WSLOT = V_F16 ? (SL + 1) % kSNV : -1;
         const uint32_t k1 = k_at((SL + 1) % kSNK), k2 = k_at((SL + 2) % kSNK);
-        if (has_next) first_half(par_c, std::true_type{}, std::true_type{}, k1, v_at(SL));
-        else first_half(par_c, std::false_type{}, std::true_type{}, k1, v_at(SL)); // (harmless without a tile: p of stale scores, never used)
+        if (has_next) first_half(par_c, std::true_type{}, std::true_type{}, k1, v_at(SL), WSLOT);
+        else first_half(par_c, std::false_type{}, std::true_type{}, k1, v_at(SL), WSLOT); // (harmless without a tile: p of stale scores, never used)
         if (has_cur) {
             if (__any(!(psum < 32768.0f))) move_maximum(s[PAR], s[PAR ^ 1]);
             l_run += psum;
             if (has_next) mask_tile(j + 1, s[PAR ^ 1]);
-            second_half(std::true_type{}, v_at(SL), k2);
+            second_half(std::true_type{}, v_at(SL), k2, WSLOT);
         } else {
-            second_half(std::false_type{}, v_at(SL), k2);
+            second_half(std::false_type{}, v_at(SL), k2, WSLOT);
         }
     };
     // full needs: tiles j .. j+2 computed by this wave, tile j+1 unmasked, and the tiles it copies whole and in range
