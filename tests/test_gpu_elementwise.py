@@ -81,3 +81,12 @@ def test_add_residual_bit_exact(dtype):
     torch.cuda.synchronize()
     assert np.array_equal(to_host_bits(bd), want)
     assert np.array_equal(to_host_bits(ad), a)
+
+
+def test_calls_go_to_the_current_stream():
+    """Without a stream argument a call goes to torch's current stream, whichever that is."""
+    side = torch.cuda.Stream()
+    assert K._stream(None) == torch.cuda.current_stream().cuda_stream
+    with torch.cuda.stream(side):
+        assert K._stream(None) == side.cuda_stream == torch.cuda.current_stream().cuda_stream
+    assert K._stream(side.cuda_stream) == side.cuda_stream
