@@ -963,7 +963,7 @@ __global__ __launch_bounds__(D / 4 * HB * S) void decode_step_finish_kernel(cons
     load4_f32(krow + dp, k_par);
     load4_f32(vrow + d0, v_in);
     const float ksc = a.k_scale ? a.k_scale[kvr] : 1.0f, vsc = a.v_scale ? a.v_scale[kvr] : 1.0f;
-    constexpr int NB = 4; // partials per batch of loads
+    constexpr int NB = S >= 16 ? 8 : 4; // partials per batch of loads
     auto load_batch = [&](int j0, float* li, float4* oi) {
 #pragma unroll
         for (int k = 0; k < NB; ++k) {
@@ -1177,24 +1177,41 @@ int decode_fast_path(const DecodePlan* p, const void* q, void* out, float* lse, 
 
 template <typename QT, typename PT, typename OT, int D>
 static int launch_step_finish(const DecodePlan* p, const StepFinishArgs& a, hipStream_t s) {
-    // heads of a unit per workgroup: 4 where the group allows it (two waves), else 2 (one wave), 1 for single heads
+    // Heads of a unit per workgroup, and slices over its partials.  Every batch of partials that a slice loads is a memory
+    // round trip behind the last one, so a unit's partials are spread over slices until one round holds them, where the
+    // launch is small enough that the additional waves cost less than the round trips.  (us, with the shapes that came out second.)
+    //   up to 4 partials, or up to 16 in a launch of more than 256 units (large batches): one slice; heads 4 at a time where the
+    //     group allows it (two waves), else 2 (one wave), 1 for single heads.  Four slices there: 40 sequences of 500 .. 900
+    //     tokens (320 units) 27.8 against 27.5, 96 of 600 .. 1 100 66.5 against 64.3.
+    //   5 .. 16, up to 256 units: four slices.  32 layers of 16 sequences of 500 .. 900 tokens 659 -> 620, of 24 of 700 .. 1 300
+    //     903 -> 872; 4 sequences of 32 single heads, 600 .. 900 tokens, 18.4 -> 16.6 (one head per workgroup; 16.8 with two).
+    //   17 .. 32 (batches of eight sequences or so): eight slices, one head per workgroup.  32 layers at batch 8: 497 against 505
+    //     with two heads per workgroup (eight waves), 527 with four (sixteen), 507 with four slices of two heads.
+    //   more (few long sequences): sixteen slices with eight partials to a batch, one round up to 128.  32 layers of 1 x 8 000
+    //     tokens 669 -> 571; 1 x 131 072 94.4 -> 91.5; two of 40 001 .. 90 001, 64/8 heads, 77.0 -> 75.3; 1 x 30 000 with 4/1 heads
+    //     30.1 -> 16.0.  (Eight slices of four before.  Thirty-two of eight from 129 partials on: as fast as sixteen.)
     const uint32_t G = a.group;
-    if (p->mfma_unit_max_count <= 16) { // what large batches produce
-        if (G >= 4)
-            hipLaunchKernelGGL((decode_step_finish_kernel<QT, PT, OT, 1, 4, D>), dim3(p->mfma_units, (G + 3) / 4), dim3(D / 4, 4, 1), 0, s, a.units, a.steps_ahead, a);
-        else if (G >= 2)
-            hipLaunchKernelGGL((decode_step_finish_kernel<QT, PT, OT, 1, 2, D>), dim3(p->mfma_units, (G + 1) / 2), dim3(D / 4, 2, 1), 0, s, a.units, a.steps_ahead, a);
-        else
-            hipLaunchKernelGGL((decode_step_finish_kernel<QT, PT, OT, 1, 1, D>), dim3(p->mfma_units, G), dim3(D / 4, 1, 1), 0, s, a.units, a.steps_ahead, a);
-    } else if (p->mfma_unit_max_count > 32 && p->mfma_unit_max_count <= 64) {
-        hipLaunchKernelGGL((decode_step_finish_kernel<QT, PT, OT, 4, 2, D>), dim3(p->mfma_units, (G + 1) / 2), dim3(D / 4, 2, 4), 0, s, a.units, a.steps_ahead, a);
+    auto launch = [&](auto s_c, auto hb_c) {
+        constexpr int S = decltype(s_c)::value, HB = decltype(hb_c)::value;
+        hipLaunchKernelGGL((decode_step_finish_kernel<QT, PT, OT, S, HB, D>), dim3(p->mfma_units, (G + HB - 1) / HB), dim3(D / 4, HB, S),
+                           0, s, a.units, a.steps_ahead, a);
+    };
+    const std::integral_constant<int, 1> c1{};
+    const std::integral_constant<int, 2> c2{};
+    const std::integral_constant<int, 4> c4{};
+    const std::integral_constant<int, 8> c8{};
+    const std::integral_constant<int, 16> c16{};
+    if (p->mfma_unit_max_count <= 4 || (p->mfma_unit_max_count <= 16 && p->mfma_units > 256)) {
+        if (G >= 4) launch(c1, c4);
+        else if (G >= 2) launch(c1, c2);
+        else launch(c1, c1);
+    } else if (p->mfma_unit_max_count <= 16) {
+        if (G >= 2) launch(c4, c2);
+        else launch(c4, c1);
+    } else if (p->mfma_unit_max_count <= 32) {
+        launch(c8, c1);
     } else {
-        // 17..32 partials (batches of eight sequences or so): eight slices, so one batch of four per slice and a single
-        // round of loads, and one head per workgroup -- four waves.  Measured on 32 layers at batch 8: 497 us per step
-        // against 505 with two heads per workgroup (eight waves), 527 with four (sixteen), 507 with four slices of two
-        // heads.  More than 64 partials (a few very long sequences): the same shape (4 x 32 768 tokens: 90.8 against
-        // 91.8 us with two heads).
-        hipLaunchKernelGGL((decode_step_finish_kernel<QT, PT, OT, 8, 1, D>), dim3(p->mfma_units, G), dim3(D / 4, 1, 8), 0, s, a.units, a.steps_ahead, a);
+        launch(c16, c1);
     }
     BZ_LAUNCH_CHECK();
     return 0;

@@ -242,3 +242,23 @@ def test_step_replays_from_a_hip_graph_and_runs_steps_ahead():
         got = outs.float().cpu().numpy()
         assert (np.abs(got - ref) <= ulp_tol(ref, p.dtype, 2e-3)).all(), (i, float(np.abs(got - ref).max()))
     assert int(counter.item()) == 0
+
+
+@pytest.mark.parametrize("heads", [(2, 2), (6, 2), (20, 4)])
+@pytest.mark.parametrize("tiles", [4, 5, 16, 17, 32, 33, 128, 130])
+def test_step_at_the_edges_of_the_finishing_kernels_slices(tiles, heads):
+    """One partial result per tile of 32 tokens, in numbers on both sides of every change of the finishing kernel's shape
+    (slices over the partials, heads per workgroup), beside a sequence of one partial and one of the new token alone; groups
+    that are no multiple of the heads of a workgroup."""
+    ctx = [32 * tiles, 20, 1]
+    dev, _, _ = run_step(DecodeProblem(400 + tiles, ctx, *heads, 128, 16, BZ_F16), split_tokens=32)
+    assert dev.handler.host_schedule(7)[:, 3].max() == tiles
+
+
+@pytest.mark.parametrize("tiles", [5, 16])
+@pytest.mark.parametrize("batch", [128, 129])
+def test_step_at_the_edge_of_a_large_launch(tiles, batch):
+    """256 units and 258: the same partials in four slices and in one."""
+    dev, _, _ = run_step(DecodeProblem(430 + tiles, [32 * tiles] * batch, 4, 2, 128, 16, BZ_BF16), split_tokens=32)
+    units = dev.handler.host_schedule(7)
+    assert len(units) == 2 * batch and units[:, 3].max() == tiles
