@@ -19,22 +19,26 @@ __device__ __forceinline__ float block_sum(float v, float* smem /* [16] */) {
 
 // out[n,:] = x[n,:] * rsqrt(mean(x^2)+eps) * w.  ADD: residual += input first (rounded to storage),
 // x is the rounded residual and the result overwrites input.
-template <typename T, bool ADD>
+// WHOLE: a lane has at most one vector of eight (rows of up to 8 192, the workgroup is made that wide): the row stays in
+// registers between the sum and the scaling and the weights are asked for with it, one memory round trip where the other
+// form has two, which is what bounds the kernel at a few rows and half of it at a thousand.  Same sums, same bits.
+template <typename T, bool ADD, bool WHOLE>
 __global__ __launch_bounds__(1024) void rms_norm_kernel(T* input, T* residual, const T* weight, T* output,
                                                          uint32_t h, float eps) {
     __shared__ float smem[16];
     const size_t row = (size_t)blockIdx.x * h;
     const uint32_t nvec = h / 8;
     float ss = 0.f;
+    float x[8];
+    Vec8<T> w;
     for (uint32_t i = threadIdx.x; i < nvec; i += blockDim.x) {
-        Vec8<T> v;
-        float x[8];
+        Vec8<T> v, r;
         v.load(input + row + i * 8);
+        if (ADD) r.load(residual + row + i * 8);
+        if (WHOLE) w.load(weight + i * 8);
         v.to_float(x);
         if (ADD) {
-            Vec8<T> r;
             float y[8];
-            r.load(residual + row + i * 8);
             r.to_float(y);
 #pragma unroll
             for (int e = 0; e < 8; ++e) x[e] += y[e];
@@ -44,21 +48,25 @@ __global__ __launch_bounds__(1024) void rms_norm_kernel(T* input, T* residual, c
         }
 #pragma unroll
         for (int e = 0; e < 8; ++e) ss += x[e] * x[e];
+        if (WHOLE) break;
     }
     ss = block_sum(ss, smem);
     const float rr = rsqrtf(ss / (float)h + eps);
     const T* src = ADD ? residual : input;
     for (uint32_t i = threadIdx.x; i < nvec; i += blockDim.x) {
-        Vec8<T> v, w;
-        float x[8], g[8];
-        v.load(src + row + i * 8);
-        w.load(weight + i * 8);
-        v.to_float(x);
+        Vec8<T> v;
+        float g[8];
+        if (!WHOLE) {
+            v.load(src + row + i * 8);
+            w.load(weight + i * 8);
+            v.to_float(x);
+        }
         w.to_float(g);
 #pragma unroll
         for (int e = 0; e < 8; ++e) x[e] = x[e] * rr * g[e];
         v.from_float(x);
         v.store(output + row + i * 8);
+        if (WHOLE) break;
     }
 }
 
@@ -116,11 +124,17 @@ __global__ __launch_bounds__(256) void add_residual_kernel(const T* input, T* re
     r.store(residual + i * 8);
 }
 
-static inline uint32_t norm_block(uint32_t h) {
+template <typename T, bool ADD>
+static void launch_rms_norm(void* input, void* residual, const void* weight, void* output, uint32_t rows, uint32_t h, float eps,
+                            hipStream_t s) {
     uint32_t t = (h / 8 + 63) / 64 * 64;
-    if (t > 1024) t = 1024;
-    if (t < 64) t = 64;
-    return t;
+    t = t > 1024 ? 1024 : (t < 64 ? 64 : t);
+    if (h / 8 <= t)
+        hipLaunchKernelGGL((rms_norm_kernel<T, ADD, true>), dim3(rows), dim3(t), 0, s, (T*)input, (T*)residual, (const T*)weight,
+                           (T*)output, h, eps);
+    else
+        hipLaunchKernelGGL((rms_norm_kernel<T, ADD, false>), dim3(rows), dim3(t), 0, s, (T*)input, (T*)residual, (const T*)weight,
+                           (T*)output, h, eps);
 }
 
 } // namespace bz
@@ -132,14 +146,9 @@ extern "C" int bz_rms_norm(const void* input, const void* weight, void* output, 
     if (!input || !weight || !output) return BZ_ERR_BAD_ARG;
     if (hidden_size % 8) return BZ_ERR_UNSUPPORTED;
     if (num_tokens == 0) return 0;
-    hipStream_t s = (hipStream_t)stream;
-    const dim3 grid(num_tokens), block(norm_block(hidden_size));
-    if (dtype == BZ_F16)
-        hipLaunchKernelGGL((rms_norm_kernel<f16_t, false>), grid, block, 0, s, (f16_t*)input, (f16_t*)nullptr,
-                           (const f16_t*)weight, (f16_t*)output, hidden_size, eps);
-    else if (dtype == BZ_BF16)
-        hipLaunchKernelGGL((rms_norm_kernel<bf16_t, false>), grid, block, 0, s, (bf16_t*)input, (bf16_t*)nullptr,
-                           (const bf16_t*)weight, (bf16_t*)output, hidden_size, eps);
+    void* in = const_cast<void*>(input);
+    if (dtype == BZ_F16) launch_rms_norm<f16_t, false>(in, nullptr, weight, output, num_tokens, hidden_size, eps, (hipStream_t)stream);
+    else if (dtype == BZ_BF16) launch_rms_norm<bf16_t, false>(in, nullptr, weight, output, num_tokens, hidden_size, eps, (hipStream_t)stream);
     else return BZ_ERR_UNSUPPORTED;
     BZ_LAUNCH_CHECK();
     return 0;
@@ -150,14 +159,8 @@ extern "C" int bz_add_rms_norm(void* input, void* residual, const void* weight, 
     if (!input || !weight || !residual) return BZ_ERR_BAD_ARG;
     if (hidden_size % 8) return BZ_ERR_UNSUPPORTED;
     if (num_tokens == 0) return 0;
-    hipStream_t s = (hipStream_t)stream;
-    const dim3 grid(num_tokens), block(norm_block(hidden_size));
-    if (dtype == BZ_F16)
-        hipLaunchKernelGGL((rms_norm_kernel<f16_t, true>), grid, block, 0, s, (f16_t*)input, (f16_t*)residual,
-                           (const f16_t*)weight, (f16_t*)input, hidden_size, eps);
-    else if (dtype == BZ_BF16)
-        hipLaunchKernelGGL((rms_norm_kernel<bf16_t, true>), grid, block, 0, s, (bf16_t*)input, (bf16_t*)residual,
-                           (const bf16_t*)weight, (bf16_t*)input, hidden_size, eps);
+    if (dtype == BZ_F16) launch_rms_norm<f16_t, true>(input, residual, weight, input, num_tokens, hidden_size, eps, (hipStream_t)stream);
+    else if (dtype == BZ_BF16) launch_rms_norm<bf16_t, true>(input, residual, weight, input, num_tokens, hidden_size, eps, (hipStream_t)stream);
     else return BZ_ERR_UNSUPPORTED;
     BZ_LAUNCH_CHECK();
     return 0;
