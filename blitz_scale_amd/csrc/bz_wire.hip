@@ -7,8 +7,7 @@
 // large transfer then replaces one send per (page, layer).  With an e4m3 wire and a 16-bit pool the
 // elements travel as x/scale in e4m3 (half the bytes) and come back as e4m3*scale.
 //
-// HBM-bound copies: every lane moves four 8-element vectors, all four loads in flight before the
-// first store.
+// HBM-bound copies: every lane moves 8-element vectors, all its loads in flight before the first store.
 #include <cstdio>
 
 #include "bz_common.hpp"
@@ -38,7 +37,11 @@ template <typename T> __device__ __forceinline__ void wire_store(const Vec8<T>& 
     }
 }
 
-constexpr int kWirePer = 4; // vectors per lane
+// Vectors per lane.  Where a workgroup's vectors all lie in one chunk its address arithmetic is scalar (else every vector
+// pays two 64-bit divisions), and what the lanes then want is few bytes each and many workgroups in flight: five prompts of
+// 400 .. 1 500 tokens, 32 layers, 8 heads, bf16, packed and unpacked (1.36 GB moved by each): 496 us with four vectors and the
+// divisions, 486 with four, 481 with two, 443 (6.1 TB/s) with one; over an e4m3 wire 508, 471 (four), 447 (two), 462 (one).
+constexpr int wire_per(bool within, bool same_size) { return !within ? 4 : (same_size ? 1 : 2); }
 
 struct WireArgs {
     char* pool;            // base of the whole pool (layer 0)
@@ -56,9 +59,10 @@ struct WireArgs {
 };
 
 // PT: pool element type, WT: wire element type, PACK: pool -> wire (else wire -> pool)
-template <typename PT, typename WT, bool PACK>
+// WITHIN: a chunk is a whole number of workgroups' vectors, so a workgroup's chunk, page and addresses are scalar.
+template <typename PT, typename WT, bool PACK, bool WITHIN>
 __global__ __launch_bounds__(256) void wire_kernel(WireArgs a) {
-    constexpr int kPer = kWirePer;
+    constexpr int kPer = wire_per(WITHIN, sizeof(PT) == sizeof(WT));
     const uint64_t g0 = (uint64_t)blockIdx.x * (256 * kPer) + threadIdx.x;
     using ST = typename std::conditional<PACK, PT, WT>::type; // what is read
     using DT = typename std::conditional<PACK, WT, PT>::type; // what is written
@@ -72,7 +76,15 @@ __global__ __launch_bounds__(256) void wire_kernel(WireArgs a) {
         live[u] = g < a.total_vecs;
         scale[u] = nullptr;
         if (!live[u]) continue;
-        const uint32_t c = (uint32_t)(g / a.vecs_per_chunk), e = (uint32_t)(g % a.vecs_per_chunk) * 8;
+        uint32_t c, e;
+        if constexpr (WITHIN) {
+            const uint32_t per_chunk = a.vecs_per_chunk / (256 * kPer);
+            c = blockIdx.x / per_chunk;
+            e = ((blockIdx.x - c * per_chunk) * (256 * kPer) + u * 256 + threadIdx.x) * 8;
+        } else {
+            c = (uint32_t)(g / a.vecs_per_chunk);
+            e = (uint32_t)(g % a.vecs_per_chunk) * 8;
+        }
         const uint32_t i = c / a.layer_cnt, l = c % a.layer_cnt;
         const int32_t page = a.page_ids[i];
         if ((uint64_t)(uint32_t)page >= a.max_pages) { // not a page of this pool: nothing is read from or written to
@@ -122,11 +134,14 @@ __global__ __launch_bounds__(256) void wire_kernel(WireArgs a) {
 
 template <typename PT, typename WT, bool PACK>
 static int launch_wire(const WireArgs& a, hipStream_t s) {
-    const uint64_t per_wg = 256 * kWirePer;
+    constexpr bool same = sizeof(PT) == sizeof(WT);
+    const bool within = a.vecs_per_chunk % (256 * wire_per(true, same)) == 0;
+    const uint64_t per_wg = 256 * wire_per(within, same);
     const uint64_t grid = (a.total_vecs + per_wg - 1) / per_wg;
     if (grid == 0) return 0;
     if (grid > 0x7fffffffull) return BZ_ERR_UNSUPPORTED;
-    hipLaunchKernelGGL((wire_kernel<PT, WT, PACK>), dim3((uint32_t)grid), dim3(256), 0, s, a);
+    if (within) hipLaunchKernelGGL((wire_kernel<PT, WT, PACK, true>), dim3((uint32_t)grid), dim3(256), 0, s, a);
+    else hipLaunchKernelGGL((wire_kernel<PT, WT, PACK, false>), dim3((uint32_t)grid), dim3(256), 0, s, a);
     BZ_LAUNCH_CHECK();
     return 0;
 }
