@@ -429,9 +429,13 @@ __global__ void decode_combine_kernel(const DecodeCombine* combos, const float* 
                                       void* out, float* lse, uint32_t num_qo_heads, uint32_t D) {
     const DecodeCombine c = combos[blockIdx.x];
     const uint32_t h = blockIdx.y, d = threadIdx.x;
+    // (four partials' loads at a time: one at a time is a memory round trip each, 4 sequences of 1 000 .. 3 000 tokens, raw K,
+    // 34.0 -> 30.7 us, 48 of 200 .. 2 048 71.8 -> 70.4)
     float M = -INFINITY;
+#pragma unroll 4
     for (int i = 0; i < c.count; ++i) M = fmaxf(M, part_lse[(size_t)(c.first + i) * num_qo_heads + h]);
     float wsum = 0.f, o = 0.f;
+#pragma unroll 4
     for (int i = 0; i < c.count; ++i) {
         const float li = part_lse[(size_t)(c.first + i) * num_qo_heads + h];
         const float w = (li == -INFINITY) ? 0.f : exp2f(li - M);

@@ -171,6 +171,24 @@ def test_shapes_outside_the_matrix_core_kernel_get_segments_only():
     assert [tuple(c) for c in s["combos"]] == [(0, 0, 16, 0)]
 
 
+@pytest.mark.parametrize("batch,Hq,Hkv,P,one_round", [
+    (48, 32, 8, 8, True),    # halving comes to 1.7 rounds of workgroups
+    (100, 32, 8, 8, False),  # whole sequences of every length in one round would end with the longest of them
+    (24, 32, 8, 24, False),  # fewer workgroups than places already, at the shortest pieces
+    (48, 40, 8, 16, False),  # groups of five: a workgroup for every q head
+])
+def test_general_pieces_that_fill_the_chip_once(batch, Hq, Hkv, P, one_round):
+    lens = np.random.default_rng(3).integers(200, 2049, size=batch)
+    s = schedule(lens, Hq, Hkv, 64, P)
+    check_general_schedule(s, P)
+    sizes = s["segments"][:, 2] - s["segments"][:, 1]
+    assert sizes.max() * P <= 2048
+    longest_of_halving = 256 if batch == 48 else (1024 if batch == 100 else 256 // P * P)
+    assert (sizes.max() * P > longest_of_halving) == one_round
+    if one_round:
+        assert 4 * CUS * 0.9 < len(sizes) * Hkv <= 4 * CUS
+
+
 def test_fewer_compute_units_mean_fewer_longer_shares():
     lens = [2048] * 64
     a = schedule(lens, 32, 8, 128, 16, 2048, cus=256)
