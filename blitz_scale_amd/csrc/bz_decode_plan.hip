@@ -82,35 +82,48 @@ static int build_schedule(DecodePlan* p, const int32_t* indptr_h, const int32_t*
     const bool never_split = split_tokens == 0xffffffffu;
     while (!never_split && piece > min_pages && count_items(piece) < (uint64_t)cus * 4)
         piece = std::max(min_pages, piece / 2);
-    // What halving comes to is often a round of workgroups and a part of one.  Pieces just long enough for all of them to
-    // find a place at once (four per CU) are taken instead where that ends sooner: a workgroup takes its longest piece's
-    // tokens and about 64 more to begin and to end; of more than a round the last is waited for half a workgroup long.
-    // 48 sequences of 200 .. 2 048 tokens, 32/8 heads, us before and now: raw K 70.4 -> 65.4, pages of 8 tokens 84.0 -> 67.4,
-    // heads of 64 over an fp8 pool 64.2 -> 50.5; 48 of 2 000 .. 6 000, raw K, 171 -> 164.  Without the comparison 100 of 200 ..
-    // 2 048 with raw K, whose lengths differ too much for one round, go from 120.2 to 123.5.
-    const uint32_t group = num_qo_heads / num_kv_heads, wgs_per_kv_head = group % 8 == 0 ? group / 8 : group % 4 == 0 ? group / 4 : group % 2 == 0 ? group / 2 : group;
-    const uint64_t places = (uint64_t)cus * 4;
-    auto time_of = [&](uint32_t pc) { // in tokens
-        uint64_t n = 0, pages = 0, longest = 0;
-        for (uint32_t b = 0; b < batch_size; ++b) {
-            const uint64_t np = indptr_h[b + 1] > indptr_h[b] ? (uint64_t)(indptr_h[b + 1] - indptr_h[b]) : 0;
-            if (np == 0) continue;
-            const uint64_t pieces = (np + pc - 1) / pc;
-            n += pieces;
-            pages += np;
-            longest = std::max(longest, (np + pieces - 1) / pieces);
+    // What halving comes to is often some rounds of workgroups and a part of one (two find a place on a compute unit, by the
+    // registers of groups of two and more; single q heads, three or four to a unit, are left as they are).  Pieces that come to
+    // one, two or three rounds are taken instead where that is sure to end sooner: a workgroup takes the tokens of its piece
+    // and about 256 more to begin and to end; the rounds take the mean piece each, the last one the longest.
+    // Sequences of 200 .. 2 048 tokens, 32/8 heads, whole calls, us (halving alone in brackets): 48 with raw K 65.9 (70.4), with
+    // pages of 8 tokens 68.1 (84.4), with heads of 64 over an fp8 pool 50.6 (64.2); 30 with pages of 8 43.5 (61.0), raw K 46.5
+    // (51.7); 24 raw K 39.7 (45.7); 30 with 64/8 heads and pages of 8 80.0 (109.1); 48 of 2 000 .. 6 000, raw K, 164 (171).  An
+    // eighth is asked for because lengths that differ much make the estimate worth less: 100 with raw K go from 120 to 124 in
+    // two rounds, 70 with 64/8 heads from 126 to 129.
+    const uint32_t group = num_qo_heads / num_kv_heads;
+    if (!never_split && piece < max_pages_cap && group % 2 == 0) {
+        // (the dispatch splits groups of more than eight, and those that are no power of two)
+        const uint64_t wgs_per_kv_head = group % 8 == 0 ? group / 8 : group % 4 == 0 ? group / 4 : group / 2;
+        const uint64_t places = (uint64_t)cus * 2, heads = num_kv_heads * wgs_per_kv_head;
+        auto time_of = [&](uint32_t pc) { // in tokens
+            uint64_t n = 0, pages = 0, longest = 0;
+            for (uint32_t b = 0; b < batch_size; ++b) {
+                const uint64_t np = indptr_h[b + 1] > indptr_h[b] ? (uint64_t)(indptr_h[b + 1] - indptr_h[b]) : 0;
+                if (np == 0) continue;
+                const uint64_t pieces = (np + pc - 1) / pc;
+                n += pieces;
+                pages += np;
+                longest = std::max(longest, (np + pieces - 1) / pieces);
+            }
+            if (n == 0) return (uint64_t)0;
+            const uint64_t rounds = (n * heads + places - 1) / places;
+            return (rounds - 1) * pages * page_size / n + longest * page_size + 256 * rounds;
+        };
+        const uint32_t halved = piece;
+        uint64_t best = time_of(halved) * 7 / 8;
+        for (uint32_t rounds = 1; rounds <= 3; ++rounds) {
+            uint32_t lo = halved, hi = max_pages_cap; // the shortest pieces that come to so many rounds, if any do
+            while (lo < hi) {
+                const uint32_t mid = (lo + hi) / 2;
+                if (count_items(mid) * wgs_per_kv_head <= rounds * places) hi = mid; else lo = mid + 1;
+            }
+            const uint64_t t = time_of(lo);
+            if (t < best) {
+                best = t;
+                piece = lo;
+            }
         }
-        const uint64_t heads = (uint64_t)num_kv_heads * wgs_per_kv_head, one = longest * page_size + 64;
-        if (n * heads <= places) return one;
-        return std::max(one, (pages * page_size + 64 * n) * heads / places + one / 2);
-    };
-    if (!never_split && piece < max_pages_cap) {
-        uint32_t lo = piece, hi = max_pages_cap; // the shortest pieces that are one round, if any are
-        while (lo < hi) {
-            const uint32_t mid = (lo + hi) / 2;
-            if (count_items(mid) * wgs_per_kv_head <= places) hi = mid; else lo = mid + 1;
-        }
-        if (time_of(lo) * 20 < time_of(piece) * 19) piece = lo;
     }
 
     std::vector<DecodeSegment>& segs = p->h_segs;

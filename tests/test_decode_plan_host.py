@@ -171,22 +171,27 @@ def test_shapes_outside_the_matrix_core_kernel_get_segments_only():
     assert [tuple(c) for c in s["combos"]] == [(0, 0, 16, 0)]
 
 
-@pytest.mark.parametrize("batch,Hq,Hkv,P,one_round", [
-    (48, 32, 8, 8, True),    # halving comes to 1.7 rounds of workgroups
-    (100, 32, 8, 8, False),  # whole sequences of every length in one round would end with the longest of them
-    (24, 32, 8, 24, False),  # fewer workgroups than places already, at the shortest pieces
-    (48, 40, 8, 16, False),  # groups of five: a workgroup for every q head
+@pytest.mark.parametrize("batch,Hq,Hkv,P,rounds", [
+    (48, 32, 8, 8, 2),    # halving comes to three rounds of workgroups, two to a compute unit, and a part of one
+    (24, 32, 8, 24, 1),   # ... to one and a part
+    (3, 32, 8, 16, 0),    # fewer workgroups than places already, at the shortest pieces
+    (100, 32, 8, 8, 0),   # whole sequences of every length: full rounds would end with the longest of them
+    (48, 40, 8, 16, 0),   # groups of five: a workgroup for every q head
+    (48, 32, 32, 16, 0),  # single heads
 ])
-def test_general_pieces_that_fill_the_chip_once(batch, Hq, Hkv, P, one_round):
+def test_general_pieces_that_fill_the_chip(batch, Hq, Hkv, P, rounds):
     lens = np.random.default_rng(3).integers(200, 2049, size=batch)
     s = schedule(lens, Hq, Hkv, 64, P)
     check_general_schedule(s, P)
     sizes = s["segments"][:, 2] - s["segments"][:, 1]
     assert sizes.max() * P <= 2048
-    longest_of_halving = 256 if batch == 48 else (1024 if batch == 100 else 256 // P * P)
-    assert (sizes.max() * P > longest_of_halving) == one_round
-    if one_round:
-        assert 4 * CUS * 0.9 < len(sizes) * Hkv <= 4 * CUS
+    halved = 2048 // P  # the rule without full rounds
+    while halved > 256 // P and Hkv * sum(-(-int(n) // (halved * P)) for n in lens) < 4 * CUS:
+        halved = max(256 // P, halved // 2)
+    if rounds:
+        assert sizes.max() > halved and 0.9 * rounds * 2 * CUS < len(sizes) * Hkv <= rounds * 2 * CUS
+    else:
+        assert sizes.max() <= halved
 
 
 def test_fewer_compute_units_mean_fewer_longer_shares():
