@@ -912,7 +912,7 @@ template <> __device__ __forceinline__ void store4<float>(float* p, const float*
     *reinterpret_cast<float4*>(p) = make_float4(v[0], v[1], v[2], v[3]);
 }
 
-template <typename QT, typename PT, typename OT, int S, int HB, int D>
+template <typename QT, typename PT, typename OT, int S, int HB, int NB, int D>
 __global__ __launch_bounds__(D / 4 * HB * S) void decode_step_finish_kernel(const MfmaUnit* __restrict__ units_p,
                                                                          const int32_t* __restrict__ ahead_p, StepFinishArgs a) {
     constexpr int LPH = D / 4; // lanes of a head
@@ -963,7 +963,6 @@ __global__ __launch_bounds__(D / 4 * HB * S) void decode_step_finish_kernel(cons
     load4_f32(krow + dp, k_par);
     load4_f32(vrow + d0, v_in);
     const float ksc = a.k_scale ? a.k_scale[kvr] : 1.0f, vsc = a.v_scale ? a.v_scale[kvr] : 1.0f;
-    constexpr int NB = S >= 16 ? 8 : 4; // partials per batch of loads
     auto load_batch = [&](int j0, float* li, float4* oi) {
 #pragma unroll
         for (int k = 0; k < NB; ++k) {
@@ -1185,15 +1184,18 @@ static int launch_step_finish(const DecodePlan* p, const StepFinishArgs& a, hipS
     //     tokens (320 units) 27.8 against 27.5, 96 of 600 .. 1 100 66.5 against 64.3.
     //   5 .. 16, up to 256 units: four slices.  32 layers of 16 sequences of 500 .. 900 tokens 659 -> 620, of 24 of 700 .. 1 300
     //     903 -> 872; 4 sequences of 32 single heads, 600 .. 900 tokens, 18.4 -> 16.6 (one head per workgroup; 16.8 with two).
-    //   17 .. 32 (batches of eight sequences or so): eight slices, one head per workgroup.  32 layers at batch 8: 497 against 505
-    //     with two heads per workgroup (eight waves), 527 with four (sixteen), 507 with four slices of two heads.
-    //   more (few long sequences): sixteen slices with eight partials to a batch, one round up to 128.  32 layers of 1 x 8 000
-    //     tokens 669 -> 571; 1 x 131 072 94.4 -> 91.5; two of 40 001 .. 90 001, 64/8 heads, 77.0 -> 75.3; 1 x 30 000 with 4/1 heads
-    //     30.1 -> 16.0.  (Eight slices of four before.  Thirty-two of eight from 129 partials on: as fast as sixteen.)
+    //   17 .. 32 (batches of eight sequences or so): four slices with eight partials to a batch, one head per workgroup.  9 sequences
+    //     of 1 000 .. 3 000 tokens over an fp8 pool 18.0 -> 17.5, 32 layers of 12 of 1 000 .. 1 400 688 -> 685 (eight slices of four
+    //     before; those with two and four heads per workgroup: 32 layers at batch 8 497 against 505 and 527).
+    //   33 .. 64: eight slices with eight partials to a batch.  32 layers of 4 x 1 500 tokens 538 -> 491, of 2 x 1 500 427 -> 396; 4 x
+    //     9 000 34.2 -> 32.5 (four slices of four for two heads before; sixteen slices: 505, 412, 33.0).
+    //   more (few long sequences): sixteen slices of eight, one round up to 128.  32 layers of 1 x 8 000 tokens 669 -> 571; 1 x
+    //     131 072 94.4 -> 91.5; two of 40 001 .. 90 001, 64/8 heads, 77.0 -> 75.3; 1 x 30 000 with 4/1 heads 30.1 -> 16.0.  (Eight
+    //     slices of four before.  Thirty-two of eight from 129 partials on: as fast as sixteen.)
     const uint32_t G = a.group;
-    auto launch = [&](auto s_c, auto hb_c) {
-        constexpr int S = decltype(s_c)::value, HB = decltype(hb_c)::value;
-        hipLaunchKernelGGL((decode_step_finish_kernel<QT, PT, OT, S, HB, D>), dim3(p->mfma_units, (G + HB - 1) / HB), dim3(D / 4, HB, S),
+    auto launch = [&](auto s_c, auto hb_c, auto nb_c) {
+        constexpr int S = decltype(s_c)::value, HB = decltype(hb_c)::value, NB = decltype(nb_c)::value; // NB: partials per batch of loads
+        hipLaunchKernelGGL((decode_step_finish_kernel<QT, PT, OT, S, HB, NB, D>), dim3(p->mfma_units, (G + HB - 1) / HB), dim3(D / 4, HB, S),
                            0, s, a.units, a.steps_ahead, a);
     };
     const std::integral_constant<int, 1> c1{};
@@ -1202,16 +1204,18 @@ static int launch_step_finish(const DecodePlan* p, const StepFinishArgs& a, hipS
     const std::integral_constant<int, 8> c8{};
     const std::integral_constant<int, 16> c16{};
     if (p->mfma_unit_max_count <= 4 || (p->mfma_unit_max_count <= 16 && p->mfma_units > 256)) {
-        if (G >= 4) launch(c1, c4);
-        else if (G >= 2) launch(c1, c2);
-        else launch(c1, c1);
+        if (G >= 4) launch(c1, c4, c4);
+        else if (G >= 2) launch(c1, c2, c4);
+        else launch(c1, c1, c4);
     } else if (p->mfma_unit_max_count <= 16) {
-        if (G >= 2) launch(c4, c2);
-        else launch(c4, c1);
+        if (G >= 2) launch(c4, c2, c4);
+        else launch(c4, c1, c4);
     } else if (p->mfma_unit_max_count <= 32) {
-        launch(c8, c1);
+        launch(c4, c1, c8);
+    } else if (p->mfma_unit_max_count <= 64) {
+        launch(c8, c1, c8);
     } else {
-        launch(c16, c1);
+        launch(c16, c1, c8);
     }
     BZ_LAUNCH_CHECK();
     return 0;

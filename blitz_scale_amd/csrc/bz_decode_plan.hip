@@ -97,23 +97,26 @@ static int build_schedule(DecodePlan* p, const int32_t* indptr_h, const int32_t*
         const uint64_t wgs_per_kv_head = group % 8 == 0 ? group / 8 : group % 4 == 0 ? group / 4 : group / 2;
         const uint64_t places = (uint64_t)cus * 2, heads = num_kv_heads * wgs_per_kv_head;
         auto time_of = [&](uint32_t pc) { // in tokens
-            uint64_t n = 0, pages = 0, longest = 0;
+            uint64_t n = 0, pages = 0;
+            uint32_t longest = 0;
             for (uint32_t b = 0; b < batch_size; ++b) {
-                const uint64_t np = indptr_h[b + 1] > indptr_h[b] ? (uint64_t)(indptr_h[b + 1] - indptr_h[b]) : 0;
+                const uint32_t np = indptr_h[b + 1] > indptr_h[b] ? (uint32_t)(indptr_h[b + 1] - indptr_h[b]) : 0;
                 if (np == 0) continue;
-                const uint64_t pieces = (np + pc - 1) / pc;
+                const uint32_t pieces = (np + pc - 1) / pc;
                 n += pieces;
                 pages += np;
-                longest = std::max(longest, (np + pieces - 1) / pieces);
+                longest = std::max(longest, pieces == 1 ? np : (np + pieces - 1) / pieces);
             }
             if (n == 0) return (uint64_t)0;
             const uint64_t rounds = (n * heads + places - 1) / places;
-            return (rounds - 1) * pages * page_size / n + longest * page_size + 256 * rounds;
+            return (rounds - 1) * pages * page_size / n + (uint64_t)longest * page_size + 256 * rounds;
         };
         const uint32_t halved = piece;
+        const uint64_t wgs_halved = count_items(halved) * wgs_per_kv_head, wgs_longest = count_items(max_pages_cap) * wgs_per_kv_head;
         uint64_t best = time_of(halved) * 7 / 8;
-        for (uint32_t rounds = 1; rounds <= 3; ++rounds) {
-            uint32_t lo = halved, hi = max_pages_cap; // the shortest pieces that come to so many rounds, if any do
+        for (uint32_t rounds = 1; rounds <= 3 && wgs_halved > rounds * places; ++rounds) {
+            if (wgs_longest > rounds * places) continue;
+            uint32_t lo = halved, hi = max_pages_cap; // the shortest pieces that come to so many rounds
             while (lo < hi) {
                 const uint32_t mid = (lo + hi) / 2;
                 if (count_items(mid) * wgs_per_kv_head <= rounds * places) hi = mid; else lo = mid + 1;
