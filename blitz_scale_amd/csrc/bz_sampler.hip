@@ -19,8 +19,10 @@ namespace bz {
 
 // grid (rows), block 256: row r of dst <- row src_row(r) of src, hidden % 8 == 0 elements of 2 bytes.
 // HBM-bound.  A row of the table is seldom wanted twice: non-temporal loads leave the caches to the rows going out, which the
-// first layer reads next.  Embedding of 8 192 rows of 4 096 with the gather and the argmax behind it 35.0 -> 30.8 us, of 8 192
-// 66.3 -> 62.5.  (Non-temporal stores as well: 32.0 and 56.3; four loads at a time: no difference.)
+// first layer reads next; the last tokens' rows have just been written and are read as they are.  (A condition on two kinds of
+// loads in one kernel makes both plain.)  Embedding of 8 192 rows of 4 096 with the gather and the argmax behind it 34.8 -> 30.4
+// us, of 8 192 66.2 -> 63.1.  (Non-temporal stores as well: 32.0 and 56.3; four loads at a time: no difference.)
+template <bool TABLE> // rows of the embedding table, or the last tokens' rows of a batch
 __global__ __launch_bounds__(256) void gather_rows_kernel(uint4* __restrict__ dst, const uint4* __restrict__ src,
                                                            const uint32_t* __restrict__ token_ids,
                                                            const int32_t* __restrict__ out_loc,
@@ -28,7 +30,7 @@ __global__ __launch_bounds__(256) void gather_rows_kernel(uint4* __restrict__ ds
                                                            uint32_t row_vecs) {
     const uint32_t r = blockIdx.x;
     int64_t s, d = r;
-    if (ragged_indptr) { // last token of request r; a request without tokens yields a zero row
+    if constexpr (!TABLE) { // last token of request r; a request without tokens yields a zero row
         s = (int64_t)ragged_indptr[r + 1] - 1;
         if (ragged_indptr[r + 1] <= ragged_indptr[r]) s = -1;
     } else {
@@ -40,7 +42,8 @@ __global__ __launch_bounds__(256) void gather_rows_kernel(uint4* __restrict__ ds
     const u32x4* srow = reinterpret_cast<const u32x4*>(src + (size_t)max(s, (int64_t)0) * row_vecs);
     for (uint32_t i = threadIdx.x; i < row_vecs; i += blockDim.x) {
         u32x4 v = {0, 0, 0, 0};
-        if (s >= 0) v = __builtin_nontemporal_load(srow + i);
+        if constexpr (TABLE) v = __builtin_nontemporal_load(srow + i);
+        else if (s >= 0) v = srow[i];
         drow[i] = v;
     }
 }
@@ -155,7 +158,7 @@ extern "C" int bz_embedding(void* output, const uint32_t* token_ids, const int32
     if (int rc = check_rows(output, weight, dtype, hidden_size)) return rc;
     if (!token_ids) return BZ_ERR_BAD_ARG;
     if (num_tokens == 0) return 0;
-    hipLaunchKernelGGL(gather_rows_kernel, dim3(num_tokens), dim3(256), 0, (hipStream_t)stream, (uint4*)output,
+    hipLaunchKernelGGL(gather_rows_kernel<true>, dim3(num_tokens), dim3(256), 0, (hipStream_t)stream, (uint4*)output,
                        (const uint4*)weight, token_ids, out_loc, (const int32_t*)nullptr, hidden_size / 8);
     BZ_LAUNCH_CHECK();
     return 0;
@@ -167,7 +170,7 @@ extern "C" int bz_gather_last_token(void* output, const void* tokens, const int3
     if (int rc = check_rows(output, tokens, dtype, hidden_size)) return rc;
     if (!ragged_indptr) return BZ_ERR_BAD_ARG;
     if (batch_size == 0) return 0;
-    hipLaunchKernelGGL(gather_rows_kernel, dim3(batch_size), dim3(256), 0, (hipStream_t)stream, (uint4*)output,
+    hipLaunchKernelGGL(gather_rows_kernel<false>, dim3(batch_size), dim3(256), 0, (hipStream_t)stream, (uint4*)output,
                        (const uint4*)tokens, (const uint32_t*)nullptr, (const int32_t*)nullptr, ragged_indptr,
                        hidden_size / 8);
     BZ_LAUNCH_CHECK();
