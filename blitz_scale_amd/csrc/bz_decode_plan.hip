@@ -69,8 +69,13 @@ static int build_schedule(DecodePlan* p, const int32_t* indptr_h, const int32_t*
     // shortened further, down to 256 tokens, until the launch holds about four workgroups per CU.
     const uint32_t max_pages_cap = std::max<uint32_t>(1, split_tokens / page_size);
     const uint32_t min_pages = std::min<uint32_t>(max_pages_cap, std::max<uint32_t>(1, 256 / page_size));
+    // (pieces longer than the longest sequence all cut alike; held to it, the sums below stay under 2^32 for every split_tokens)
+    uint32_t longest_pages = 1;
+    for (uint32_t b = 0; b < batch_size; ++b)
+        if (indptr_h[b + 1] > indptr_h[b]) longest_pages = std::max(longest_pages, (uint32_t)(indptr_h[b + 1] - indptr_h[b]));
     uint32_t piece = max_pages_cap;
     auto count_items = [&](uint32_t pc) {
+        pc = std::min(pc, longest_pages);
         uint64_t n = 0;
         for (uint32_t b = 0; b < batch_size; ++b) {
             const int32_t np = indptr_h[b + 1] - indptr_h[b];
@@ -82,6 +87,7 @@ static int build_schedule(DecodePlan* p, const int32_t* indptr_h, const int32_t*
     const bool never_split = split_tokens == 0xffffffffu;
     while (!never_split && piece > min_pages && count_items(piece) < (uint64_t)cus * 4)
         piece = std::max(min_pages, piece / 2);
+    piece = std::min(piece, longest_pages);
     // What halving comes to is often some rounds of workgroups and a part of one (two find a place on a compute unit, by the
     // registers of groups of two and more; single q heads, three or four to a unit, are left as they are).  Pieces that come to
     // one, two or three rounds are taken instead where that is sure to end sooner: a workgroup takes the tokens of its piece
@@ -92,7 +98,8 @@ static int build_schedule(DecodePlan* p, const int32_t* indptr_h, const int32_t*
     // eighth is asked for because lengths that differ much make the estimate worth less: 100 with raw K go from 120 to 124 in
     // two rounds, 70 with 64/8 heads from 126 to 129.
     const uint32_t group = num_qo_heads / num_kv_heads;
-    if (!never_split && piece < max_pages_cap && group % 2 == 0) {
+    const uint32_t longest_piece = std::min(max_pages_cap, longest_pages);
+    if (!never_split && piece < longest_piece && group % 2 == 0) {
         // (the dispatch splits groups of more than eight, and those that are no power of two)
         const uint64_t wgs_per_kv_head = group % 8 == 0 ? group / 8 : group % 4 == 0 ? group / 4 : group / 2;
         const uint64_t places = (uint64_t)cus * 2, heads = num_kv_heads * wgs_per_kv_head;
@@ -112,13 +119,13 @@ static int build_schedule(DecodePlan* p, const int32_t* indptr_h, const int32_t*
             return (rounds - 1) * pages * page_size / n + (uint64_t)longest * page_size + 256 * rounds;
         };
         const uint32_t halved = piece;
-        const uint64_t wgs_halved = count_items(halved) * wgs_per_kv_head, wgs_longest = count_items(max_pages_cap) * wgs_per_kv_head;
+        const uint64_t wgs_halved = count_items(halved) * wgs_per_kv_head, wgs_longest = count_items(longest_piece) * wgs_per_kv_head;
         uint64_t best = time_of(halved) * 7 / 8;
         for (uint32_t rounds = 1; rounds <= 3 && wgs_halved > rounds * places; ++rounds) {
             if (wgs_longest > rounds * places) continue;
-            uint32_t lo = halved, hi = max_pages_cap; // the shortest pieces that come to so many rounds
+            uint32_t lo = halved, hi = longest_piece; // the shortest pieces that come to so many rounds
             while (lo < hi) {
-                const uint32_t mid = (lo + hi) / 2;
+                const uint32_t mid = lo + (hi - lo) / 2;
                 if (count_items(mid) * wgs_per_kv_head <= rounds * places) hi = mid; else lo = mid + 1;
             }
             const uint64_t t = time_of(lo);

@@ -194,6 +194,19 @@ def test_general_pieces_that_fill_the_chip(batch, Hq, Hkv, P, rounds):
         assert sizes.max() <= halved
 
 
+@pytest.mark.parametrize("P", [1, 3, 16])
+@pytest.mark.parametrize("split", [0x7FFFFFFF, 0x80000000, 0xFFFFFF00, 0xFFFFFFFE, 0xFFFFFFFF])
+def test_piece_lengths_up_to_the_largest_of_their_type(split, P):
+    """Pieces longer than any sequence: no sum of pages wraps around, in counting pieces or in looking for full rounds."""
+    lens = np.random.default_rng(3).integers(200, 2049, size=48)
+    s = schedule(lens, 32, 8, 64, P, split)
+    check_general_schedule(s, P)
+    if split == 0xFFFFFFFF:  # never split
+        assert len(s["segments"]) == 48 and len(s["combos"]) == 0
+    else:
+        assert len(s["segments"]) > 48
+
+
 def test_fewer_compute_units_mean_fewer_longer_shares():
     lens = [2048] * 64
     a = schedule(lens, 32, 8, 128, 16, 2048, cus=256)
