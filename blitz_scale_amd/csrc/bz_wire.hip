@@ -132,17 +132,43 @@ __global__ __launch_bounds__(256) void wire_kernel(WireArgs a) {
     }
 }
 
+// A launch has fewer than 2^32 work-items: where the short form would have more (64 GiB of a 16-bit pool at one vector per
+// lane), the four vectors per lane of the general form cover four times as much; what is longer still is refused.
+struct WireLaunch {
+    bool within;
+    uint32_t per, workgroups;
+};
+static int wire_launch_shape(uint64_t total_vecs, uint32_t vecs_per_chunk, bool same_size, WireLaunch* w) {
+    constexpr uint64_t kMost = 0xffffffffull / 256; // workgroups
+    auto workgroups = [&](bool within) {
+        const uint64_t per_wg = 256 * wire_per(within, same_size);
+        return (total_vecs + per_wg - 1) / per_wg;
+    };
+    w->within = vecs_per_chunk % (256 * wire_per(true, same_size)) == 0 && workgroups(true) <= kMost;
+    if (workgroups(w->within) > kMost) return BZ_ERR_UNSUPPORTED;
+    w->per = (uint32_t)wire_per(w->within, same_size);
+    w->workgroups = (uint32_t)workgroups(w->within);
+    return 0;
+}
+
 template <typename PT, typename WT, bool PACK>
 static int launch_wire(const WireArgs& a, hipStream_t s) {
-    constexpr bool same = sizeof(PT) == sizeof(WT);
-    const bool within = a.vecs_per_chunk % (256 * wire_per(true, same)) == 0;
-    const uint64_t per_wg = 256 * wire_per(within, same);
-    const uint64_t grid = (a.total_vecs + per_wg - 1) / per_wg;
-    if (grid == 0) return 0;
-    if (grid > 0x7fffffffull) return BZ_ERR_UNSUPPORTED;
-    if (within) hipLaunchKernelGGL((wire_kernel<PT, WT, PACK, true>), dim3((uint32_t)grid), dim3(256), 0, s, a);
-    else hipLaunchKernelGGL((wire_kernel<PT, WT, PACK, false>), dim3((uint32_t)grid), dim3(256), 0, s, a);
+    WireLaunch w;
+    if (int rc = wire_launch_shape(a.total_vecs, a.vecs_per_chunk, sizeof(PT) == sizeof(WT), &w)) return rc;
+    if (w.workgroups == 0) return 0;
+    if (w.within) hipLaunchKernelGGL((wire_kernel<PT, WT, PACK, true>), dim3(w.workgroups), dim3(256), 0, s, a);
+    else hipLaunchKernelGGL((wire_kernel<PT, WT, PACK, false>), dim3(w.workgroups), dim3(256), 0, s, a);
     BZ_LAUNCH_CHECK();
+    return 0;
+}
+
+// What the two directions look at before anything else: the geometry and the types.
+static int wire_check(const bz_paged_kv_t* kv, int wire_dtype) {
+    if (kv->stride_page == 0 || kv->stride_page % 16 || kv->stride_h == 0 || kv->num_kv_heads == 0) return BZ_ERR_BAD_ARG;
+    if (kv->stride_page / 8 > 0xffffffffull) return BZ_ERR_UNSUPPORTED;
+    const int pd = kv->kv_dtype;
+    if (pd != BZ_F16 && pd != BZ_BF16 && pd != BZ_E4M3) return BZ_ERR_BAD_ARG;
+    if (wire_dtype != pd && !(wire_dtype == BZ_E4M3 && (pd == BZ_F16 || pd == BZ_BF16))) return BZ_ERR_UNSUPPORTED;
     return 0;
 }
 
@@ -153,11 +179,8 @@ static int wire_dispatch(void* pool_base, uint64_t max_pages, const bz_paged_kv_
     if (!kv) return BZ_ERR_BAD_ARG;
     if (num_pages == 0 || layer_cnt == 0) return 0;
     if (!pool_base || !page_ids || !wire) return BZ_ERR_BAD_ARG;
-    if (kv->stride_page == 0 || kv->stride_page % 16 || kv->stride_h == 0 || kv->num_kv_heads == 0) return BZ_ERR_BAD_ARG;
-    if (kv->stride_page / 8 > 0xffffffffull) return BZ_ERR_UNSUPPORTED;
+    if (int rc = wire_check(kv, wire_dtype)) return rc;
     const int pd = kv->kv_dtype;
-    if (pd != BZ_F16 && pd != BZ_BF16 && pd != BZ_E4M3) return BZ_ERR_BAD_ARG;
-    if (wire_dtype != pd && !(wire_dtype == BZ_E4M3 && (pd == BZ_F16 || pd == BZ_BF16))) return BZ_ERR_UNSUPPORTED;
     WireArgs a;
     a.pool = (char*)pool_base;
     a.wire = (char*)wire;
@@ -189,6 +212,19 @@ using namespace bz;
 extern "C" uint64_t bz_kv_wire_bytes(uint32_t num_pages, uint32_t layer_cnt, const bz_paged_kv_t* kv, int wire_dtype) {
     if (!kv) return 0;
     return (uint64_t)num_pages * layer_cnt * kv->stride_page * dtype_bytes(wire_dtype);
+}
+
+extern "C" int bz_kv_wire_launch_shape(uint32_t num_pages, uint32_t layer_cnt, const bz_paged_kv_t* kv, int wire_dtype,
+                                       uint32_t* vectors_per_lane, uint32_t* workgroups) {
+    if (!kv || !vectors_per_lane || !workgroups) return BZ_ERR_BAD_ARG;
+    if (int rc = wire_check(kv, wire_dtype)) return rc;
+    const uint32_t vecs_per_chunk = (uint32_t)(kv->stride_page / 8);
+    WireLaunch w;
+    if (int rc = wire_launch_shape((uint64_t)num_pages * layer_cnt * vecs_per_chunk, vecs_per_chunk, wire_dtype == kv->kv_dtype, &w))
+        return rc;
+    *vectors_per_lane = w.per;
+    *workgroups = w.workgroups;
+    return 0;
 }
 
 extern "C" int bz_kv_pages_pack(const void* pool_base, uint64_t max_pages, const bz_paged_kv_t* kv,

@@ -370,6 +370,11 @@ int bz_batch_find_max(uint32_t* output_indices, const void* input, int dtype, ui
  * it).  Pages listed twice in an unpack race.  Launch only; no allocation, copy or synchronisation.
  * ------------------------------------------------------------------------------------- */
 uint64_t bz_kv_wire_bytes(uint32_t num_pages, uint32_t layer_cnt, const bz_paged_kv_t* kv, int wire_dtype);
+/* How one call of bz_kv_pages_pack / _unpack over so many pages and layers is launched: vectors of eight elements per
+ * lane, workgroups of 256 lanes.  BZ_ERR_UNSUPPORTED for a call that has more work-items than a launch can (256 GiB of a
+ * 16-bit pool, 128 GiB of an fp8 pool).  Host only. */
+int bz_kv_wire_launch_shape(uint32_t num_pages, uint32_t layer_cnt, const bz_paged_kv_t* kv, int wire_dtype,
+                            uint32_t* vectors_per_lane, uint32_t* workgroups);
 int bz_kv_pages_pack(const void* pool_base, uint64_t max_pages, const bz_paged_kv_t* kv, const int32_t* page_ids,
                      uint32_t num_pages, uint32_t start_layer, uint32_t layer_cnt, void* wire, int wire_dtype,
                      const float* k_scale, const float* v_scale, void* stream);

@@ -109,3 +109,24 @@ def test_pool_offsets_beyond_four_gib():
     torch.cuda.synchronize()
     for s_id, d_id in zip(ids_high, dst):
         assert np.array_equal(hp.page_bits(d_id), hp.page_bits(s_id))
+
+
+def test_pack_of_more_than_64_gib():
+    """One call whose launch, at one vector per lane, would have more than 2^32 work-items: a small pool's pages, listed over and
+    over, on a wire of 64 GiB and two pages."""
+    layers, max_pages, sp, pages = 32, 40, 2 * 8 * 16 * 128, 32770
+    if torch.cuda.mem_get_info()[0] < 72 << 30:
+        pytest.skip("needs 72 GiB of device memory")
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(11)
+    pool = torch.randint(-2 ** 15, 2 ** 15, (layers, max_pages, sp), dtype=torch.int16, device="cuda", generator=gen)
+    ids = torch.randint(0, max_pages, (pages,), dtype=torch.int32, device="cuda", generator=gen)
+    wire = torch.empty(pages * layers * sp, dtype=torch.int16, device="cuda")
+    wire[-2 * layers * sp:] = -1
+    pt = K.PageTable(1, 16, 8, 128, pool.view(torch.bfloat16).view(-1))
+    assert K.kv_wire_bytes(pt, pages, layers) == 2 * wire.numel() > 64 << 30
+    K.pack_kv_pages(pt, max_pages, ids, 0, layers, wire)
+    got = wire.view(pages, layers, sp)
+    by_page = pool.transpose(0, 1).contiguous()
+    for lo in range(0, pages, 1024):
+        assert torch.equal(got[lo:lo + 1024], by_page[ids[lo:lo + 1024].long()]), lo
