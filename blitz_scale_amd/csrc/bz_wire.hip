@@ -38,10 +38,12 @@ template <typename T> __device__ __forceinline__ void wire_store(const Vec8<T>& 
 }
 
 // Vectors per lane.  Where a workgroup's vectors all lie in one chunk its address arithmetic is scalar (else every vector
-// pays two 64-bit divisions), and what the lanes then want is few bytes each and many workgroups in flight: five prompts of
-// 400 .. 1 500 tokens, 32 layers, 8 heads, bf16, packed and unpacked (1.36 GB moved by each): 496 us with four vectors and the
-// divisions, 486 with four, 481 with two, 443 (6.1 TB/s) with one; over an e4m3 wire 508, 471 (four), 447 (two), 462 (one).
-constexpr int wire_per(bool within, bool same_size) { return !within ? 4 : (same_size ? 1 : 2); }
+// pays two 64-bit divisions), and what the lanes then want is 16 bytes each and many workgroups in flight: one vector of a
+// 16-bit pool, two where either side has one byte an element.  Five prompts of 400 .. 1 500 tokens, 32 layers, 8 heads, packed
+// and unpacked, us with four vectors and the divisions / four / two / one:
+//   bf16 pool (1.36 GB moved by each) 496 / 486 / 481 / 443 (6.1 TB/s); over an e4m3 wire 508 / 471 / 447 / 462
+//   fp8 pool (0.68 GB) 283 / 261 / 257 / 280; one prompt of 250 19.3 / 18.0 / 16.4 / 17.4
+constexpr int wire_per(bool within, size_t pool_bytes, size_t wire_bytes) { return !within ? 4 : (pool_bytes + wire_bytes == 4 ? 1 : 2); }
 
 struct WireArgs {
     char* pool;            // base of the whole pool (layer 0)
@@ -62,7 +64,7 @@ struct WireArgs {
 // WITHIN: a chunk is a whole number of workgroups' vectors, so a workgroup's chunk, page and addresses are scalar.
 template <typename PT, typename WT, bool PACK, bool WITHIN>
 __global__ __launch_bounds__(256) void wire_kernel(WireArgs a) {
-    constexpr int kPer = wire_per(WITHIN, sizeof(PT) == sizeof(WT));
+    constexpr int kPer = wire_per(WITHIN, sizeof(PT), sizeof(WT));
     const uint64_t g0 = (uint64_t)blockIdx.x * (256 * kPer) + threadIdx.x;
     using ST = typename std::conditional<PACK, PT, WT>::type; // what is read
     using DT = typename std::conditional<PACK, WT, PT>::type; // what is written
@@ -138,15 +140,15 @@ struct WireLaunch {
     bool within;
     uint32_t per, workgroups;
 };
-static int wire_launch_shape(uint64_t total_vecs, uint32_t vecs_per_chunk, bool same_size, WireLaunch* w) {
+static int wire_launch_shape(uint64_t total_vecs, uint32_t vecs_per_chunk, size_t pool_bytes, size_t wire_bytes, WireLaunch* w) {
     constexpr uint64_t kMost = 0xffffffffull / 256; // workgroups
     auto workgroups = [&](bool within) {
-        const uint64_t per_wg = 256 * wire_per(within, same_size);
+        const uint64_t per_wg = 256 * wire_per(within, pool_bytes, wire_bytes);
         return (total_vecs + per_wg - 1) / per_wg;
     };
-    w->within = vecs_per_chunk % (256 * wire_per(true, same_size)) == 0 && workgroups(true) <= kMost;
+    w->within = vecs_per_chunk % (256 * wire_per(true, pool_bytes, wire_bytes)) == 0 && workgroups(true) <= kMost;
     if (workgroups(w->within) > kMost) return BZ_ERR_UNSUPPORTED;
-    w->per = (uint32_t)wire_per(w->within, same_size);
+    w->per = (uint32_t)wire_per(w->within, pool_bytes, wire_bytes);
     w->workgroups = (uint32_t)workgroups(w->within);
     return 0;
 }
@@ -154,7 +156,7 @@ static int wire_launch_shape(uint64_t total_vecs, uint32_t vecs_per_chunk, bool 
 template <typename PT, typename WT, bool PACK>
 static int launch_wire(const WireArgs& a, hipStream_t s) {
     WireLaunch w;
-    if (int rc = wire_launch_shape(a.total_vecs, a.vecs_per_chunk, sizeof(PT) == sizeof(WT), &w)) return rc;
+    if (int rc = wire_launch_shape(a.total_vecs, a.vecs_per_chunk, sizeof(PT), sizeof(WT), &w)) return rc;
     if (w.workgroups == 0) return 0;
     if (w.within) hipLaunchKernelGGL((wire_kernel<PT, WT, PACK, true>), dim3(w.workgroups), dim3(256), 0, s, a);
     else hipLaunchKernelGGL((wire_kernel<PT, WT, PACK, false>), dim3(w.workgroups), dim3(256), 0, s, a);
@@ -220,7 +222,8 @@ extern "C" int bz_kv_wire_launch_shape(uint32_t num_pages, uint32_t layer_cnt, c
     if (int rc = wire_check(kv, wire_dtype)) return rc;
     const uint32_t vecs_per_chunk = (uint32_t)(kv->stride_page / 8);
     WireLaunch w;
-    if (int rc = wire_launch_shape((uint64_t)num_pages * layer_cnt * vecs_per_chunk, vecs_per_chunk, wire_dtype == kv->kv_dtype, &w))
+    if (int rc = wire_launch_shape((uint64_t)num_pages * layer_cnt * vecs_per_chunk, vecs_per_chunk, dtype_bytes(kv->kv_dtype),
+                                   dtype_bytes(wire_dtype), &w))
         return rc;
     *vectors_per_lane = w.per;
     *workgroups = w.workgroups;

@@ -164,31 +164,31 @@ def test_empty_and_rejected_arguments():
         K.pack_kv_pages(pt8, 4, torch.zeros(1, dtype=torch.int32, device="cuda"), 0, 1, wire, wire_dtype=BZ_F16)
 
 
-@pytest.mark.parametrize("wire_dtype", [BZ_BF16, BZ_E4M3])
-@pytest.mark.parametrize("Hkv", [1, 2, 3, 5])
-def test_chunks_at_the_size_of_a_workgroup(wire_dtype, Hkv):
-    """Chunks of 2048 elements times the heads: whole numbers of workgroups' vectors (of 2048 elements for a copy, of 4096
-    where the wire has another type) and not."""
+@pytest.mark.parametrize("dtype,wire_dtype", [(BZ_BF16, BZ_BF16), (BZ_BF16, BZ_E4M3), (BZ_E4M3, BZ_E4M3)])
+@pytest.mark.parametrize("Hkv,P", [(1, 16), (2, 16), (3, 16), (5, 16), (1, 20), (2, 20), (8, 20)])
+def test_chunks_at_the_size_of_a_workgroup(dtype, wire_dtype, Hkv, P):
+    """Chunks of 2048 (pages of 16) and 2560 (20) elements times the heads: whole numbers of workgroups' vectors (of 2048
+    elements where a 16-bit pool is copied, of 4096 where either side is fp8) and not, in each direction."""
     rng = np.random.default_rng(25 + Hkv)
-    layers, max_pages, P, D = 3, 11, 16, 64
-    bits, pool, pt, sp = make(rng, layers, max_pages, Hkv, P, D, BZ_BF16)
+    layers, max_pages, D = 3, 11, 64
+    bits, pool, pt, sp = make(rng, layers, max_pages, Hkv, P, D, dtype)
     _, _, stride_h = wl.strides(BZ_LAYOUT_HND, Hkv, P, D)
     ids = rng.permutation(max_pages)[:5].astype(np.int32)
     scales = rng.uniform(4.0, 5.0, (2, 2, Hkv)).astype(np.float32) / np.float32(448)
     okw, kw = {}, {}
-    if wire_dtype == BZ_E4M3:
+    if wire_dtype != dtype:
         okw = dict(wire_dtype=BZ_E4M3, num_kv_heads=Hkv, stride_h=stride_h, k_scale=scales[0], v_scale=scales[1])
         kw = dict(wire_dtype=BZ_E4M3, k_scale=torch.from_numpy(scales[0]).cuda(), v_scale=torch.from_numpy(scales[1]).cuda())
-    want = oracle.kv_pages_pack(bits, BZ_BF16, max_pages, sp, ids, 1, 2, **okw)
+    want = oracle.kv_pages_pack(bits, dtype, max_pages, sp, ids, 1, 2, **okw)
     wire = wire_tensor(want.nbytes + 64)
     K.pack_kv_pages(pt, max_pages, torch.from_numpy(ids).cuda(), 1, 2, wire, **kw)
     torch.cuda.synchronize()
     got = wire.cpu().numpy()
     assert np.array_equal(got[:want.nbytes], want.view(np.uint8)) and (got[want.nbytes:] == 0xA5).all()
     there = rng.permutation(max_pages)[:5].astype(np.int32)
-    dst_bits = np.full(layers * max_pages * sp, 0x7bcd, bits.dtype)
-    dst = to_dev(dst_bits, BZ_BF16)
+    dst_bits = np.full(layers * max_pages * sp, 0x5a if dtype == BZ_E4M3 else 0x7bcd, bits.dtype)
+    dst = to_dev(dst_bits, dtype)
     K.unpack_kv_pages(K.PageTable(1, P, Hkv, D, dst), max_pages, torch.from_numpy(there).cuda(), 1, 2, wire, **kw)
     torch.cuda.synchronize()
-    oracle.kv_pages_unpack(dst_bits, BZ_BF16, max_pages, sp, there, 1, 2, want, **okw)
+    oracle.kv_pages_unpack(dst_bits, dtype, max_pages, sp, there, 1, 2, want, **okw)
     assert np.array_equal(to_host_bits(dst), dst_bits)

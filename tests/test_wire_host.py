@@ -39,3 +39,8 @@ def test_chunks_that_are_no_whole_number_of_workgroups_take_the_general_form():
     assert launch_shape(10, 2, 3, 4, 8, BZ_F16, BZ_F16)[1:3] == (4, 1)  # 24 vectors per chunk
     assert launch_shape(10, 2, 3, 16, 64, BZ_BF16, BZ_E4M3)[1] == 4     # 768: no multiple of 512
     assert launch_shape(10, 2, 4, 16, 64, BZ_BF16, BZ_E4M3)[1] == 2
+
+
+@pytest.mark.parametrize("dtype,wire,per", [(BZ_BF16, BZ_BF16, 1), (BZ_F16, BZ_F16, 1), (BZ_F16, BZ_E4M3, 2), (BZ_E4M3, BZ_E4M3, 2)])
+def test_a_lane_moves_16_bytes_of_the_narrower_side(dtype, wire, per):
+    assert launch_shape(1000, 32, 8, 16, 128, dtype, wire)[:2] == (0, per)
