@@ -88,21 +88,33 @@ static int build_schedule(DecodePlan* p, const int32_t* indptr_h, const int32_t*
     while (!never_split && piece > min_pages && count_items(piece) < (uint64_t)cus * 4)
         piece = std::max(min_pages, piece / 2);
     piece = std::min(piece, longest_pages);
-    // What halving comes to is often some rounds of workgroups and a part of one (two find a place on a compute unit, by the
-    // registers of groups of two and more; single q heads, three or four to a unit, are left as they are).  Pieces that come to
-    // one, two or three rounds are taken instead where that is sure to end sooner: a workgroup takes the tokens of its piece
-    // and about 256 more to begin and to end; the rounds take the mean piece each, the last one the longest.
+    // What halving comes to is often some rounds of workgroups and a part of one.  Pieces that come to one, two or three rounds
+    // are taken instead where that is sure to end sooner: a workgroup takes the tokens of its piece and about 256 more to begin
+    // and to end; the rounds take the mean piece each, the last one the longest.
+    // Places on a compute unit, by the registers of the kernel that will run: two for groups of four in every form and for
+    // groups of eight with the angle table or over fp8 pools of heads of 64; one for other groups of eight, whose rounds of two
+    // are full rounds of one as well; groups of two (and six, ten: workgroups of two heads) three with the angle table and over
+    // fp8 pools, which is what comes here with heads of 64 in pages of whole sixteens, else two or three.  Single q heads, three or
+    // four to a unit, are left as they are.
     // Sequences of 200 .. 2 048 tokens, 32/8 heads, whole calls, us (halving alone in brackets): 48 with raw K 65.9 (70.4), with
     // pages of 8 tokens 68.1 (84.4), with heads of 64 over an fp8 pool 50.6 (64.2); 30 with pages of 8 43.5 (61.0), raw K 46.5
-    // (51.7); 24 raw K 39.7 (45.7); 30 with 64/8 heads and pages of 8 80.0 (109.1); 48 of 2 000 .. 6 000, raw K, 164 (171).  An
-    // eighth is asked for because lengths that differ much make the estimate worth less: 100 with raw K go from 120 to 124 in
-    // two rounds, 70 with 64/8 heads from 126 to 129.
-    const uint32_t group = num_qo_heads / num_kv_heads;
-    const uint32_t longest_piece = std::min(max_pages_cap, longest_pages);
-    if (!never_split && piece < longest_piece && group % 2 == 0) {
+    // (51.7); 24 raw K 39.7 (45.7); 30 with 64/8 heads and pages of 8 80.0 (109.1); 48 of 2 000 .. 6 000, raw K, 164 (171).
+    // Where the estimate is not good enough, by about 700 batches timed with and without these pieces:
+    //   an eighth is asked for, two ninths where halving ends at pieces of more than 512 tokens, or over raw-K rows of 128 at more
+    //     than 256: those differ in length, so that a part of a round fills up by itself (90 sequences, 32/8 heads, 109 -> 116 us
+    //     over a raw-K cache, 110 -> 112 in pages of 8; 42 with 64/16 heads, raw K, 101 -> 108);
+    //   over raw-K rows of 128, rounds are not cut to less than a third (42 with 64/8 heads, three rounds to one: 90 -> 93; to two:
+    //     82);
+    //   workgroups of two heads over raw-K rows of 128 keep the halving (half of the choices gained 2 to 12 %, half lost as much,
+    //     in rounds of two and of three places: 60 with 48/8 heads 163 -> 199, 20 with 40/4 heads 54 -> 60).  Of heads of 64 the
+    //     planner cannot tell a raw-K cache, 5 % faster in the mean of 68 batches (20 with 40/4 heads 38.7 -> 41.0, the worst), from
+    //     an fp8 pool, 21 % faster.
+    const uint32_t group = num_qo_heads / num_kv_heads, longest_piece = std::min(max_pages_cap, longest_pages);
+    const bool whole16 = page_size % 16 == 0, raw_rows = head_dim == 128 && whole16; // (the matrix-core kernel takes the other calls)
+    if (!never_split && piece < longest_piece && group % 2 == 0 && !(group % 4 && raw_rows)) {
         // (the dispatch splits groups of more than eight, and those that are no power of two)
         const uint64_t wgs_per_kv_head = group % 8 == 0 ? group / 8 : group % 4 == 0 ? group / 4 : group / 2;
-        const uint64_t places = (uint64_t)cus * 2, heads = num_kv_heads * wgs_per_kv_head;
+        const uint64_t places = (uint64_t)cus * (group % 4 && whole16 ? 3 : 2), heads = num_kv_heads * wgs_per_kv_head;
         auto time_of = [&](uint32_t pc) { // in tokens
             uint64_t n = 0, pages = 0;
             uint32_t longest = 0;
@@ -120,9 +132,10 @@ static int build_schedule(DecodePlan* p, const int32_t* indptr_h, const int32_t*
         };
         const uint32_t halved = piece;
         const uint64_t wgs_halved = count_items(halved) * wgs_per_kv_head, wgs_longest = count_items(longest_piece) * wgs_per_kv_head;
-        uint64_t best = time_of(halved) * 7 / 8;
+        const bool uneven = (uint64_t)halved * page_size > 512 || (raw_rows && halved > min_pages);
+        uint64_t best = time_of(halved) * 7 / (uneven ? 9 : 8);
         for (uint32_t rounds = 1; rounds <= 3 && wgs_halved > rounds * places; ++rounds) {
-            if (wgs_longest > rounds * places) continue;
+            if (wgs_longest > rounds * places || (raw_rows && wgs_halved > 3 * rounds * places)) continue;
             uint32_t lo = halved, hi = longest_piece; // the shortest pieces that come to so many rounds
             while (lo < hi) {
                 const uint32_t mid = lo + (hi - lo) / 2;

@@ -194,6 +194,30 @@ def test_general_pieces_that_fill_the_chip(batch, Hq, Hkv, P, rounds):
         assert sizes.max() <= halved
 
 
+@pytest.mark.parametrize("batch,Hq,Hkv,D,P,places,rounds", [
+    (48, 32, 8, 128, 16, 2, 2),   # rows of 128 in pages of whole sixteens: raw-K calls, groups of four
+    (42, 64, 8, 128, 16, 2, 2),   # from three rounds and a bit to two, not to one
+    (60, 48, 8, 128, 16, 2, 0),   # workgroups of two heads over raw-K rows
+    (24, 16, 8, 128, 16, 2, 0),
+    (24, 16, 8, 64, 16, 3, 1),    # heads of 64: three workgroups of two heads to a compute unit
+    (24, 16, 8, 64, 8, 2, 1),     # pages of 8: two
+    (90, 32, 8, 64, 8, 2, 0),     # halving ends at pieces of up to 1024 tokens, which differ in length
+])
+def test_general_pieces_by_the_kernel_that_runs(batch, Hq, Hkv, D, P, places, rounds):
+    lens = np.random.default_rng(0x5EED).integers(200, 2049, size=batch)
+    s = schedule(lens, Hq, Hkv, D, P)
+    check_general_schedule(s, P)
+    sizes, group = s["segments"][:, 2] - s["segments"][:, 1], Hq // Hkv
+    wgs = len(sizes) * Hkv * (group // next(g for g in (8, 4, 2) if group % g == 0))
+    halved = 2048 // P
+    while halved > 256 // P and Hkv * sum(-(-int(n) // (halved * P)) for n in lens) < 4 * CUS:
+        halved = max(256 // P, halved // 2)
+    if rounds:
+        assert sizes.max() > halved and 0.9 * rounds * places * CUS < wgs <= rounds * places * CUS
+    else:
+        assert sizes.max() <= halved
+
+
 @pytest.mark.parametrize("P", [1, 3, 16])
 @pytest.mark.parametrize("split", [0x7FFFFFFF, 0x80000000, 0xFFFFFF00, 0xFFFFFFFE, 0xFFFFFFFF])
 def test_piece_lengths_up_to_the_largest_of_their_type(split, P):
