@@ -944,7 +944,7 @@ __global__ __launch_bounds__(D / 4 * HB * S) void decode_step_finish_kernel(cons
     const bool upper = d0 >= D / 2;           // they are the second elements of their rotate-half pairs
     const uint32_t i0 = d0 & (D / 2 - 1), dp = upper ? d0 - D / 2 : d0 + D / 2;
     // Everything that depends on the unit record alone is requested at once: the caller's rows, the scales
-    // and the first four partial results of this slice.  (The sequence's length and its place in the page
+    // and the first NB partial results of this slice.  (The sequence's length and its place in the page
     // list come with the unit record, from the host table the plan was made from, like the lengths the
     // decode kernel works with.)
     const int seq_len = u.seq_len - max(ahead_raw, 0);
@@ -1178,7 +1178,9 @@ template <typename QT, typename PT, typename OT, int D>
 static int launch_step_finish(const DecodePlan* p, const StepFinishArgs& a, hipStream_t s) {
     // Heads of a unit per workgroup, and slices over its partials.  Every batch of partials that a slice loads is a memory
     // round trip behind the last one, so a unit's partials are spread over slices until one round holds them, where the
-    // launch is small enough that the additional waves cost less than the round trips.  (us, with the shapes that came out second.)
+    // launch is small enough that the additional waves cost less than the round trips: all units get the shape that the
+    // largest asks for, and one long sequence among many short ones makes a large launch whose waves mostly find nothing to
+    // load.  (us, with the shapes that came out second; rows: units times heads of a unit; heads 32/8 if not said.)
     //   up to 4 partials, or up to 16 in a launch of more than 256 units (large batches): one slice; heads 4 at a time where the
     //     group allows it (two waves), else 2 (one wave), 1 for single heads.  Four slices there: 40 sequences of 500 .. 900
     //     tokens (320 units) 27.8 against 27.5, 96 of 600 .. 1 100 66.5 against 64.3.
@@ -1186,12 +1188,18 @@ static int launch_step_finish(const DecodePlan* p, const StepFinishArgs& a, hipS
     //     903 -> 872; 4 sequences of 32 single heads, 600 .. 900 tokens, 18.4 -> 16.6 (one head per workgroup; 16.8 with two).
     //   17 .. 32 (batches of eight sequences or so): four slices with eight partials to a batch, one head per workgroup.  9 sequences
     //     of 1 000 .. 3 000 tokens over an fp8 pool 18.0 -> 17.5, 32 layers of 12 of 1 000 .. 1 400 688 -> 685 (eight slices of four
-    //     before; those with two and four heads per workgroup: 32 layers at batch 8 497 against 505 and 527).
-    //   33 .. 64: eight slices with eight partials to a batch.  32 layers of 4 x 1 500 tokens 538 -> 491, of 2 x 1 500 427 -> 396; 4 x
-    //     9 000 34.2 -> 32.5 (four slices of four for two heads before; sixteen slices: 505, 412, 33.0).
-    //   more (few long sequences): sixteen slices of eight, one round up to 128.  32 layers of 1 x 8 000 tokens 669 -> 571; 1 x
-    //     131 072 94.4 -> 91.5; two of 40 001 .. 90 001, 64/8 heads, 77.0 -> 75.3; 1 x 30 000 with 4/1 heads 30.1 -> 16.0.  (Eight
-    //     slices of four before.  Thirty-two of eight from 129 partials on: as fast as sixteen.)
+    //     before; those with two and four heads per workgroup: 32 layers at batch 8 497 against 505 and 527).  127 of 500 and one of
+    //     7 000: 60.6 (eight slices of four 63.8, sixteen of eight 80.6).
+    //   33 .. 64, up to 512 rows: eight slices with eight partials to a batch.  32 layers of 4 x 1 500 tokens 538 -> 491, of 2 x 1 500
+    //     427 -> 396; 4 x 9 000 34.2 -> 32.5 (four slices of four for two heads before; sixteen slices: 505, 412, 33.0).
+    //   more, up to 256 rows, or 512 with more than 128 partials (few long sequences): sixteen slices of eight, one round up to 128.
+    //     32 layers of 1 x 8 000 tokens 669 -> 571; 1 x 131 072 94.4 -> 91.5; 1 x 30 000 with 4/1 heads 30.1 -> 16.0; one of 30 000
+    //     and 7 of 300 34.8 -> 32.6, and 15 of 500 34.7 -> 33.5 (eight slices of four before).
+    //   65 and more, up to 1 024 rows: eight slices of eight.  20 of 700 and one of 9 000 26.2 .. 26.6 (sixteen 28.5, eight of four 26.5), 31
+    //     of 300 and one of 30 000 43.9 (45.2, 44.9), 200 of 200 and one of 20 000, 4/1 heads, 20.4 (21.2, 23.0).
+    //   33 and more in the launches that are left: four slices of eight, two heads per workgroup.  30 of 500 and one of 5 000 24.2
+    //     (eight slices of eight 24.8, four of four 25.2); 63 of 800 and one of 30 000 62.5 .. 64.0 (sixteen slices 71.5, eight of four 63.8);
+    //     127 of 500 and one of 32 768 79.8 (99.6, 83.3), 255 of 300 and one of 60 000 109 (150, 116).
     const uint32_t G = a.group;
     auto launch = [&](auto s_c, auto hb_c, auto nb_c) {
         constexpr int S = decltype(s_c)::value, HB = decltype(hb_c)::value, NB = decltype(nb_c)::value; // NB: partials per batch of loads
@@ -1212,10 +1220,17 @@ static int launch_step_finish(const DecodePlan* p, const StepFinishArgs& a, hipS
         else launch(c4, c1, c4);
     } else if (p->mfma_unit_max_count <= 32) {
         launch(c4, c1, c8);
-    } else if (p->mfma_unit_max_count <= 64) {
-        launch(c8, c1, c8);
     } else {
-        launch(c16, c1, c8);
+        const uint32_t most = p->mfma_unit_max_count;
+        const uint64_t rows = (uint64_t)p->mfma_units * G;
+        if (rows > (most <= 64 ? 512 : 1024)) {
+            if (G >= 2) launch(c4, c2, c8);
+            else launch(c4, c1, c8);
+        } else if (most <= 64 || rows > (most <= 128 ? 256 : 512)) {
+            launch(c8, c1, c8);
+        } else {
+            launch(c16, c1, c8);
+        }
     }
     BZ_LAUNCH_CHECK();
     return 0;

@@ -262,3 +262,15 @@ def test_step_at_the_edge_of_a_large_launch(tiles, batch):
     dev, _, _ = run_step(DecodeProblem(430 + tiles, [32 * tiles] * batch, 4, 2, 128, 16, BZ_BF16), split_tokens=32)
     units = dev.handler.host_schedule(7)
     assert len(units) == 2 * batch and units[:, 3].max() == tiles
+
+
+@pytest.mark.parametrize("heads", [(16, 2), (10, 2), (2, 2)])
+@pytest.mark.parametrize("tiles,rows", [(33, 512), (33, 528), (64, 512), (64, 528), (65, 256), (65, 272), (65, 1024), (65, 1040),
+                                        (128, 512), (129, 512), (129, 528)])
+def test_step_of_one_long_sequence_among_short_ones(tiles, rows, heads):
+    """The finishing kernel's shape by the largest unit and by the rows of the launch (units times heads of a unit), on both sides
+    of every change: one unit of many partials, the others of one, in each shape's full and ragged groups of heads."""
+    batch = rows // heads[0]  # (rows of the launch: q heads times sequences)
+    dev, _, _ = run_step(DecodeProblem(440 + tiles, [20] * (batch - 1) + [32 * tiles], *heads, 128, 16, BZ_BF16), split_tokens=32)
+    units = dev.handler.host_schedule(7)
+    assert len(units) == heads[1] * batch and units[:, 3].max() == tiles and (units[:, 3] == 1).sum() == len(units) - heads[1]
