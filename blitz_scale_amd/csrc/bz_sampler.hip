@@ -18,11 +18,11 @@
 namespace bz {
 
 // grid (rows), block 256: row r of dst <- row src_row(r) of src, hidden % 8 == 0 elements of 2 bytes.
-// HBM-bound.  A row of the table is seldom wanted twice: non-temporal loads leave the caches to the rows going out, which the
-// first layer reads next; the last tokens' rows have just been written and are read as they are.  (A condition on two kinds of
-// loads in one kernel makes both plain.)  Embedding of 8 192 rows of 4 096 with the gather and the argmax behind it 34.8 -> 30.4
-// us, of 8 192 66.2 -> 63.1.  (Non-temporal stores as well: 32.0 and 56.3; four loads at a time: no difference.)
-template <bool TABLE> // rows of the embedding table, or the last tokens' rows of a batch
+// HBM-bound.  Plain loads: a few hundred tokens make up half of a text, and their rows of the table come from the caches from
+// the second time on.  Embedding, last-token gather and argmax over 8 192 tokens, ids by rank (1 / (rank + 2.7)), 128 256 rows, us
+// with plain and with non-temporal loads of the table: rows of 4 096 33.6 and 34.6, of 8 192 54.8 and 64.3, 1 500 rows of 5 120
+// 24.5 and 26.2, with the norm that reads the rows next 57.3 and 61.6, 107 and 104, 33.9 and 34.4.  (Where every row is wanted
+// once, as with ids drawn evenly, non-temporal loads are the faster: 40.1 and 33.6, 65.9 and 62.9, 25.0 and 24.2.)
 __global__ __launch_bounds__(256) void gather_rows_kernel(uint4* __restrict__ dst, const uint4* __restrict__ src,
                                                            const uint32_t* __restrict__ token_ids,
                                                            const int32_t* __restrict__ out_loc,
@@ -30,22 +30,16 @@ __global__ __launch_bounds__(256) void gather_rows_kernel(uint4* __restrict__ ds
                                                            uint32_t row_vecs) {
     const uint32_t r = blockIdx.x;
     int64_t s, d = r;
-    if constexpr (!TABLE) { // last token of request r; a request without tokens yields a zero row
+    if (ragged_indptr) { // last token of request r; a request without tokens yields a zero row
         s = (int64_t)ragged_indptr[r + 1] - 1;
         if (ragged_indptr[r + 1] <= ragged_indptr[r]) s = -1;
     } else {
         s = token_ids[r];
         if (out_loc) d = out_loc[r];
     }
-    typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
-    u32x4* drow = reinterpret_cast<u32x4*>(dst + (size_t)d * row_vecs);
-    const u32x4* srow = reinterpret_cast<const u32x4*>(src + (size_t)max(s, (int64_t)0) * row_vecs);
-    for (uint32_t i = threadIdx.x; i < row_vecs; i += blockDim.x) {
-        u32x4 v = {0, 0, 0, 0};
-        if constexpr (TABLE) v = __builtin_nontemporal_load(srow + i);
-        else if (s >= 0) v = srow[i];
-        drow[i] = v;
-    }
+    uint4* drow = dst + (size_t)d * row_vecs;
+    for (uint32_t i = threadIdx.x; i < row_vecs; i += blockDim.x)
+        drow[i] = s >= 0 ? src[(size_t)s * row_vecs + i] : make_uint4(0, 0, 0, 0);
 }
 
 template <typename T> __device__ __forceinline__ float elem_f32(uint16_t bits);
@@ -158,7 +152,7 @@ extern "C" int bz_embedding(void* output, const uint32_t* token_ids, const int32
     if (int rc = check_rows(output, weight, dtype, hidden_size)) return rc;
     if (!token_ids) return BZ_ERR_BAD_ARG;
     if (num_tokens == 0) return 0;
-    hipLaunchKernelGGL(gather_rows_kernel<true>, dim3(num_tokens), dim3(256), 0, (hipStream_t)stream, (uint4*)output,
+    hipLaunchKernelGGL(gather_rows_kernel, dim3(num_tokens), dim3(256), 0, (hipStream_t)stream, (uint4*)output,
                        (const uint4*)weight, token_ids, out_loc, (const int32_t*)nullptr, hidden_size / 8);
     BZ_LAUNCH_CHECK();
     return 0;
@@ -170,7 +164,7 @@ extern "C" int bz_gather_last_token(void* output, const void* tokens, const int3
     if (int rc = check_rows(output, tokens, dtype, hidden_size)) return rc;
     if (!ragged_indptr) return BZ_ERR_BAD_ARG;
     if (batch_size == 0) return 0;
-    hipLaunchKernelGGL(gather_rows_kernel<false>, dim3(batch_size), dim3(256), 0, (hipStream_t)stream, (uint4*)output,
+    hipLaunchKernelGGL(gather_rows_kernel, dim3(batch_size), dim3(256), 0, (hipStream_t)stream, (uint4*)output,
                        (const uint4*)tokens, (const uint32_t*)nullptr, (const int32_t*)nullptr, ragged_indptr,
                        hidden_size / 8);
     BZ_LAUNCH_CHECK();
