@@ -22,7 +22,7 @@ def _close(got_bits, ref_f32, dtype):
 
 
 @pytest.mark.parametrize("dtype", [BZ_F16, BZ_BF16])
-@pytest.mark.parametrize("N,h", [(64, 4096), (1, 4096), (7, 5120), (3, 8192), (5, 256), (2, 11008)])
+@pytest.mark.parametrize("N,h", [(64, 4096), (1, 4096), (7, 5120), (3, 8192), (3, 8200), (5, 256), (2, 11008)])
 def test_rms_norm(dtype, N, h):
     rng = np.random.default_rng(60 + N)
     x, w = wl.randn_bits(rng, (N, h), dtype), wl.randn_bits(rng, (h,), dtype, mean=1.0, std=0.02)
@@ -40,7 +40,7 @@ def test_rms_norm(dtype, N, h):
 
 
 @pytest.mark.parametrize("dtype", [BZ_F16, BZ_BF16])
-@pytest.mark.parametrize("N,h", [(64, 4096), (3, 5120)])
+@pytest.mark.parametrize("N,h", [(64, 4096), (3, 5120), (2, 8192), (2, 8200), (3, 16384)])  # (the row in registers up to 8192)
 def test_add_rms_norm(dtype, N, h):
     rng = np.random.default_rng(70)
     x, r = wl.randn_bits(rng, (N, h), dtype), wl.randn_bits(rng, (N, h), dtype)
