@@ -19,7 +19,7 @@ from blitz_scale_amd import workloads as wl
 from blitz_scale_amd._lib import BZ_BF16, BZ_E4M3, BZ_F16, BZ_F32, BZ_LAYOUT_HND, BZ_LAYOUT_NHD, BZ_ROPE_NONE, BZ_ROPE_Q_ONLY
 
 from _gpu import TORCH_OF, DeviceDecode, to_dev, to_host_bits, to_host_f32
-from _util import DecodeProblem, ulp_tol
+from _util import DecodeProblem, dense_attention_f64, ulp_tol
 
 pytestmark = pytest.mark.gpu
 
@@ -274,3 +274,29 @@ def test_step_of_one_long_sequence_among_short_ones(tiles, rows, heads):
     dev, _, _ = run_step(DecodeProblem(440 + tiles, [20] * (batch - 1) + [32 * tiles], *heads, 128, 16, BZ_BF16), split_tokens=32)
     units = dev.handler.host_schedule(7)
     assert len(units) == heads[1] * batch and units[:, 3].max() == tiles and (units[:, 3] == 1).sum() == len(units) - heads[1]
+
+
+@pytest.mark.parametrize("P,bound", [
+    (16, 2.0 ** -16),  # bf16 head + tail of q and of the probabilities: 2^-17 of a logit and 2^-17 of a weight
+    (8, 2.0 ** -20),   # the general kernel and its combine: fp32 throughout, sums of 128 products and of thousands of tokens
+])
+@pytest.mark.parametrize("ctx", [[8000], [1500] * 4, [100] * 140 + [9000]])
+def test_fp32_rows_against_float64(ctx, P, bound):
+    """2-norm of the error of fp32 rows against float64, with many partials per unit in each shape of the finishing kernel."""
+    p = DecodeProblem(460, ctx, 8, 2, 128, P, BZ_BF16)
+    rng = np.random.default_rng(461)
+    k, v = (to_dev(wl.randn_bits(rng, (p.B, p.Hkv, p.D), p.dtype), p.dtype) for _ in range(2))
+    dev = DeviceDecode(p, float_ws_bytes=128 << 20)
+    dev.plan()
+    assert dev.handler.step_form() == ("one_call" if P == 16 else "two_calls")
+    out = torch.full((p.B, p.Hq, p.D), float("nan"), dtype=torch.float32, device="cuda")
+    K.decode_step(dev.handler, dev.q, k, v, dev.pt, out, p.Hq, rope=False)
+    torch.cuda.synchronize()
+    p.pool = to_host_bits(dev.pool)
+    q, num, den = wl.to_f32(p.q, p.dtype), 0.0, 0.0
+    for b, got in enumerate(out.cpu().numpy().astype(np.float64)):
+        if len(ctx) > 100 and 4 <= b < 138:
+            continue
+        ref = dense_attention_f64(q[b], *p.gather_kv(b), p.D ** -0.5)
+        num, den = num + ((got - ref) ** 2).sum(), den + (ref ** 2).sum()
+    assert num <= bound ** 2 * den
