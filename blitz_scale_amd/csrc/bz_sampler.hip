@@ -22,7 +22,8 @@ namespace bz {
 // the second time on.  Embedding, last-token gather and argmax over 8 192 tokens, ids by rank (1 / (rank + 2.7)), 128 256 rows, us
 // with plain and with non-temporal loads of the table: rows of 4 096 33.6 and 34.6, of 8 192 54.8 and 64.3, 1 500 rows of 5 120
 // 24.5 and 26.2, with the norm that reads the rows next 57.3 and 61.6, 107 and 104, 33.9 and 34.4.  (Where every row is wanted
-// once, as with ids drawn evenly, non-temporal loads are the faster: 40.1 and 33.6, 65.9 and 62.9, 25.0 and 24.2.)
+// once, as with ids drawn evenly, non-temporal loads are the faster: 40.1 and 33.6, 65.9 and 62.9, 25.0 and 24.2.  Non-temporal
+// stores help the gather, 21.6 -> 17.6 us for 8 192 rows of 4 096 by rank, and cost the norm behind it more: 43.7 -> 46.2.)
 __global__ __launch_bounds__(256) void gather_rows_kernel(uint4* __restrict__ dst, const uint4* __restrict__ src,
                                                            const uint32_t* __restrict__ token_ids,
                                                            const int32_t* __restrict__ out_loc,
