@@ -110,6 +110,7 @@ struct PrefillArgs {
     const float4* rope_table; // ROPE_Q: [32 couples of pairs][rope_pitch positions] x (cos i, sin i, cos i+1, sin i+1), i even
     uint32_t rope_pitch;
     uint32_t num_qo_heads, num_kv_heads;
+    uint32_t group_inv; // ceil(2^32 / (q heads per kv head)): a q head's kv head is the upper half of the product; 0 without groups
     // Grouped-query attention: log2 of the heads whose tiles are worked on in slices of rows (0, 1 or 2: sets of 1, 2 or
     // 4 q heads of one kv head).  A workgroup that takes 32 rows of four heads instead of 128 rows of one reads the same
     // K/V tiles for as many rows, but its waves end on the same diagonal tile -- with 128 consecutive rows three of the
@@ -183,7 +184,7 @@ __device__ __forceinline__ uint32_t& pf_u4(uint4& v, int i) { return reinterpret
 // global -> LDS with LDS-direct loads, kSNK (K) and kSNV (V) tiles deep, two to three tiles (about two
 // microseconds) ahead of their first read; there is one workgroup barrier per tile, at the top of the iteration,
 // where the tiles read next are published and the buffers of the tiles just finished are handed back to the
-// copies.  The steady state (`full`) has no conditions in it; everything ragged or masked goes through `generic`.
+// copies.  The steady state (`full`) has no conditions in it; everything ragged or masked goes through `tail`.
 //
 // Softmax without a maximum per tile: q rows that are rotated here carry sm_scale * log2(e) in the one rounding of
 // the rotated row (rows that arrive as they are keep their bits and the scale stays on the score), and the first
@@ -212,7 +213,7 @@ constexpr int kSTile = kSN * 256;            // bytes of one K or V tile in LDS
 #define BZ_PF_NV 4
 #endif
 constexpr int kSNK = BZ_PF_NK, kSNV = BZ_PF_NV; // K and V tiles in flight per workgroup
-constexpr int kSLds = (kSNK + kSNV) * kSTile;   // 65 536 bytes per workgroup: K slots, then V slots
+constexpr int kSLds = (kSNK + kSNV + 1) * kSTile; // 73 728 bytes per workgroup: K slots, V slots, and one more for q rows
 static_assert(kSNK == 4 && kSNV == 4, "the steady state is unrolled over four slots");
 
 __device__ __forceinline__ void lds_direct_load16x2(const char* uniform_base, uint32_t o0, uint32_t o1, uint32_t lds_addr) {
@@ -226,20 +227,13 @@ __device__ __forceinline__ void lds_direct_load16x2(const char* uniform_base, ui
 // Loads the compiler keeps no count of: the kernel waits for them itself (sp_wait_copies counts them like copies),
 // so that a wait for the q rows does not become a wait for every tile copy in flight.  The registers must not be
 // read before sp_loads_arrived() has been passed over them.
-__device__ __forceinline__ uint4 sp_load16(const void* p) {
+__device__ __forceinline__ uint4 sp_load16_at(const char* uniform_base, uint32_t lane_offset) {
     typedef uint32_t __attribute__((ext_vector_type(4))) u32x4;
     u32x4 r;
-    asm volatile("global_load_dwordx4 %0, %1, off" : "=v"(r) : "v"(p) : "memory");
+    asm volatile("global_load_dwordx4 %0, %1, %2" : "=v"(r) : "v"(lane_offset), "s"(uniform_base) : "memory");
     return make_uint4(r.x, r.y, r.z, r.w);
 }
-__device__ __forceinline__ float2 sp_load8(const void* p) {
-    typedef float __attribute__((ext_vector_type(2))) f32x2;
-    f32x2 r;
-    asm volatile("global_load_dwordx2 %0, %1, off" : "=v"(r) : "v"(p) : "memory");
-    return make_float2(r.x, r.y);
-}
 __device__ __forceinline__ void sp_loads_arrived(uint4& r) { asm volatile("" : "+v"(r.x), "+v"(r.y), "+v"(r.z), "+v"(r.w)); }
-__device__ __forceinline__ void sp_loads_arrived(float2& r) { asm volatile("" : "+v"(r.x), "+v"(r.y)); }
 
 // workgroup barrier that the compiler moves no memory access across (it waits for nothing by itself)
 __device__ __forceinline__ void sp_barrier() {
@@ -270,27 +264,18 @@ template <int BEHIND> __device__ __forceinline__ void sp_wait_lds() {
 }
 // Copies are issued in pairs (K(i + kSNK), V(i + kSNV - 1)) at the top of iteration i, the first kSNK pairs
 // (i = -kSNK .. -1, tiles below 0 left out) in the prologue.  The tiles first read in iteration j are K(j+2) and
-// V(j); with V_NEXT also V(j+1), which is then converted in place during iteration j.  This counts the copies that
-// exist (tile < n) behind the last of them, up to those of iteration j-1.
-__device__ __forceinline__ int sp_copies_behind(int j, int n, bool v_next) {
-    const int pk = 2 * (j + 2 - kSNK), pv = 2 * (j + 1 - kSNV) + 1; // positions of K(j+2), V(j) in the issue order
-    int p = max(pk, pv);
-    if (v_next && j + 1 < n) p = max(p, pv + 2);
-    int c = 0;
-    for (int pos = p + 1; pos <= 2 * j - 1; ++pos) {
-        const int i = pos >> 1; // (arithmetic shift: positions may be negative in the first iterations)
-        const int tile = (pos & 1) ? i + kSNV - 1 : i + kSNK;
-        c += (tile >= 0 && tile < n) ? 1 : 0;
-    }
-    return c;
+// V(j); with V_NEXT also V(j+1), which is then converted in place during iteration j.  Behind the last of them were
+// issued, up to iteration j-1, V(j+1) (without V_NEXT), K(j+3) and V(j+2): as many of them are in flight as there are
+// tiles left, `left` = n - 1 - j behind tile j.
+constexpr int sp_copies_behind_steady(bool v_next) { return v_next ? 2 : 3; } // every tile exists
+template <bool V_NEXT> __device__ __forceinline__ void sp_wait_tail(int left) {
+    constexpr int kMost = sp_copies_behind_steady(V_NEXT);
+    const int behind = left - (V_NEXT ? 1 : 0);
+    if (behind >= kMost) sp_wait_copies(kMost);
+    else if (behind <= 0) sp_wait_copies(0);
+    else if (behind == 1) sp_wait_copies(1);
+    else sp_wait_copies(2);
 }
-constexpr int sp_copies_behind_steady(bool v_next) { // the same when every tile exists
-    const int pk = 2 * (2 - kSNK), pv = 2 * (1 - kSNV) + 1;
-    int p = pk > pv ? pk : pv;
-    if (v_next && pv + 2 > p) p = pv + 2;
-    return -1 - p;
-}
-__device__ __forceinline__ int sp_wrap(int x, int m) { return x >= m ? x - m : x; } // x < 2 m
 
 #ifdef BZ_PF_TIMING
 // Diagnostic build: every workgroup leaves the shader clock at a few points of its life in bz_pf_wg (read
@@ -352,7 +337,7 @@ __global__ __launch_bounds__(256, 2) void prefill_kernel(PrefillArgs a, const ch
     const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int head = it.head - sub + (wv & set_mask);
     const int Hq = (int)a.num_qo_heads, Hkv = (int)a.num_kv_heads;
-    const int kvh = head / (Hq / Hkv);
+    const int kvh = a.group_inv ? (int)__umulhi((uint32_t)head, a.group_inv) : head; // head / (Hq / Hkv)
     const int qn = lane & 31, h = lane >> 5;
     // Lq q rows attend to L K/V rows (L >= Lq); q row i of the request sits at position off + i: it sees, when
     // causal, the tokens up to that position, and is rotated by that position.
@@ -390,77 +375,114 @@ __global__ __launch_bounds__(256, 2) void prefill_kernel(PrefillArgs a, const ch
     const char* const v_wave = v_ptr + kv_row0 + (size_t)(8 * wv) * row_stride;
     const uint32_t m0_wave = lds0 + (uint32_t)(8 * wv * 256);
     const size_t tile_stride = (size_t)kSN * row_stride;
-    // a whole tile inside the request: one wave-uniform base, lane constants for the rest
-    auto issue_k_fast = [&](int t, int slot) __attribute__((always_inline)) {
-        lds_direct_load16x2(k_wave + (size_t)t * tile_stride, kfast[0], kfast[1], m0_wave + (uint32_t)(slot * kSTile));
+    // a whole tile inside the request: one wave-uniform base (this wave's first row of the tile), lane constants for the rest
+    auto issue_k_fast = [&](const char* rows, int slot) __attribute__((always_inline)) {
+        lds_direct_load16x2(rows, kfast[0], kfast[1], m0_wave + (uint32_t)(slot * kSTile));
     };
-    auto issue_v_fast = [&](int t, int slot) __attribute__((always_inline)) {
-        lds_direct_load16x2(v_wave + (size_t)t * tile_stride, vfast[0], vfast[1], m0_wave + (uint32_t)((kSNK + slot) * kSTile));
+    auto issue_v_fast = [&](const char* rows, int slot) __attribute__((always_inline)) {
+        lds_direct_load16x2(rows, vfast[0], vfast[1], m0_wave + (uint32_t)((kSNK + slot) * kSTile));
     };
-    auto issue_k = [&](int t, int slot) __attribute__((always_inline)) {
-        if ((t + 1) * kSN <= L) {
-            issue_k_fast(t, slot);
-        } else { // rows past the end of the request re-read its last row (masked later)
-            const char* base = k_ptr + kv_row0 + (size_t)t * tile_stride;
-            const uint32_t m0 = m0_wave + (uint32_t)(slot * kSTile);
-#pragma unroll
-            for (int i = 0; i < 2; ++i) {
-                const int row = min(t * kSN + 8 * wv + 4 * i + r4, L - 1) - t * kSN;
-                lds_direct_load16(base, (uint32_t)row * row_stride + kcol[i], m0 + i * 1024);
-            }
-        }
+    // any tile t: rows past the end of the request re-read its last row (masked later)
+    auto issue_ragged = [&](const char* rows, int t, const uint32_t col0, const uint32_t col1, uint32_t m0) __attribute__((always_inline)) {
+        int lane_row = 8 * wv + r4;
+        asm volatile("" : "+v"(lane_row)); // (formed here: kept across the loops, the rows below cost ten registers)
+        const char* base = rows - (size_t)(8 * wv) * row_stride;
+        const int last = L - 1 - t * kSN;
+        lds_direct_load16(base, (uint32_t)min(lane_row, last) * row_stride + col0, m0);
+        lds_direct_load16(base, (uint32_t)min(lane_row + 4, last) * row_stride + col1, m0 + 1024);
     };
-    auto issue_v = [&](int t, int slot) __attribute__((always_inline)) {
-        if ((t + 1) * kSN <= L) {
-            issue_v_fast(t, slot);
-        } else {
-            const char* base = v_ptr + kv_row0 + (size_t)t * tile_stride;
-            const uint32_t m0 = m0_wave + (uint32_t)((kSNK + slot) * kSTile);
-#pragma unroll
-            for (int i = 0; i < 2; ++i) {
-                const int row = min(t * kSN + 8 * wv + 4 * i + r4, L - 1) - t * kSN;
-                lds_direct_load16(base, (uint32_t)row * row_stride + vcol, m0 + i * 1024);
-            }
-        }
+    auto issue_k = [&](const char* rows, int t, int slot) __attribute__((always_inline)) {
+        if ((t + 1) * kSN <= L) issue_k_fast(rows, slot);
+        else issue_ragged(rows, t, kcol[0], kcol[1], m0_wave + (uint32_t)(slot * kSTile));
     };
+    auto issue_v = [&](const char* rows, int t, int slot) __attribute__((always_inline)) {
+        if ((t + 1) * kSN <= L) issue_v_fast(rows, slot);
+        else issue_ragged(rows, t, vcol, vcol, m0_wave + (uint32_t)((kSNK + slot) * kSTile));
+    };
+    // the tiles that are copied next
+    const char *k_next = k_wave, *v_next = v_wave;
     // ---- Q rows as B operands: lane (q, h) holds q[q][16*ks + 8*h .. +7], ks = 0..7.  The
     // loads of the q rows and of the angles go first, the tile copies of the prologue behind them; the rotation
-    // is done while the copies travel.
+    // is done while the copies travel.  The rows travel like K rows, whole and straight into LDS (the same XOR), into slots
+    // that no tile needs yet: K3, V2 and V3, and one of their own, for waves 0 to 3.  Read into the operand's layout
+    // directly, each of eight loads touches 32 rows for 32 bytes of each, and the wave stands until they have all gone out:
+    // from a job's record to the last of these loads 4 350 cycles then and 2 800 now, where a job of 61 prompts of 16 .. 400 tokens
+    // takes 18 000 (32/8 heads; the whole call 111 -> 101 us with the last tiles below), 6 030 and 4 100 of 64 000 for 16 of
+    // 128 .. 4 096 with 40 heads (1 028 -> 1 000 us; 32 of 200 .. 1 403 523 -> 493).
+    const uint32_t q_slot = (uint32_t)((wv == 0 ? kSNK - 1 : kSNK + kSNV - 3 + wv) * kSTile);
     uint4 qreg[8];
     uint4 cs[ROPE_Q ? 16 : 1];
     {
-        const size_t qtok = (size_t)it.tok0 + (size_t)min(q_pos, Lq - 1);
-        const char* qrow = q_ptr + (qtok * Hq + head) * 256;
+        const int base_row = min(wave_q_lo, Lq - 1), last_row = Lq - 1 - base_row;
+        const char* qrow = q_ptr + (((size_t)it.tok0 + base_row) * Hq + head) * 256;
 #pragma unroll
-        for (int ks = 0; ks < 8; ++ks) qreg[ks] = sp_load16(qrow + ks * 32 + h * 16);
+        for (int i = 0; i < 8; ++i) { // rows 4i .. 4i+3 (those past the end of the request re-read its last row)
+            const int row = 4 * i + r4;
+            lds_direct_load16(qrow, (uint32_t)min(row, last_row) * (uint32_t)(Hq * 256) + (uint32_t)((p16 ^ (row & 15)) * 16),
+                              lds0 + q_slot + (uint32_t)(i * 1024));
+        }
         if constexpr (ROPE_Q) {
             // d = 16 ks + 8 h + e (ks < 4) pairs with d + 64, which this lane holds at step ks + 4.  The table is
             // laid out couple of pairs by couple of pairs, so the 32 rows of a half-wave read 512 consecutive bytes
             // per load.
-            const float4* tab = a.rope_table + (skip + off + min(q_pos, Lq - 1));
+            const uint32_t lane_at = ((uint32_t)(skip + off + min(q_pos, Lq - 1)) + 4u * (uint32_t)h * a.rope_pitch) * 16u;
 #pragma unroll
-            for (int e = 0; e < 16; ++e) cs[e] = sp_load16(tab + (size_t)(8 * (e >> 2) + 4 * h + (e & 3)) * a.rope_pitch);
+            for (int e = 0; e < 16; ++e)
+                cs[e] = sp_load16_at((const char*)(a.rope_table + (size_t)(8 * (e >> 2) + (e & 3)) * a.rope_pitch), lane_at);
         }
     }
-    int copies = 0; // tile copies issued so far
-    if (L >= kSNK * kSN && n >= kSNK) { // the common case: the first tiles all exist and are whole
+    // Operand reads.  K: lane (row qn, half h) needs chunk 2 ks + h of its row for step ks, which sits at position
+    // (2 ks + h) ^ (qn % 16); V, through the transposing read: chunk 4 db + zl' of its row for d block db (see
+    // the kernel's header).  One address register per step / d block (complete LDS addresses inside slot 0); the slot and
+    // the token offsets of the V operands go into the instruction's offset field where they are compile-time constants.
+    uint32_t koff[8], voff[4];
+    {
+        const int y = h ^ (qn & 15);
 #pragma unroll
-        for (int i = -kSNK; i < 0; ++i) {
-            issue_k_fast(i + kSNK, i + kSNK);
-            if (i + kSNV - 1 >= 0) issue_v_fast(i + kSNV - 1, i + kSNV - 1);
+        for (int ks = 0; ks < 8; ++ks) {
+            koff[ks] = lds0 + (uint32_t)(qn * 256 + (((2 * ks) ^ y) * 16));
+            asm volatile("" : "+v"(koff[ks])); // keep the sum: the compiler would rebuild it at every use
         }
-        copies = kSNK + kSNV - 1;
-        sp_wait_copies(kSNK + kSNV - 1); // the q rows (and the angles) are here
+        const int srow = (lane & 15) >> 2;
+        const int zl = ((((lane >> 4) & 1) << 1) | ((lane & 3) >> 1)) ^ BZ_VSWZ(srow);
+#pragma unroll
+        for (int db = 0; db < 4; ++db) {
+            voff[db] = lds0 + (uint32_t)(kSNK * kSTile + (4 * h + srow) * 256 + ((((db << 2)) ^ zl) * 16) + (lane & 1) * 8);
+            asm volatile("" : "+v"(voff[db]));
+        }
+    }
+    // The first tiles in the order K0 | K1 V0 | K2 V1; K3 and V2 follow when the q rows have left their slots.
+    int copies = 0; // tile copies issued so far
+    if (L >= (kSNK - 1) * kSN && n >= kSNK - 1) { // the common case: the first tiles all exist and are whole
+#pragma unroll
+        for (int i = 0; i < kSNK - 1; ++i) {
+            issue_k_fast(k_next, i);
+            k_next += tile_stride;
+            if (i > 0) {
+                issue_v_fast(v_next, i - 1);
+                v_next += tile_stride;
+            }
+        }
+        copies = kSNK + kSNV - 3;
+        sp_wait_copies(kSNK + kSNV - 3); // the q rows (and the angles) are here
     } else {
 #pragma unroll
-        for (int i = -kSNK; i < 0; ++i) {
-            if (i + kSNK < n) { issue_k(i + kSNK, i + kSNK); ++copies; }
-            if (i + kSNV - 1 >= 0 && i + kSNV - 1 < n) { issue_v(i + kSNV - 1, i + kSNV - 1); ++copies; }
+        for (int i = 0; i < kSNK - 1; ++i) {
+            if (i < n) { issue_k(k_next, i, i); ++copies; }
+            k_next += tile_stride;
+            if (i > 0) {
+                if (i - 1 < n) { issue_v(v_next, i - 1, i - 1); ++copies; }
+                v_next += tile_stride;
+            }
         }
         sp_wait_copies(copies);
     }
 #pragma unroll
-    for (int ks = 0; ks < 8; ++ks) sp_loads_arrived(qreg[ks]);
+    for (int ks = 0; ks < 8; ++ks) {
+        typedef uint32_t __attribute__((ext_vector_type(4))) u32x4;
+        const u32x4 r = *(const u32x4 __attribute__((address_space(3)))*)(uintptr_t)(koff[ks] + q_slot);
+        qreg[ks] = make_uint4(r.x, r.y, r.z, r.w);
+    }
     if constexpr (ROPE_Q) {
 #pragma unroll
         for (int e = 0; e < 16; ++e) sp_loads_arrived(cs[e]);
@@ -482,26 +504,6 @@ __global__ __launch_bounds__(256, 2) void prefill_kernel(PrefillArgs a, const ch
             }
     }
 
-    // Operand reads.  K: lane (row qn, half h) needs chunk 2 ks + h of its row for step ks, which sits at position
-    // (2 ks + h) ^ (qn % 16); V, through the transposing read: chunk 4 db + zl' of its row for d block db (see
-    // the kernel's header).  One address register per step / d block (complete LDS addresses inside slot 0); the slot and
-    // the token offsets of the V operands go into the instruction's offset field where they are compile-time constants.
-    uint32_t koff[8], voff[4];
-    {
-        const int y = h ^ (qn & 15);
-#pragma unroll
-        for (int ks = 0; ks < 8; ++ks) {
-            koff[ks] = lds0 + (uint32_t)(qn * 256 + (((2 * ks) ^ y) * 16));
-            asm volatile("" : "+v"(koff[ks])); // keep the sum: the compiler would rebuild it at every use
-        }
-        const int srow = (lane & 15) >> 2;
-        const int zl = ((((lane >> 4) & 1) << 1) | ((lane & 3) >> 1)) ^ BZ_VSWZ(srow);
-#pragma unroll
-        for (int db = 0; db < 4; ++db) {
-            voff[db] = lds0 + (uint32_t)(kSNK * kSTile + (4 * h + srow) * 256 + ((((db << 2)) ^ zl) * 16) + (lane & 1) * 8);
-            asm volatile("" : "+v"(voff[db]));
-        }
-    }
     uint4 kring[4], vring[4]; // operands of the matrix instructions, read four instructions ahead of their use
     typedef uint32_t __attribute__((ext_vector_type(4))) pf_u32x4;
     // (these issue the reads; the first use of a register waits for it.  `soff`: byte offset of the tile's slot)
@@ -568,11 +570,9 @@ __global__ __launch_bounds__(256, 2) void prefill_kernel(PrefillArgs a, const ch
     auto mask_tile = [&](int t, pf_f32x16& sc) __attribute__((always_inline)) {
         // element 4b+r of a score block is token 32t + 8b + 4h + r
         if (t >= t_diag || (t + 1) * kSN > L) {
+            const int last = kv_max - t * kSN - 4 * h;
 #pragma unroll
-            for (int i = 0; i < 16; ++i) {
-                const int kv = t * kSN + 8 * (i >> 2) + 4 * h + (i & 3);
-                sc[i] = kv > kv_max ? -INFINITY : sc[i];
-            }
+            for (int i = 0; i < 16; ++i) sc[i] = 8 * (i >> 2) + (i & 3) > last ? -INFINITY : sc[i];
         }
     };
     auto exp_of = [&](float x, float shift) __attribute__((always_inline)) {
@@ -603,8 +603,8 @@ __global__ __launch_bounds__(256, 2) void prefill_kernel(PrefillArgs a, const ch
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
             if (QK) s[PAR ^ 1] = M::run(kring[i & 3], qreg[i], i == 0 ? cinit : s[PAR ^ 1]);
-            if (i < 4) read_k(kring[i], k1, i + 4);
-            else read_v(vring[i - 4], vj, i - 4);
+            if (i >= 4) read_v(vring[i - 4], vj, i - 4);
+            else if (QK) read_k(kring[i], k1, i + 4);
             if (V_F16 && (i == 4 || i == 5) && wslot >= 0) wide[i - 4] = *widen_at(wslot, i - 4);
             if (EX) {
                 const float n0 = exp_of(s[PAR][2 * i], 0.f), n1 = exp_of(s[PAR][2 * i + 1], 0.f);
@@ -621,15 +621,12 @@ __global__ __launch_bounds__(256, 2) void prefill_kernel(PrefillArgs a, const ch
     // (at k2) into the rings.  V_F16: the widening ends here, in the shadow of the first six steps, whose matrix
     // instructions have no vector work of their own beside them; behind its last write come kWidenBehind operand reads.
     constexpr int kWidenBehind = 2;
-    auto second_half = [&](auto pv_c, uint32_t vj, uint32_t k2, int wslot) __attribute__((always_inline)) {
-        constexpr bool PV = decltype(pv_c)::value;
+    auto second_half = [&](uint32_t vj, uint32_t k2, int wslot) __attribute__((always_inline)) {
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
-            if (PV) {
-                acc[i & 3] = MP::run(vring[i & 3], pa[i >> 2], acc[i & 3]);
-                if (SPLIT_P) acc[i & 3] = MP::run(vring[i & 3], pb[i >> 2], acc[i & 3]);
-            }
+            acc[i & 3] = MP::run(vring[i & 3], pa[i >> 2], acc[i & 3]);
+            if (SPLIT_P) acc[i & 3] = MP::run(vring[i & 3], pb[i >> 2], acc[i & 3]);
             if (i < 4) read_v(vring[i], vj, i + 4);
             else read_k(kring[i - 4], k2, i - 4);
             if (V_F16 && i < 6 && wslot >= 0) {
@@ -665,18 +662,44 @@ __global__ __launch_bounds__(256, 2) void prefill_kernel(PrefillArgs a, const ch
     };
 
     // ---- prologue: scores of tile 0 set the reference maximum, the ring takes the first K operands of tile 1.
-    // The copies were issued in the order K0 | K1 V0 | K2 V1 | K3 V2 (those that exist).
     BZ_PF_WG(1);
-    sp_wait_copies(copies - 1); // K0 has landed
+    sp_wait_copies(max(copies - (V_F16 ? 3 : 2), 0)); // K0 and K1 have landed (if there is one); V_F16: V0 as well
+    sp_wait_lds<0>();                                 // the q rows have left LDS
     sp_barrier();
+    // copies of tile t of K and of tile t - 1 of V, the next ones in order, as far as they exist
+    auto issue_next = [&](int t, int slot) __attribute__((always_inline)) { // slot: t % 4
+        if (t - 1 < n) {
+            if (t < n) issue_k(k_next, t, slot);
+            issue_v(v_next, t - 1, (slot + kSNV - 1) % kSNV);
+        }
+        k_next += tile_stride;
+        v_next += tile_stride;
+    };
+    issue_next(kSNK - 1, kSNK - 1);
     BZ_PF_WG(2);
     {
         uint4 k0[8];
 #pragma unroll
         for (int i = 0; i < 8; ++i) read_k(k0[i], k_at(0), i);
+        if (V_F16) {
+#pragma unroll
+            for (int i = 0; i < 2; ++i) wide[i] = *widen_at(0, i);
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) read_k(kring[i], k_at(1 % kSNK), i);
         if (n_w > 0) {
 #pragma unroll
             for (int i = 0; i < 8; ++i) s[0] = M::run(k0[i], qreg[i], i == 0 ? cinit : s[0]);
+        }
+        if (V_F16) { // (beside the scores; waited for in front of the next barrier)
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                widen_words(i, 0, 4);
+                *widen_at(0, i) = wide[i];
+            }
+            sp_wait_lds<0>();
+        }
+        if (n_w > 0) {
             mask_tile(0, s[0]);
             float tmax = -INFINITY;
 #pragma unroll
@@ -689,22 +712,13 @@ __global__ __launch_bounds__(256, 2) void prefill_kernel(PrefillArgs a, const ch
                 cinit[i] = -tmax;
             }
         }
-        sp_wait_copies(max(copies - (V_F16 ? 3 : 2), 0)); // K1 has landed (if there is one); V_F16: V0 as well
-        sp_barrier();
-#pragma unroll
-        for (int i = 0; i < 4; ++i) read_k(kring[i], k_at(1 % kSNK), i);
-        if (V_F16) {
-            widen_v(0);
-            sp_wait_lds<0>();
-        }
     }
     BZ_PF_WG(3);
 
     // ---- the steady state: every tile touched exists, is whole and needs no mask.  SL = j % 4 is the slot of
     // K(j) and of V(j), a compile-time constant (the loop is unrolled by four), so that LDS addresses are one
     // register plus an immediate and the copies' LDS targets are constants as well.
-    const char* k_next = k_wave + (size_t)kSNK * tile_stride;       // K(j + kSNK)
-    const char* v_next = v_wave + (size_t)(kSNV - 1) * tile_stride; // V(j + kSNV - 1)
+    // (k_next and v_next are at K(j + kSNK), V(j + kSNV - 1))
     auto full = [&](int j, auto par_c, auto sl_c) __attribute__((always_inline)) {
         constexpr int PAR = decltype(par_c)::value, SL = decltype(sl_c)::value;
         BZ_PF_PH_START();
@@ -721,35 +735,30 @@ __global__ __launch_bounds__(256, 2) void prefill_kernel(PrefillArgs a, const ch
         constexpr int WSLOT = V_F16 ? (SL + 1) % kSNV : -1; // V(j+1), first read after the next barrier
         first_half(par_c, std::true_type{}, std::true_type{}, k_at((SL + 1) % kSNK), v_at(SL), WSLOT);
         BZ_PF_PH(3);
-        if (__any(!(psum < 32768.0f))) move_maximum(s[PAR], s[PAR ^ 1]);
+        if (__builtin_expect(__any(!(psum < 32768.0f)), 0)) move_maximum(s[PAR], s[PAR ^ 1]);
         l_run += psum;
-        second_half(std::true_type{}, v_at(SL), k_at((SL + 2) % kSNK), WSLOT);
+        second_half(v_at(SL), k_at((SL + 2) % kSNK), WSLOT);
         BZ_PF_PH(4);
     };
-    // ---- the same with every condition checked (the slots are still compile-time constants: j % 4 == SL).  The operand
-    // reads are issued by every wave, also one that has nothing to compute, so that the registers have one definition
-    // per iteration.
-    auto generic = [&](int j, auto par_c, auto sl_c) __attribute__((always_inline)) {
+    // ---- the last tiles of this wave: copies as far as there are tiles left, the next tile masked where it has to be.  (A tile
+    // takes 1 400 cycles here and 850 to 1 250 above; 2 000 while the copies in flight were counted by a loop over them, the
+    // copies' addresses multiplied out per tile, and waves without a tile sent through the same code.)
+    auto tail = [&](int j, auto par_c, auto sl_c) __attribute__((always_inline)) {
         constexpr int PAR = decltype(par_c)::value, SL = decltype(sl_c)::value;
-        const bool has_cur = j < n_w, has_next = j + 1 < n_w;
-        sp_wait_copies(sp_copies_behind(j, n, V_F16));
+        sp_wait_tail<V_F16>(n - 1 - j);
         if (V_F16) sp_wait_lds<kWidenBehind>();
         sp_barrier();
-        if (j + kSNK < n) issue_k(j + kSNK, SL);
-        if (j + kSNV - 1 < n) issue_v(j + kSNV - 1, (SL + kSNV - 1) % kSNV);
+        issue_next(j + kSNK, SL);
         // (V(j+1) is widened whether there is one or not: the slot is this wave's to write, what it holds then is read by nobody)
         constexpr int WSLOT = V_F16 ? (SL + 1) % kSNV : -1;
-        const uint32_t k1 = k_at((SL + 1) % kSNK), k2 = k_at((SL + 2) % kSNK);
-        if (has_next) first_half(par_c, std::true_type{}, std::true_type{}, k1, v_at(SL), WSLOT);
-        else first_half(par_c, std::false_type{}, std::true_type{}, k1, v_at(SL), WSLOT); // (harmless without a tile: p of stale scores, never used)
-        if (has_cur) {
-            if (__any(!(psum < 32768.0f))) move_maximum(s[PAR], s[PAR ^ 1]);
-            l_run += psum;
-            if (has_next) mask_tile(j + 1, s[PAR ^ 1]);
-            second_half(std::true_type{}, v_at(SL), k2, WSLOT);
-        } else {
-            second_half(std::false_type{}, v_at(SL), k2, WSLOT);
-        }
+        // (the scores of a next tile are taken whether there is one or not, from whatever its slot holds, and read by nobody
+        // then: with a branch there the compiler gathers the vector work that both sides have in front of it and behind it,
+        // out of the shadow of the matrix instructions)
+        first_half(par_c, std::true_type{}, std::true_type{}, k_at((SL + 1) % kSNK), v_at(SL), WSLOT);
+        if (__builtin_expect(__any(!(psum < 32768.0f)), 0)) move_maximum(s[PAR], s[PAR ^ 1]);
+        l_run += psum;
+        if (j + 1 < n_w) mask_tile(j + 1, s[PAR ^ 1]);
+        second_half(v_at(SL), k_at((SL + 2) % kSNK), WSLOT);
     };
     // full needs: tiles j .. j+2 computed by this wave, tile j+1 unmasked, and the tiles it copies whole and in range
     const int j_full = min(min(n_w - 2, t_diag - 1), min(L / kSN, n) - kSNK);
@@ -767,15 +776,23 @@ __global__ __launch_bounds__(256, 2) void prefill_kernel(PrefillArgs a, const ch
     BZ_PF_WG(4);
     // the rest (j is a multiple of four): the last tiles of the job, the diagonal ones and everything ragged.  Nested,
     // not one condition after the other: a tile's registers are then defined on one path only.
-    for (; j < n; j += 4) {
-        generic(j, c0, c0);
-        if (j + 1 < n) {
-            generic(j + 1, c1, c1);
-            if (j + 2 < n) {
-                generic(j + 2, c0, c2);
-                if (j + 3 < n) generic(j + 3, c1, c3);
+    for (; j < n_w; j += 4) {
+        tail(j, c0, c0);
+        if (j + 1 < n_w) {
+            tail(j + 1, c1, c1);
+            if (j + 2 < n_w) {
+                tail(j + 2, c0, c2);
+                if (j + 3 < n_w) tail(j + 3, c1, c3);
             }
         }
+    }
+    // tiles that other waves of the workgroup still need and this one does not: its share of the copies and of the widening
+    for (j = n_w; j < n; ++j) {
+        sp_wait_tail<V_F16>(n - 1 - j);
+        if (V_F16) sp_wait_lds<0>();
+        sp_barrier();
+        issue_next(j + kSNK, j & 3);
+        if (V_F16) widen_v((j + 1) & 3);
     }
     sp_barrier(); // nobody reads a tile any more: the epilogue takes their place
     BZ_PF_WG(5);
@@ -809,16 +826,19 @@ __global__ __launch_bounds__(256, 2) void prefill_kernel(PrefillArgs a, const ch
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    // (one uniform base per four rows and one lane offset; only rows past the end of the request need a look at each lane)
+    char* const o_wave = (char*)a.out + (((size_t)it.tok0 + wave_q_lo) * Hq + head) * 256;
+    const uint32_t o_lane = (uint32_t)r4 * (uint32_t)(Hq * 256) + (uint32_t)(p16 * 16);
+    auto store_rows = [&](auto whole_c) __attribute__((always_inline)) {
 #pragma unroll
-    for (int ps = 0; ps < 8; ++ps) {
-        const int row = 4 * ps + (lane >> 4);
-        const int pos = wave_q_lo + row;
-        if (pos < Lq) {
-            const uint4 v = *reinterpret_cast<const uint4*>(o_lds + row * 256 + (((lane & 15) ^ (row & 15)) * 16));
-            char* orow = (char*)a.out + (((size_t)it.tok0 + pos) * Hq + head) * 256;
-            *reinterpret_cast<uint4*>(orow + (lane & 15) * 16) = v;
+        for (int ps = 0; ps < 8; ++ps) {
+            const uint4 v = *reinterpret_cast<const uint4*>(o_lds + r4 * 256 + ps * 1024 + ((p16 ^ r4) ^ (4 * (ps & 3))) * 16);
+            if (decltype(whole_c)::value || wave_q_lo + 4 * ps + r4 < Lq)
+                *reinterpret_cast<uint4*>(o_wave + (size_t)(4 * ps) * (Hq * 256) + o_lane) = v;
         }
-    }
+    };
+    if (wave_q_lo + 32 <= Lq) store_rows(std::true_type{});
+    else store_rows(std::false_type{});
 #ifdef BZ_PF_PHASES
     if ((wv == 0 || wv == 3) && lane == 0 && blockIdx.x < kPftMaxWg) {
         unsigned long long* dst = bz_pf_ph + ((size_t)blockIdx.x * 2 + (wv == 3 ? 1 : 0)) * 8;
@@ -1516,6 +1536,8 @@ extern "C" int bz_batch_prefill_ragged(bz_prefill_plan_t* plan_, void* q, const 
     a.rope_table = (const float4*)p->rope_table;
     a.rope_pitch = p->max_len;
     a.num_qo_heads = num_qo_heads; a.num_kv_heads = num_kv_heads;
+    const uint32_t group = num_qo_heads / num_kv_heads;
+    a.group_inv = group > 1 ? (uint32_t)(((1ull << 32) + group - 1) / group) : 0;
     a.head_shift = prefill_head_shift(num_qo_heads, num_kv_heads);
     a.causal = causal ? 1 : 0;
     if (!(sm_scale > 0.f)) sm_scale = 1.0f / sqrtf((float)head_dim);

@@ -98,6 +98,23 @@ def test_grouped_heads_share_a_workgroup(kind, causal, Hq, Hkv):
 
 
 @pytest.mark.parametrize("kind", KINDS, ids=KIND_IDS)
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("Hq,Hkv", [(2, 2), (4, 1), (10, 2)])
+def test_every_number_of_tiles_around_the_copies_ahead(kind, causal, Hq, Hkv):
+    """Jobs of one to ten tiles of 32 K/V rows, whole and with a ragged end: four tiles are copied ahead, so the first tiles, the
+    last ones without copies and the steady ones between them meet in every combination.  128 rows of one head, 32 of four,
+    and a group (5) whose q heads are found by a product instead of a shift."""
+    dtype = kind[0]
+    lens = [32 * n - cut for n in range(1, 11) for cut in (0, 13)]
+    pf = Prefill(230 + Hq, lens, Hq, Hkv, 128, dtype, kind[1])
+    got = pf.run(causal=causal, rope_mode=BZ_ROPE_Q_ONLY)
+    ref = oracle.batch_prefill_ragged(pf.q_as_fed(1e4), pf.k, pf.v, dtype, pf.indptr, Hq, Hkv, 128, causal=causal, sm_scale=LN2,
+                                      parallel=True)
+    assert not np.isnan(got).any()
+    assert (np.abs(got - ref) <= kind_tol(ref, kind)).all(), np.abs(got - ref).max()
+
+
+@pytest.mark.parametrize("kind", KINDS, ids=KIND_IDS)
 @pytest.mark.parametrize("float_ws_bytes", [1 << 20, 1 << 10])
 def test_rope_inside_the_call(kind, float_ws_bytes):
     """BZ_ROPE_FULL, the reference's kRoPELlama: k rows are rotated in place (the page store that follows
