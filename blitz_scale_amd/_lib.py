@@ -4,6 +4,8 @@ The shared library is the product: there is no Python or CPU fallback.  Loading 
 when blitz_scale_amd/lib/libbz_hip.so has not been built (python -m blitz_scale_amd.build).
 """
 import ctypes as C
+import importlib.machinery
+import importlib.util
 import os
 
 HERE = os.path.dirname(os.path.abspath(__file__))
@@ -121,6 +123,23 @@ def load():
         fn.argtypes = args
     _lib = lib
     return lib
+
+
+PYCALL_PATH = os.path.join(HERE, "lib", "bz_pycall.so")
+_pycall = None
+
+
+def load_pycall():
+    """Load the native calling side (csrc/bz_pycall.cpp).  Raises if it is not built."""
+    global _pycall
+    if _pycall is None:
+        if not os.path.exists(PYCALL_PATH):
+            raise RuntimeError(f"{PYCALL_PATH} is missing: build it first (python -m blitz_scale_amd.build).")
+        loader = importlib.machinery.ExtensionFileLoader("bz_pycall", PYCALL_PATH)
+        module = importlib.util.module_from_spec(importlib.util.spec_from_loader("bz_pycall", loader))
+        loader.exec_module(module)
+        _pycall = module
+    return _pycall
 
 
 class BzError(RuntimeError):

@@ -6,6 +6,7 @@ HIP + a C ABI (include/bz_hip.h); it does not link against torch.
 import os
 import subprocess
 import sys
+import sysconfig
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(HERE)
@@ -75,7 +76,22 @@ def build(verbose=True, jobs=8):
     if verbose:
         print(" ".join(cmd), flush=True)
     subprocess.check_call(cmd)
+    build_pycall(verbose)
     return LIB_PATH
+
+
+PYCALL_PATH = os.path.join(LIB_DIR, "bz_pycall.so")
+
+
+def build_pycall(verbose=True):
+    """The extension module through which kernel.py calls the library (host code only)."""
+    cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-Wno-missing-field-initializers",
+           "-I", sysconfig.get_paths()["include"], "-I", os.path.join(ROOT, "include"), os.path.join(CSRC, "bz_pycall.cpp"),
+           "-o", PYCALL_PATH]
+    if verbose:
+        print(" ".join(cmd), flush=True)
+    subprocess.check_call(cmd)
+    return PYCALL_PATH
 
 
 PROBE_SRC = os.path.join(HERE, "probes", "mfma_ceiling.hip")

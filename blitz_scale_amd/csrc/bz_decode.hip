@@ -463,10 +463,10 @@ static int launch_general_g(const DecodeArgs& a, int G, dim3 grid, hipStream_t s
     if constexpr (std::is_same<QT, KVT>::value) {
         if (a.rope_mode == BZ_ROPE_FULL && a.rope_table) { // angles from the table
             switch (G) {
-                case 1: hipLaunchKernelGGL((decode_general_kernel<QT, KVT, OT, D, 1, true>), grid, dim3(256), 0, s, a); break;
-                case 2: hipLaunchKernelGGL((decode_general_kernel<QT, KVT, OT, D, 2, true>), grid, dim3(256), 0, s, a); break;
-                case 4: hipLaunchKernelGGL((decode_general_kernel<QT, KVT, OT, D, 4, true>), grid, dim3(256), 0, s, a); break;
-                case 8: hipLaunchKernelGGL((decode_general_kernel<QT, KVT, OT, D, 8, true>), grid, dim3(256), 0, s, a); break;
+                case 1: launch_kernel((decode_general_kernel<QT, KVT, OT, D, 1, true>), grid, dim3(256), 0, s, a); break;
+                case 2: launch_kernel((decode_general_kernel<QT, KVT, OT, D, 2, true>), grid, dim3(256), 0, s, a); break;
+                case 4: launch_kernel((decode_general_kernel<QT, KVT, OT, D, 4, true>), grid, dim3(256), 0, s, a); break;
+                case 8: launch_kernel((decode_general_kernel<QT, KVT, OT, D, 8, true>), grid, dim3(256), 0, s, a); break;
                 default: return BZ_ERR_UNSUPPORTED;
             }
             BZ_LAUNCH_CHECK();
@@ -474,10 +474,10 @@ static int launch_general_g(const DecodeArgs& a, int G, dim3 grid, hipStream_t s
         }
     }
     switch (G) {
-        case 1: hipLaunchKernelGGL((decode_general_kernel<QT, KVT, OT, D, 1>), grid, dim3(256), 0, s, a); break;
-        case 2: hipLaunchKernelGGL((decode_general_kernel<QT, KVT, OT, D, 2>), grid, dim3(256), 0, s, a); break;
-        case 4: hipLaunchKernelGGL((decode_general_kernel<QT, KVT, OT, D, 4>), grid, dim3(256), 0, s, a); break;
-        case 8: hipLaunchKernelGGL((decode_general_kernel<QT, KVT, OT, D, 8>), grid, dim3(256), 0, s, a); break;
+        case 1: launch_kernel((decode_general_kernel<QT, KVT, OT, D, 1>), grid, dim3(256), 0, s, a); break;
+        case 2: launch_kernel((decode_general_kernel<QT, KVT, OT, D, 2>), grid, dim3(256), 0, s, a); break;
+        case 4: launch_kernel((decode_general_kernel<QT, KVT, OT, D, 4>), grid, dim3(256), 0, s, a); break;
+        case 8: launch_kernel((decode_general_kernel<QT, KVT, OT, D, 8>), grid, dim3(256), 0, s, a); break;
         default: return BZ_ERR_UNSUPPORTED;
     }
     BZ_LAUNCH_CHECK();
@@ -502,12 +502,12 @@ static int launch_general_kv(const DecodeArgs& a, int kv_dtype, int q_dtype, int
 template <typename OT>
 static void launch_combine(const DecodePlan* p, const float* part_o, const float* part_lse, void* out, float* lse,
                            uint32_t Hq, uint32_t D, hipStream_t s) {
-    hipLaunchKernelGGL((decode_combine_kernel<OT>), dim3(p->num_combos, Hq), dim3(D), 0, s, p->combos_d, part_o,
+    launch_kernel((decode_combine_kernel<OT>), dim3(p->num_combos, Hq), dim3(D), 0, s, p->combos_d, part_o,
                        part_lse, out, lse, Hq, D);
 }
 template <typename OT>
 static void launch_zero(const DecodePlan* p, void* out, uint32_t row_elems, hipStream_t s) {
-    hipLaunchKernelGGL((decode_zero_rows_kernel<OT>), dim3(p->num_empty), dim3(256), 0, s, p->empty_d, out, row_elems);
+    launch_kernel((decode_zero_rows_kernel<OT>), dim3(p->num_empty), dim3(256), 0, s, p->empty_d, out, row_elems);
 }
 
 int decode_fast_path(const DecodePlan* p, const void* q, void* out, float* lse, int q_dtype, int out_dtype,
@@ -604,7 +604,7 @@ static int batch_decode_impl(DecodePlan* p, const void* q, int q_dtype, const bz
                 if (off + tbytes <= p->float_buffer_bytes) {
                     float2* table = reinterpret_cast<float2*>(reinterpret_cast<char*>(p->part_o) + off);
                     const uint32_t n = positions * (uint32_t)(D / 2);
-                    hipLaunchKernelGGL(decode_rope_table_kernel, dim3((n + 255) / 256), dim3(256), 0, s, table, positions,
+                    launch_kernel(decode_rope_table_kernel, dim3((n + 255) / 256), dim3(256), 0, s, table, positions,
                                        (uint32_t)(D / 2), a.freqs);
                     BZ_LAUNCH_CHECK();
                     a.rope_table = table;

@@ -1101,11 +1101,11 @@ struct DecodeArgs; // general-kernel argument block (bz_decode.hip); only its sc
 template <bool BF16, typename OT, bool ROPE_Q, bool KV8, int D>
 static void launch_mfma_k(const DecodePlan* p, const MfmaDecodeArgs& a, hipStream_t s) {
     if (p->mfma_streaming)
-        hipLaunchKernelGGL((decode_mfma_kernel<BF16, OT, ROPE_Q, KV8, true, D>), dim3(p->mfma_slots), dim3(64), 0, s, a.heads, a,
+        launch_kernel((decode_mfma_kernel<BF16, OT, ROPE_Q, KV8, true, D>), dim3(p->mfma_slots), dim3(64), 0, s, a.heads, a,
                            (const char*)a.q, a.k_data, a.v_data, a.indices, a.pieces, a.tiles, a.k_scale,
                            a.v_scale);
     else
-        hipLaunchKernelGGL((decode_mfma_kernel<BF16, OT, ROPE_Q, KV8, false, D>), dim3(p->mfma_slots), dim3(64), 0, s, a.heads, a,
+        launch_kernel((decode_mfma_kernel<BF16, OT, ROPE_Q, KV8, false, D>), dim3(p->mfma_slots), dim3(64), 0, s, a.heads, a,
                            (const char*)a.q, a.k_data, a.v_data, a.indices, a.pieces, a.tiles, a.k_scale,
                            a.v_scale);
 }
@@ -1121,13 +1121,13 @@ static int launch_mfma(const DecodePlan* p, const MfmaDecodeArgs& a, hipStream_t
     if (p->mfma_combos > 0) {
         const dim3 cgrid(p->mfma_combos, a.group);
         if (p->mfma_max_count <= 16)
-            hipLaunchKernelGGL((decode_mfma_combine_kernel<OT, 1, D>), cgrid, dim3(D, 1), 0, s, p->mfma_combos_d,
+            launch_kernel((decode_mfma_combine_kernel<OT, 1, D>), cgrid, dim3(D, 1), 0, s, p->mfma_combos_d,
                                a.part_o, a.part_lse, a.out, a.lse, a.num_qo_heads, a.group);
         else if (p->mfma_max_count <= 64)
-            hipLaunchKernelGGL((decode_mfma_combine_kernel<OT, 4, D>), cgrid, dim3(D, 4), 0, s, p->mfma_combos_d,
+            launch_kernel((decode_mfma_combine_kernel<OT, 4, D>), cgrid, dim3(D, 4), 0, s, p->mfma_combos_d,
                                a.part_o, a.part_lse, a.out, a.lse, a.num_qo_heads, a.group);
         else
-            hipLaunchKernelGGL((decode_mfma_combine_kernel<OT, 8, D>), cgrid, dim3(D, 8), 0, s, p->mfma_combos_d,
+            launch_kernel((decode_mfma_combine_kernel<OT, 8, D>), cgrid, dim3(D, 8), 0, s, p->mfma_combos_d,
                                a.part_o, a.part_lse, a.out, a.lse, a.num_qo_heads, a.group);
         BZ_LAUNCH_CHECK();
     }
@@ -1203,7 +1203,7 @@ static int launch_step_finish(const DecodePlan* p, const StepFinishArgs& a, hipS
     const uint32_t G = a.group;
     auto launch = [&](auto s_c, auto hb_c, auto nb_c) {
         constexpr int S = decltype(s_c)::value, HB = decltype(hb_c)::value, NB = decltype(nb_c)::value; // NB: partials per batch of loads
-        hipLaunchKernelGGL((decode_step_finish_kernel<QT, PT, OT, S, HB, NB, D>), dim3(p->mfma_units, (G + HB - 1) / HB), dim3(D / 4, HB, S),
+        launch_kernel((decode_step_finish_kernel<QT, PT, OT, S, HB, NB, D>), dim3(p->mfma_units, (G + HB - 1) / HB), dim3(D / 4, HB, S),
                            0, s, a.units, a.steps_ahead, a);
     };
     const std::integral_constant<int, 1> c1{};

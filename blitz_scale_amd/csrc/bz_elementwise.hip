@@ -130,10 +130,10 @@ static void launch_rms_norm(void* input, void* residual, const void* weight, voi
     uint32_t t = (h / 8 + 63) / 64 * 64;
     t = t > 1024 ? 1024 : (t < 64 ? 64 : t);
     if (h / 8 <= t)
-        hipLaunchKernelGGL((rms_norm_kernel<T, ADD, true>), dim3(rows), dim3(t), 0, s, (T*)input, (T*)residual, (const T*)weight,
+        launch_kernel((rms_norm_kernel<T, ADD, true>), dim3(rows), dim3(t), 0, s, (T*)input, (T*)residual, (const T*)weight,
                            (T*)output, h, eps);
     else
-        hipLaunchKernelGGL((rms_norm_kernel<T, ADD, false>), dim3(rows), dim3(t), 0, s, (T*)input, (T*)residual, (const T*)weight,
+        launch_kernel((rms_norm_kernel<T, ADD, false>), dim3(rows), dim3(t), 0, s, (T*)input, (T*)residual, (const T*)weight,
                            (T*)output, h, eps);
 }
 
@@ -174,9 +174,9 @@ extern "C" int bz_silu_and_mul(const void* input, void* output, int dtype, uint3
     hipStream_t s = (hipStream_t)stream;
     const dim3 block(256), grid((inter_size / 8 + 255) / 256, num_tokens);
     if (dtype == BZ_F16)
-        hipLaunchKernelGGL((silu_and_mul_kernel<f16_t>), grid, block, 0, s, (const f16_t*)input, (f16_t*)output, inter_size);
+        launch_kernel((silu_and_mul_kernel<f16_t>), grid, block, 0, s, (const f16_t*)input, (f16_t*)output, inter_size);
     else if (dtype == BZ_BF16)
-        hipLaunchKernelGGL((silu_and_mul_kernel<bf16_t>), grid, block, 0, s, (const bf16_t*)input, (bf16_t*)output, inter_size);
+        launch_kernel((silu_and_mul_kernel<bf16_t>), grid, block, 0, s, (const bf16_t*)input, (bf16_t*)output, inter_size);
     else return BZ_ERR_UNSUPPORTED;
     BZ_LAUNCH_CHECK();
     return 0;
@@ -192,9 +192,9 @@ extern "C" int bz_add_residual(const void* input, void* residual, int dtype, uin
     const size_t nvec = n / 8;
     const dim3 block(256), grid((unsigned)((nvec + 255) / 256));
     if (dtype == BZ_F16)
-        hipLaunchKernelGGL((add_residual_kernel<f16_t>), grid, block, 0, s, (const f16_t*)input, (f16_t*)residual, nvec);
+        launch_kernel((add_residual_kernel<f16_t>), grid, block, 0, s, (const f16_t*)input, (f16_t*)residual, nvec);
     else if (dtype == BZ_BF16)
-        hipLaunchKernelGGL((add_residual_kernel<bf16_t>), grid, block, 0, s, (const bf16_t*)input, (bf16_t*)residual, nvec);
+        launch_kernel((add_residual_kernel<bf16_t>), grid, block, 0, s, (const bf16_t*)input, (bf16_t*)residual, nvec);
     else return BZ_ERR_UNSUPPORTED;
     BZ_LAUNCH_CHECK();
     return 0;

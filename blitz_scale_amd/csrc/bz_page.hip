@@ -354,13 +354,13 @@ template <typename ST, typename PT, bool PREFILL>
 static int launch_page_write_d(const PageWriteArgs& a, int D, uint32_t grid, hipStream_t s) {
     if (grid == 0) return 0;
     if constexpr (PREFILL) {
-        auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3(grid), dim3(256), 0, s, a.ragged_indptr, a.indptr, a.indices, a); };
+        auto launch = [&](auto kernel) { launch_kernel(kernel, dim3(grid), dim3(256), 0, s, a.ragged_indptr, a.indptr, a.indices, a); };
         if (D == 128) a.rows_held == kPwRowsMany ? launch(page_write_kernel<ST, PT, 128, kPwRowsMany>) : launch(page_write_kernel<ST, PT, 128, kPwRowsFew>);
         else if (D == 64) a.rows_held == kPwRowsMany ? launch(page_write_kernel<ST, PT, 64, kPwRowsMany>) : launch(page_write_kernel<ST, PT, 64, kPwRowsFew>);
         else return BZ_ERR_UNSUPPORTED;
     } else {
-        if (D == 128) hipLaunchKernelGGL((append_kernel<ST, PT, 128>), dim3(grid), dim3(256), 0, s, a);
-        else if (D == 64) hipLaunchKernelGGL((append_kernel<ST, PT, 64>), dim3(grid), dim3(256), 0, s, a);
+        if (D == 128) launch_kernel((append_kernel<ST, PT, 128>), dim3(grid), dim3(256), 0, s, a);
+        else if (D == 64) launch_kernel((append_kernel<ST, PT, 64>), dim3(grid), dim3(256), 0, s, a);
         else return BZ_ERR_UNSUPPORTED;
     }
     BZ_LAUNCH_CHECK();
@@ -470,7 +470,7 @@ using namespace bz;
 
 extern "C" int bz_steps_ahead_advance(int32_t* steps_ahead, void* stream) {
     if (!steps_ahead) return BZ_ERR_BAD_ARG;
-    hipLaunchKernelGGL(steps_ahead_advance_kernel, dim3(1), dim3(1), 0, (hipStream_t)stream, steps_ahead);
+    launch_kernel(steps_ahead_advance_kernel, dim3(1), dim3(1), 0, (hipStream_t)stream, steps_ahead);
     BZ_LAUNCH_CHECK();
     return 0;
 }
@@ -547,11 +547,11 @@ extern "C" int bz_rope_cached_k(const bz_paged_kv_t* kv, float rope_theta, int i
     const dim3 grid(kv->batch_size, 32);
     hipStream_t s = (hipStream_t)stream;
     if (kv->kv_dtype == BZ_F16) {
-        if (D == 128) hipLaunchKernelGGL((rope_cached_k_kernel<f16_t, 128>), grid, dim3(256), lds, s, a);
-        else hipLaunchKernelGGL((rope_cached_k_kernel<f16_t, 64>), grid, dim3(256), lds, s, a);
+        if (D == 128) launch_kernel((rope_cached_k_kernel<f16_t, 128>), grid, dim3(256), lds, s, a);
+        else launch_kernel((rope_cached_k_kernel<f16_t, 64>), grid, dim3(256), lds, s, a);
     } else {
-        if (D == 128) hipLaunchKernelGGL((rope_cached_k_kernel<bf16_t, 128>), grid, dim3(256), lds, s, a);
-        else hipLaunchKernelGGL((rope_cached_k_kernel<bf16_t, 64>), grid, dim3(256), lds, s, a);
+        if (D == 128) launch_kernel((rope_cached_k_kernel<bf16_t, 128>), grid, dim3(256), lds, s, a);
+        else launch_kernel((rope_cached_k_kernel<bf16_t, 64>), grid, dim3(256), lds, s, a);
     }
     BZ_LAUNCH_CHECK();
     return 0;

@@ -687,7 +687,7 @@ __global__ __launch_bounds__(256, 2) void prefill_kernel(PrefillArgs a, const ch
         }
 #pragma unroll
         for (int i = 0; i < 4; ++i) read_k(kring[i], k_at(1 % kSNK), i);
-        if (n_w > 0) {
+        {
 #pragma unroll
             for (int i = 0; i < 8; ++i) s[0] = M::run(k0[i], qreg[i], i == 0 ? cinit : s[0]);
         }
@@ -699,7 +699,7 @@ __global__ __launch_bounds__(256, 2) void prefill_kernel(PrefillArgs a, const ch
             }
             sp_wait_lds<0>();
         }
-        if (n_w > 0) {
+        {
             mask_tile(0, s[0]);
             float tmax = -INFINITY;
 #pragma unroll
@@ -1432,13 +1432,13 @@ static int launch_prefill_kernel(PrefillPlan* p, const PrefillArgs& a, const voi
     std::unique_lock<std::mutex> lock(p->cut_mutex, std::defer_lock);
     if (PARTS) lock.lock();
     if (p->time_start) BZ_CHECK_HIP(hipEventRecord(p->time_start, s));
-    hipLaunchKernelGGL(kern, dim3(PARTS ? p->num_cut_items : p->num_items), dim3(256), kSLds, s, a, (const char*)q,
+    launch_kernel(kern, dim3(PARTS ? p->num_cut_items : p->num_items), dim3(256), kSLds, s, a, (const char*)q,
                        (const char*)k, (const char*)v);
     BZ_LAUNCH_CHECK();
     if (p->time_stop) BZ_CHECK_HIP(hipEventRecord(p->time_stop, s));
     if (PARTS) {
-        if (BF16) hipLaunchKernelGGL(prefill_combine_kernel<bf16_t>, dim3(p->num_joins, 4), dim3(256), 0, s, a, p->joins_d);
-        else hipLaunchKernelGGL(prefill_combine_kernel<f16_t>, dim3(p->num_joins, 4), dim3(256), 0, s, a, p->joins_d);
+        if (BF16) launch_kernel(prefill_combine_kernel<bf16_t>, dim3(p->num_joins, 4), dim3(256), 0, s, a, p->joins_d);
+        else launch_kernel(prefill_combine_kernel<f16_t>, dim3(p->num_joins, 4), dim3(256), 0, s, a, p->joins_d);
         BZ_LAUNCH_CHECK();
     }
     return 0;
@@ -1506,7 +1506,7 @@ extern "C" int bz_batch_prefill_ragged(bz_prefill_plan_t* plan_, void* q, const 
             // (every call: the workspace may be shared with other handlers between calls, calls may change streams,
             // and a captured call must replay its own fill; a few microseconds)
             const float scale = (sm_scale > 0.f ? sm_scale : 1.0f / sqrtf((float)head_dim)) * 1.4426950408889634f;
-            hipLaunchKernelGGL(rope_table_kernel, dim3((p->max_len + 255) / 256, 32), dim3(256), 0, s, (float4*)p->rope_table,
+            launch_kernel(rope_table_kernel, dim3((p->max_len + 255) / 256, 32), dim3(256), 0, s, (float4*)p->rope_table,
                                p->max_len, p->max_len, freqs, scale);
             BZ_LAUNCH_CHECK();
         }
@@ -1516,8 +1516,8 @@ extern "C" int bz_batch_prefill_ragged(bz_prefill_plan_t* plan_, void* q, const 
             ra.batch_size = batch_size; ra.num_heads = heads;
             ra.freqs = freqs;
             if (tokens == 0) return;
-            if (dtype == BZ_F16) hipLaunchKernelGGL((rope_ragged_kernel<f16_t>), dim3(tokens), dim3(256), 0, s, ra);
-            else hipLaunchKernelGGL((rope_ragged_kernel<bf16_t>), dim3(tokens), dim3(256), 0, s, ra);
+            if (dtype == BZ_F16) launch_kernel((rope_ragged_kernel<f16_t>), dim3(tokens), dim3(256), 0, s, ra);
+            else launch_kernel((rope_ragged_kernel<bf16_t>), dim3(tokens), dim3(256), 0, s, ra);
         };
         if (rope_mode == BZ_ROPE_FULL) rotate_rows(k, kv_indptr, nullptr, num_kv_heads, p->total_kv_tokens);
         if (!p->rope_table) rotate_rows(q, qo_indptr, kv_indptr, num_qo_heads, p->total_tokens); // no room for the table

@@ -153,7 +153,7 @@ extern "C" int bz_embedding(void* output, const uint32_t* token_ids, const int32
     if (int rc = check_rows(output, weight, dtype, hidden_size)) return rc;
     if (!token_ids) return BZ_ERR_BAD_ARG;
     if (num_tokens == 0) return 0;
-    hipLaunchKernelGGL(gather_rows_kernel, dim3(num_tokens), dim3(256), 0, (hipStream_t)stream, (uint4*)output,
+    launch_kernel(gather_rows_kernel, dim3(num_tokens), dim3(256), 0, (hipStream_t)stream, (uint4*)output,
                        (const uint4*)weight, token_ids, out_loc, (const int32_t*)nullptr, hidden_size / 8);
     BZ_LAUNCH_CHECK();
     return 0;
@@ -165,7 +165,7 @@ extern "C" int bz_gather_last_token(void* output, const void* tokens, const int3
     if (int rc = check_rows(output, tokens, dtype, hidden_size)) return rc;
     if (!ragged_indptr) return BZ_ERR_BAD_ARG;
     if (batch_size == 0) return 0;
-    hipLaunchKernelGGL(gather_rows_kernel, dim3(batch_size), dim3(256), 0, (hipStream_t)stream, (uint4*)output,
+    launch_kernel(gather_rows_kernel, dim3(batch_size), dim3(256), 0, (hipStream_t)stream, (uint4*)output,
                        (const uint4*)tokens, (const uint32_t*)nullptr, (const int32_t*)nullptr, ragged_indptr,
                        hidden_size / 8);
     BZ_LAUNCH_CHECK();
@@ -180,10 +180,10 @@ extern "C" int bz_batch_find_max(uint32_t* output_indices, const void* input, in
     if ((uintptr_t)input % 2) return BZ_ERR_BAD_ARG;
     if (batch_size == 0) return 0;
     if (dtype == BZ_F16)
-        hipLaunchKernelGGL(batch_find_max_kernel<f16_t>, dim3(batch_size), dim3(1024), 0, (hipStream_t)stream,
+        launch_kernel(batch_find_max_kernel<f16_t>, dim3(batch_size), dim3(1024), 0, (hipStream_t)stream,
                            output_indices, (const uint16_t*)input, length);
     else
-        hipLaunchKernelGGL(batch_find_max_kernel<bf16_t>, dim3(batch_size), dim3(1024), 0, (hipStream_t)stream,
+        launch_kernel(batch_find_max_kernel<bf16_t>, dim3(batch_size), dim3(1024), 0, (hipStream_t)stream,
                            output_indices, (const uint16_t*)input, length);
     BZ_LAUNCH_CHECK();
     return 0;

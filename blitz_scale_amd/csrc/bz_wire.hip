@@ -158,8 +158,8 @@ static int launch_wire(const WireArgs& a, hipStream_t s) {
     WireLaunch w;
     if (int rc = wire_launch_shape(a.total_vecs, a.vecs_per_chunk, sizeof(PT), sizeof(WT), &w)) return rc;
     if (w.workgroups == 0) return 0;
-    if (w.within) hipLaunchKernelGGL((wire_kernel<PT, WT, PACK, true>), dim3(w.workgroups), dim3(256), 0, s, a);
-    else hipLaunchKernelGGL((wire_kernel<PT, WT, PACK, false>), dim3(w.workgroups), dim3(256), 0, s, a);
+    if (w.within) launch_kernel((wire_kernel<PT, WT, PACK, true>), dim3(w.workgroups), dim3(256), 0, s, a);
+    else launch_kernel((wire_kernel<PT, WT, PACK, false>), dim3(w.workgroups), dim3(256), 0, s, a);
     BZ_LAUNCH_CHECK();
     return 0;
 }

@@ -53,6 +53,35 @@ def _host_i32(a):
     return np.ascontiguousarray(np.asarray(a, dtype=np.int32))
 
 
+class _Calls:
+    """The launching calls of the C ABI as Python callables, bound on first use (lib/bz_pycall.so, csrc/bz_pycall.cpp: arguments
+    that are what they usually are go through without ctypes).  A call takes the C arguments in order -- a tensor for its address
+    or for its type code, a PageTable for the struct, None for the current stream -- and raises BzError on a status."""
+
+    WHAT = {"bz_batch_decode": "batchDecodeAttention", "bz_batch_decode_noalloc": "batchDecodeAttention", "bz_decode_step": "decodeStep",
+            "bz_batch_prefill_ragged": "BatchPrefillWithRaggedKVCache", "bz_store_prefill_kv": "AppendPagedKVCache",
+            "bz_append_decode_kv": "AppendPagedKVCacheDecode", "bz_rms_norm": "rmsNorm", "bz_add_rms_norm": "fusedAddRmsNorm",
+            "bz_silu_and_mul": "siluAndMul", "bz_add_residual": "AddKernel", "bz_embedding": "EmbeddingKernel",
+            "bz_gather_last_token": "GatherLastTokenKernel", "bz_batch_find_max": "BatchFindMaxKernel"}
+
+    def __getattr__(self, name):
+        fn = getattr(_lib.load(), name)
+        native = _lib.load_pycall()
+        raw = _raw_stream or (lambda device: torch.cuda.current_stream(device).cuda_stream)
+        native.setup(torch.Tensor, torch.Tensor.data_ptr, _DTYPES, PageTable, torch.cuda.is_initialized,
+                     _current_device or torch.cuda.current_device, raw)
+        # the slow way, for arguments that the native side leaves alone: converted, and refused, as ctypes does it
+        convert = {"p": _ptr, "d": bz_dtype, "k": lambda table: C.byref(table.as_struct()), "t": int, "s": _stream}
+        ways = [convert.get(letter, lambda value: value) for letter in native.specs()[name]]
+        call = native.bind(name, C.cast(fn, C.c_void_p).value, lambda *args: fn(*[way(a) for way, a in zip(ways, args)]), check,
+                           self.WHAT[name])
+        setattr(self, name, call)
+        return call
+
+
+_calls = _Calls()
+
+
 class PageTable:
     """blitz::kernel::PageTable<DType, IdType> (src/kernel/page.h:12-64).
 
@@ -247,44 +276,32 @@ class BatchPrefillRaggedHandler:
 def batch_decode_attention(handler, q_input, paged_kv, output, num_qo_heads, *, rope_mode=BZ_ROPE_Q_ONLY,
                            rope_theta=1e4, sm_scale=0.0, k_scale=None, v_scale=None, lse=None, stream=None):
     """src/kernel/attention.h:24-31."""
-    s = paged_kv.as_struct()
-    rc = _lib.load().bz_batch_decode(handler.get(), _ptr(q_input), bz_dtype(q_input), C.byref(s), _ptr(output),
-                                     bz_dtype(output), num_qo_heads, rope_mode, rope_theta, sm_scale, _ptr(k_scale),
-                                     _ptr(v_scale), _ptr(lse), _stream(stream))
-    check(rc, "batchDecodeAttention")
+    _calls.bz_batch_decode(handler.get(), q_input, q_input, paged_kv, output, output, num_qo_heads, rope_mode, rope_theta, sm_scale,
+                           k_scale, v_scale, lse, stream)
 
 
 def decode_step(handler, q_input, k_new, v_new, paged_kv, output, num_qo_heads, *, rope=True, rope_theta=1e4,
                 sm_scale=0.0, k_scale=None, v_scale=None, lse=None, stream=None):
     """append_decode_kv_cache followed by batch_decode_attention (src/layer/attn.h:196-203) as one call: the
     new K (rotated when rope) and V rows go into the cache, q is rotated inside the kernels and left as it is."""
-    s = paged_kv.as_struct()
-    rc = _lib.load().bz_decode_step(handler.get(), _ptr(q_input), bz_dtype(q_input), _ptr(k_new), _ptr(v_new), C.byref(s),
-                                    _ptr(output), bz_dtype(output), num_qo_heads, int(rope), rope_theta, sm_scale,
-                                    _ptr(k_scale), _ptr(v_scale), _ptr(lse), _stream(stream))
-    check(rc, "decodeStep")
+    _calls.bz_decode_step(handler.get(), q_input, q_input, k_new, v_new, paged_kv, output, output, num_qo_heads, rope, rope_theta,
+                          sm_scale, k_scale, v_scale, lse, stream)
 
 
 def batch_decode_attention_noalloc(handler, q_input, paged_kv, output, num_qo_heads, *, rope_mode=BZ_ROPE_Q_ONLY,
                                    rope_theta=1e4, sm_scale=0.0, k_scale=None, v_scale=None, lse=None, stream=None):
     """batch_decode_attention with the split-K partials in the library's own fixed device array instead of
     the plan's float workspace: the call allocates nothing (no counterpart in the reference)."""
-    s = paged_kv.as_struct()
-    rc = _lib.load().bz_batch_decode_noalloc(handler.get(), _ptr(q_input), bz_dtype(q_input), C.byref(s),
-                                             _ptr(output), bz_dtype(output), num_qo_heads, rope_mode, rope_theta,
-                                             sm_scale, _ptr(k_scale), _ptr(v_scale), _ptr(lse), _stream(stream))
-    check(rc, "batchDecodeAttention")
+    _calls.bz_batch_decode_noalloc(handler.get(), q_input, q_input, paged_kv, output, output, num_qo_heads, rope_mode, rope_theta,
+                                   sm_scale, k_scale, v_scale, lse, stream)
 
 
 def batch_prefill_attention(handler, q_input, qo_indptr, k_input, v_input, kv_indptr, output, batch_size,
                             num_qo_heads, num_kv_heads, head_size, *, causal=True, rope_mode=BZ_ROPE_NONE,
                             rope_theta=1e4, sm_scale=0.0, stream=None):
     """src/kernel/attention.h:9-22."""
-    rc = _lib.load().bz_batch_prefill_ragged(handler.get(), _ptr(q_input), _ptr(qo_indptr), _ptr(k_input),
-                                             _ptr(v_input), _ptr(kv_indptr), _ptr(output), bz_dtype(q_input),
-                                             batch_size, num_qo_heads, num_kv_heads, head_size, int(causal),
-                                             rope_mode, rope_theta, sm_scale, _stream(stream))
-    check(rc, "BatchPrefillWithRaggedKVCache")
+    _calls.bz_batch_prefill_ragged(handler.get(), q_input, qo_indptr, k_input, v_input, kv_indptr, output, q_input, batch_size,
+                                   num_qo_heads, num_kv_heads, head_size, causal, rope_mode, rope_theta, sm_scale, stream)
 
 
 def store_prefill_kv_cache(page_table, k_data, v_data, ragged_indptr, *, num_tokens=None, q=None, num_qo_heads=0,
@@ -292,21 +309,14 @@ def store_prefill_kv_cache(page_table, k_data, v_data, ragged_indptr, *, num_tok
     """src/kernel/page.h:66-67."""
     if num_tokens is None:
         num_tokens = k_data.shape[0]
-    s = page_table.as_struct()
-    rc = _lib.load().bz_store_prefill_kv(C.byref(s), _ptr(k_data), _ptr(v_data), bz_dtype(k_data),
-                                         _ptr(ragged_indptr), num_tokens, _ptr(q), num_qo_heads, int(rope),
-                                         rope_theta, _ptr(k_scale), _ptr(v_scale), _stream(stream))
-    check(rc, "AppendPagedKVCache")
+    _calls.bz_store_prefill_kv(page_table, k_data, v_data, k_data, ragged_indptr, num_tokens, q, num_qo_heads, rope, rope_theta,
+                               k_scale, v_scale, stream)
 
 
 def append_decode_kv_cache(page_table, k_data, v_data, *, q=None, num_qo_heads=0, rope=False, rope_theta=1e4,
                            k_scale=None, v_scale=None, stream=None):
     """src/kernel/page.h:69-70."""
-    s = page_table.as_struct()
-    rc = _lib.load().bz_append_decode_kv(C.byref(s), _ptr(k_data), _ptr(v_data), bz_dtype(k_data), _ptr(q),
-                                         num_qo_heads, int(rope), rope_theta, _ptr(k_scale), _ptr(v_scale),
-                                         _stream(stream))
-    check(rc, "AppendPagedKVCacheDecode")
+    _calls.bz_append_decode_kv(page_table, k_data, v_data, k_data, q, num_qo_heads, rope, rope_theta, k_scale, v_scale, stream)
 
 
 def rope_cached_k(page_table, *, rope_theta=1e4, inverse=False, stream=None):
@@ -324,50 +334,37 @@ def steps_ahead_advance(steps_ahead, *, stream=None):
 
 def rms_norm(input, weight, output, num_tokens, hidden_size, eps=1e-5, *, stream=None):
     """src/kernel/rms_norm.h:11-19."""
-    rc = _lib.load().bz_rms_norm(_ptr(input), _ptr(weight), _ptr(output), bz_dtype(input), num_tokens, hidden_size,
-                                 eps, _stream(stream))
-    check(rc, "rmsNorm")
+    _calls.bz_rms_norm(input, weight, output, input, num_tokens, hidden_size, eps, stream)
 
 
 def add_rms_norm(input, residual, weight, num_tokens, hidden_size, eps=1e-5, *, stream=None):
     """src/kernel/rms_norm.h:26-34."""
-    rc = _lib.load().bz_add_rms_norm(_ptr(input), _ptr(residual), _ptr(weight), bz_dtype(input), num_tokens,
-                                     hidden_size, eps, _stream(stream))
-    check(rc, "fusedAddRmsNorm")
+    _calls.bz_add_rms_norm(input, residual, weight, input, num_tokens, hidden_size, eps, stream)
 
 
 def silu_and_mul(input, output, num_tokens, inter_size, *, stream=None):
     """src/kernel/activation.h:10-16."""
-    rc = _lib.load().bz_silu_and_mul(_ptr(input), _ptr(output), bz_dtype(input), num_tokens, inter_size,
-                                     _stream(stream))
-    check(rc, "siluAndMul")
+    _calls.bz_silu_and_mul(input, output, input, num_tokens, inter_size, stream)
 
 
 def add_residual(input, residual, num_tokens, dim, *, stream=None):
     """src/kernel/add.h:8-14."""
-    rc = _lib.load().bz_add_residual(_ptr(input), _ptr(residual), bz_dtype(input), num_tokens, dim, _stream(stream))
-    check(rc, "AddKernel")
+    _calls.bz_add_residual(input, residual, input, num_tokens, dim, stream)
 
 
 def embedding(output, token_ids, weight, num_tokens, hidden_size, *, out_loc=None, stream=None):
     """src/kernel/embedding.h:7-36: output[loc] = weight[token_ids[t]]; loc = t or out_loc[t]."""
-    rc = _lib.load().bz_embedding(_ptr(output), _ptr(token_ids), _ptr(out_loc) if out_loc is not None else None,
-                                  _ptr(weight), bz_dtype(weight), num_tokens, hidden_size, _stream(stream))
-    check(rc, "EmbeddingKernel")
+    _calls.bz_embedding(output, token_ids, out_loc, weight, weight, num_tokens, hidden_size, stream)
 
 
 def gather_last_token(output, tokens, ragged_indptr, num_tokens, batch_size, hidden_size, *, stream=None):
     """src/kernel/sampler.h:8-16: output[b] = tokens[ragged_indptr[b+1] - 1]."""
-    rc = _lib.load().bz_gather_last_token(_ptr(output), _ptr(tokens), _ptr(ragged_indptr), bz_dtype(tokens),
-                                          num_tokens, batch_size, hidden_size, _stream(stream))
-    check(rc, "GatherLastTokenKernel")
+    _calls.bz_gather_last_token(output, tokens, ragged_indptr, tokens, num_tokens, batch_size, hidden_size, stream)
 
 
 def batch_find_max(output_indices, input, batch_size, length, *, stream=None):
     """src/kernel/sampler.h:18-26: output_indices[b] = argmax(input[b])."""
-    rc = _lib.load().bz_batch_find_max(_ptr(output_indices), _ptr(input), bz_dtype(input), batch_size, length,
-                                       _stream(stream))
-    check(rc, "BatchFindMaxKernel")
+    _calls.bz_batch_find_max(output_indices, input, input, batch_size, length, stream)
 
 
 def kv_wire_bytes(page_table, num_pages, layer_cnt, wire_dtype=None):
