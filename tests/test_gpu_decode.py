@@ -428,3 +428,52 @@ def test_general_kernel_with_page_ids_of_a_set_ahead(kv_dtype, Hq, Hkv, D, P):
     groups that take their page ids with the rows, a set ahead, or either by the segment's length."""
     p = DecodeProblem(680 + Hq + D + P, [1, 63, 64, 65, 127, 128, 129, 0, 191, 193, 256, 257, 385], Hq, Hkv, D, P, BZ_BF16, kv_dtype=kv_dtype)
     check(p)
+
+
+@pytest.mark.parametrize("dtype", [BZ_F16, BZ_BF16])
+@pytest.mark.parametrize("Hq,Hkv,P,layout", [(1, 1, 16, BZ_LAYOUT_HND), (8, 2, 32, BZ_LAYOUT_NHD), (5, 1, 16, BZ_LAYOUT_HND),
+                                             (12, 2, 48, BZ_LAYOUT_NHD), (32, 2, 64, BZ_LAYOUT_HND), (20, 1, 16, BZ_LAYOUT_NHD)])
+@pytest.mark.parametrize("split_tokens", [0, 96, 0xFFFFFFFF])
+def test_raw_k_rows_on_the_matrix_cores(dtype, Hq, Hkv, P, layout, split_tokens):
+    """16-bit rows over a raw-K cache of heads of 128: sequences that end on either side of a subtile of 16 and a tile of 32, one
+    piece after another in a wave slot, pieces that begin anywhere, groups up to 16 and one of two parts, no sequence at all."""
+    p = DecodeProblem(700 + Hq + P, [1, 15, 16, 17, 31, 32, 33, 0, 47, 48, 49, 95, 97, 700, 2100], Hq, Hkv, 128, P, dtype, layout=layout)
+    dev = DeviceDecode(p)
+    dev.plan(split_tokens)
+    for theta in (1e4, 5e5):
+        ref = oracle.batch_decode(p.q, dtype, p.oracle_kv(), Hq, rope_mode=BZ_ROPE_FULL, rope_theta=theta, parallel=True)
+        got = dev.decode(None, BZ_ROPE_FULL, theta)
+        assert (np.abs(got - ref) <= ulp_tol(ref, dtype)).all(), np.abs(got - ref).max()
+
+
+@pytest.mark.parametrize("dtype", [BZ_F16, BZ_BF16])
+def test_raw_k_rows_under_a_table_that_runs_ahead(dtype):
+    """The table lists five tokens more than there are: q and every K row are rotated at their present positions."""
+    ctx, ahead = [22, 43, 166, 1030], 5  # (the last page keeps a token without them)
+    p = DecodeProblem(730, ctx, 8, 2, 128, 16, dtype)
+    assert (p.last_page_len > ahead).all()
+    dev = DeviceDecode(p)
+    dev.plan(256)
+    dev.pt.steps_ahead_d = torch.tensor([ahead], dtype=torch.int32, device="cuda")
+    got = dev.decode(None, BZ_ROPE_FULL, 1e4)
+    p.last_page_len = p.last_page_len - ahead
+    ref = oracle.batch_decode(p.q, dtype, p.oracle_kv(), 8, rope_mode=BZ_ROPE_FULL, rope_theta=1e4, parallel=True)
+    assert (np.abs(got - ref) <= ulp_tol(ref, dtype)).all(), np.abs(got - ref).max()
+
+
+def test_raw_k_rows_in_f16_keep_the_range_of_fp32():
+    """Two values near the largest f16 rotate to as much as 92 600, and many tokens far below the largest have to count: both
+    are beyond an f16 operand that is not scaled.  K rows whose largest values meet in one pair, q that picks them out."""
+    p = DecodeProblem(731, [4000], 1, 1, 128, 16, BZ_F16)
+    f = np.zeros((p.pool_pages, 2, 1, 16, 128), np.float32)
+    f[:, 0, 0, :, 0] = f[:, 0, 0, :, 64] = 65504.0  # pair 0 turns by a radian a token
+    f[:, 1] = 1.0
+    p.pool = wl.to_bits(f.reshape(-1), BZ_F16)
+    q = np.zeros((1, 1, 128), np.float32)
+    q[0, 0, 0], q[0, 0, 64] = 2e-3, 1e-3
+    p.q = wl.to_bits(q, BZ_F16)
+    dev = DeviceDecode(p)
+    dev.plan(0)
+    ref = oracle.batch_decode(p.q, BZ_F16, p.oracle_kv(), 1, rope_mode=BZ_ROPE_FULL, rope_theta=1e4, parallel=True)
+    got = dev.decode(None, BZ_ROPE_FULL, 1e4)
+    assert np.isfinite(got).all() and (np.abs(got - ref) <= ulp_tol(ref, BZ_F16)).all(), np.abs(got - ref).max()
