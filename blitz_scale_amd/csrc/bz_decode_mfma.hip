@@ -979,6 +979,7 @@ struct StepFinishArgs {
     const float* v_scale;
     uint64_t stride_page, stride_n, stride_h;
     uint32_t page_size, num_qo_heads, num_kv_heads, group, parts;
+    int page_shift; // log2 of page_size, negative where that is no power of two
     int rope;
     float sm_scale_log2;
     alignas(8) RopeFreqs freqs; // (read two at a time)
@@ -1024,7 +1025,7 @@ __global__ __launch_bounds__(D / 4 * HB * S) void decode_step_finish_kernel(cons
     asm volatile("" ::"s"(a.q), "s"(a.k_new), "s"(a.v_new), "s"(a.k_data), "s"(a.v_data), "s"(a.indices), "s"(a.part_o),
                  "s"(a.part_lse), "s"(a.out), "s"(a.lse), "s"(a.k_scale), "s"(a.v_scale), "s"(a.stride_page),
                  "s"(a.stride_n), "s"(a.stride_h), "s"(a.page_size), "s"(a.num_qo_heads), "s"(a.num_kv_heads),
-                 "s"(a.group), "s"(a.parts), "s"(a.rope), "s"(a.sm_scale_log2));
+                 "s"(a.group), "s"(a.parts), "s"(a.page_shift), "s"(a.rope), "s"(a.sm_scale_log2));
     // The angles of the new token's position: lane t of a head works out pairs 2t and 2t + 1, and the lanes of the
     // head then pass them round (no LDS table, no workgroup barrier).  The two frequencies are asked for here, beside
     // the unit record, not where they are used.
@@ -1033,7 +1034,7 @@ __global__ __launch_bounds__(D / 4 * HB * S) void decode_step_finish_kernel(cons
     const bool head_live = g_raw < a.group;           // a group that is no multiple of HB leaves lanes idle
     const uint32_t g = head_live ? g_raw : a.group - 1;
     const int b = u.seq;
-    const int kvr = u.unit / (int)a.parts; // the kv head whose K/V the unit reads
+    const int kvr = a.parts == 1 ? u.unit : u.unit / (int)a.parts; // the kv head whose K/V the unit reads
     const uint32_t hq = (uint32_t)u.unit * a.group + g;
     const uint32_t d0 = 4 * t;             // this lane's four output dimensions
     const bool upper = d0 >= D / 2;           // they are the second elements of their rotate-half pairs
@@ -1046,8 +1047,9 @@ __global__ __launch_bounds__(D / 4 * HB * S) void decode_step_finish_kernel(cons
     // (the page of the newest token is asked for beside the rows, not where it is used: one dependent round trip less
     // between the unit record and the append -- and by every workgroup, needed or not: a unit's sequence has pages,
     // and a load under a condition would be waited for on the spot)
-    const bool appends = g_raw == 0 && sl == 0 && u.unit % (int)a.parts == 0; // one head's lanes per (sequence, kv head)
-    const int64_t page = a.indices[u.ip0 + max(seq_len - 1, 0) / (int)a.page_size];
+    const bool appends = g_raw == 0 && sl == 0 && u.unit == kvr * (int)a.parts; // one head's lanes per (sequence, kv head)
+    const int newest = max(seq_len - 1, 0), newest_page = a.page_shift >= 0 ? newest >> a.page_shift : newest / (int)a.page_size;
+    const int64_t page = a.indices[u.ip0 + newest_page];
     const QT* qrow = reinterpret_cast<const QT*>(a.q) + ((size_t)b * a.num_qo_heads + hq) * D;
     const QT* krow = reinterpret_cast<const QT*>(a.k_new) + ((size_t)b * a.num_kv_heads + kvr) * D;
     const QT* vrow = reinterpret_cast<const QT*>(a.v_new) + ((size_t)b * a.num_kv_heads + kvr) * D;
@@ -1058,13 +1060,20 @@ __global__ __launch_bounds__(D / 4 * HB * S) void decode_step_finish_kernel(cons
     load4_f32(krow + dp, k_par);
     load4_f32(vrow + d0, v_in);
     const float ksc = a.k_scale ? a.k_scale[kvr] : 1.0f, vsc = a.v_scale ? a.v_scale[kvr] : 1.0f;
+    // (Partials past the last one are the last one again, with a weight of zero: a load under a condition is a branch of its own.
+    // One uniform base and 32-bit offsets, and no division by a page size that is a power of two: 165 instructions stood in
+    // front of the last of these loads where 350 did, and the waves of this kernel mostly issue instructions.  32 layers of 8
+    // sequences of 700 .. 1 350 tokens 533 -> 526 us, of 12 x 1 200 683 -> 673, of 1 x 8 000 566 -> 557; one layer of two of
+    // 40 000 .. 90 000 74.8 -> 74.4, 96 with heads of 64 44.9 -> 44.7, 128 sequences, 32/8 heads, 107.4 -> 107.2.)
+    const char* lse_rows = reinterpret_cast<const char*>(a.part_lse + (size_t)u.first_piece * 16);
+    const char* o_rows = reinterpret_cast<const char*>(a.part_o + (size_t)u.first_piece * (16 * D));
+    const uint32_t lse_lane = g * 4, o_lane = (g * D + d0) * 4;
     auto load_batch = [&](int j0, float* li, float4* oi) {
 #pragma unroll
         for (int k = 0; k < NB; ++k) {
-            const bool live = j0 + k < u.count;
-            const size_t slot = (size_t)(u.first_piece + (live ? j0 + k : 0));
-            li[k] = live ? a.part_lse[slot * 16 + g] : -INFINITY;
-            oi[k] = *reinterpret_cast<const float4*>(a.part_o + (slot * 16 + g) * D + d0);
+            const uint32_t at = (uint32_t)min(j0 + k, u.count - 1);
+            li[k] = *reinterpret_cast<const float*>(lse_rows + (at * 64u + lse_lane));
+            oi[k] = *reinterpret_cast<const float4*>(o_rows + (at * (64u * D) + o_lane));
         }
     };
     float li0[NB];
@@ -1113,7 +1122,7 @@ __global__ __launch_bounds__(D / 4 * HB * S) void decode_step_finish_kernel(cons
             v_term[e] = pool_to_f32(v_st[e]) * vsc;
         }
         if (appends) { // the append
-            const size_t off = (size_t)page * a.stride_page + (size_t)(pos % (int)a.page_size) * a.stride_n +
+            const size_t off = (size_t)page * a.stride_page + (size_t)(pos - newest_page * (int)a.page_size) * a.stride_n +
                                (size_t)kvr * a.stride_h + d0;
             store4(reinterpret_cast<PT*>(a.k_data) + off, k_st);
             store4(reinterpret_cast<PT*>(a.v_data) + off, v_st);
@@ -1125,10 +1134,13 @@ __global__ __launch_bounds__(D / 4 * HB * S) void decode_step_finish_kernel(cons
 
     // ---- the partial results of the older tokens (normalised rows and base-2 log-sum-exp per piece)
     float M = -INFINITY, wsum = 0.f, o[4] = {0.f, 0.f, 0.f, 0.f};
-    auto merge_batch = [&](const float* li, const float4* oi) {
+    auto merge_batch = [&](int j0, float* li, const float4* oi) {
         float m2 = M;
 #pragma unroll
-        for (int k = 0; k < NB; ++k) m2 = fmaxf(m2, li[k]);
+        for (int k = 0; k < NB; ++k) {
+            li[k] = j0 + k < u.count ? li[k] : -INFINITY;
+            m2 = fmaxf(m2, li[k]);
+        }
         if (m2 == -INFINITY) return;
         const float sc = __builtin_amdgcn_exp2f(M - m2); // 0 while nothing has been merged yet
         wsum *= sc;
@@ -1145,12 +1157,12 @@ __global__ __launch_bounds__(D / 4 * HB * S) void decode_step_finish_kernel(cons
         }
         M = m2;
     };
-    merge_batch(li0, oi0);
+    merge_batch(NB * (int)sl, li0, oi0);
     for (int j0 = NB * (int)sl + NB * S; j0 < u.count; j0 += NB * S) {
         float li[NB];
         float4 oi[NB];
         load_batch(j0, li, oi);
-        merge_batch(li, oi);
+        merge_batch(j0, li, oi);
     }
     if constexpr (S > 1) {
         __shared__ float sm_m[S][HB][LPH], sm_w[S][HB][LPH];
@@ -1370,6 +1382,7 @@ int decode_step_fast_path(const DecodePlan* p, const void* q, const void* k_new,
     a.stride_page = kv->stride_page; a.stride_n = kv->stride_n; a.stride_h = kv->stride_h;
     a.page_size = kv->page_size; a.num_qo_heads = num_qo_heads; a.num_kv_heads = kv->num_kv_heads;
     a.parts = p->mfma_parts;
+    a.page_shift = (kv->page_size & (kv->page_size - 1)) ? -1 : __builtin_ctz(kv->page_size);
     a.group = num_qo_heads / kv->num_kv_heads / p->mfma_parts;
     a.rope = rope ? 1 : 0;
     a.sm_scale_log2 = sm_scale_log2;

@@ -300,3 +300,12 @@ def test_fp32_rows_against_float64(ctx, P, bound):
         ref = dense_attention_f64(q[b], *p.gather_kv(b), p.D ** -0.5)
         num, den = num + ((got - ref) ** 2).sum(), den + (ref ** 2).sum()
     assert num <= bound ** 2 * den
+
+
+@pytest.mark.parametrize("P", [16, 48, 64])
+@pytest.mark.parametrize("lens", [[5000, 1], [33, 64, 900], [2100] * 9])
+def test_step_with_pieces_around_the_batches_of_partials(P, lens):
+    """Units of one partial and of many, so that a slice's batch of loads ends inside, at and past the last partial; pages whose
+    size is a power of two and one that is not; 32 q heads on one kv head are two units of one kv head."""
+    for Hq, Hkv in ((4, 1), (32, 1)):
+        run_step(DecodeProblem(750 + P + Hq, lens, Hq, Hkv, 128, P, BZ_F16), split_tokens=96)
