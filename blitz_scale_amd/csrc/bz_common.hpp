@@ -8,6 +8,7 @@
 #include <stdint.h>
 
 #include <tuple>
+#include <type_traits>
 
 #include "../../include/bz_hip.h"
 
@@ -230,15 +231,18 @@ template <> struct Vec8<float> {
 template <typename T> __device__ __forceinline__ constexpr size_t elem_size() { return sizeof(T); }
 
 // ---- wave64 reductions -------------------------------------------------------------------
+// Sum over the wave, left in every lane: the pairs of a butterfly (xor 32, 16, 8, 4, 2, 1) through the vector ALU -- lane swaps,
+// row rotations (by 8, and by 4 where lanes 8 apart hold the same) and quad permutes -- instead of six LDS round trips.
 __device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-    return v;
-}
-__device__ __forceinline__ float wave_max(float v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, 64));
-    return v;
+    auto dpp_add = [](float x, auto ctrl) {
+        constexpr int C = decltype(ctrl)::value;
+        return x + __uint_as_float(__builtin_amdgcn_update_dpp(0u, __float_as_uint(x), C, 0xF, 0xF, false));
+    };
+    v = lane_sum_xor16(lane_sum_xor32(v));
+    v = dpp_add(v, std::integral_constant<int, 0x128>{}); // row_ror:8
+    v = dpp_add(v, std::integral_constant<int, 0x124>{}); // row_ror:4
+    v = dpp_add(v, std::integral_constant<int, 0x4E>{});  // quad_perm [2,3,0,1]
+    return dpp_add(v, std::integral_constant<int, 0xB1>{}); // quad_perm [1,0,3,2]
 }
 
 // Llama rotate-half frequencies, f_i = theta^(-2i/D), evaluated in double on the host and rounded

@@ -5,15 +5,19 @@
 
 namespace bz {
 
-// sum over the workgroup; every lane gets the result
-__device__ __forceinline__ float block_sum(float v, float* smem /* [16] */) {
+// sum over the workgroup, wave by wave; every lane gets the result (called once per kernel: smem is not handed back)
+__device__ __forceinline__ float block_sum(float v, float (&smem)[16]) {
     v = wave_sum(v);
     const int wave = threadIdx.x / 64, lane = threadIdx.x % 64, nw = (blockDim.x + 63) / 64;
     if (lane == 0) smem[wave] = v;
     __syncthreads();
-    float t = 0.f;
-    for (int w = 0; w < nw; ++w) t += smem[w];
-    __syncthreads();
+    float part[8], t = 0.f; // (eight asked for at once; a loop over the waves that there are waits for each)
+    for (int w0 = 0; w0 < nw; w0 += 8) {
+#pragma unroll
+        for (int w = 0; w < 8; w += 4) *reinterpret_cast<float4*>(&part[w]) = *reinterpret_cast<const float4*>(&smem[w0 + w]);
+#pragma unroll
+        for (int w = 0; w < 8; ++w) t += w0 + w < nw ? part[w] : 0.f;
+    }
     return t;
 }
 
@@ -25,7 +29,7 @@ __device__ __forceinline__ float block_sum(float v, float* smem /* [16] */) {
 template <typename T, bool ADD, bool WHOLE>
 __global__ __launch_bounds__(1024) void rms_norm_kernel(T* input, T* residual, const T* weight, T* output,
                                                          uint32_t h, float eps) {
-    __shared__ float smem[16];
+    __shared__ __attribute__((aligned(16))) float smem[16];
     const size_t row = (size_t)blockIdx.x * h;
     const uint32_t nvec = h / 8;
     float ss = 0.f;
