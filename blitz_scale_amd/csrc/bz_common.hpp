@@ -38,6 +38,9 @@ inline void launch_kernel(void (*kernel)(P...), dim3 grid, dim3 block, size_t ld
     }, values);
 }
 
+// Host: a plan's tables, `bytes` of pinned memory, to device memory, in order with the stream (bz_decode_plan.hip).
+int upload_tables(void* to, const void* staging, size_t bytes, hipStream_t s);
+
 constexpr int kWave = 64;
 
 struct f16_t { uint16_t bits; };

@@ -1373,7 +1373,7 @@ extern "C" int bz_prefill_plan(bz_prefill_plan_t* plan_, void* float_buffer, siz
         p->staging = nullptr;
         p->staging_bytes = 0;
         const size_t want = std::max<size_t>(pf_align_up(bytes * 2, 4096), 1 << 16);
-        BZ_CHECK_HIP(hipHostMalloc(&p->staging, want, hipHostMallocDefault));
+        BZ_CHECK_HIP(hipHostMalloc(&p->staging, want, hipHostMallocPortable));
         p->staging_bytes = want;
     }
     uint32_t launched = 0;
@@ -1386,7 +1386,7 @@ extern "C" int bz_prefill_plan(bz_prefill_plan_t* plan_, void* float_buffer, siz
             memcpy(to + parts_at, cut.parts.data(), cut.parts.size() * sizeof(PrefillPart));
             memcpy(to + joins_at, cut.joins.data(), cut.joins.size() * sizeof(PrefillJoin));
         }
-        BZ_CHECK_HIP(hipMemcpyAsync(int_buffer, p->staging, bytes, hipMemcpyHostToDevice, s));
+        if (const int rc = upload_tables(int_buffer, p->staging, bytes, s)) return rc;
     }
     BZ_CHECK_HIP(hipEventRecord(p->upload_done, s));
     p->items_d = (const PrefillItem*)int_buffer;

@@ -477,3 +477,16 @@ def test_raw_k_rows_in_f16_keep_the_range_of_fp32():
     ref = oracle.batch_decode(p.q, BZ_F16, p.oracle_kv(), 1, rope_mode=BZ_ROPE_FULL, rope_theta=1e4, parallel=True)
     got = dev.decode(None, BZ_ROPE_FULL, 1e4)
     assert np.isfinite(got).all() and (np.abs(got - ref) <= ulp_tol(ref, BZ_F16)).all(), np.abs(got - ref).max()
+
+
+@pytest.mark.parametrize("offset", [0, 16, 4])
+def test_tables_reach_a_workspace_that_begins_anywhere(offset):
+    """The schedule goes up by a kernel where the workspace begins on a vector, by a copy where it does not; planned twice, so that
+    the second schedule meets the first one's staging buffer."""
+    p = DecodeProblem(760, [700, 64, 3000, 17], 8, 2, 128, 16, BZ_F16)
+    dev = DeviceDecode(p)
+    dev.int_ws = torch.full((8 << 20,), 255, dtype=torch.uint8, device="cuda")[offset:]
+    ref = oracle.batch_decode(p.q, p.dtype, p.oracle_kv(), p.Hq, parallel=True)
+    for split_tokens in (256, 0):
+        dev.plan(split_tokens)
+        assert (np.abs(dev.decode() - ref) <= ulp_tol(ref, p.dtype)).all()
