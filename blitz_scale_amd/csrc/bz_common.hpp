@@ -40,6 +40,9 @@ inline void launch_kernel(void (*kernel)(P...), dim3 grid, dim3 block, size_t ld
 
 // Host: a plan's tables, `bytes` of pinned memory, to device memory, in order with the stream (bz_decode_plan.hip).
 int upload_tables(void* to, const void* staging, size_t bytes, hipStream_t s);
+// What that buffer is allocated as: a kernel reads it again after the host has written the next plan, so the device may not
+// keep its lines, and a plan may go up on another device than the last one did.
+constexpr unsigned kStagingMemory = hipHostMallocPortable | hipHostMallocCoherent;
 
 constexpr int kWave = 64;
 

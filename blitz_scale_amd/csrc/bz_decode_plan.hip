@@ -412,7 +412,7 @@ extern "C" int bz_decode_plan(bz_decode_plan_t* plan_, void* float_buffer, size_
         p->staging = nullptr;
         p->staging_bytes = 0;
         const size_t want = std::max<size_t>(align_up(total * 2, 4096), 1 << 16);
-        BZ_CHECK_HIP(hipHostMalloc(&p->staging, want, hipHostMallocPortable));
+        BZ_CHECK_HIP(hipHostMalloc(&p->staging, want, kStagingMemory));
         p->staging_bytes = want;
     }
     char* st = (char*)p->staging;

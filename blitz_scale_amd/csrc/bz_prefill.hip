@@ -1373,7 +1373,7 @@ extern "C" int bz_prefill_plan(bz_prefill_plan_t* plan_, void* float_buffer, siz
         p->staging = nullptr;
         p->staging_bytes = 0;
         const size_t want = std::max<size_t>(pf_align_up(bytes * 2, 4096), 1 << 16);
-        BZ_CHECK_HIP(hipHostMalloc(&p->staging, want, hipHostMallocPortable));
+        BZ_CHECK_HIP(hipHostMalloc(&p->staging, want, kStagingMemory));
         p->staging_bytes = want;
     }
     uint32_t launched = 0;
