@@ -497,12 +497,13 @@ extern "C" int bz_decode_plan(bz_decode_plan_t* plan_, void* float_buffer, size_
     // writes its final rows at once.  So the one call pays where most of them are split over wave slots
     // anyway (batches with fewer of them than the launch has slots), and the two calls are taken where most
     // are whole (1024 sequences of 64 tokens: 63 us against 77 us).  The one call also needs room for one
-    // partial per piece in the float workspace.
+    // partial per piece in the float workspace, and no (sequence, kv head) with 4 GiB of them: its kernel's offsets have 32 bits.
     {
         const size_t part_o_bytes = ((size_t)p->mfma_pieces * 16 * head_dim * sizeof(float) + 255) / 256 * 256;
         const size_t part_lse_bytes = ((size_t)p->mfma_pieces * 16 * sizeof(float) + 255) / 256 * 256;
         const bool applies = p->mfma_ok && !p->force_general && p->mfma_slots > 0 && p->mfma_units_d &&
-                             p->mfma_units > 0 && part_o_bytes + part_lse_bytes <= p->float_buffer_bytes;
+                             p->mfma_units > 0 && part_o_bytes + part_lse_bytes <= p->float_buffer_bytes &&
+                             (uint64_t)p->mfma_unit_max_count * 16 * head_dim * sizeof(float) <= (uint64_t)1 << 32;
         const bool mostly_split = 2 * (uint64_t)p->mfma_combos >= p->mfma_units;
         p->step_one_call = applies && (force_one_call || mostly_split);
     }
