@@ -490,3 +490,16 @@ def test_tables_reach_a_workspace_that_begins_anywhere(offset):
     for split_tokens in (256, 0):
         dev.plan(split_tokens)
         assert (np.abs(dev.decode() - ref) <= ulp_tol(ref, p.dtype)).all()
+
+
+def test_tables_above_half_a_megabyte_take_the_copy_engine():
+    """800 sequences of a tile, eight kv heads each: 0.9 MB of tables, then few again from the same handle, then many."""
+    many, few = DecodeProblem(761, [20] * 800, 8, 8, 128, 16, BZ_F16), DecodeProblem(762, [90, 1, 700], 8, 8, 128, 16, BZ_F16)
+    handler = None
+    for p in (many, few, many):
+        dev = DeviceDecode(p)
+        dev.handler = handler = handler or dev.handler
+        dev.plan(0)
+        ref = oracle.batch_decode(p.q, p.dtype, p.oracle_kv(), p.Hq, parallel=True)
+        got = dev.decode()
+        assert (np.abs(got - ref) <= ulp_tol(ref, p.dtype)).all()
