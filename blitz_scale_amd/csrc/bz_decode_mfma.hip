@@ -186,15 +186,18 @@ constexpr int kInfoChunk = 16; // tile descriptions fetched per round trip (one 
 //
 // ROPE_K: the pool holds K as projected (BZ_ROPE_FULL), 16-bit rows of 128.  Every K value is multiplied by factors of its token
 // and pair before it becomes an operand; 64 floats of angles per lane and tile have no place beside two waves per SIMD.  They
-// are put together instead, from the angle of a subtile's first token (one sincosf per lane, passed around through LDS) and the
-// lane's own offset of 0 to 15 tokens, whose sixteen pairs of factors a lane keeps for the whole slot.  That, the rotation and
-// the split into head and tail are 560 vector instructions per tile, about 15 of the 44 us below, and run while the other wave of
-// the SIMD has its tile in flight.  The same rule as for heads of 64 keeps fp32 rows and log-sum-exps with the general kernel.
+// are put together instead, from the angle of a subtile's first token (one sincosf per lane and tile, the second subtile's turned
+// on from it by sixteen tokens; passed around through LDS) and the lane's own offset of 0 to 15 tokens, whose sixteen pairs of
+// factors a lane keeps for the whole slot.  That, the rotation and the split into head and tail are some 500 vector instructions
+// per tile, about a third of the 43 us below, and run while the other wave of the SIMD has its tile in flight.  The same rule as
+// for heads of 64 keeps fp32 rows and log-sum-exps with the general kernel.
 // 48 sequences of 200 .. 2 048 tokens, 32/8 heads, bf16, the whole call with append and combine: 65.8 us on the general kernel,
-// whose vector units do the contractions too, 51.0 here (the kernel alone 60 -> 44, and no table of angles in front of it);
-// 60 with 48/8 heads 164 -> 62, 42 with 64/8 82 -> 48, 128 x 100 .. 500 with 40/8 140 -> 44, 64 x 512 .. 1 500 with 32/32 236 ->
-// 193, 1 x 100 16.5 -> 13.0.  Against float64 (2-norm): 2.08e-4 and 1.66e-3 as before in f16 and bf16, 7.9e-4 -> 7.5e-4 and
-// 1.78e-3 -> 1.77e-3 for three sequences of 20 000 .. 60 000, whose angles lose less to fp32.
+// whose vector units do the contractions too, 49.3 here (the kernel alone 60 -> 43, and no table of angles in front of it);
+// 60 with 48/8 heads 164 -> 61, 42 with 64/8 82 -> 48, 128 x 100 .. 500 with 40/8 140 -> 43, 64 x 512 .. 1 500 with 32/32 238 ->
+// 179, 4 x 9 000 .. 30 000 with 64/8 130 -> 71, 128 x 1 024 112 -> 97, 1 x 100 15.5 -> 13.0.  (A sincosf for each subtile:
+// 48 sequences 49.6, 64 181, 4 72.1, 128 x 1 024 98.7.)  Against float64 (2-norm): 2.08e-4 and 1.65e-3 as before in f16 and bf16; three sequences of 20 000
+// .. 60 000, whose angles lose less to fp32, 2.77e-4 -> 2.64e-4 (theta 5e5, f16), 3.37e-4 -> 3.18e-4 (1e4, f16), 1.684e-3 ->
+// 1.680e-3 (1e4, bf16).
 template <bool BF16, typename OT, bool ROPE_Q, bool KV8, bool NT, int D, bool ROPE_K>
 __global__ __launch_bounds__(64, 2) void decode_mfma_kernel(const MfmaSlotHead* __restrict__ heads, MfmaDecodeArgs a,
                                                             const char* __restrict__ q_ptr,
@@ -429,14 +432,13 @@ __global__ __launch_bounds__(64, 2) void decode_mfma_kernel(const MfmaSlotHead* 
     // Raw-K pools: cos and sin of n * frequency for this lane's token n of a subtile and its sixteen pairs (steps ks and
     // ks + 2 of the contraction hold the two halves of a row).  One lane per pair evaluates the sixteen tokens, the LDS of the V
     // tile, still unused, turns the table around.
-    float tok_c[ROPE_K ? 16 : 1], tok_s[ROPE_K ? 16 : 1];
+    float tok_c[ROPE_K ? 16 : 1], tok_s[ROPE_K ? 16 : 1], step_c = 1.f, step_s = 0.f; // (step: of 16 tokens, for the lane's own pair)
     if constexpr (ROPE_K) {
         float2* table = reinterpret_cast<float2*>(v_lds); // [16 tokens][64 pairs]
 #pragma nounroll
-        for (int t = 0; t < 16; ++t) {
-            float sn, cs;
-            sincosf((float)t * lane_freq, &sn, &cs);
-            table[t * 64 + lane] = make_float2(cs, sn);
+        for (int t = 0; t <= 16; ++t) {
+            sincosf((float)t * lane_freq, &step_s, &step_c);
+            if (t < 16) table[t * 64 + lane] = make_float2(step_c, step_s);
         }
         wave_lds_sync();
 #pragma unroll
@@ -524,16 +526,22 @@ __global__ __launch_bounds__(64, 2) void decode_mfma_kernel(const MfmaSlotHead* 
     // per lane, passed around through LDS) and, in the same products, by the lane's own offset from it; the rotated rows are
     // split into head and tail like q.
     auto scores_raw_k = [&](const uint4 (&kop)[2][4], const TileUni& uc, f32x4_t (&s)[2]) __attribute__((always_inline)) {
+        // (with the part of position * frequency that fp32 drops: the offsets are small, so the angles of all 32 tokens are then
+        // as good as their frequency; those of the second subtile are the first one's, turned on by sixteen tokens)
+        const float first_tok = (float)(uc.t * kTileTok), angle = first_tok * lane_freq, dropped = fmaf(first_tok, lane_freq, -angle);
+        float sn1, cs1;
+        sincosf(angle, &sn1, &cs1);
+        float base_c = kRotatedK * fmaf(-sn1, dropped, cs1), base_s = kRotatedK * fmaf(cs1, dropped, sn1);
 #pragma unroll
         for (int u = 0; u < 2; ++u) {
-            // (with the part of position * frequency that fp32 drops: the offsets are small, so the angles of all sixteen tokens
-            // are then as good as their frequency)
-            const float first_tok = (float)(uc.t * kTileTok + 16 * u), angle = first_tok * lane_freq, dropped = fmaf(first_tok, lane_freq, -angle);
-            float sn1, cs1;
-            sincosf(angle, &sn1, &cs1);
+            if (u) {
+                const float c = base_c;
+                base_c = c * step_c - base_s * step_s;
+                base_s = base_s * step_c + c * step_s;
+            }
             wave_lds_sync();
-            rope_cs[0][lane] = kRotatedK * fmaf(-sn1, dropped, cs1);
-            rope_cs[ROPE_Q ? 1 : 0][lane] = kRotatedK * fmaf(cs1, dropped, sn1);
+            rope_cs[0][lane] = base_c;
+            rope_cs[ROPE_Q ? 1 : 0][lane] = base_s;
             wave_lds_sync();
             s[u] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
