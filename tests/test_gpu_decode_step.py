@@ -309,3 +309,15 @@ def test_step_with_pieces_around_the_batches_of_partials(P, lens):
     size is a power of two and one that is not; 32 q heads on one kv head are two units of one kv head."""
     for Hq, Hkv in ((4, 1), (32, 1)):
         run_step(DecodeProblem(750 + P + Hq, lens, Hq, Hkv, 128, P, BZ_F16), split_tokens=96)
+
+
+def test_form_of_a_step_whose_partials_of_one_unit_pass_4_gib():
+    """One sequence cut into as many one-tile pieces as 32-bit offsets into its partials reach, and one more: planned, not run."""
+    float_ws = torch.empty((4 << 30) + (64 << 20), dtype=torch.uint8, device="cuda")
+    int_ws = torch.empty(256 << 20, dtype=torch.uint8, device="cuda")
+    for tiles, form in ((1 << 19, "one_call"), ((1 << 19) + 1, "two_calls")):
+        handler = K.BlitzBatchDecodeHandler()
+        handler.plan(float_ws, float_ws.numel(), int_ws, int_ws.numel(), np.array([0, 2 * tiles], np.int32), np.array([16], np.int32),
+                     1, 1, 1, 128, 16, split_tokens=32)
+        assert handler.step_form() == form
+    torch.cuda.synchronize()
