@@ -183,22 +183,7 @@ constexpr int kInfoChunk = 16; // tile descriptions fetched per round trip (one 
 // whose results are 16-bit rows come this way (decode_fast_path), and an f16 operand, whose range is what head + tail runs
 // out of at both ends, is scaled by a power of two: the rotated q by 1/2 (two values near 65 504 rotate to as much as
 // 92 600), the probabilities by 2^kProbLog2, so that a long tail of small ones beside a large one is not flushed.
-//
-// ROPE_K: the pool holds K as projected (BZ_ROPE_FULL), 16-bit rows of 128.  Every K value is multiplied by factors of its token
-// and pair before it becomes an operand; 64 floats of angles per lane and tile have no place beside two waves per SIMD.  They
-// are put together instead, from the angle of a subtile's first token (one sincosf per lane and tile, the second subtile's turned
-// on from it by sixteen tokens; passed around through LDS) and the lane's own offset of 0 to 15 tokens, whose sixteen pairs of
-// factors a lane keeps for the whole slot.  That, the rotation and the split into head and tail are some 500 vector instructions
-// per tile, about a third of the 43 us below, and run while the other wave of the SIMD has its tile in flight.  The same rule as
-// for heads of 64 keeps fp32 rows and log-sum-exps with the general kernel.
-// 48 sequences of 200 .. 2 048 tokens, 32/8 heads, bf16, the whole call with append and combine: 65.8 us on the general kernel,
-// whose vector units do the contractions too, 49.3 here (the kernel alone 60 -> 43, and no table of angles in front of it);
-// 60 with 48/8 heads 164 -> 61, 42 with 64/8 82 -> 48, 128 x 100 .. 500 with 40/8 140 -> 43, 64 x 512 .. 1 500 with 32/32 238 ->
-// 179, 4 x 9 000 .. 30 000 with 64/8 130 -> 71, 128 x 1 024 112 -> 97, 1 x 100 15.5 -> 13.0.  (A sincosf for each subtile:
-// 48 sequences 49.6, 64 181, 4 72.1, 128 x 1 024 98.7.)  Against float64 (2-norm): 2.08e-4 and 1.65e-3 as before in f16 and bf16; three sequences of 20 000
-// .. 60 000, whose angles lose less to fp32, 2.77e-4 -> 2.64e-4 (theta 5e5, f16), 3.37e-4 -> 3.18e-4 (1e4, f16), 1.684e-3 ->
-// 1.680e-3 (1e4, bf16).
-template <bool BF16, typename OT, bool ROPE_Q, bool KV8, bool NT, int D, bool ROPE_K>
+template <bool BF16, typename OT, bool ROPE_Q, bool KV8, bool NT, int D>
 __global__ __launch_bounds__(64, 2) void decode_mfma_kernel(const MfmaSlotHead* __restrict__ heads, MfmaDecodeArgs a,
                                                             const char* __restrict__ q_ptr,
                                                             const char* __restrict__ k_data,
@@ -209,13 +194,11 @@ __global__ __launch_bounds__(64, 2) void decode_mfma_kernel(const MfmaSlotHead* 
                                                             const float* __restrict__ k_scale,
                                                             const float* __restrict__ v_scale) {
     static_assert(D == 128 || (D == 64 && !KV8), "head sizes");
-    static_assert(!ROPE_K || (D == 128 && !KV8 && ROPE_Q), "raw-K pools: 16-bit rows of 128, q rotated as well");
     using M = Mma<BF16>;
     constexpr bool TWO_SETS = KV8 || D == 64;   // a tile is 8 KiB: two of them in flight per wave
     constexpr int KS = D / 32, DB = D / 16;     // matrix steps of the scores; 16-wide blocks of the output
-    constexpr bool F16_RANGE = (D == 64 || ROPE_K) && !BF16;
+    constexpr bool F16_RANGE = D == 64 && !BF16;
     constexpr float kRotatedQ = F16_RANGE ? 0.5f : 1.f, kProbLog2 = F16_RANGE ? 14.f : 0.f;
-    constexpr float kRotatedK = F16_RANGE ? 0.5f : 1.f;
     constexpr int kVRowBytes = 2 * D + kVRowPad;
     __shared__ __attribute__((aligned(16))) unsigned char v_lds[kTileTok * kVRowBytes];
     __shared__ __attribute__((aligned(16))) int info_lds[2][kInfoChunk][kInfoInts];
@@ -315,10 +298,8 @@ __global__ __launch_bounds__(64, 2) void decode_mfma_kernel(const MfmaSlotHead* 
         return make_desc(rec, fetch_dep(rec));
     };
     auto stash_info = [&](const Desc& d, int buf) {
-        int lane_here = lane;
-        if constexpr (ROPE_K) asm volatile("" : "+v"(lane_here)); // (see the end of a piece)
-        if (lane_here < kInfoChunk) {
-            int* dst = &info_lds[buf][lane_here][0];
+        if (lane < kInfoChunk) {
+            int* dst = &info_lds[buf][lane][0];
             *reinterpret_cast<int4*>(dst) = make_int4(d.v[0], d.v[1], d.v[2], d.v[3]);
             *reinterpret_cast<int4*>(dst + 4) = make_int4(d.v[4], d.v[5], d.v[6], d.v[7]);
             *reinterpret_cast<int2*>(dst + 8) = make_int2(d.v[8], d.v[9]);
@@ -341,10 +322,7 @@ __global__ __launch_bounds__(64, 2) void decode_mfma_kernel(const MfmaSlotHead* 
         return u;
     };
 
-    uint4 kreg[2][4], vreg[8], qhi[KS], qlo[KS], qnext_regs[ROPE_K ? 1 : KS];
-    // (raw-K pools: the next piece's rows land where the head operands lie, which nothing reads between the scores of a piece's
-    // last tile and the next one's first: sixteen registers less)
-    uint4(&qnext)[KS] = [&]() -> uint4(&)[KS] { if constexpr (ROPE_K) return qhi; else return qnext_regs; }();
+    uint4 kreg[2][4], vreg[8], qnext[KS];
     // byte offsets of the two 16-token subtiles of a tile inside the pool
     struct TileBase { size_t b[2]; };
     auto tile_base = [&](const TileUni& u) -> TileBase {
@@ -429,31 +407,10 @@ __global__ __launch_bounds__(64, 2) void decode_mfma_kernel(const MfmaSlotHead* 
         stash_info(make_desc(rec0, raw0), 0);
         wave_lds_sync();
     }
-    // Raw-K pools: cos and sin of n * frequency for this lane's token n of a subtile and its sixteen pairs (steps ks and
-    // ks + 2 of the contraction hold the two halves of a row).  One lane per pair evaluates the sixteen tokens, the LDS of the V
-    // tile, still unused, turns the table around.
-    float tok_c[ROPE_K ? 16 : 1], tok_s[ROPE_K ? 16 : 1], step_c = 1.f, step_s = 0.f; // (step: of 16 tokens, for the lane's own pair)
-    if constexpr (ROPE_K) {
-        float2* table = reinterpret_cast<float2*>(v_lds); // [16 tokens][64 pairs]
-#pragma nounroll
-        for (int t = 0; t <= 16; ++t) {
-            sincosf((float)t * lane_freq, &step_s, &step_c);
-            if (t < 16) table[t * 64 + lane] = make_float2(step_c, step_s);
-        }
-        wave_lds_sync();
-#pragma unroll
-        for (int ks = 0; ks < 2; ++ks)
-#pragma unroll
-            for (int e = 0; e < 8; e += 2) {
-                const float4 v = *reinterpret_cast<const float4*>(&table[n * 64 + 32 * ks + 8 * j + e]);
-                tok_c[8 * ks + e] = v.x; tok_s[8 * ks + e] = v.y;
-                tok_c[8 * ks + e + 1] = v.z; tok_s[8 * ks + e + 1] = v.w;
-            }
-        wave_lds_sync();
-    }
     int chunk_base = g_begin, buf = 0;
     Desc dnext;
 
+    uint4 qhi[KS], qlo[KS];
     float m_run = -INFINITY, l_run = 0.f;
     f32x4_t acc[DB];
 
@@ -465,7 +422,7 @@ __global__ __launch_bounds__(64, 2) void decode_mfma_kernel(const MfmaSlotHead* 
     };
     // (positive; the floor keeps masked scores at -inf instead of NaN should a head's K scale be zero)
     auto score_scale_of = [&](const TileUni& uc) __attribute__((always_inline)) {
-        return fmaxf(a.sm_scale_log2 * ((KV8 && k_scale) ? k_scale[uc.kvr] : 1.0f), 1e-30f) * (ROPE_Q ? 1.f / kRotatedQ : 1.f) * (ROPE_K ? 1.f / kRotatedK : 1.f);
+        return fmaxf(a.sm_scale_log2 * ((KV8 && k_scale) ? k_scale[uc.kvr] : 1.0f), 1e-30f) * (ROPE_Q ? 1.f / kRotatedQ : 1.f);
     };
     // ================= first tile of a piece =================
     auto open_piece = [&](const TileUni& uc) __attribute__((always_inline)) {
@@ -519,60 +476,6 @@ __global__ __launch_bounds__(64, 2) void decode_mfma_kernel(const MfmaSlotHead* 
             if (ROPE_Q) {
 #pragma unroll
                 for (int ks = 0; ks < KS; ++ks) s[u] = M::run(kop[u][ks], qlo[ks], s[u]);
-            }
-        }
-    };
-    // ---- the same over a raw-K pool: the rows of a subtile are rotated on the way, by the angle of its first token (one pair
-    // per lane, passed around through LDS) and, in the same products, by the lane's own offset from it; the rotated rows are
-    // split into head and tail like q.
-    auto scores_raw_k = [&](const uint4 (&kop)[2][4], const TileUni& uc, f32x4_t (&s)[2]) __attribute__((always_inline)) {
-        // (with the part of position * frequency that fp32 drops: the offsets are small, so the angles of all 32 tokens are then
-        // as good as their frequency; those of the second subtile are the first one's, turned on by sixteen tokens)
-        const float first_tok = (float)(uc.t * kTileTok), angle = first_tok * lane_freq, dropped = fmaf(first_tok, lane_freq, -angle);
-        float sn1, cs1;
-        sincosf(angle, &sn1, &cs1);
-        float base_c = kRotatedK * fmaf(-sn1, dropped, cs1), base_s = kRotatedK * fmaf(cs1, dropped, sn1);
-#pragma unroll
-        for (int u = 0; u < 2; ++u) {
-            if (u) {
-                const float c = base_c;
-                base_c = c * step_c - base_s * step_s;
-                base_s = base_s * step_c + c * step_s;
-            }
-            wave_lds_sync();
-            rope_cs[0][lane] = base_c;
-            rope_cs[ROPE_Q ? 1 : 0][lane] = base_s;
-            wave_lds_sync();
-            s[u] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-            for (int ks = 0; ks < 2; ++ks) {
-                uint4 xh, yh, xl, yl;
-#pragma unroll
-                for (int w = 0; w < 4; ++w) {
-                    const uint32_t xw = reinterpret_cast<const uint32_t*>(&kop[u][ks])[w], yw = reinterpret_cast<const uint32_t*>(&kop[u][ks + 2])[w];
-                    const float x[2] = {M::unpack_lo(xw), M::unpack_hi(xw)}, y[2] = {M::unpack_lo(yw), M::unpack_hi(yw)};
-                    float xr[2], yr[2];
-#pragma unroll
-                    for (int e = 0; e < 2; ++e) {
-                        const int i = 2 * w + e;
-                        const float cb = rope_cs[0][32 * ks + 8 * j + i], sb = rope_cs[ROPE_Q ? 1 : 0][32 * ks + 8 * j + i];
-                        const float ct = tok_c[8 * ks + i], st = tok_s[8 * ks + i];
-                        const float c = cb * ct - sb * st, sn = sb * ct + cb * st;
-                        xr[e] = x[e] * c - y[e] * sn;
-                        yr[e] = y[e] * c + x[e] * sn;
-                    }
-                    const uint32_t xp = M::pack2(xr[0], xr[1]), yp = M::pack2(yr[0], yr[1]);
-                    u4(xh, w) = xp;
-                    u4(yh, w) = yp;
-                    u4(xl, w) = M::pack2(xr[0] - M::unpack_lo(xp), xr[1] - M::unpack_hi(xp));
-                    u4(yl, w) = M::pack2(yr[0] - M::unpack_lo(yp), yr[1] - M::unpack_hi(yp));
-                }
-                s[u] = M::run(xh, qhi[ks], s[u]);
-                s[u] = M::run(yh, qhi[ks + 2], s[u]);
-                s[u] = M::run(xh, qlo[ks], s[u]);
-                s[u] = M::run(yh, qlo[ks + 2], s[u]);
-                s[u] = M::run(xl, qhi[ks], s[u]);
-                s[u] = M::run(yl, qhi[ks + 2], s[u]);
             }
         }
     };
@@ -699,11 +602,6 @@ __global__ __launch_bounds__(64, 2) void decode_mfma_kernel(const MfmaSlotHead* 
             // the normalised rows are parked in LDS, head-major (store_rows above says why)
             if (pend_rows + G > kStageRows || pend_n == kStagePieces) store_rows();
             float* rows = stage_lds + pend_rows * kStageRow;
-            // (raw-K pools: addresses formed here; kept from the start they would be spilled, and the reload, a load like any
-            // other, would wait here for the next tile)
-            int lane_here = lane;
-            if constexpr (ROPE_K) asm volatile("" : "+v"(lane_here));
-            const int n = lane_here & 15, j = lane_here >> 4;
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 const int head = 4 * j + i;
@@ -871,8 +769,7 @@ __global__ __launch_bounds__(64, 2) void decode_mfma_kernel(const MfmaSlotHead* 
             // been requested they held the next tile's V loads back until q had arrived.
             __builtin_amdgcn_s_waitcnt(0x0F70); // vmcnt(0)
             f32x4_t s[2];
-            if constexpr (ROPE_K) scores_raw_k(kreg, uc, s);
-            else scores(kreg, s);
+            scores(kreg, s);
             __builtin_amdgcn_sched_barrier(0); // the loads below overwrite the operands of the instructions above
             if (g + 1 < g_end) {
                 if (i + 1 == kInfoChunk) { chunk_base += kInfoChunk; buf ^= 1; }
@@ -1213,24 +1110,22 @@ __global__ __launch_bounds__(D / 4 * HB * S) void decode_step_finish_kernel(cons
 
 struct DecodeArgs; // general-kernel argument block (bz_decode.hip); only its scalar fields are forwarded here
 
-template <bool BF16, typename OT, bool ROPE_Q, bool KV8, int D, bool ROPE_K = false>
+template <bool BF16, typename OT, bool ROPE_Q, bool KV8, int D>
 static void launch_mfma_k(const DecodePlan* p, const MfmaDecodeArgs& a, hipStream_t s) {
     if (p->mfma_streaming)
-        launch_kernel((decode_mfma_kernel<BF16, OT, ROPE_Q, KV8, true, D, ROPE_K>), dim3(p->mfma_slots), dim3(64), 0, s, a.heads, a,
+        launch_kernel((decode_mfma_kernel<BF16, OT, ROPE_Q, KV8, true, D>), dim3(p->mfma_slots), dim3(64), 0, s, a.heads, a,
                            (const char*)a.q, a.k_data, a.v_data, a.indices, a.pieces, a.tiles, a.k_scale,
                            a.v_scale);
     else
-        launch_kernel((decode_mfma_kernel<BF16, OT, ROPE_Q, KV8, false, D, ROPE_K>), dim3(p->mfma_slots), dim3(64), 0, s, a.heads, a,
+        launch_kernel((decode_mfma_kernel<BF16, OT, ROPE_Q, KV8, false, D>), dim3(p->mfma_slots), dim3(64), 0, s, a.heads, a,
                            (const char*)a.q, a.k_data, a.v_data, a.indices, a.pieces, a.tiles, a.k_scale,
                            a.v_scale);
 }
 
 template <bool BF16, typename OT, bool KV8, int D>
-static int launch_mfma(const DecodePlan* p, const MfmaDecodeArgs& a, bool raw_k, hipStream_t s) {
+static int launch_mfma(const DecodePlan* p, const MfmaDecodeArgs& a, hipStream_t s) {
     if (p->time_start) BZ_CHECK_HIP(hipEventRecord(p->time_start, s));
-    if (raw_k) {
-        if constexpr (!KV8 && D == 128 && !std::is_same<OT, float>::value) launch_mfma_k<BF16, OT, true, KV8, D, true>(p, a, s);
-    } else if (a.rope_q) launch_mfma_k<BF16, OT, true, KV8, D>(p, a, s);
+    if (a.rope_q) launch_mfma_k<BF16, OT, true, KV8, D>(p, a, s);
     else launch_mfma_k<BF16, OT, false, KV8, D>(p, a, s);
     BZ_LAUNCH_CHECK();
     if (p->time_stop) BZ_CHECK_HIP(hipEventRecord(p->time_stop, s));
@@ -1251,10 +1146,10 @@ static int launch_mfma(const DecodePlan* p, const MfmaDecodeArgs& a, bool raw_k,
     return 0;
 }
 template <bool BF16, typename OT>
-static int launch_mfma_any(const DecodePlan* p, const MfmaDecodeArgs& a, bool kv8, bool raw_k, hipStream_t s) {
+static int launch_mfma_any(const DecodePlan* p, const MfmaDecodeArgs& a, bool kv8, hipStream_t s) {
     if constexpr (!std::is_same<OT, float>::value)
-        if (p->head_dim == 64) return launch_mfma<BF16, OT, false, 64>(p, a, false, s);
-    return kv8 ? launch_mfma<BF16, OT, true, 128>(p, a, false, s) : launch_mfma<BF16, OT, false, 128>(p, a, raw_k, s);
+        if (p->head_dim == 64) return launch_mfma<BF16, OT, false, 64>(p, a, s);
+    return kv8 ? launch_mfma<BF16, OT, true, 128>(p, a, s) : launch_mfma<BF16, OT, false, 128>(p, a, s);
 }
 
 int decode_fast_path(const DecodePlan* p, const void* q, void* out, float* lse, int q_dtype, int out_dtype,
@@ -1263,9 +1158,7 @@ int decode_fast_path(const DecodePlan* p, const void* q, void* out, float* lse, 
                      float* part_lse, bool step_mode, hipStream_t s) {
     if (!p->mfma_ok || p->mfma_slots == 0) return BZ_ERR_UNSUPPORTED;
     const bool kv8 = kv->kv_dtype == BZ_E4M3;
-    const bool raw_k = rope_mode == BZ_ROPE_FULL;
-    if (!kv8 && kv->kv_dtype != q_dtype) return BZ_ERR_UNSUPPORTED;
-    if (raw_k && (p->head_dim != 128 || kv8 || out_dtype == BZ_F32 || lse)) return BZ_ERR_UNSUPPORTED;
+    if ((!kv8 && kv->kv_dtype != q_dtype) || rope_mode == BZ_ROPE_FULL) return BZ_ERR_UNSUPPORTED;
     if (!kv8 && (k_scale || v_scale)) return BZ_ERR_UNSUPPORTED;
     // Heads of 64: calls whose results are 16-bit rows.  fp32 rows and log-sum-exps come from the general kernel, whose fp32 q
     // and probabilities show there (largest error of a row about 5e-7 against 2e-6 with head + tail operands).
@@ -1283,14 +1176,14 @@ int decode_fast_path(const DecodePlan* p, const void* q, void* out, float* lse, 
     a.stride_page = kv->stride_page; a.stride_n = kv->stride_n; a.stride_h = kv->stride_h;
     a.page_size = kv->page_size; a.num_qo_heads = num_qo_heads;
     a.group = num_qo_heads / kv->num_kv_heads / p->mfma_parts;
-    a.rope_q = rope_mode != BZ_ROPE_NONE;
+    a.rope_q = rope_mode == BZ_ROPE_Q_ONLY;
     a.step_mode = step_mode ? 1 : 0;
     a.sm_scale_log2 = sm_scale_log2;
     a.k_scale = k_scale; a.v_scale = v_scale;
     a.freqs = freqs;
     if (q_dtype == BZ_BF16)
-        return out_dtype == BZ_F32 ? launch_mfma_any<true, float>(p, a, kv8, raw_k, s) : launch_mfma_any<true, bf16_t>(p, a, kv8, raw_k, s);
-    return out_dtype == BZ_F32 ? launch_mfma_any<false, float>(p, a, kv8, raw_k, s) : launch_mfma_any<false, f16_t>(p, a, kv8, raw_k, s);
+        return out_dtype == BZ_F32 ? launch_mfma_any<true, float>(p, a, kv8, s) : launch_mfma_any<true, bf16_t>(p, a, kv8, s);
+    return out_dtype == BZ_F32 ? launch_mfma_any<false, float>(p, a, kv8, s) : launch_mfma_any<false, f16_t>(p, a, kv8, s);
 }
 
 template <typename QT, typename PT, typename OT, int D>

@@ -158,10 +158,9 @@ int bz_decode_plan_set_timing_events(bz_decode_plan_t* plan, void* start_event, 
  * (NULL = 1).  lse: optional device fp32 [batch, num_qo_heads] (reference passes nullptr).
  * Heads of 64 run on the matrix-core kernel where the pool is a 16-bit one, `out` has q's type and lse is NULL; fp32 rows and
  * log-sum-exps, whose low bits would show it, come from the general kernel, which keeps q and the probabilities in fp32.
- * BZ_ROPE_FULL (raw K in the cache, the reference's kRoPELlama): 16-bit rows of heads of 128 in pages of whole sixteens run on
- * the matrix-core kernel, which puts the angles together as it goes.  For the rest every call builds a table of angles, 4 *
- * head_dim bytes per position of the longest sequence, in the plan's float workspace behind the split-K partials when there is
- * room (it is only faster with it).
+ * BZ_ROPE_FULL (raw K in the cache, the reference's kRoPELlama): the general kernel, whose rotated K, q and probabilities are
+ * fp32.  Every call builds a table of angles, 4 * head_dim bytes per position of the longest sequence, in the plan's float
+ * workspace behind the split-K partials when there is room (it is only faster with it; bz_batch_decode_noalloc does without).
  */
 int bz_batch_decode(bz_decode_plan_t* plan, const void* q, int q_dtype, const bz_paged_kv_t* kv, void* out,
                     int out_dtype, uint32_t num_qo_heads, int rope_mode, float rope_theta, float sm_scale,

@@ -18,7 +18,7 @@ from blitz_scale_amd._lib import (BZ_BF16, BZ_E4M3, BZ_F16, BZ_F32, BZ_LAYOUT_HN
                                   BZ_ROPE_NONE, BZ_ROPE_Q_ONLY)
 
 from _gpu import DeviceDecode, to_dev, to_host_bits
-from _util import DecodeProblem, ulp_tol
+from _util import DecodeProblem, dense_attention_f64, rope_f64, ulp_tol
 
 pytestmark = pytest.mark.gpu
 
@@ -434,9 +434,9 @@ def test_general_kernel_with_page_ids_of_a_set_ahead(kv_dtype, Hq, Hkv, D, P):
 @pytest.mark.parametrize("Hq,Hkv,P,layout", [(1, 1, 16, BZ_LAYOUT_HND), (8, 2, 32, BZ_LAYOUT_NHD), (5, 1, 16, BZ_LAYOUT_HND),
                                              (12, 2, 48, BZ_LAYOUT_NHD), (32, 2, 64, BZ_LAYOUT_HND), (20, 1, 16, BZ_LAYOUT_NHD)])
 @pytest.mark.parametrize("split_tokens", [0, 96, 0xFFFFFFFF])
-def test_raw_k_rows_on_the_matrix_cores(dtype, Hq, Hkv, P, layout, split_tokens):
-    """16-bit rows over a raw-K cache of heads of 128: sequences that end on either side of a subtile of 16 and a tile of 32, one
-    piece after another in a wave slot, pieces that begin anywhere, groups up to 16 and one of two parts, no sequence at all."""
+def test_raw_k_rows_of_16_bits(dtype, Hq, Hkv, P, layout, split_tokens):
+    """16-bit rows over a raw-K cache of heads of 128: sequences that end on either side of 16, 32 and 64 tokens, whole and in
+    pieces, groups of 1 to 20, no sequence at all."""
     p = DecodeProblem(700 + Hq + P, [1, 15, 16, 17, 31, 32, 33, 0, 47, 48, 49, 95, 97, 700, 2100], Hq, Hkv, 128, P, dtype, layout=layout)
     dev = DeviceDecode(p)
     dev.plan(split_tokens)
@@ -461,22 +461,96 @@ def test_raw_k_rows_under_a_table_that_runs_ahead(dtype):
     assert (np.abs(got - ref) <= ulp_tol(ref, dtype)).all(), np.abs(got - ref).max()
 
 
-def test_raw_k_rows_in_f16_keep_the_range_of_fp32():
-    """Two values near the largest f16 rotate to as much as 92 600, and many tokens far below the largest have to count: both
-    are beyond an f16 operand that is not scaled.  K rows whose largest values meet in one pair, q that picks them out."""
-    p = DecodeProblem(731, [4000], 1, 1, 128, 16, BZ_F16)
-    f = np.zeros((p.pool_pages, 2, 1, 16, 128), np.float32)
-    f[:, 0, 0, :, 0] = f[:, 0, 0, :, 64] = 65504.0  # pair 0 turns by a radian a token
-    f[:, 1] = 1.0
-    p.pool = wl.to_bits(f.reshape(-1), BZ_F16)
-    q = np.zeros((1, 1, 128), np.float32)
-    q[0, 0, 0], q[0, 0, 64] = 2e-3, 1e-3
-    p.q = wl.to_bits(q, BZ_F16)
-    dev = DeviceDecode(p)
-    dev.plan(0)
-    ref = oracle.batch_decode(p.q, BZ_F16, p.oracle_kv(), 1, rope_mode=BZ_ROPE_FULL, rope_theta=1e4, parallel=True)
+def raw_k_rows_f64(p, theta):
+    """The rows of a raw-K call in float64, from the stored bits."""
+    out = np.zeros((p.B, p.Hq, p.D))
+    for b in range(p.B):
+        L = int(p.ctx[b])
+        k, v = p.gather_kv(b)
+        k = rope_f64(k, np.arange(L)[:, None, None], theta)
+        out[b] = dense_attention_f64(rope_f64(wl.to_f32(p.q[b], p.dtype), L - 1, theta), k, v, p.D ** -0.5)
+    return out
+
+
+def with_values_of_one(p, seed):
+    """V of standard normal values beside whatever K holds."""
+    half = p.stride_page // 2
+    planes = p.pool.reshape(-1, 2, half)
+    planes[:, 1] = wl.randn_bits(np.random.default_rng(seed), (len(planes), half), p.dtype)
+    return p
+
+
+# The rounding of the stored rows alone is 2.1e-4 (f16) and 1.66e-3 (bf16) of their 2-norm.
+ROWS_2NORM = {BZ_F16: 2.4e-4, BZ_BF16: 1.9e-3}
+
+
+@pytest.mark.parametrize("dtype", [BZ_F16, BZ_BF16])
+@pytest.mark.parametrize("split_tokens", [0, 0xFFFFFFFF])
+def test_raw_k_rows_are_as_good_as_their_rounding(dtype, split_tokens):
+    """Scores of a standard deviation of 4, so that what K, q and the probabilities lose in front of the softmax shows in the rows."""
+    p = DecodeProblem(731, [300, 700, 1025, 2047], 8, 2, 128, 16, dtype)
+    p.q = wl.to_bits(4 * wl.to_f32(p.q, dtype), dtype)
+    dev, ref = DeviceDecode(p), raw_k_rows_f64(p, 1e4)
+    dev.plan(split_tokens)
     got = dev.decode(None, BZ_ROPE_FULL, 1e4)
-    assert np.isfinite(got).all() and (np.abs(got - ref) <= ulp_tol(ref, BZ_F16)).all(), np.abs(got - ref).max()
+    assert np.linalg.norm(got - ref) <= ROWS_2NORM[dtype] * np.linalg.norm(ref)
+
+
+@pytest.mark.parametrize("dtype", [BZ_F16, BZ_BF16])
+def test_raw_k_rows_of_a_long_sequence(dtype):
+    """30 000 tokens, theta 5e5.  The frequency and position * frequency in fp32 are each off by up to half a unit in the last
+    place: over the 64 pairs 1.2e-4 rad rms for a K row (mean over the positions) and 2.1e-4 for q, at the end.  Scores of 1 are
+    off by as much, together 2.4e-4, and the rows by that beside their rounding."""
+    p = DecodeProblem(732, [30000], 4, 2, 128, 16, dtype)
+    dev, ref = DeviceDecode(p), raw_k_rows_f64(p, 5e5)
+    dev.plan()
+    got = dev.decode(None, BZ_ROPE_FULL, 5e5)
+    assert np.linalg.norm(got - ref) <= np.hypot(ROWS_2NORM[dtype], 2.4e-4) * np.linalg.norm(ref)
+
+
+def test_raw_k_rows_of_small_values_keep_their_bits():
+    """K of 1e-5, all of it below f16's normal range: a rotated value in fp32 has its 24 bits there, an f16 operand and what it
+    leaves behind would have seven.  q of +-6e4 makes scores of 0.6 of it (and leaves f16's range itself when it is rotated)."""
+    p = with_values_of_one(DecodeProblem(733, [1, 33, 300, 1000], 8, 2, 128, 16, BZ_F16, kv_std=1e-5), 733)
+    p.q = wl.to_bits(np.where(np.random.default_rng(7).random((p.B, p.Hq, p.D)) < 0.5, -6e4, 6e4).astype(np.float32), BZ_F16)
+    dev, ref = DeviceDecode(p), raw_k_rows_f64(p, 1e4)
+    dev.plan()
+    got = dev.decode(None, BZ_ROPE_FULL, 1e4)
+    assert np.linalg.norm(got - ref) <= ROWS_2NORM[BZ_F16] * np.linalg.norm(ref)
+
+
+def test_raw_k_rows_in_f16_keep_the_range_of_fp32():
+    """K rows whose two largest values meet in one pair rotate to as much as 92 600: q picks them out, and V differs from token to
+    token, so that the weights show."""
+    p = with_values_of_one(DecodeProblem(734, [4000], 1, 1, 128, 16, BZ_F16), 734)
+    k = np.zeros((len(p.pool) // p.stride_page, 16, 128), np.float32)
+    k[..., 0] = k[..., 64] = 65504.0  # pair 0 turns by a radian a token
+    p.pool.reshape(-1, 2, 16, 128)[:, 0] = wl.to_bits(k, BZ_F16)
+    q = np.zeros((1, 1, 128), np.float32)
+    q[0, 0, 0], q[0, 0, 64] = 2e-4, 1e-4
+    p.q = wl.to_bits(q, BZ_F16)
+    dev, ref = DeviceDecode(p), raw_k_rows_f64(p, 1e4)
+    dev.plan()
+    got = dev.decode(None, BZ_ROPE_FULL, 1e4)
+    # (128 values, whose rounding comes to a fifth more or less than many do)
+    assert np.linalg.norm(got - ref) <= 1.2 * ROWS_2NORM[BZ_F16] * np.linalg.norm(ref)
+
+
+def test_raw_k_rows_of_a_long_tail_of_small_probabilities():
+    """4 000 tokens in one piece whose probabilities lie 2^-26 below the largest one's and carry the whole result."""
+    p = DecodeProblem(735, [4000], 4, 2, 128, 16, BZ_F16, oversub=1.0)
+    planes = p.pool.reshape(-1, 2, 2, 16, 128)  # [page][K | V][kv head][token][dim]
+    planes[:, 0] = 0
+    planes[:, 1] = wl.to_bits(np.ones(1, np.float32), BZ_F16)
+    page, slot = p.indices[-1], (4000 - 1) % 16  # the newest token: q and K turned by the same angles
+    planes[page, 0, :, slot] = wl.to_bits(np.full(1, 26 * np.log(2) / 128 ** 0.5, np.float32), BZ_F16)
+    planes[page, 1, :, slot] = 0
+    p.q = wl.to_bits(np.ones((1, 4, 128), np.float32), BZ_F16)
+    ref = raw_k_rows_f64(p, 1e4)
+    assert 5e-5 < ref.min() and ref.max() < 7e-5
+    dev = DeviceDecode(p)
+    dev.plan(0xFFFFFFFF)
+    assert np.abs(dev.decode(None, BZ_ROPE_FULL, 1e4) / ref - 1).max() < 2e-3  # (a step of the stored f16 there is 1e-3)
 
 
 @pytest.mark.parametrize("offset", [0, 16, 4])
