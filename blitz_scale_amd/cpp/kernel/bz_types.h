@@ -47,7 +47,7 @@ struct AttentionOptions {
     bool store_rotates_k = false;           // store_prefill_kv_cache: k was rotated by the attention call before it
     bool append_rotates_k = true;           // append_decode_kv_cache rotates the new K row
     int decode_rope_mode = BZ_ROPE_Q_ONLY;  // batch_decode_attention: rotate q only, cached K is rotated
-    uint32_t split_tokens = 0;              // 0: the library's choice
+    uint32_t split_tokens = 0;              // 0: library default (2048)
     int prefill_bf16_mode = BZ_PREFILL_BF16_WIDEN_V; // bf16 prefill: second product in f16 with V widened (exact for
                                             // |v| in f16's range), or BZ_PREFILL_BF16_HEAD_TAIL for any range of V
     void* stream = nullptr;                 // hipStream_t; nullptr = the legacy default stream the reference uses

@@ -86,8 +86,7 @@ struct ScheduleLayout {
 static int build_schedule(DecodePlan* p, const int32_t* indptr_h, const int32_t* last_page_len_h, uint32_t batch_size,
                           uint32_t num_qo_heads, uint32_t num_kv_heads, uint32_t head_dim, uint32_t page_size,
                           uint32_t split_tokens, int cus, bool small_heads, ScheduleCounts* counts) {
-    const bool library_split = split_tokens == 0;
-    if (library_split) split_tokens = 2048;
+    if (split_tokens == 0) split_tokens = 2048;
     // ---- choose the piece length (in pages) -------------------------------------------------
     // Pieces never exceed split_tokens (contexts longer than that are always split); they are
     // shortened further, down to 256 tokens, until the launch holds about four workgroups per CU.
@@ -205,7 +204,7 @@ static int build_schedule(DecodePlan* p, const int32_t* indptr_h, const int32_t*
     // The flattened (sequence, kv head, 32-token tile) space is divided into equal shares, one per
     // wave slot of the chip (8 single-wave workgroups per CU).  A share that crosses a (sequence, kv
     // head) boundary becomes several pieces; a (sequence, kv head) that ends up in more than one
-    // piece, or is longer than the split_tokens asked for, is folded from partial results.  Every tile of a share
+    // piece, or is longer than split_tokens, is folded from partial results.  Every tile of a share
     // gets a 16-byte record so that the kernel never has to chase the piece list tile by tile.
     std::vector<MfmaPiece>& mp = p->h_pieces;
     RawArray<MfmaTile>& mt = p->h_tiles;
@@ -235,11 +234,10 @@ static int build_schedule(DecodePlan* p, const int32_t* indptr_h, const int32_t*
         const uint64_t max_slots = (uint64_t)cus * 8;
         const uint64_t share = std::max<uint64_t>(1, (total_tiles + max_slots - 1) / max_slots);
         p->mfma_streaming = share >= 2;
-        // The library's own split_tokens is the general kernel's, whose pieces are its workgroups.  A wave slot takes its share one
-        // tile after another whatever the pieces, and a piece that ends in it costs a partial row written and read again: 256
-        // sequences of 4 096 tokens, 64/8 heads, fp8 pool, where a slot has one (sequence, kv head) of 128 tiles, 351 us a step
-        // when they were cut at 2 048 tokens, 334 whole (and the step then runs as its two calls).
-        const uint32_t cap_tiles = never_split || library_split ? 0x7fffffffu : std::max<uint32_t>(1, split_tokens / 32);
+        // (Shares left whole unless a split is asked for: 256 sequences of 4 096 tokens, 64/8 heads, fp8 pool, 352 -> 333 us a step,
+        // 256 of 8 192, 32/8 heads, f16, 1 311 -> 1 278; but one chain of fp32 sums then spans the share: error of fp32 rows against
+        // float64 2.27e-6 -> 2.35e-6 and 5.4e-7 -> 9.1e-7.  A caller who wants that passes a longer split_tokens.)
+        const uint32_t cap_tiles = never_split ? 0x7fffffffu : std::max<uint32_t>(1, split_tokens / 32);
         // Workgroups are dealt round-robin to the 8 XCDs.  With plain K/V loads the odd XCDs streamed HBM
         // about a tenth slower than the even ones under full load (measured per wave with wall_clock64)
         // and a 9 % smaller share for their slots paid; with the non-temporal loads of the streaming

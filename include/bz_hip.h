@@ -102,8 +102,8 @@ void bz_kv_layer_view(bz_paged_kv_t* kv, void* pool_base, uint32_t layer, uint64
  * over the compute units and copies the schedule into int_buffer (device).  float_buffer
  * (device) receives the split-K partial results at run time.  Synchronous host work plus
  * one async H2D copy on `stream`, like the reference's plan().
- * split_tokens: contexts longer than this are always split (0 = the library's choice: 2048 for the general kernel, and
- * wherever a wave slot's share ends for the matrix-core kernel; UINT32_MAX = never split: one piece per sequence).
+ * split_tokens: contexts longer than this are always split (0 = library default 2048,
+ * UINT32_MAX = never split: one piece per sequence).
  * ------------------------------------------------------------------------------------- */
 typedef struct bz_decode_plan bz_decode_plan_t;
 

@@ -155,24 +155,18 @@ def test_matrix_core_schedule_invariants(name, lens, Hq, Hkv, P, split):
         assert ip0 == s["indptr"][b] and ntok == lens[b]
 
 
-def test_a_wave_slot_takes_its_share_whole_unless_a_split_is_asked_for():
-    """Sixteen slots of 94 tiles: without split_tokens a piece ends only where a share or a (sequence, kv head) does; asked for,
-    no piece is longer than it says.  The general kernel's segments are held to 2 048 tokens either way."""
-    lens, share = [6000, 3000, 6000, 40, 9000], (2 * sum((l + 31) // 32 for l in [6000, 3000, 6000, 40, 9000]) + 15) // 16
-    own = schedule(lens, 8, 2, 128, 16, 0, cus=2)
-    ends = set(own["slot_ptr"][:, 0])
-    at = 0
-    for seq, kvh, t0, t1 in own["pieces"][:, :4]:
-        at += t1 - t0
-        assert at in ends or t1 == (lens[seq] + 31) // 32
-    longest = (own["pieces"][:, 3] - own["pieces"][:, 2]).max()
-    assert 64 < longest <= share + 1
-    asked = schedule(lens, 8, 2, 128, 16, 2048, cus=2)
-    assert (asked["pieces"][:, 3] - asked["pieces"][:, 2]).max() == 64
-    check_mfma_schedule(asked, 2, 16, 2048)
+def test_no_chain_of_partial_sums_is_longer_than_2048_tokens_unless_that_is_asked_for():
+    """Sixteen slots of 94 tiles.  A piece's sums run from its first token to its last, so the default holds the pieces of both
+    kernels to 2 048 tokens, as asked for by name; a longer split_tokens leaves the shares whole."""
+    lens = [6000, 3000, 6000, 40, 9000]
+    own, asked, longer = (schedule(lens, 8, 2, 128, 16, split, cus=2) for split in (0, 2048, 1 << 20))
     for s in (own, asked):
+        assert (s["pieces"][:, 3] - s["pieces"][:, 2]).max() == 64
         assert (s["segments"][:, 2] - s["segments"][:, 1]).max() * 16 <= 2048
+        check_mfma_schedule(s, 2, 16, 2048)
         check_general_schedule(s, 16)
+    assert all(np.array_equal(own[key], asked[key]) for key in ("pieces", "segments", "slot_ptr"))
+    assert (longer["pieces"][:, 3] - longer["pieces"][:, 2]).max() > 64
 
 
 def test_shapes_outside_the_matrix_core_kernel_get_segments_only():
