@@ -25,7 +25,7 @@ static int device_cu_count() {
 
 // A plan's tables from its pinned staging buffer into the caller's workspace, a lane a vector: on the compute queue, in line with
 // the launches around it, where the copy engine has a signal to wait for in front of its copy and another behind it.  The
-// schedule of eight sequences of 1 000 tokens, 0.3 MB: plan and wait 47.5 us by the copy engine, 43.7 here; a model step of 32
+// schedule of eight sequences of 1 000 tokens, 0.3 MB: plan and wait 47 us by the copy engine, 44.6 here; a model step of 32
 // layers with its plan 523 -> 512.  The engine moves more bytes a second: 48 x 1 100 tokens, 0.48 MB, 59.5 and 58.9, 128 x 1 024,
 // 0.84 MB, 85.5 and 86.5, 256 x 4 096, 4.5 MB, 371 and 386; it keeps what is above half a megabyte.
 constexpr size_t kUploadByKernel = 512 << 10;
@@ -33,10 +33,22 @@ static __global__ __launch_bounds__(256) void table_copy_kernel(uint4* __restric
     const uint32_t i = blockIdx.x * 256 + threadIdx.x;
     if (i < n) to[i] = from[i];
 }
+// Whether `to` is memory of the current GPU, and `s` one of its streams.  (0.7 us; looked up in every call, since an address may
+// be another device's memory by the next one.)
+static bool kernel_reaches(const void* to, hipStream_t s) {
+    int current = 0, of_stream = 0;
+    hipPointerAttribute_t at;
+    bool known = hipGetDevice(&current) == hipSuccess && hipPointerGetAttributes(&at, to) == hipSuccess;
+    // (the null streams are the current device's)
+    if (!s || s == hipStreamPerThread || s == hipStreamLegacy) of_stream = current;
+    else known = known && hipStreamGetDevice(s, &of_stream) == hipSuccess;
+    if (!known) (void)hipGetLastError(); // memory that the runtime does not know is for the copy to judge
+    return known && at.type == hipMemoryTypeDevice && at.device == current && of_stream == current;
+}
 int upload_tables(void* to, const void* staging, size_t bytes, hipStream_t s) {
     if (bytes == 0) return 0;
     // (whole vectors; a workspace that begins inside one takes the copy engine)
-    if (bytes <= kUploadByKernel && bytes % sizeof(uint4) == 0 && (uintptr_t)to % sizeof(uint4) == 0) {
+    if (bytes <= kUploadByKernel && bytes % sizeof(uint4) == 0 && (uintptr_t)to % sizeof(uint4) == 0 && kernel_reaches(to, s)) {
         const uint32_t n = (uint32_t)(bytes / sizeof(uint4));
         launch_kernel(table_copy_kernel, dim3((n + 255) / 256), dim3(256), 0, s, (uint4*)to, (const uint4*)staging, n);
         BZ_LAUNCH_CHECK();

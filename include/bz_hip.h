@@ -101,7 +101,8 @@ void bz_kv_layer_view(bz_paged_kv_t* kv, void* pool_base, uint32_t layer, uint64
  * last_page_len: cuts every sequence into page-aligned segments (split-K), balances them
  * over the compute units and copies the schedule into int_buffer (device).  float_buffer
  * (device) receives the split-K partial results at run time.  Synchronous host work plus
- * one async H2D copy on `stream`, like the reference's plan().
+ * one async upload on `stream`, like the reference's plan(): by a kernel where the tables are small and int_buffer is memory of
+ * the current device, else by a copy, which reaches any GPU's.
  * split_tokens: contexts longer than this are always split (0 = library default 2048,
  * UINT32_MAX = never split: one piece per sequence).
  * ------------------------------------------------------------------------------------- */
