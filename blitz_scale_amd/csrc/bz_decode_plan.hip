@@ -27,7 +27,8 @@ static int device_cu_count() {
 // the launches around it, where the copy engine has a signal to wait for in front of its copy and another behind it.  The
 // schedule of eight sequences of 1 000 tokens, 0.3 MB: plan and wait 47 us by the copy engine, 44.6 here; a model step of 32
 // layers with its plan 523 -> 512.  The engine moves more bytes a second: 48 x 1 100 tokens, 0.48 MB, 59.5 and 58.9, 128 x 1 024,
-// 0.84 MB, 85.5 and 86.5, 256 x 4 096, 4.5 MB, 371 and 386; it keeps what is above half a megabyte.
+// 0.84 MB, 85.5 and 86.5, 256 x 4 096, 4.5 MB, 371 and 386; it keeps what is above half a megabyte,
+// and whatever a kernel on this stream may not write: a copy reaches a workspace on any GPU, or in host memory.
 constexpr size_t kUploadByKernel = 512 << 10;
 static __global__ __launch_bounds__(256) void table_copy_kernel(uint4* __restrict__ to, const uint4* __restrict__ from, uint32_t n) {
     const uint32_t i = blockIdx.x * 256 + threadIdx.x;

@@ -227,10 +227,10 @@ __device__ __forceinline__ void lds_direct_load16x2(const char* uniform_base, ui
 // Loads the compiler keeps no count of: the kernel waits for them itself (sp_wait_copies counts them like copies),
 // so that a wait for the q rows does not become a wait for every tile copy in flight.  The registers must not be
 // read before sp_loads_arrived() has been passed over them.
-__device__ __forceinline__ uint4 sp_load16_at(const char* uniform_base, uint32_t lane_offset) {
+__device__ __forceinline__ uint4 sp_load16(const void* p) {
     typedef uint32_t __attribute__((ext_vector_type(4))) u32x4;
     u32x4 r;
-    asm volatile("global_load_dwordx4 %0, %1, %2" : "=v"(r) : "v"(lane_offset), "s"(uniform_base) : "memory");
+    asm volatile("global_load_dwordx4 %0, %1, off" : "=v"(r) : "v"(p) : "memory");
     return make_uint4(r.x, r.y, r.z, r.w);
 }
 __device__ __forceinline__ void sp_loads_arrived(uint4& r) { asm volatile("" : "+v"(r.x), "+v"(r.y), "+v"(r.z), "+v"(r.w)); }
@@ -424,11 +424,10 @@ __global__ __launch_bounds__(256, 2) void prefill_kernel(PrefillArgs a, const ch
         if constexpr (ROPE_Q) {
             // d = 16 ks + 8 h + e (ks < 4) pairs with d + 64, which this lane holds at step ks + 4.  The table is
             // laid out couple of pairs by couple of pairs, so the 32 rows of a half-wave read 512 consecutive bytes
-            // per load.
-            const uint32_t lane_at = ((uint32_t)(skip + off + min(q_pos, Lq - 1)) + 4u * (uint32_t)h * a.rope_pitch) * 16u;
+            // per load.  (Addresses of 64 bits: the half-waves' rows of the table are 64 bytes times its positions apart.)
+            const float4* tab = a.rope_table + (size_t)(skip + off + min(q_pos, Lq - 1)) + (size_t)(4 * h) * a.rope_pitch;
 #pragma unroll
-            for (int e = 0; e < 16; ++e)
-                cs[e] = sp_load16_at((const char*)(a.rope_table + (size_t)(8 * (e >> 2) + (e & 3)) * a.rope_pitch), lane_at);
+            for (int e = 0; e < 16; ++e) cs[e] = sp_load16(tab + (size_t)(8 * (e >> 2) + (e & 3)) * a.rope_pitch);
         }
     }
     // Operand reads.  K: lane (row qn, half h) needs chunk 2 ks + h of its row for step ks, which sits at position

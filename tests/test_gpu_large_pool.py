@@ -13,7 +13,7 @@ import torch
 import oracle
 from blitz_scale_amd import kernel as K
 from blitz_scale_amd import workloads as wl
-from blitz_scale_amd._lib import BZ_BF16, BZ_LAYOUT_HND, BZ_ROPE_NONE
+from blitz_scale_amd._lib import BZ_BF16, BZ_LAYOUT_HND, BZ_ROPE_NONE, BZ_ROPE_Q_ONLY
 
 from _gpu import TORCH_OF, to_dev, to_host_bits
 from _util import DecodeProblem, ulp_tol
@@ -130,3 +130,35 @@ def test_pack_of_more_than_64_gib():
     by_page = pool.transpose(0, 1).contiguous()
     for lo in range(0, pages, 1024):
         assert torch.equal(got[lo:lo + 1024], by_page[ids[lo:lo + 1024].long()]), lo
+
+
+def test_angles_of_q_rows_past_53_million_positions():
+    """A chunk of 64 tokens behind 54 million: the second half of an angle table's couple of pairs lies more than 4 GiB behind the
+    first one's.  K is zero but for a row per q row that is the q row itself, turned by its position, 2.5 times as large: its score
+    is 19 to 37 against 54 million of 0, and nearly all of the result is that row's V."""
+    L, Lq, theta, f16 = 54_000_000, 64, 1e4, torch.float16
+    if torch.cuda.mem_get_info()[0] < 64 << 30:
+        pytest.skip("needs 64 GiB of device memory")
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(12)
+    k, v = torch.zeros((L, 1, 128), dtype=f16, device="cuda"), torch.zeros((L, 1, 128), dtype=f16, device="cuda")
+    q = torch.randn((Lq, 1, 128), dtype=f16, device="cuda", generator=gen)
+    v[-Lq:] = torch.randn((Lq, 1, 128), dtype=f16, device="cuda", generator=gen)
+    # the angles as the table has them: position and frequency in fp32, their product rounded to it
+    freqs = torch.tensor(theta ** (-2.0 * np.arange(64) / 128), dtype=torch.float32, device="cuda")
+    angle = (torch.arange(L - Lq, L, device="cuda").float()[:, None] * freqs).double()
+    lo, hi = q[:, 0, :64].double(), q[:, 0, 64:].double()
+    c, s = angle.cos(), angle.sin()
+    k[-Lq:, 0] = 2.5 * torch.cat([lo * c - hi * s, hi * c + lo * s], -1).half()
+    qo, kv = np.array([0, Lq], np.int32), np.array([0, L], np.int32)
+    float_ws = torch.empty(512 * L + (64 << 20), dtype=torch.uint8, device="cuda")
+    int_ws = torch.empty(8 << 20, dtype=torch.uint8, device="cuda")
+    handler = K.BatchPrefillRaggedHandler()
+    handler.plan(float_ws, float_ws.numel(), int_ws, int_ws.numel(), qo, kv, 1, 1, 1, 128, 16)
+    out = torch.empty_like(q)
+    K.batch_prefill_attention(handler, q, torch.from_numpy(qo).cuda(), k, v, torch.from_numpy(kv).cuda(), out, 1, 1, 1, 128,
+                              rope_mode=BZ_ROPE_Q_ONLY, rope_theta=theta)
+    own = ((q[:, 0].double() ** 2).sum(-1) * 2.5 / 128 ** 0.5).exp()
+    want = v[-Lq:, 0].double() * (own / (own + L))[:, None]
+    # (a causal row sees the rows before it as well, at scores of 2.5 times a standard normal value: at most e^10 of e^20)
+    assert (out[:, 0].double() - want).abs().max() < 0.02
