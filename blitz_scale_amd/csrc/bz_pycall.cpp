@@ -117,9 +117,8 @@ int stream_of(PyObject* o, uint64_t& to) {
 }
 int table_of(PyObject* o, bz_paged_kv_t& kv) {
     if ((PyObject*)Py_TYPE(o) != g_table) return 0;
-    PyObject** at = _PyObject_GetDictPtr(o);
-    PyObject* d = at ? *at : nullptr;
-    if (!d) return 0;
+    PyObject* d = PyObject_GenericGetDict(o, nullptr);
+    if (!d) return -1;
     int rc = 1;
     auto get = [&](PyObject* name, int (*convert)(PyObject*, uint64_t&)) -> uint64_t {
         if (rc != 1) return 0;
@@ -146,6 +145,7 @@ int table_of(PyObject* o, bz_paged_kv_t& kv) {
     kv.stride_h = get(s_stride_h, whole_of);
     kv.kv_dtype = (int)get(s_kv_dtype, whole_of);
     kv.steps_ahead = (const int32_t*)get(s_steps_ahead_d, address_of);
+    Py_DECREF(d);
     return rc;
 }
 
@@ -207,7 +207,9 @@ void call_free(PyObject* self_) {
     Py_XDECREF(self->slow);
     Py_XDECREF(self->check);
     Py_XDECREF(self->what);
-    Py_TYPE(self_)->tp_free(self_);
+    PyTypeObject* type = Py_TYPE(self_);
+    type->tp_free(self_);
+    Py_DECREF(type); // (an instance of a heap type holds it)
 }
 
 PyMemberDef call_members[] = {{"__vectorcalloffset__", T_PYSSIZET, offsetof(Call, vectorcall), READONLY, nullptr}, {nullptr}};
@@ -244,6 +246,7 @@ PyObject* setup(PyObject*, PyObject* args) {
         Py_INCREF(o[i]);
         Py_XSETREF(*to[i], o[i]);
     }
+    g_gpu_up = false; // (as the function before this one saw it)
     Py_RETURN_NONE;
 }
 

@@ -136,3 +136,13 @@ def test_every_call_is_bound_to_the_library():
         assert callable(getattr(K._calls, name)) and K._calls.__dict__[name]
     with pytest.raises(BzError):  # (refused on the host, before anything is launched)
         K._calls.bz_silu_and_mul(None, None, torch.zeros(1, dtype=torch.float16), 1, 8, 0)
+
+
+def test_whether_the_gpu_is_up_is_asked_again_after_a_setup():
+    b = Bound("bz_rms_norm")
+    args = [_usual(x, i) for i, x in enumerate(b.spec)]
+    b.call(*args)
+    assert b.slow == 0
+    _lib.load_pycall().setup(torch.Tensor, torch.Tensor.data_ptr, K._DTYPES, K.PageTable, lambda: False, lambda: 5, lambda dev: 1)
+    b.call(*args)
+    assert b.slow == 1 and b.seen[0] == b.seen[1]
