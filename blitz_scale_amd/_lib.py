@@ -125,16 +125,15 @@ def load():
     return lib
 
 
-PYCALL_PATH = os.path.join(HERE, "lib", "bz_pycall.so")
+# (named for the interpreter it is built for: another one does not find it)
+PYCALL_PATH = os.path.join(HERE, "lib", "bz_pycall" + importlib.machinery.EXTENSION_SUFFIXES[0])
 _pycall = None
 
 
 def load_pycall():
-    """Load the native calling side (csrc/bz_pycall.cpp).  Raises if it is not built."""
+    """The native calling side (csrc/bz_pycall.cpp), or None where this interpreter has none: kernel.py then calls through ctypes."""
     global _pycall
-    if _pycall is None:
-        if not os.path.exists(PYCALL_PATH):
-            raise RuntimeError(f"{PYCALL_PATH} is missing: build it first (python -m blitz_scale_amd.build).")
+    if _pycall is None and os.path.exists(PYCALL_PATH):
         loader = importlib.machinery.ExtensionFileLoader("bz_pycall", PYCALL_PATH)
         module = importlib.util.module_from_spec(importlib.util.spec_from_loader("bz_pycall", loader))
         loader.exec_module(module)

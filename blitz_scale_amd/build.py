@@ -3,7 +3,9 @@
 `python -m blitz_scale_amd.build` writes blitz_scale_amd/lib/libbz_hip.so.  The library is plain
 HIP + a C ABI (include/bz_hip.h); it does not link against torch.
 """
+import importlib.machinery
 import os
+import shutil
 import subprocess
 import sys
 import sysconfig
@@ -80,18 +82,22 @@ def build(verbose=True, jobs=8):
     return LIB_PATH
 
 
-PYCALL_PATH = os.path.join(LIB_DIR, "bz_pycall.so")
-
-
 def build_pycall(verbose=True):
-    """The extension module through which kernel.py calls the library (host code only)."""
-    cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-Wno-missing-field-initializers",
-           "-I", sysconfig.get_paths()["include"], "-I", os.path.join(ROOT, "include"), os.path.join(CSRC, "bz_pycall.cpp"),
-           "-o", PYCALL_PATH]
+    """The extension module through which kernel.py calls the library (host code only), for the interpreter that runs this.
+    Optional: without a C++ compiler or this Python's headers (3.9 or newer) the calls go through ctypes, at 1 to 3 us more each."""
+    path = os.path.join(LIB_DIR, "bz_pycall" + importlib.machinery.EXTENSION_SUFFIXES[0])
+    cxx, include = os.environ.get("CXX", "g++"), sysconfig.get_paths()["include"]
+    if sys.version_info < (3, 9) or not shutil.which(cxx.split()[0]) or not os.path.exists(os.path.join(include, "Python.h")):
+        if os.path.exists(path):
+            os.remove(path)  # (of an earlier build: its list of calls may be another one)
+        print(f"bz_pycall: no C++ compiler ({cxx}) or no Python headers ({include}); calls go through ctypes", flush=True)
+        return None
+    cmd = [*cxx.split(), "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-Wno-missing-field-initializers",
+           "-I", include, "-I", os.path.join(ROOT, "include"), os.path.join(CSRC, "bz_pycall.cpp"), "-o", path]
     if verbose:
         print(" ".join(cmd), flush=True)
     subprocess.check_call(cmd)
-    return PYCALL_PATH
+    return path
 
 
 PROBE_SRC = os.path.join(HERE, "probes", "mfma_ceiling.hip")

@@ -54,27 +54,46 @@ def _host_i32(a):
 
 
 class _Calls:
-    """The launching calls of the C ABI as Python callables, bound on first use (lib/bz_pycall.so, csrc/bz_pycall.cpp: arguments
-    that are what they usually are go through without ctypes).  A call takes the C arguments in order -- a tensor for its address
-    or for its type code, a PageTable for the struct, None for the current stream -- and raises BzError on a status."""
+    """The launching calls of the C ABI as Python callables, bound on first use: through the native calling side (csrc/bz_pycall.cpp,
+    arguments that are what they usually are go through without ctypes) where there is one for this interpreter, else through
+    ctypes.  A call takes the C arguments in order -- a tensor for its address or for its type code, a PageTable for the struct,
+    None for the current stream -- and raises BzError on a status."""
 
     WHAT = {"bz_batch_decode": "batchDecodeAttention", "bz_batch_decode_noalloc": "batchDecodeAttention", "bz_decode_step": "decodeStep",
             "bz_batch_prefill_ragged": "BatchPrefillWithRaggedKVCache", "bz_store_prefill_kv": "AppendPagedKVCache",
             "bz_append_decode_kv": "AppendPagedKVCacheDecode", "bz_rms_norm": "rmsNorm", "bz_add_rms_norm": "fusedAddRmsNorm",
             "bz_silu_and_mul": "siluAndMul", "bz_add_residual": "AddKernel", "bz_embedding": "EmbeddingKernel",
             "bz_gather_last_token": "GatherLastTokenKernel", "bz_batch_find_max": "BatchFindMaxKernel"}
+    # a letter per C argument: p address, d type code of a tensor, k PageTable, u unsigned, i int, t truth value as int, f float,
+    # s stream
+    SPECS = {"bz_batch_decode": "ppdkpduiffppps", "bz_batch_decode_noalloc": "ppdkpduiffppps", "bz_decode_step": "ppdppkpdutffppps",
+             "bz_batch_prefill_ragged": "pppppppduuuutiffs", "bz_store_prefill_kv": "kppdpuputfpps",
+             "bz_append_decode_kv": "kppdputfpps", "bz_rms_norm": "pppduufs", "bz_add_rms_norm": "pppduufs",
+             "bz_silu_and_mul": "ppduus", "bz_add_residual": "ppduus", "bz_embedding": "ppppduus",
+             "bz_gather_last_token": "pppduuus", "bz_batch_find_max": "ppduus"}
 
     def __getattr__(self, name):
-        fn = getattr(_lib.load(), name)
-        native = _lib.load_pycall()
-        raw = _raw_stream or (lambda device: torch.cuda.current_stream(device).cuda_stream)
-        native.setup(torch.Tensor, torch.Tensor.data_ptr, _DTYPES, PageTable, torch.cuda.is_initialized,
-                     _current_device or torch.cuda.current_device, raw)
+        if name not in self.SPECS:
+            raise AttributeError(name)
+        fn, what, spec = getattr(_lib.load(), name), self.WHAT[name], self.SPECS[name]
         # the slow way, for arguments that the native side leaves alone: converted, and refused, as ctypes does it
         convert = {"p": _ptr, "d": bz_dtype, "k": lambda table: C.byref(table.as_struct()), "t": int, "s": _stream}
-        ways = [convert.get(letter, lambda value: value) for letter in native.specs()[name]]
-        call = native.bind(name, C.cast(fn, C.c_void_p).value, lambda *args: fn(*[way(a) for way, a in zip(ways, args)]), check,
-                           self.WHAT[name])
+        ways = [convert.get(letter, lambda value: value) for letter in spec]
+
+        def slowly(*args):
+            return fn(*[way(a) for way, a in zip(ways, args)])
+
+        native = _lib.load_pycall()
+        if native is not None:
+            raw = _raw_stream or (lambda device: torch.cuda.current_stream(device).cuda_stream)
+            native.setup(torch.Tensor, torch.Tensor.data_ptr, _DTYPES, PageTable, torch.cuda.is_initialized,
+                         _current_device or torch.cuda.current_device, raw)
+            call = native.bind(name, C.cast(fn, C.c_void_p).value, slowly, check, what)
+        else:
+            def call(*args):
+                if len(args) != len(spec):
+                    raise TypeError(f"{name} takes {len(spec)} positional arguments")
+                check(slowly(*args), what)
         setattr(self, name, call)
         return call
 

@@ -1,6 +1,8 @@
 """The native calling side (csrc/bz_pycall.cpp) hands the C ABI what ctypes would: every call is bound to a recording function
 of the same C signature and made twice, through the native conversion and through the Python one that it falls back to."""
 import ctypes as C
+import importlib.machinery
+import os
 
 import numpy as np
 import pytest
@@ -138,6 +140,10 @@ def test_every_call_is_bound_to_the_library():
         K._calls.bz_silu_and_mul(None, None, torch.zeros(1, dtype=torch.float16), 1, 8, 0)
 
 
+def test_both_sides_know_the_same_arguments():
+    assert _lib.load_pycall().specs() == K._Calls.SPECS
+
+
 def test_whether_the_gpu_is_up_is_asked_again_after_a_setup():
     b = Bound("bz_rms_norm")
     args = [_usual(x, i) for i, x in enumerate(b.spec)]
@@ -146,3 +152,30 @@ def test_whether_the_gpu_is_up_is_asked_again_after_a_setup():
     _lib.load_pycall().setup(torch.Tensor, torch.Tensor.data_ptr, K._DTYPES, K.PageTable, lambda: False, lambda: 5, lambda dev: 1)
     b.call(*args)
     assert b.slow == 1 and b.seen[0] == b.seen[1]
+
+
+def test_without_the_native_side_calls_go_through_ctypes(monkeypatch):
+    """As on an interpreter that bz_pycall was not built for."""
+    suffix = importlib.machinery.EXTENSION_SUFFIXES[0]
+    assert _lib.PYCALL_PATH.endswith("bz_pycall" + suffix) and suffix != ".so"
+    monkeypatch.setattr(_lib, "PYCALL_PATH", _lib.PYCALL_PATH.replace(suffix, ".cpython-399-other.so"))
+    monkeypatch.setattr(_lib, "_pycall", None)
+    assert _lib.load_pycall() is None
+    K._calls.__dict__.clear()
+    x = torch.zeros(8, dtype=torch.float16)
+    for name in NAMES:
+        assert callable(getattr(K._calls, name))
+    with pytest.raises(BzError, match="siluAndMul"):  # (refused on the host, before anything is launched)
+        K._calls.bz_silu_and_mul(None, None, x, 1, 8, 0)
+    with pytest.raises(TypeError):
+        K._calls.bz_silu_and_mul(None, None, x, 1, 8)
+    with pytest.raises(C.ArgumentError):
+        K._calls.bz_silu_and_mul(x, x, x, 1.5, 8, 0)
+
+
+def test_building_without_a_compiler_leaves_no_native_side(monkeypatch, tmp_path):
+    from blitz_scale_amd import build
+    monkeypatch.setattr(build, "LIB_DIR", str(tmp_path))
+    assert os.path.basename(build.build_pycall(verbose=False)) == os.path.basename(_lib.PYCALL_PATH)
+    monkeypatch.setenv("CXX", str(tmp_path / "no-such-compiler"))
+    assert build.build_pycall(verbose=False) is None and not os.listdir(tmp_path)
