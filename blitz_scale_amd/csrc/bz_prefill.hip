@@ -241,18 +241,17 @@ __device__ __forceinline__ void sp_barrier() {
     asm volatile("s_barrier" ::: "memory");
     __builtin_amdgcn_sched_barrier(0);
 }
-// wait until at most `tiles` of this wave's tile copies (two instructions each) are still in flight
+// wait until at most `tiles` of this wave's tile copies (two instructions each) are still in flight; any count but 1 .. 5, the
+// most that are issued at a time, waits for all
 __device__ __forceinline__ void sp_wait_copies(int tiles) {
     __builtin_amdgcn_sched_barrier(0);
     switch (tiles) {
-        case 0: __builtin_amdgcn_s_waitcnt(0x0F70); break;
         case 1: __builtin_amdgcn_s_waitcnt(0x0F72); break;
         case 2: __builtin_amdgcn_s_waitcnt(0x0F74); break;
         case 3: __builtin_amdgcn_s_waitcnt(0x0F76); break;
         case 4: __builtin_amdgcn_s_waitcnt(0x0F78); break;
         case 5: __builtin_amdgcn_s_waitcnt(0x0F7A); break;
-        case 6: __builtin_amdgcn_s_waitcnt(0x0F7C); break;
-        default: __builtin_amdgcn_s_waitcnt(0x0F7E); break;
+        default: __builtin_amdgcn_s_waitcnt(0x0F70); break;
     }
     __builtin_amdgcn_sched_barrier(0);
 }
@@ -589,34 +588,31 @@ __global__ __launch_bounds__(256, 2) void prefill_kernel(PrefillArgs a, const ch
             psum = MP::add_pair(tw, psum);
         }
     };
-    // The first half of an iteration: scores of the next tile into s[PAR ^ 1] (QK) from K at k1 (steps 0..3 are in
-    // the ring), probabilities of this tile from s[PAR] (EX), first V operands of this tile (at vj) into the ring.
+    // The first half of an iteration: scores of the next tile into s[PAR ^ 1] from K at k1 (steps 0..3 are in
+    // the ring), probabilities of this tile from s[PAR], first V operands of this tile (at vj) into the ring.
     // The exponentials of step i are consumed in step i + 1 (their latency is longer than one instruction).
     // `wslot`: V_F16, the slot of the V tile whose widening starts here (negative: none).
-    auto first_half = [&](auto par_c, auto qk_c, auto ex_c, uint32_t k1, uint32_t vj, int wslot) __attribute__((always_inline)) {
+    auto first_half = [&](auto par_c, uint32_t k1, uint32_t vj, int wslot) __attribute__((always_inline)) {
         constexpr int PAR = decltype(par_c)::value;
-        constexpr bool QK = decltype(qk_c)::value, EX = decltype(ex_c)::value;
         float e0 = 0.f, e1 = 0.f;
-        if (EX) psum = 0.f;
+        psum = 0.f;
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
-            if (QK) s[PAR ^ 1] = M::run(kring[i & 3], qreg[i], i == 0 ? cinit : s[PAR ^ 1]);
-            if (i >= 4) read_v(vring[i - 4], vj, i - 4);
-            else if (QK) read_k(kring[i], k1, i + 4);
+            s[PAR ^ 1] = M::run(kring[i & 3], qreg[i], i == 0 ? cinit : s[PAR ^ 1]);
+            if (i < 4) read_k(kring[i], k1, i + 4);
+            else read_v(vring[i - 4], vj, i - 4);
             if (V_F16 && (i == 4 || i == 5) && wslot >= 0) wide[i - 4] = *widen_at(wslot, i - 4);
-            if (EX) {
-                const float n0 = exp_of(s[PAR][2 * i], 0.f), n1 = exp_of(s[PAR][2 * i + 1], 0.f);
-                if (i > 0) take_pair(e0, e1, i - 1);
-                e0 = n0;
-                e1 = n1;
-            }
+            const float n0 = exp_of(s[PAR][2 * i], 0.f), n1 = exp_of(s[PAR][2 * i + 1], 0.f);
+            if (i > 0) take_pair(e0, e1, i - 1);
+            e0 = n0;
+            e1 = n1;
             __builtin_amdgcn_sched_barrier(0);
         }
-        if (EX) take_pair(e0, e1, 7);
+        take_pair(e0, e1, 7);
         __builtin_amdgcn_sched_barrier(0);
     };
-    // The second half: O += V^T P^T (PV), the rest of V (at vj) and the first K operands of the tile after the next
+    // The second half: O += V^T P^T, the rest of V (at vj) and the first K operands of the tile after the next
     // (at k2) into the rings.  V_F16: the widening ends here, in the shadow of the first six steps, whose matrix
     // instructions have no vector work of their own beside them; behind its last write come kWidenBehind operand reads.
     constexpr int kWidenBehind = 2;
@@ -686,10 +682,9 @@ __global__ __launch_bounds__(256, 2) void prefill_kernel(PrefillArgs a, const ch
         }
 #pragma unroll
         for (int i = 0; i < 4; ++i) read_k(kring[i], k_at(1 % kSNK), i);
-        {
+        // (waves without rows do as the others do: token 0 exists, and nobody reads what they make of it)
 #pragma unroll
-            for (int i = 0; i < 8; ++i) s[0] = M::run(k0[i], qreg[i], i == 0 ? cinit : s[0]);
-        }
+        for (int i = 0; i < 8; ++i) s[0] = M::run(k0[i], qreg[i], i == 0 ? cinit : s[0]);
         if (V_F16) { // (beside the scores; waited for in front of the next barrier)
 #pragma unroll
             for (int i = 0; i < 2; ++i) {
@@ -698,18 +693,16 @@ __global__ __launch_bounds__(256, 2) void prefill_kernel(PrefillArgs a, const ch
             }
             sp_wait_lds<0>();
         }
-        {
-            mask_tile(0, s[0]);
-            float tmax = -INFINITY;
+        mask_tile(0, s[0]);
+        float tmax = -INFINITY;
 #pragma unroll
-            for (int i = 0; i < 16; ++i) tmax = fmaxf(tmax, s[0][i]);
-            tmax = lane_max_xor32(tmax); // finite: token 0 is visible to every row
-            m_run = tmax;
+        for (int i = 0; i < 16; ++i) tmax = fmaxf(tmax, s[0][i]);
+        tmax = lane_max_xor32(tmax); // finite: token 0 is visible to every row
+        m_run = tmax;
 #pragma unroll
-            for (int i = 0; i < 16; ++i) {
-                s[0][i] -= tmax;
-                cinit[i] = -tmax;
-            }
+        for (int i = 0; i < 16; ++i) {
+            s[0][i] -= tmax;
+            cinit[i] = -tmax;
         }
     }
     BZ_PF_WG(3);
@@ -732,7 +725,7 @@ __global__ __launch_bounds__(256, 2) void prefill_kernel(PrefillArgs a, const ch
         v_next += tile_stride;
         BZ_PF_PH(2);
         constexpr int WSLOT = V_F16 ? (SL + 1) % kSNV : -1; // V(j+1), first read after the next barrier
-        first_half(par_c, std::true_type{}, std::true_type{}, k_at((SL + 1) % kSNK), v_at(SL), WSLOT);
+        first_half(par_c, k_at((SL + 1) % kSNK), v_at(SL), WSLOT);
         BZ_PF_PH(3);
         if (__builtin_expect(__any(!(psum < 32768.0f)), 0)) move_maximum(s[PAR], s[PAR ^ 1]);
         l_run += psum;
@@ -753,7 +746,7 @@ __global__ __launch_bounds__(256, 2) void prefill_kernel(PrefillArgs a, const ch
         // (the scores of a next tile are taken whether there is one or not, from whatever its slot holds, and read by nobody
         // then: with a branch there the compiler gathers the vector work that both sides have in front of it and behind it,
         // out of the shadow of the matrix instructions)
-        first_half(par_c, std::true_type{}, std::true_type{}, k_at((SL + 1) % kSNK), v_at(SL), WSLOT);
+        first_half(par_c, k_at((SL + 1) % kSNK), v_at(SL), WSLOT);
         if (__builtin_expect(__any(!(psum < 32768.0f)), 0)) move_maximum(s[PAR], s[PAR ^ 1]);
         l_run += psum;
         if (j + 1 < n_w) mask_tile(j + 1, s[PAR ^ 1]);
