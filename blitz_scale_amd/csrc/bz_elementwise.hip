@@ -1,6 +1,6 @@
 // Row-wise element-wise kernels for gfx950: RMSNorm, fused add+RMSNorm, SiLU-gate and residual
 // add.  Replace src/kernel/norm.cu, activation.cu and add.cu of the BlitzScale worker.  All of
-// them move 16 bytes per lane and reduce in fp32 with wave64 shuffles.
+// them move 16 bytes per lane and reduce in fp32, within a wave through the vector ALU's lane permutes.
 #include "bz_common.hpp"
 
 namespace bz {
