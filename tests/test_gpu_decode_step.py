@@ -321,3 +321,34 @@ def test_form_of_a_step_whose_partials_of_one_unit_pass_4_gib():
                      1, 1, 1, 128, 16, split_tokens=32)
         assert handler.step_form() == form
     torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("dtype", [BZ_F16, BZ_BF16])
+@pytest.mark.parametrize("Hkv,D", [(2, 128), (1, 128), (2, 64)])
+@pytest.mark.parametrize("ctx", [312, 1496, 5016])
+def test_infinite_values_come_out_as_in_the_two_calls(ctx, Hkv, D, dtype):
+    """V is infinite for a token of the first piece, in one dimension, and for one of the last, in another.  A probability's tail
+    makes some of these rows NaN on the way (zero or less times infinity); the others stay infinite, whichever piece is read again
+    where a batch of the finishing kernel's loads has more places than there are pieces."""
+    p = DecodeProblem(850 + D, [ctx], 16, Hkv, D, 16, dtype)
+    planes = p.pool.reshape(-1, 2, Hkv, 16, D)  # [page][K | V][kv head][token][dim]
+    for token, dim in ((5, 3), (ctx - 7, 9)):
+        planes[p.indices[token // 16], 1, :, token % 16, dim] = 0x7C00 if dtype == BZ_F16 else 0x7F80
+    # (the newest token, whose score is 0, has the largest of no piece: 23 others of the last tile would all have to be negative)
+    k = np.zeros((1, Hkv, D), np.uint16)
+    v = wl.randn_bits(np.random.default_rng(851), (1, Hkv, D), dtype)
+    two, one = DeviceDecode(p), DeviceDecode(p, float_ws_bytes=128 << 20)
+    two.plan()
+    K.append_decode_kv_cache(two.pt, to_dev(k, dtype), to_dev(v, dtype))
+    want = two.decode(None, BZ_ROPE_NONE)
+    os.environ["BZ_DECODE_PATH"] = "one_call"
+    try:
+        one.plan()
+    finally:
+        del os.environ["BZ_DECODE_PATH"]
+    assert one.handler.step_form() == "one_call"
+    out = torch.empty((1, 16, D), dtype=TORCH_OF[dtype], device="cuda")
+    K.decode_step(one.handler, one.q, to_dev(k, dtype), to_dev(v, dtype), one.pt, out, 16, rope=False)
+    got = to_host_f32(out)
+    assert all(np.isposinf(want[..., dim]).any() for dim in (3, 9)) and np.isfinite(np.delete(want, (3, 9), -1)).all()
+    assert np.array_equal(np.isposinf(got), np.isposinf(want)) and np.array_equal(np.isnan(got), np.isnan(want))
